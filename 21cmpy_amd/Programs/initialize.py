@@ -76,20 +76,13 @@ def init(DIM=None, HII_DIM=None, BOX_LEN=None, seed=0, box_id=0, pspec="planck",
         spec = gpu.grf_init_table(DIM, L, table[0], table[1], seed, box_id)
     deltax = gpu.c2r(spec)                                   # initialize.py:79-82
     R = smoothing_radius(L, HII_DIM)
-    work = gpu.hii_filter(spec, L, R, filter_type=0, ref_fallthrough=True, korder=1)
-    large = gpu.c2r(work, preserve_input=False)              # initialize.py:86-93
-    smoothed = gpu.subsample(large, HII_DIM)
+    # initialize.py:86-109: the smoothed box and the displacement boxes, picked to HII_DIM
+    smoothed, *vs = gpu.smoothed_fields(spec, L, HII_DIM, R, displacements=with_velocity)
     out = {"spec": spec, "deltax": deltax, "smoothed": smoothed}
     if table is not None:
         out["pk_table"] = table
     if with_velocity:
-        vs = []
-        for comp in range(3):                                # initialize.py:102-109
-            gpu.velocity(spec, L, comp, filter_type=0, R=R, out=work)
-            gpu.c2r(work, out=large, preserve_input=False)
-            vs.append(gpu.subsample(large, HII_DIM))
         out["v"] = tuple(vs)
-    del work, large
     if save:
         d = os.path.join(out_dir or P.IO_DIR, "Boxes")
         os.makedirs(d, exist_ok=True)

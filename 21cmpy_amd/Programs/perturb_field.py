@@ -126,16 +126,7 @@ def velocities_at(z, deltax, HII_DIM=None, box_len=None, ddt_over_d=None, save=F
     f = planck.ddt_growth_over_growth(float(z)) if ddt_over_d is None else float(ddt_over_d)
     spec = gpu.r2c(deltax)  # DIM^3 times the c2r-ready spectrum
     R = initialize.smoothing_radius(L, HII)
-    work = torch.empty_like(spec)
-    large = torch.empty((DIM, DIM, DIM), dtype=torch.float32, device=deltax.device)
-    scale = np.float32(f / float(DIM) ** 3)
-    vs = []
-    for comp in range(3):
-        gpu.velocity(spec, L, comp, filter_type=0, R=R, out=work)
-        gpu.c2r(work, out=large, preserve_input=False)
-        v = gpu.subsample(large, HII)
-        v.mul_(scale)
-        vs.append(v)
+    vs = gpu.smoothed_fields(spec, L, HII, R, smoothed=False, scale=np.float32(f / float(DIM) ** 3))
     if save:
         d = os.path.join(out_dir or P.IO_DIR, "Boxes")
         os.makedirs(d, exist_ok=True)

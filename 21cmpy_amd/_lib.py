@@ -124,6 +124,7 @@ SIGNATURES = {
     "cm21_grf_init_table": (I, [VP, I, D, VP, VP, I, U32, U32, VP]),
     "cm21_subsample": (I, [VP, VP, I, I, F, VP]),
     "cm21_velocity": (I, [VP, VP, I, F, I, I, F, VP]),
+    "cm21_fold_fields": (I, [VP, VP, I, I, F, F, F, I, I, VP]),
     "cm21_move_mass": (I, [VP, VP, VP, VP, VP, I, I, F, F, I, VP]),
     "cm21_delta_T": (I, [VP, VP, VP, I, F, VP, VP, VP]),
     "cm21_pk_workspace_bytes": (SZ, [I, I]),

@@ -4,6 +4,7 @@
 //
 // Reference: Programs/initialize.cu:58-95 (init_kernel), :133-146 (subsample),
 // :148-190 (set_velocity); Programs/initialize.py:33-111 (driver).
+#include <algorithm>
 #include <cmath>
 
 #include "cm21_internal.hpp"
@@ -215,6 +216,85 @@ __global__ void k_velocity(float2* __restrict__ out, const float2* __restrict__ 
     out[idx] = r;
 }
 
+// Spectra of boxes that are only read on every q-th cell (q = D/d): a field
+// of the D^3 grid picked at multiples of q is the inverse transform on the
+// d^3 grid of its spectrum folded modulo d, Y[m] = sum of W(n) X[n] over n = m
+// (mod d).  One thread per mode m of the small half spectrum adds the one to
+// eight modes n inside the window's cut (|n|^2 <= m2max; negative n_c through
+// the conjugate of -n), in a fixed order, and forms the smoothed spectrum and
+// the three displacement spectra i k/k^2 W X from one read of X, in the
+// arithmetic of k_filter and k_velocity.
+//
+// What bounds it: the writes of the small spectra (four of 68 MB at d = 256)
+// and the FP64 sine and cosine of the window, 8.4 M modes instead of the 67 M
+// of the 512^3 spectrum.  At 512 -> 256 it takes 216 us and the four 256^3
+// inverse transforms 600 us, for a filter (585 us), three displacement passes
+// (3 x 500), four 512^3 transforms (4 x 1450) and four picks (4 x 50):
+// initial conditions 10.2 -> 3.0 ms, velocity boxes at z 7.4 -> 2.1 ms.
+__global__ void k_fold_fields(float2* __restrict__ out, const float2* __restrict__ in, int D, int d, WindowParams wp,
+                              float scale, int bm, long m2max, int smoothed, int velocity) {
+    const int H = D / 2 + 1, h = d / 2 + 1;
+    const int mc = blockIdx.x * kModeBlockX + threadIdx.x, mb = blockIdx.y * kModeBlockY + threadIdx.y;
+    const int ma = blockIdx.z;
+    if (mc >= h || mb >= d) return;
+    const int lo = -min(bm, D / 2 - 1), hi = min(bm, D / 2);  // index D/2 is the mode +D/2
+    float2 y[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) y[q] = make_float2(0.0f, 0.0f);
+    // the largest n <= hi with n = m (mod d), then down to lo
+    for (int na = ma + (hi - ma >= 0 ? (hi - ma) / d : -((ma - hi + d - 1) / d)) * d; na >= lo; na -= d) {
+        for (int nb = mb + (hi - mb >= 0 ? (hi - mb) / d : -((mb - hi + d - 1) / d)) * d; nb >= lo; nb -= d) {
+            for (int nc = mc + (hi - mc >= 0 ? (hi - mc) / d : -((mc - hi + d - 1) / d)) * d; nc >= lo; nc -= d) {
+                if ((long)na * na + (long)nb * nb + (long)nc * nc > m2max) continue;
+                // the stored mode: n, or -n for negative n_c
+                const bool neg = nc < 0;
+                int a = neg ? -na : na, b = neg ? -nb : nb;
+                const int c = neg ? -nc : nc;
+                if (a < 0) a += D;
+                if (b < 0) b += D;
+                const float k0 = __fmul_rn((float)mode_of(a, D), wp.dk);
+                const float k1 = __fmul_rn((float)mode_of(b, D), wp.dk);
+                const float k2 = __fmul_rn((float)c, wp.dk);
+                const float ksq = __fadd_rn(__fadd_rn(__fmul_rn(k0, k0), __fmul_rn(k1, k1)), __fmul_rn(k2, k2));
+                float w0, w2;
+                bool cut;
+                window_of(sqrt_rn(ksq), wp, w0, cut, w2);
+                if (cut) continue;
+                float2 v = in[((size_t)a * D + b) * H + c];
+                const float sgn = neg ? -1.0f : 1.0f;
+                if (smoothed) {
+                    const float2 r = apply_window(v, w0, false, w2, scale);
+                    y[0].x += r.x;
+                    y[0].y += sgn * r.y;
+                }
+                if (velocity && ksq != 0.0f) {
+                    const float kk[3] = {k0, k1, k2};
+                    const int idx[3] = {a, b, c};
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        if (idx[q] == D / 2) continue;
+                        const float f = __fdiv_rn(kk[q], ksq);
+                        float2 r = make_float2(-__fmul_rn(f, v.y), __fmul_rn(f, v.x));  // (i f) * v
+                        r = apply_window(r, w0, false, w2, scale);
+                        y[q + 1].x += r.x;
+                        y[q + 1].y += sgn * r.y;
+                    }
+                }
+            }
+        }
+    }
+    const size_t nc = (size_t)d * d * h, idx = ((size_t)ma * d + mb) * h + mc;
+    float2* o = out + idx;
+    if (smoothed) {
+        *o = y[0];
+        o += nc;
+    }
+    if (velocity) {
+#pragma unroll
+        for (int q = 1; q < 4; ++q, o += nc) *o = y[q];
+    }
+}
+
 bool valid_dim(int D) { return D >= 2 && D <= 2048 && D % 2 == 0; }
 
 dim3 grf_grid(int D) { return dim3(1u, (unsigned)((D + kGrfRows - 1) / kGrfRows), (unsigned)D); }
@@ -270,5 +350,26 @@ extern "C" int cm21_velocity(void* spec_out, const void* spec_in, int D, float d
     k_velocity<<<mode_grid(D, D / 2 + 1), mode_block(), 0, (hipStream_t)stream>>>(
         (float2*)spec_out, (const float2*)spec_in, D, delta_k, comp, filter_type, R);
     CM21_LAUNCH_CHECK("k_velocity");
+    return CM21_OK;
+}
+
+extern "C" int cm21_fold_fields(void* spec_out, const void* spec_in, int D, int sw, float delta_k, float R,
+                                float scale, int smoothed, int velocity, void* stream) {
+    CM21_REQUIRE(spec_out && spec_in, "cm21_fold_fields: NULL spectrum");
+    CM21_REQUIRE(valid_dim(D), "cm21_fold_fields: D=%d must be even in [2,2048]", D);
+    CM21_REQUIRE(valid_dim(sw) && sw <= D && D % sw == 0, "cm21_fold_fields: sw=%d must be even and divide D=%d", sw, D);
+    CM21_REQUIRE(smoothed || velocity, "cm21_fold_fields: no field asked for");
+    CM21_REQUIRE(delta_k > 0.0f, "cm21_fold_fields: delta_k must be positive");
+    // the type-0 window cuts kR > 1/0.413566994 (the kernel's float32 test
+    // decides inside a shell of 1e-5)
+    const int hd = D / 2;
+    const double all = 3.0 * hd * hd, kcut = 1.0 / (0.413566994 * (double)delta_k * (double)R);
+    const double m2 = std::floor(kcut * kcut * (1.0 + 1e-5));
+    const long m2max = (R > 0.0f && m2 < all) ? (long)m2 : (long)all;
+    const int bm = (int)std::min<double>(std::sqrt((double)m2max) + 1.0, (double)hd);
+    WindowParams wp{delta_k, R, 0, 1, 1};
+    k_fold_fields<<<mode_grid(sw, sw / 2 + 1), mode_block(), 0, (hipStream_t)stream>>>(
+        (float2*)spec_out, (const float2*)spec_in, D, sw, wp, scale, bm, m2max, smoothed ? 1 : 0, velocity ? 1 : 0);
+    CM21_LAUNCH_CHECK("k_fold_fields");
     return CM21_OK;
 }

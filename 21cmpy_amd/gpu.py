@@ -148,6 +148,36 @@ def velocity(spec, box_len, comp, filter_type=0, R=0.0, out=None):
     return out
 
 
+def smoothed_fields(spec, box_len, sw, R, smoothed=True, displacements=True, scale=1.0):
+    """The box smoothed with the type-0 window at R (smoothed) and the three
+    displacement boxes of the smoothed field (displacements), each on every D/sw-th
+    cell and times ``scale``: float32 (sw, sw, sw) boxes, the smoothed one
+    first.  An even sw takes the boxes from the folded spectrum
+    (cm21_fold_fields) and sw^3 transforms; the transforms need an even side,
+    so an odd sw picks its cells from the D^3 boxes."""
+    D = spec.shape[0]
+    _check_spec(spec, D, "spec")
+    if sw < 1 or D % sw:
+        raise ValueError(f"sw={sw} must divide D={D}")
+    if sw % 2:
+        work = torch.empty_like(spec)
+        large = torch.empty((D, D, D), dtype=torch.float32, device=spec.device)
+        out = []
+        if smoothed:
+            hii_filter(spec, box_len, R, filter_type=0, ref_fallthrough=True, korder=1, scale=scale, out=work)
+            out.append(subsample(c2r(work, out=large, preserve_input=False), sw))
+        for comp in range(3 if displacements else 0):
+            velocity(spec, box_len, comp, filter_type=0, R=R, out=work)
+            v = subsample(c2r(work, out=large, preserve_input=False), sw)
+            out.append(v if scale == 1.0 else v.mul_(scale))
+        return out
+    n = int(bool(smoothed)) + 3 * int(bool(displacements))
+    fold = torch.empty((n, sw, sw, sw // 2 + 1), dtype=torch.complex64, device=spec.device)
+    _lib.call("cm21_fold_fields", _lib.ptr(fold), _lib.ptr(spec), D, int(sw), delta_k(box_len), float(R), float(scale),
+              1 if smoothed else 0, 1 if displacements else 0, _lib.stream_handle())
+    return [c2r(f, preserve_input=False) for f in fold]
+
+
 def move_mass(deltax, vx, vy, vz, disp_scale, growth_init, scheme="cic", out=None):
     DIM = deltax.shape[0]
     sw = vx.shape[0]

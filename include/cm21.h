@@ -190,6 +190,16 @@ int cm21_subsample(float* small, const float* large, int D, int sw,
 int cm21_velocity(void* spec_out, const void* spec_in, int D, float delta_k,
                   int comp, int filter_type, float R, void* stream);
 
+/* The spectra of the smoothed box (smoothed != 0) and of the three displacement
+ * boxes (velocity != 0), each picked at multiples of D/sw cells: spec_out holds
+ * 1, 3 or 4 half spectra (sw,sw,sw/2+1), the smoothed one first, whose
+ * cm21_c2r on the sw^3 grid is what cm21_hii_filter(filter 0, fall-through,
+ * korder 1, scale) or cm21_velocity(comp, filter 0, R) of spec_in followed by
+ * cm21_c2r and cm21_subsample give (initialize.py:86-109), up to rounding.  sw
+ * must be even and divide D. */
+int cm21_fold_fields(void* spec_out, const void* spec_in, int D, int sw, float delta_k, float R, float scale,
+                     int smoothed, int velocity, void* stream);
+
 /* ------------------------------------------------------------------ perturb
  * Replaces move_mass + the renormalisation (Programs/perturb_field.cu:90-133;
  * perturb_field.py:93-105): the DIM^3 particles at cell centres move by
