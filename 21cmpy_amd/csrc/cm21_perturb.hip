@@ -1,16 +1,13 @@
 // Zel'dovich mass move on the GPU (perturb_field stage).
 //
 // Reference: Programs/perturb_field.cu:90-133 (move_mass) and
-// Programs/perturb_field.py:93-105.  One thread per DIM^3 particle, in the
-// reference's float32 position arithmetic.  NGP deposits the whole mass in the
-// truncated cell (bit-exact indices); CIC shares it over the 8 nearest cell
-// centres.  Deposits are float atomics: the summation order varies from run
+// Programs/perturb_field.py:93-105, in the reference's float32 position
+// arithmetic.  NGP deposits the whole mass in the truncated cell (bit-exact
+// indices); CIC shares it over the 8 nearest cell centres.  Deposits are float atomics: the summation order varies from run
 // to run at the 1e-7 relative level, the target cells never do.
 //
-// Particles of a block come from a 16^3 patch of the DIM grid whose
-// displacements are small, so the block first accumulates into an LDS tile
-// around the patch's HII footprint and flushes it once; deposits that fall
-// outside the tile go straight to global memory.
+// The particles of one HII cell share their displacement and deposit
+// together (k_move_cells), through an LDS tile around their block's patch.
 #include <cmath>
 
 #include "cm21_internal.hpp"
@@ -20,20 +17,22 @@ using namespace cm21;
 namespace {
 
 struct MoveParams {
-    int DIM, sw;
+    int DIM, sw, q;     // q = DIM / sw
     float disp_scale;   // (D(z) - D_init)/BOX_LEN
     float growth_init;  // D_init
-    double pf;          // PIXEL_FACTOR = DIM / sw
 };
 
-// Position of particle index i on one axis after the wrap loops of
+// Start of particle index i on one axis, in box units.
+__device__ inline float particle_start(int i, int DIM) { return (float)(((double)i + 0.5) / (double)DIM); }
+
+// Position on one axis from the start, after the wrap loops of
 // perturb_field.cu:102-118.  Returns false for a non-finite position.
-__device__ inline bool particle_coord(int i, float v, const MoveParams& mp, float& f) {
+__device__ __forceinline__ bool particle_coord(float start, float v, const MoveParams& mp, float& f) {
     const float swf = (float)mp.sw;
-    f = (float)(((double)i + 0.5) / (double)mp.DIM);
-    f = __fadd_rn(f, __fmul_rn(v, mp.disp_scale));
+    f = __fadd_rn(start, __fmul_rn(v, mp.disp_scale));
     f = __fmul_rn(f, swf);
     if (!isfinite(f)) return false;
+    if (f >= 0.0f && f < swf) return true;
     // The reference loops until in range; bound the loop and finish with an
     // exact floor-based wrap for displacements of many box lengths.
     int it = 0;
@@ -46,178 +45,322 @@ __device__ inline bool particle_coord(int i, float v, const MoveParams& mp, floa
     return true;
 }
 
-__device__ inline int hii_index(int i, double pf) { return (int)floor((double)i / pf); }
-
-__device__ inline bool particle_pos(size_t p, const float* vx, const float* vy, const float* vz,
-                                    const MoveParams& mp, float& xf, float& yf, float& zf) {
-    const int DIM = mp.DIM;
-    const int k = (int)(p % DIM);
-    const int j = (int)((p / DIM) % DIM);
-    const int i = (int)(p / ((size_t)DIM * DIM));
-    const int hi = hii_index(i, mp.pf), hj = hii_index(j, mp.pf), hk = hii_index(k, mp.pf);
-    const size_t h = ((size_t)hi * mp.sw + hj) * mp.sw + hk;  // C_INDEX(HII_k, HII_j, HII_i, sw)
-    return particle_coord(i, vx[h], mp, xf) && particle_coord(j, vy[h], mp, yf) && particle_coord(k, vz[h], mp, zf);
-}
-
 __device__ inline float particle_mass(float delta, float growth_init) {
     return (float)(1.0 + (double)__fmul_rn(growth_init, delta));
 }
 
-__device__ inline int wrap_cell(int x, int sw) {
-    if (x >= sw) x -= sw;
-    if (x < 0) x += sw;
-    return x;
-}
-
-__global__ void k_move_ngp(float* __restrict__ acc, const float* __restrict__ delta, const float* __restrict__ vx,
-                           const float* __restrict__ vy, const float* __restrict__ vz, MoveParams mp) {
-    const size_t n = (size_t)mp.DIM * mp.DIM * mp.DIM;
-    const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    float xf, yf, zf;
-    if (!particle_pos(p, vx, vy, vz, mp, xf, yf, zf)) return;
-    const int sw = mp.sw;
-    const int xi = wrap_cell((int)xf, sw), yi = wrap_cell((int)yf, sw), zi = wrap_cell((int)zf, sw);
-    if ((unsigned)xi >= (unsigned)sw || (unsigned)yi >= (unsigned)sw || (unsigned)zi >= (unsigned)sw) return;
-    atomicAdd(&acc[((size_t)xi * sw + yi) * sw + zi], particle_mass(delta[p], mp.growth_init));
-}
-
-// Tiled deposit.  A block of 256 threads moves the 16^3 particles of one
-// patch of the DIM grid (thread t owns (j,k) = (t/16, t%16) and walks 16
-// values of i).  Their HII targets lie near the patch's HII footprint, so the
-// block accumulates into an LDS tile covering the footprint plus a halo of
-// kHalo cells (plus one for the CIC neighbour) and flushes each non-zero tile
-// cell with one global atomic; deposits outside the tile go straight to
-// global memory.  scheme 0 = NGP, 1 = CIC.
+// Deposit by displacement cells.  The q^3 particles of one HII cell share
+// their displacement (q = DIM/sw), so they move as a rigid lattice less than
+// one HII cell wide: along each axis their target cells are base + {0, 1}
+// (NGP) or base + {0, 1, 2} (CIC; one less at q = 1), and the CIC weight of a particle in a cell
+// is the product of its three axis weights.  A thread therefore takes one HII
+// cell, forms the C weights of each of its q planes per axis (C = 1, 2 or 3) and
+// contracts the q^3 masses with them, along z, then y, then x, into C^3 sums:
+// 27 deposits for q^3 particles instead of 8 q^3 (q > 1).
 //
-// CIC: along a thread's walk in i the particles advance by 1/PIXEL_FACTOR
-// HII cells in x and share (y, z) cells while their displacement cells do, so
-// the thread keeps the deposits of the two x cells {base, base+1} times the
-// four (y, z) cells in registers and writes a cell to the tile only when the
-// walk leaves it: about 40 LDS atomics per 16 particles instead of 128.
-constexpr int kPatch = 16;
-constexpr int kHalo = 4;
+// A block of 512 threads takes kNY x kNZ columns of HII cells, each column
+// shared by two threads that walk half of its PX cells in x; it accumulates
+// into an LDS tile of the patch and the cells within kHalo of it, room for
+// displacements of 3.25 cells either way.  Cells whose lattice leaves the
+// tile deposit straight into global memory, and cells with a non-finite mass
+// or position go particle by particle, so that one bad particle reaches only
+// the cells that it touches.
+//
+// The tile is FP64 because the float32 LDS atomic is slow on this hardware:
+// ds_add_f32 takes 195 cycles of a CU's LDS per wavefront, ds_add_f64 9 (and
+// ds_add_u32 5), all on distinct addresses.  The float atomics were the bound
+// of every earlier form (2.1 to 2.3 ms at 512 -> 256, per particle or per
+// cell alike: 27 a cell are 7 M of them, 2.2 ms).
+//
+// Then each non-zero tile cell is one global atomic.  Storing the tiles and
+// adding those that cover a cell in a second kernel, without atomics, was
+// slower at every size (512 -> 256: 432 against 305 us, 128 -> 64: 35 against
+// 24).  In all, with the clearing and the renormalisation, 512 -> 256 takes
+// 305 us (CIC; 2.14 ms before), of which reading delta and the displacements
+// is 0.16 ms at the rate of a copy.
+constexpr int kHalo = 4, kReach = 2 * kHalo;  // tile side: patch side + kReach
+constexpr int kNY = 16, kNZ = 16, kWalk = 8, kMoveThreads = 512;
 
-__device__ inline int mod_sw(int x, int sw) {
-    x %= sw;
-    return x < 0 ? x + sw : x;
-}
+struct Tile {
+    float* acc;
+    int ox, oy, oz, Tx, Ty, Tz, sw;
+    bool use;
 
-// One deposit into the block's tile, or into global memory when the cell
-// lies outside the tile.  x, y, z are unwrapped HII cells.
-__device__ __forceinline__ void deposit(float* tile, float* acc, int x, int y, int z, float w, int ox, int oy,
-                                        int oz, int T, int sw, bool use_tile) {
-    if (w == 0.0f) return;
-    const int lx = mod_sw(x - ox, sw), ly = mod_sw(y - oy, sw), lz = mod_sw(z - oz, sw);
-    if (use_tile && lx < T && ly < T && lz < T)
-        atomicAdd(&tile[(lx * T + ly) * T + lz], w);
-    else
-        atomicAdd(&acc[((size_t)mod_sw(x, sw) * sw + mod_sw(y, sw)) * sw + mod_sw(z, sw)], w);
-}
+    __device__ __forceinline__ int local(int x, int o) const {  // (x - o) mod sw, x in [-1, sw), o in [-kHalo, sw)
+        int l = x - o;
+        l += l < 0 ? sw : 0;
+        return l >= sw ? l - sw : l;
+    }
+    __device__ __forceinline__ static int cell(int x, int sw) {
+        x %= sw;
+        return x < 0 ? x + sw : x;
+    }
+    __device__ __forceinline__ void add_global(int x, int y, int z, float w) const {
+        atomicAdd(&acc[((size_t)cell(x, sw) * sw + cell(y, sw)) * sw + cell(z, sw)], w);
+    }
+};
 
-// The register accumulator of one thread's CIC walk: cells (base + a, y0 + b,
-// z0 + c) for a, b, c in {0, 1}.
-struct CicRun {
-    int base, y0, z0;
-    bool live;
-    float v[2][4];  // [a][2b + c]
+// Target of one plane of a cell's lattice on one axis: its offset from the
+// base cell and its C weights.
+template <int SCHEME, int Q>
+struct AxisWeights {
+    static constexpr int C = (SCHEME == 0 ? 2 : 3) - (Q == 1 ? 1 : 0);
+    float w[C];
+    int cell;  // NGP: the target; CIC: the lower target
+    float t;   // CIC: share of the upper target
 
-    __device__ __forceinline__ void flush_x(int a, float* tile, float* acc, int ox, int oy, int oz, int T, int sw,
-                                            bool use_tile) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            deposit(tile, acc, base + a, y0 + (q >> 1), z0 + (q & 1), v[a][q], ox, oy, oz, T, sw, use_tile);
-            v[a][q] = 0.0f;
+    // f: position in [0, sw)
+    __device__ __forceinline__ void place(float f) {
+        if (SCHEME == 0) {
+            cell = (int)f;
+            t = 0.0f;
+        } else {
+            const float c = __fsub_rn(f, 0.5f), fl = floorf(c);
+            cell = (int)fl;
+            t = __fsub_rn(c, fl);
+        }
+    }
+    // weights relative to `base`; false when the offset is not 0 or 1
+    __device__ __forceinline__ bool weigh(int base, int sw) {
+        int o = cell - base;
+        o += o < 0 ? sw : 0;
+        const float lo = SCHEME == 0 ? 1.0f : __fsub_rn(1.0f, t);
+        if constexpr (Q == 1) {  // one plane: its own cell is the base
+            w[0] = lo;
+            if constexpr (C == 2) w[1] = t;
+            return true;
+        } else {
+            w[0] = o ? 0.0f : lo;
+            w[1] = o ? lo : t;
+            if constexpr (C == 3) w[2] = o ? t : 0.0f;
+            return o == 0 || o == 1;
         }
     }
 };
 
-template <int SCHEME>
-__global__ void k_move_tile(float* __restrict__ acc, const float* __restrict__ delta, const float* __restrict__ vx,
-                            const float* __restrict__ vy, const float* __restrict__ vz, MoveParams mp, int T) {
-    extern __shared__ float tile[];
-    const int DIM = mp.DIM, sw = mp.sw;
-    const int np = DIM / kPatch;
-    const int bk = blockIdx.x % np, bj = (blockIdx.x / np) % np, bi = blockIdx.x / (np * np);
+// Q: DIM/sw when it is 1 to 4 (the weights of every plane stay in registers),
+// or 0 for a larger ratio (formed again per row).
+template <int SCHEME, int Q>
+__global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__ acc, const float* __restrict__ delta,
+                                                    const float* __restrict__ vx, const float* __restrict__ vy,
+                                                    const float* __restrict__ vz, MoveParams mp, int PX, int Tx, int Ty,
+                                                    int Tz) {
+    using W = AxisWeights<SCHEME, Q>;
+    constexpr int C = W::C, NQ = Q > 0 ? Q : 1;
+    extern __shared__ double tile[];
+    __shared__ float startx[kWalk * NQ];  // particle_start of the walk's planes
+    const int DIM = mp.DIM, sw = mp.sw, q = Q > 0 ? Q : mp.q;
+    const int nz = (sw + kNZ - 1) / kNZ, ny = (sw + kNY - 1) / kNY;
+    const int z0 = (blockIdx.x % nz) * kNZ, y0 = (blockIdx.x / nz % ny) * kNY, x0 = (int)(blockIdx.x / (nz * ny)) * PX;
     const int t = threadIdx.x;
-    const int j = bj * kPatch + (t >> 4), k = bk * kPatch + (t & 15);
-    // Tile origin in unwrapped HII cells: footprint start minus the halo.
-    const int ox = hii_index(bi * kPatch, mp.pf) - kHalo;
-    const int oy = hii_index(bj * kPatch, mp.pf) - kHalo;
-    const int oz = hii_index(bk * kPatch, mp.pf) - kHalo;
-    const bool use_tile = sw >= T;
-    const int T3 = T * T * T;
-    if (use_tile) {
-        for (int q = t; q < T3; q += blockDim.x) tile[q] = 0.0f;
-        __syncthreads();
-    }
-    CicRun run;
-    run.live = false;
-    run.base = run.y0 = run.z0 = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) run.v[0][q] = run.v[1][q] = 0.0f;
-    for (int ii = 0; ii < kPatch; ++ii) {
-        const int i = bi * kPatch + ii;
-        const size_t p = ((size_t)i * DIM + j) * DIM + k;
-        float xf, yf, zf;
-        if (!particle_pos(p, vx, vy, vz, mp, xf, yf, zf)) continue;
-        const float m = particle_mass(delta[p], mp.growth_init);
-        if (SCHEME == 0) {
-            const int xi = wrap_cell((int)xf, sw), yi = wrap_cell((int)yf, sw), zi = wrap_cell((int)zf, sw);
-            if ((unsigned)xi >= (unsigned)sw || (unsigned)yi >= (unsigned)sw || (unsigned)zi >= (unsigned)sw) continue;
-            const int lx = mod_sw(xi - ox, sw), ly = mod_sw(yi - oy, sw), lz = mod_sw(zi - oz, sw);
-            if (use_tile && lx < T && ly < T && lz < T)
-                atomicAdd(&tile[(lx * T + ly) * T + lz], m);
-            else
-                atomicAdd(&acc[((size_t)xi * sw + yi) * sw + zi], m);
-        } else {
-            const float cx = __fsub_rn(xf, 0.5f), cy = __fsub_rn(yf, 0.5f), cz = __fsub_rn(zf, 0.5f);
-            const float fx = floorf(cx), fy = floorf(cy), fz = floorf(cz);
-            const float tx = __fsub_rn(cx, fx), ty = __fsub_rn(cy, fy), tz = __fsub_rn(cz, fz);
-            const int x0 = (int)fx, y0 = (int)fy, z0 = (int)fz;
-            if (run.live && (y0 != run.y0 || z0 != run.z0 || x0 < run.base || x0 > run.base + 1)) {
-                run.flush_x(0, tile, acc, ox, oy, oz, T, sw, use_tile);
-                run.flush_x(1, tile, acc, ox, oy, oz, T, sw, use_tile);
-                run.live = false;
-            }
-            if (!run.live) {
-                run.base = x0;
-                run.y0 = y0;
-                run.z0 = z0;
-                run.live = true;
-            } else if (x0 == run.base + 1) {
-                // the walk leaves cell `base`: write it, slide the window
-                run.flush_x(0, tile, acc, ox, oy, oz, T, sw, use_tile);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    run.v[0][q] = run.v[1][q];
-                    run.v[1][q] = 0.0f;
-                }
-                run.base = x0;
-            }
-            const float wx[2] = {__fsub_rn(1.0f, tx), tx};
-            const float wy[2] = {__fsub_rn(1.0f, ty), ty};
-            const float wz[2] = {__fsub_rn(1.0f, tz), tz};
-#pragma unroll
-            for (int dx = 0; dx < 2; ++dx)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    run.v[dx][q] += __fmul_rn(__fmul_rn(__fmul_rn(m, wx[dx]), wy[q >> 1]), wz[q & 1]);
-        }
-    }
-    if (SCHEME == 1 && run.live) {
-        run.flush_x(0, tile, acc, ox, oy, oz, T, sw, use_tile);
-        run.flush_x(1, tile, acc, ox, oy, oz, T, sw, use_tile);
-    }
-    if (!use_tile) return;
+    const int hy = y0 + t / kNZ % kNY, hz = z0 + t % kNZ;
+    const int half = t / (kNY * kNZ), xa = x0 + half * (PX / 2);  // this thread's part of the walk
+    const Tile tl{acc, x0 - kHalo, y0 - kHalo, z0 - kHalo, Tx, Ty, Tz, sw, sw >= Tx && sw >= Ty && sw >= Tz};
+    if (tl.use)
+        for (int c = t; c < Tx * Ty * Tz; c += kMoveThreads) tile[c] = 0.0;
+    if (t < kWalk * NQ) startx[t] = particle_start(x0 * NQ + t, DIM);
     __syncthreads();
-    for (int q = t; q < T3; q += blockDim.x) {
-        const float v = tile[q];
-        if (v != 0.0f) {
-            const int lz = q % T, ly = (q / T) % T, lx = q / (T * T);
-            atomicAdd(&acc[((size_t)mod_sw(ox + lx, sw) * sw + mod_sw(oy + ly, sw)) * sw + mod_sw(oz + lz, sw)], v);
+    const int xb = hy < sw && hz < sw ? min(sw, xa + PX / 2) : xa;
+    for (int hx = xa; hx < xb; ++hx) {
+        const size_t h = ((size_t)hx * sw + hy) * sw + hz;  // C_INDEX(HII_k, HII_j, HII_i, sw)
+        const float pv[3] = {vx[h], vy[h], vz[h]};
+        const int i0 = hx * q, j0 = hy * q, k0 = hz * q;  // the cell's first particle
+        const float* dp = delta + ((size_t)i0 * DIM + j0) * DIM + k0;
+        float m[NQ][NQ][NQ];
+        if (Q > 0) {
+#pragma unroll
+            for (int i = 0; i < NQ; ++i)
+#pragma unroll
+                for (int j = 0; j < NQ; ++j) {
+                    const float* row = dp + ((size_t)i * DIM + j) * DIM;
+                    // rows start at multiples of q floats and DIM is a multiple of 8
+                    if constexpr (Q == 2) {
+                        const float2 d = *(const float2*)row;
+                        m[i][j][0] = d.x, m[i][j][1] = d.y;
+                    } else if constexpr (Q == 4) {
+                        const float4 d = *(const float4*)row;
+                        m[i][j][0] = d.x, m[i][j][1] = d.y, m[i][j][2] = d.z, m[i][j][3] = d.w;
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < NQ; ++k) m[i][j][k] = row[k];
+                    }
+                }
+        }
+        W w[3][NQ];
+        int base[3];
+        bool ok = true;
+        const int first[3] = {i0, j0, k0};
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            float f;
+            auto start = [&](int p) {
+                return Q > 0 && ax == 0 ? startx[(hx - x0) * NQ + p] : particle_start(first[ax] + p, DIM);
+            };
+            ok = particle_coord(start(0), pv[ax], mp, f) && ok;
+            w[ax][0].place(f);
+            base[ax] = w[ax][0].cell;
+            w[ax][0].weigh(base[ax], sw);
+#pragma unroll
+            for (int p = 1; p < NQ; ++p) {
+                ok = particle_coord(start(p), pv[ax], mp, f) && ok;
+                w[ax][p].place(f);
+                ok = w[ax][p].weigh(base[ax], sw) && ok;
+            }
+        }
+        float s[C][C][C];
+#pragma unroll
+        for (int a = 0; a < C; ++a)
+#pragma unroll
+            for (int b = 0; b < C; ++b)
+#pragma unroll
+                for (int c = 0; c < C; ++c) s[a][b][c] = 0.0f;
+        float total = 0.0f;
+        auto weight = [&](int ax, int p, W& o) {
+            float f;
+            ok = particle_coord(particle_start(first[ax] + p, DIM), pv[ax], mp, f) && ok;
+            o.place(f);
+            ok = o.weigh(base[ax], sw) && ok;
+        };
+        if (Q > 0) {
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                float p2[C][C];
+#pragma unroll
+                for (int j = 0; j < NQ; ++j) {
+                    float p1[C];
+#pragma unroll
+                    for (int k = 0; k < NQ; ++k) {
+                        const float mass = particle_mass(m[i][j][k], mp.growth_init);
+                        total += mass;
+#pragma unroll
+                        for (int c = 0; c < C; ++c) p1[c] = k ? fmaf(w[2][k].w[c], mass, p1[c]) : w[2][k].w[c] * mass;
+                    }
+#pragma unroll
+                    for (int b = 0; b < C; ++b)
+#pragma unroll
+                        for (int c = 0; c < C; ++c)
+                            p2[b][c] = j ? fmaf(w[1][j].w[b], p1[c], p2[b][c]) : w[1][j].w[b] * p1[c];
+                }
+#pragma unroll
+                for (int a = 0; a < C; ++a)
+#pragma unroll
+                    for (int b = 0; b < C; ++b)
+#pragma unroll
+                        for (int c = 0; c < C; ++c) s[a][b][c] = fmaf(w[0][i].w[a], p2[b][c], s[a][b][c]);
+            }
+        } else {
+            for (int i = 0; i < q; ++i) {
+                float p2[C][C];
+#pragma unroll
+                for (int b = 0; b < C; ++b)
+#pragma unroll
+                    for (int c = 0; c < C; ++c) p2[b][c] = 0.0f;
+                for (int j = 0; j < q; ++j) {
+                    float p1[C];
+#pragma unroll
+                    for (int c = 0; c < C; ++c) p1[c] = 0.0f;
+                    const float* row = dp + ((size_t)i * DIM + j) * DIM;
+                    for (int k = 0; k < q; ++k) {
+                        W wk;
+                        weight(2, k, wk);
+                        const float mass = particle_mass(row[k], mp.growth_init);
+                        total += mass;
+#pragma unroll
+                        for (int c = 0; c < C; ++c) p1[c] = fmaf(wk.w[c], mass, p1[c]);
+                    }
+                    W wj;
+                    weight(1, j, wj);
+#pragma unroll
+                    for (int b = 0; b < C; ++b)
+#pragma unroll
+                        for (int c = 0; c < C; ++c) p2[b][c] = fmaf(wj.w[b], p1[c], p2[b][c]);
+                }
+                W wi;
+                weight(0, i, wi);
+#pragma unroll
+                for (int a = 0; a < C; ++a)
+#pragma unroll
+                    for (int b = 0; b < C; ++b)
+#pragma unroll
+                        for (int c = 0; c < C; ++c) s[a][b][c] = fmaf(wi.w[a], p2[b][c], s[a][b][c]);
+            }
+        }
+        if (!(ok && isfinite(total))) {
+            for (int p = 0; p < q * q * q; ++p) {
+                const int i = p / (q * q), j = p / q % q, k = p % q;
+                W o[3];
+                float f[3];
+                if (!(particle_coord(particle_start(i0 + i, DIM), pv[0], mp, f[0]) &&
+                      particle_coord(particle_start(j0 + j, DIM), pv[1], mp, f[1]) &&
+                      particle_coord(particle_start(k0 + k, DIM), pv[2], mp, f[2])))
+                    continue;
+                const float mass = particle_mass(dp[((size_t)i * DIM + j) * DIM + k], mp.growth_init);
+#pragma unroll
+                for (int ax = 0; ax < 3; ++ax) o[ax].place(f[ax]);
+                for (int c = 0; c < (SCHEME == 0 ? 1 : 8); ++c) {
+                    const int a = c >> 2, b = (c >> 1) & 1, e = c & 1;
+                    float wt = mass;
+                    if (SCHEME == 1) {
+                        wt = __fmul_rn(wt, a ? o[0].t : __fsub_rn(1.0f, o[0].t));
+                        wt = __fmul_rn(wt, b ? o[1].t : __fsub_rn(1.0f, o[1].t));
+                        wt = __fmul_rn(wt, e ? o[2].t : __fsub_rn(1.0f, o[2].t));
+                    }
+                    if (wt != 0.0f) tl.add_global(o[0].cell + a, o[1].cell + b, o[2].cell + e, wt);
+                }
+            }
+            continue;
+        }
+        const int lx = tl.local(base[0], tl.ox), ly = tl.local(base[1], tl.oy), lz = tl.local(base[2], tl.oz);
+        if (tl.use && lx <= Tx - C && ly <= Ty - C && lz <= Tz - C) {
+            double* p = tile + (lx * Ty + ly) * Tz + lz;
+#pragma unroll
+            for (int a = 0; a < C; ++a)
+#pragma unroll
+                for (int b = 0; b < C; ++b)
+#pragma unroll
+                    for (int c = 0; c < C; ++c) atomicAdd(p + (a * Ty + b) * Tz + c, (double)s[a][b][c]);
+        } else {
+#pragma unroll
+            for (int a = 0; a < C; ++a)
+#pragma unroll
+                for (int b = 0; b < C; ++b)
+#pragma unroll
+                    for (int c = 0; c < C; ++c)
+                        if (s[a][b][c] != 0.0f) tl.add_global(base[0] + a, base[1] + b, base[2] + c, s[a][b][c]);
         }
     }
+    if (!tl.use) return;
+    __syncthreads();
+    for (int c = t; c < Ty * Tz; c += kMoveThreads) {
+        const int ly = c / Tz, lz = c - ly * Tz;
+        int gx = tl.ox < 0 ? tl.ox + sw : tl.ox, gy = tl.oy + ly, gz = tl.oz + lz;
+        gy = gy < 0 ? gy + sw : (gy >= sw ? gy - sw : gy);
+        gz = gz < 0 ? gz + sw : (gz >= sw ? gz - sw : gz);
+        float* col = acc + (size_t)gy * sw + gz;
+        for (int lx = 0; lx < Tx; ++lx) {
+            const float v = (float)tile[lx * Ty * Tz + c];
+            if (v != 0.0f) atomicAdd(col + (size_t)gx * sw * sw, v);
+            gx = gx + 1 == sw ? 0 : gx + 1;
+        }
+    }
+}
+
+template <int SCHEME>
+int launch_move(float* acc, const float* delta, const float* vx, const float* vy, const float* vz, const MoveParams& mp,
+                hipStream_t st) {
+    auto blocks = [&](int n) { return (unsigned)((mp.sw + n - 1) / n); };
+    // a walk of kWalk cells, or of 2 where that would leave CUs without a block
+    const int PX = blocks(kWalk) * blocks(kNY) * blocks(kNZ) >= 512 ? kWalk : 2;
+    const int Tx = PX + kReach, Ty = kNY + kReach, Tz = kNZ + kReach;
+    const unsigned grid = blocks(PX) * blocks(kNY) * blocks(kNZ);
+    const size_t lds = sizeof(double) * Tx * Ty * Tz;  // 72 KB, two blocks a CU (45 KB for the short walk)
+    auto* k = mp.q == 1 ? k_move_cells<SCHEME, 1>
+                        : (mp.q == 2 ? k_move_cells<SCHEME, 2>
+                                     : (mp.q == 3 ? k_move_cells<SCHEME, 3>
+                                                  : (mp.q == 4 ? k_move_cells<SCHEME, 4> : k_move_cells<SCHEME, 0>)));
+    k<<<grid, kMoveThreads, lds, st>>>(acc, delta, vx, vy, vz, mp, PX, Tx, Ty, Tz);
+    CM21_LAUNCH_CHECK("k_move_cells");
+    return CM21_OK;
 }
 
 __global__ void k_zero(float* __restrict__ p, size_t n) {
@@ -240,31 +383,15 @@ extern "C" int cm21_move_mass(float* updated, const float* deltax, const float* 
                  DIM);
     CM21_REQUIRE(sw >= 1 && sw <= DIM && DIM % sw == 0, "cm21_move_mass: sw=%d must divide DIM=%d", sw, DIM);
     CM21_REQUIRE(scheme == 0 || scheme == 1, "cm21_move_mass: scheme=%d not in {0 (NGP), 1 (CIC)}", scheme);
+    if (scheme == 1 && DIM % 16 != 0)
+        return cm21::fail(CM21_ERR_INVALID, "cm21_move_mass: CIC needs DIM %% 16 == 0");
     hipStream_t st = (hipStream_t)stream;
     const size_t n_small = (size_t)sw * sw * sw;
-    const size_t n_part = (size_t)DIM * DIM * DIM;
     const float pff = (float)DIM / (float)sw;  // PIXEL_FACTOR (INIT_PARAMS.py:7)
-    MoveParams mp{DIM, sw, disp_scale, growth_init, (double)pff};
-    // Tile edge: HII footprint of a patch (ceil(16/pf)) plus halo on both
-    // sides plus the CIC neighbour.
-    const int foot = (int)std::ceil((double)kPatch / (double)pff);
-    const int T = foot + 2 * kHalo + 1;
-    const size_t lds = sizeof(float) * (size_t)T * T * T;
-    const unsigned blocks = (unsigned)((DIM / kPatch) * (DIM / kPatch) * (DIM / kPatch));
-    if (scheme == 1 && (DIM % kPatch != 0 || lds > 64 * 1024))
-        return cm21::fail(CM21_ERR_INVALID, "cm21_move_mass: CIC needs DIM %% 16 == 0 and DIM/sw <= 16");
+    const MoveParams mp{DIM, sw, DIM / sw, disp_scale, growth_init};
     k_zero<<<grid_for(n_small), kThreads, 0, st>>>(updated, n_small);
     CM21_LAUNCH_CHECK("k_zero");
-    if (DIM % kPatch != 0 || lds > 64 * 1024) {
-        k_move_ngp<<<grid_for(n_part), kThreads, 0, st>>>(updated, deltax, vx, vy, vz, mp);
-        CM21_LAUNCH_CHECK("k_move_ngp");
-    } else if (scheme == 0) {
-        k_move_tile<0><<<blocks, kThreads, lds, st>>>(updated, deltax, vx, vy, vz, mp, T);
-        CM21_LAUNCH_CHECK("k_move_tile<NGP>");
-    } else {
-        k_move_tile<1><<<blocks, kThreads, lds, st>>>(updated, deltax, vx, vy, vz, mp, T);
-        CM21_LAUNCH_CHECK("k_move_tile<CIC>");
-    }
+    CM21_TRY((scheme ? launch_move<1> : launch_move<0>)(updated, deltax, vx, vy, vz, mp, st));
     const float mass_factor = (float)std::pow((double)pff, 3.0);  // MASS_FACTOR (INIT_PARAMS.py:8)
     k_renorm<<<grid_for(n_small), kThreads, 0, st>>>(updated, n_small, mass_factor);
     CM21_LAUNCH_CHECK("k_renorm");

@@ -1,0 +1,62 @@
+"""The mass move at the edges of its patches and tiles: sides that do not fill
+a patch, every ratio class DIM/sw, boxes smaller than a tile and displacements
+that leave it.  Against the oracle with its bars (NGP cells exact, sums 1e-5)."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import pkg
+from oracle import perturb
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("DIM,sw", [(8, 8), (8, 1), (16, 1), (16, 2), (24, 24), (32, 32), (40, 20), (48, 48), (48, 16),
+                                    (56, 28), (64, 32), (72, 24), (80, 16), (80, 8), (96, 12), (112, 56), (128, 32), (144, 144), (176, 88)])
+@pytest.mark.parametrize("amp", [0.0, 3.0, 60.0, 400.0])
+def test_move_mass_edges(gpu, DIM, sw, amp):
+    g = pkg("gpu")
+    L = 60.0
+    rng = np.random.default_rng(DIM * 1000 + sw)
+    delta = rng.standard_normal((DIM,) * 3).astype(np.float32)
+    v = [(amp * rng.standard_normal((sw,) * 3)).astype(np.float32) for _ in range(3)]
+    growth, ginit = 0.12, 0.0036
+    s = pkg("Programs.perturb_field").displacement_scale(growth, ginit, L)
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    dv = [dev(a) for a in v]
+    got = g.move_mass(dev(np.zeros_like(delta)), *dv, s, ginit, "ngp").cpu().numpy()
+    assert np.array_equal(got, perturb.move_mass_ngp(np.zeros_like(delta), *v, growth, ginit, L))
+    got = g.move_mass(dev(delta), *dv, s, ginit, "ngp").cpu().numpy()
+    assert np.allclose(got, perturb.move_mass_ngp(delta, *v, growth, ginit, L), rtol=1e-5, atol=2e-6)
+    if DIM % 16 == 0:
+        got = g.move_mass(dev(delta), *dv, s, ginit, "cic").cpu().numpy()
+        assert np.allclose(got, perturb.move_mass_cic(delta, *v, growth, ginit, L), rtol=1e-5, atol=2e-6)
+    else:
+        with pytest.raises(pkg("_lib").CM21Error):
+            g.move_mass(dev(delta), *dv, s, ginit, "cic")
+
+
+def test_move_mass_keeps_bad_particles_apart(gpu):
+    """A non-finite mass reaches only the cells of its own particle, and a
+    non-finite displacement drops the particles of its cell, as the move
+    particle by particle does."""
+    g = pkg("gpu")
+    DIM, sw, L = 64, 32, 60.0
+    rng = np.random.default_rng(5)
+    delta = np.zeros((DIM,) * 3, np.float32)
+    v = [(3.0 * rng.standard_normal((sw,) * 3)).astype(np.float32) for _ in range(3)]
+    s = pkg("Programs.perturb_field").displacement_scale(0.12, 0.0036, L)
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    delta[10, 20, 31] = np.nan
+    delta[40, 41, 42] = np.inf
+    for scheme, most in (("ngp", 1), ("cic", 8)):
+        got = g.move_mass(dev(delta), *[dev(a) for a in v], s, 0.0036, scheme).cpu().numpy()
+        assert 1 <= np.isnan(got).sum() <= most and 1 <= np.isinf(got).sum() <= most
+    delta[:] = 0.0
+    v[1][4, 5, 6] = np.nan
+    v[2][7, 8, 9] = np.inf
+    for scheme in ("ngp", "cic"):
+        got = g.move_mass(dev(delta), *[dev(a) for a in v], s, 0.0036, scheme).cpu().numpy()
+        assert np.isfinite(got).all()
+        # 16 particles of 64^3 are gone; cells hold (mass / 8) - 1
+        assert abs((got.astype(np.float64) + 1.0).sum() * 8 - (DIM ** 3 - 16)) < 0.05
