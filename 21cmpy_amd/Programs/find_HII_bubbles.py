@@ -161,9 +161,9 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
     caller = torch.cuda.current_stream()
     s = caller if stream is None else stream
     plan = _lib.plan(D, 1)
-    nbytes = _lib.query("cm21_find_bubbles_workspace_bytes", D, len(radii), int(update))
     r = np.ascontiguousarray(radii, dtype=np.float32)
     dn = np.ascontiguousarray(denoms, dtype=np.float32)
+    nbytes = _lib.query("cm21_find_bubbles_full_workspace_bytes", D, r.ctypes.data_as(_lib.c_float_p), len(r), prm)
     # Everything runs on `s`, ordered after the caller's pending work and
     # before the caller's later work: the input upload, the loop, the read-back.
     if s != caller:

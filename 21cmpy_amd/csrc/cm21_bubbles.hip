@@ -301,18 +301,76 @@ LoopWork carve(void* base, int D, int n_radii, int update) {
     w.bytes = off;
     return w;
 }
+
+// The all-radii form (sides up to 160): its buffers behind the standard
+// carve-up's spectrum, or bytes = 0 when the form does not apply.
+struct AllWork {
+    AllRadii a;
+    size_t bytes;
+};
+
+bool loop_is_fused(const FusedShape* sh, const cm21_bubble_params* prm) {
+    return prm->fused && sh && prm->update == 0 && (prm->filter_type == 1 || prm->filter_type == 2);
+}
+
+float loop_scale(int D, const cm21_bubble_params* prm) {
+    const double n = (double)((size_t)D * D * D);
+    return prm->linear_input ? (float)(1.0 / n) : (float)((double)prm->growth_inv / n);
+}
+
+float loop_delta_k(const cm21_bubble_params* prm) { return (float)(2.0 * M_PI / (double)prm->box_len); }
+
+AllWork carve_all(void* base, int D, const float* radii, const float* denoms, int n_radii,
+                  const cm21_bubble_params* prm) {
+    AllWork w{};
+    const FusedShape* sh = fused_shape(D);
+    if (!loop_is_fused(sh, prm)) return w;
+    const size_t nt = all_radii_table(*sh, loop_delta_k(prm), radii, denoms, n_radii, prm->filter_type,
+                                      prm->ref_fallthrough, loop_scale(D, prm), &w.a);
+    if (nt == 0) return w;
+    const size_t N = (size_t)D * D * D, row = (size_t)D * D * padded_row(D / 2 + 1);
+    const size_t cells = (size_t)n_radii * w.a.nblk;
+    char* p = (char*)base;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        void* q = p + off;
+        off = align_up(off + bytes, 256);
+        return q;
+    };
+    AllRadii& a = w.a;
+    a.S = (float2*)take(sizeof(float2) * row);
+    // the forward transform passes through the intermediates' region
+    a.T = (float2*)take(sizeof(float2) * std::max(nt, row));
+    a.sums = (double*)take(sizeof(double) * n_radii);
+    a.scaled = (ScaledThreshold*)take(sizeof(ScaledThreshold) * n_radii);
+    a.hits = (unsigned*)take(sizeof(unsigned) * cells);
+    a.planes = (unsigned long long*)take(sizeof(unsigned long long) * n_radii * (N / 64));
+    if (!prm->linear_input) {
+        a.partial = (double*)take(sizeof(double) * cells);
+        a.bmax = (float*)take(sizeof(float) * cells);
+    }
+    w.bytes = off;
+    return w;
+}
 }  // namespace
 
 namespace {
 int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* radii, const float* denoms,
-             int n_radii, const cm21_bubble_params* prm, const LoopWork& w, hipStream_t st);
+             int n_radii, const cm21_bubble_params* prm, void* work, size_t work_bytes, hipStream_t st);
 int graph_loop(cm21_plan* plan, const float* delta, float* ionized, const float* radii, const float* denoms,
-               int n_radii, const cm21_bubble_params* prm, const LoopWork& w, hipStream_t st);
+               int n_radii, const cm21_bubble_params* prm, void* work, size_t work_bytes, hipStream_t st);
 }  // namespace
 
 extern "C" size_t cm21_find_bubbles_workspace_bytes(int D, int n_radii, int update) {
     if (!valid_dim(D)) return 0;
     return carve(nullptr, D, n_radii, update).bytes;
+}
+
+extern "C" size_t cm21_find_bubbles_full_workspace_bytes(int D, const float* radii, int n_radii,
+                                                         const cm21_bubble_params* prm) {
+    if (!valid_dim(D) || !radii || n_radii < 1 || !prm || !(prm->box_len > 0.0f)) return 0;
+    return std::max(carve(nullptr, D, n_radii, prm->update).bytes,
+                    carve_all(nullptr, D, radii, nullptr, n_radii, prm).bytes);
 }
 
 namespace {
@@ -343,27 +401,27 @@ extern "C" int cm21_find_bubbles(cm21_plan* plan, const float* delta, float* ion
                                  size_t work_bytes, void* stream) {
     CM21_TRY(check_loop_args("cm21_find_bubbles", plan, delta, ionized, radii, denoms, n_radii, prm));
     CM21_REQUIRE(work, "cm21_find_bubbles: NULL argument");
-    const int D = plan_dim(plan);
-    LoopWork w = carve(work, D, n_radii, prm->update);
-    if (work_bytes < w.bytes)
-        return cm21::fail(CM21_ERR_NOMEM, "cm21_find_bubbles: workspace %zu bytes < required %zu", work_bytes,
-                          w.bytes);
+    const size_t need = carve(nullptr, plan_dim(plan), n_radii, prm->update).bytes;
+    if (work_bytes < need)
+        return cm21::fail(CM21_ERR_NOMEM, "cm21_find_bubbles: workspace %zu bytes < required %zu", work_bytes, need);
     hipStream_t st = (hipStream_t)stream;
-    if (prm->graph && st != nullptr && !prof_any()) return graph_loop(plan, delta, ionized, radii, denoms, n_radii, prm, w, st);
-    return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, w, st);
+    if (prm->graph && st != nullptr && !prof_any())
+        return graph_loop(plan, delta, ionized, radii, denoms, n_radii, prm, work, work_bytes, st);
+    return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, work, work_bytes, st);
 }
 
 namespace {
 int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* radii, const float* denoms,
-             int n_radii, const cm21_bubble_params* prm, const LoopWork& w, hipStream_t st) {
+             int n_radii, const cm21_bubble_params* prm, void* work, size_t work_bytes, hipStream_t st) {
     void* stream = (void*)st;
     const int D = plan_dim(plan);
     const size_t N = (size_t)D * D * D;
+    const LoopWork w = carve(work, D, n_radii, prm->update);
 
-    const float dk = (float)(2.0 * M_PI / (double)prm->box_len);
-    const float scale = prm->linear_input ? (float)(1.0 / (double)N) : (float)((double)prm->growth_inv / (double)N);
+    const float dk = loop_delta_k(prm);
+    const float scale = loop_scale(D, prm);
     const FusedShape* sh = fused_shape(D);
-    if (prm->fused && sh && prm->update == 0 && (prm->filter_type == 1 || prm->filter_type == 2)) {
+    if (loop_is_fused(sh, prm)) {
         const float2* tw = plan_twiddles(plan);
         // the forward transform forms only the modes the widest window keeps,
         // through the intermediate that radius 4 uses first
@@ -371,6 +429,19 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
         for (int r = 1; r < n_radii; ++r) {
             const FusedParams f = fused_params(D, dk, radii[r], prm->filter_type, prm->ref_fallthrough, scale);
             if (f.m2max > widest.m2max) widest = f;
+        }
+        // every radius at once where the workspace holds their intermediates
+        AllWork all = carve_all(work, D, radii, denoms, n_radii, prm);
+        if (all.bytes && work_bytes >= all.bytes) {
+            AllRadii& a = all.a;
+            a.linear = prm->linear_input ? 1 : 0;
+            a.deltac = prm->deltac;
+            a.fc_mean = prm->fc_mean;
+            a.zeta = prm->zeta;
+            a.ncells = (double)N;
+            a.out = ionized;
+            CM21_TRY(fused_forward(*sh, delta, a.T, a.S, tw, widest, st));
+            return fused_all_radii(*sh, a, tw, st);
         }
         CM21_TRY(fused_forward(*sh, delta, w.inter[kInter - 1], w.spec, tw, widest, st));
         CM21_TRY(fused_mask_clear(w.mask, (N + 63) / 64, st));
@@ -511,11 +582,13 @@ struct GraphKey {
     const void* delta;
     const void* ionized;
     const void* work;
+    size_t work_bytes;
     hipStream_t stream;
     cm21_bubble_params prm;
     std::vector<float> radii, denoms;
     bool operator==(const GraphKey& o) const {
-        return delta == o.delta && ionized == o.ionized && work == o.work && stream == o.stream &&
+        return delta == o.delta && ionized == o.ionized && work == o.work &&
+               work_bytes == o.work_bytes && stream == o.stream &&
                std::memcmp(&prm, &o.prm, sizeof(prm)) == 0 && radii == o.radii && denoms == o.denoms;
     }
 };
@@ -527,8 +600,8 @@ std::mutex g_graph_mu;
 std::unordered_map<const cm21_plan*, GraphEntry> g_graphs;
 
 int graph_loop(cm21_plan* plan, const float* delta, float* ionized, const float* radii, const float* denoms,
-               int n_radii, const cm21_bubble_params* prm, const LoopWork& w, hipStream_t st) {
-    GraphKey key{delta, ionized, w.spec, st, *prm, std::vector<float>(radii, radii + n_radii),
+               int n_radii, const cm21_bubble_params* prm, void* work, size_t work_bytes, hipStream_t st) {
+    GraphKey key{delta, ionized, work, work_bytes, st, *prm, std::vector<float>(radii, radii + n_radii),
                  std::vector<float>(denoms, denoms + n_radii)};
     std::lock_guard<std::mutex> lk(g_graph_mu);
     auto it = g_graphs.find(plan);
@@ -542,9 +615,9 @@ int graph_loop(cm21_plan* plan, const float* delta, float* ionized, const float*
     }
     if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) {
         (void)hipGetLastError();
-        return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, w, st);
+        return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, work, work_bytes, st);
     }
-    const int rc = run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, w, st);
+    const int rc = run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, work, work_bytes, st);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(st, &graph);
     hipGraphExec_t exec = nullptr;
@@ -554,7 +627,7 @@ int graph_loop(cm21_plan* plan, const float* delta, float* ionized, const float*
     if (!ok) {
         (void)hipGetLastError();
         if (rc != CM21_OK) return rc;
-        return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, w, st);
+        return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, work, work_bytes, st);
     }
     g_graphs[plan] = GraphEntry{std::move(key), exec};
     CM21_HIP_CHECK(hipGraphLaunch(exec, st));
@@ -608,10 +681,9 @@ extern "C" int cm21_find_bubbles_noalloc(cm21_plan* plan, const float* delta, fl
                           D, n_radii, prm->update, need, kScratchBytes);
     void* base = nullptr;
     CM21_TRY(scratch_on_current_device(&base));
-    LoopWork w = carve(base, D, n_radii, prm->update);
     // the launches go straight to the stream (params->graph is ignored), so a
     // caller that captures the stream records them into its own graph
-    return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, w, (hipStream_t)stream);
+    return run_loop(plan, delta, ionized, radii, denoms, n_radii, prm, base, kScratchBytes, (hipStream_t)stream);
 }
 
 namespace cm21 {

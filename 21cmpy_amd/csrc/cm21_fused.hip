@@ -85,12 +85,15 @@ __device__ void finish_box_sum(const double* partial, int n, double* out, const 
 // inside the band take the exact test, so the skip never drops a hit).  A
 // final-paint block whose cells are all ionized writes 1 without transforming.
 // `blk` is the index of the L-line group the block works on.
-template <int N1, int N2, int L, int MODE>
-__device__ __forceinline__ void lines_block(const float2* __restrict__ U, const float2* __restrict__ tw,
+// `hs` is the line stride of U.  kLinePaint is kLineFinal with the block's mask
+// words in ep.word (thread t holds word t) instead of ep.mask.
+template <int N1, int N2, int L, int MODE_>
+__device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs, const float2* __restrict__ tw,
                                             const FusedParams& fp, const LineEpilogue& ep, int blk, float2* buf,
                                             float2* stw, unsigned long long* smask) {
     using C = LinesCore<N1, N2, L>;
     constexpr int D = C::D, NT = C::NT, WORDS = C::WORDS;
+    constexpr int MODE = MODE_ == kLinePaint ? (int)kLineFinal : MODE_;
     const int t = threadIdx.x;
     const size_t line0 = (size_t)blk * L;
     const size_t word0 = line0 * D / 64;
@@ -105,7 +108,7 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, const 
             scale = s.scale;
             th = s.th;
         }
-        mword = t < WORDS ? ep.mask[word0 + t] : ~0ull;
+        mword = t < WORDS ? (MODE_ == kLinePaint ? ep.word : ep.mask[word0 + t]) : ~0ull;
         const bool all_ionized = __syncthreads_and(mword == ~0ull);
         if (all_ionized) {
             if (MODE == kLineFinal)
@@ -116,7 +119,7 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, const 
     }
     // all global loads in flight before the first LDS store
     float2 tmp[C::LOADS];
-    C::load(U + line0 * C::HO, C::HO, fp.cmax + 1, tmp);
+    C::load(U + line0 * hs, hs, fp.cmax + 1, tmp);
     for (int q = t; q < D; q += NT) stw[q] = tw[q];
     C::store(tmp, buf);
     if (MODE != kLineSum && t < WORDS) smask[t] = mword;
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(L* N1) void k_fused_lines(const float2* __restrict_
         if (blk >= *ep.nactive) return;
         blk = ep.active[blk];
     }
-    lines_block<N1, N2, L, MODE>(U, tw, fp, ep, blk, buf, stw, smask);
+    lines_block<N1, N2, L, MODE>(U, C::HO, tw, fp, ep, blk, buf, stw, smask);
 }
 
 // One launch of the pipelined radius loop.  Its blocks take one of five
@@ -247,14 +250,14 @@ __global__ __launch_bounds__(W* D1, 8) void k_fused_radius(RadiusRoles a, const 
             if (b >= *a.ep_thr.nactive) return;
             b = a.ep_thr.active[b];
         }
-        lines_block<N1, N2, L, kLineThreshold>(a.Uthr, tw, a.fp_thr, a.ep_thr, b, buf, stw, smask);
+        lines_block<N1, N2, L, kLineThreshold>(a.Uthr, C::HO, tw, a.fp_thr, a.ep_thr, b, buf, stw, smask);
         return;
     }
     if (b >= thr0 + a.n_thr) b -= a.n_thr;
     const bool mem = b >= a.n_sum;
     int i = mem ? b - a.n_sum : b;
     if (!mem) {
-        lines_block<N1, N2, L, kLineSum>(a.Usum, tw, a.fp_sum, a.ep_sum, i, buf, stw, smask);
+        lines_block<N1, N2, L, kLineSum>(a.Usum, C::HO, tw, a.fp_sum, a.ep_sum, i, buf, stw, smask);
     } else if (i < a.n_cols) {
         columns_body<D1, D2, W, kRounds, true>(a.S, a.Tcols, C::HO, tw, a.fp_cols, a.fp_cols.scale, i / a.ncg_cols,
                                 i % a.ncg_cols, lds);
@@ -262,6 +265,163 @@ __global__ __launch_bounds__(W* D1, 8) void k_fused_radius(RadiusRoles a, const 
         i -= a.n_cols;
         rows_body<D1, D2, W, kRounds>(a.Trows, C::HO, tw, a.fp_rows, i / a.ncg_rows, i % a.ncg_rows, lds);
     }
+}
+
+// ------------------------------------------------------------------ all radii at once
+// For sides up to 160 a launch per radius leaves most of the chip idle (64 to
+// 800 line groups on 2048 block slots) and the ~45 launches of a box cost more
+// than their work.  Here each role runs once, over every (radius, group): the
+// columns, the rows, the box sums, the reductions (nonlinear input), the
+// thresholds and the paint, with the same device bodies on the same tiles, so
+// the results are those of the launch per radius bit for bit.  What the loop
+// orders, the ionization mask, becomes one bit plane per radius: a group's
+// threshold block writes its hits where it has any, and the paint ORs the
+// flagged planes.  The thresholds of linear input are found by the columns
+// launch (one more block) instead of on the host.
+// A call of conv_bubbles takes 75 us at 64^3 (linear, 37 radii; 279 before)
+// and 247 us at 128^3 (nonlinear, 40 radii; 463), 130 of them the box sums.
+__device__ __forceinline__ int radius_of_block(const int* blk, int nr, int x) {
+    int lo = 0, hi = nr - 1;  // last r with blk[r] <= x
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (blk[mid] <= x)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
+}
+
+// LDS rounds and tile of the columns and rows bodies, as in k_fused_radius.
+template <int D1, int D2, int W, int N1, int N2, int L>
+struct ColumnTile {
+    using C = LinesCore<N1, N2, L>;
+    static constexpr int D = D1 * D2;
+    static constexpr int kLdsLines = L * C::HP + D + C::WORDS;
+    static constexpr int kRounds = W * (D + 1) > kLdsLines + kLdsLines / 4 ? 0 : 1;
+    static constexpr int kLdsCR = kRounds == 0 ? (W * (D + 1) + 1) / 2 : W * (D + 1);
+};
+
+template <int D1, int D2, int W, int N1, int N2, int L>
+__global__ __launch_bounds__(W* D1) void k_all_columns(AllRadii a, const float2* __restrict__ tw) {
+    using CT = ColumnTile<D1, D2, W, N1, N2, L>;
+    __shared__ float2 lds[CT::kLdsCR];
+    const int x = blockIdx.x;
+    if (x == a.cblk[a.nr]) {  // one more block: thresholds of linear input
+        const int r = threadIdx.x;
+        if (r < a.nr) {
+            ScaledThreshold s;
+            s.scale = 1.0f;
+            s.th = density_threshold(a.deltac, a.r[r].denom, a.zeta, 1.0f);
+            s.pad = 0.0f;
+            a.scaled[r] = s;
+        }
+        return;
+    }
+    const int r = radius_of_block(a.cblk, a.nr, x), i = x - a.cblk[r];
+    const AllRadius& R = a.r[r];
+    columns_body<D1, D2, W, CT::kRounds, true>(a.S, a.T + R.toff, R.ho, tw, R.fp, R.fp.scale, i / R.ncg, i % R.ncg, lds);
+}
+
+template <int D1, int D2, int W, int N1, int N2, int L>
+__global__ __launch_bounds__(W* D1) void k_all_rows(AllRadii a, const float2* __restrict__ tw) {
+    using CT = ColumnTile<D1, D2, W, N1, N2, L>;
+    __shared__ float2 lds[CT::kLdsCR];
+    const int x = blockIdx.x;
+    const int r = radius_of_block(a.rblk, a.nr, x), i = x - a.rblk[r];
+    const AllRadius& R = a.r[r];
+    rows_body<D1, D2, W, CT::kRounds>(a.T + R.toff, R.ho, tw, R.fp, i / R.ncg, i % R.ncg, lds);
+}
+
+template <int N1, int N2, int L>
+__global__ __launch_bounds__(L* N1) void k_all_sums(AllRadii a, const float2* __restrict__ tw) {
+    using C = LinesCore<N1, N2, L>;
+    __shared__ float2 buf[L * C::HP];
+    __shared__ float2 stw[C::D];
+    __shared__ unsigned long long smask[C::WORDS];
+    const int r = blockIdx.y;
+    const AllRadius& R = a.r[r];
+    LineEpilogue ep{};
+    ep.deltac = a.deltac;
+    ep.denom = R.denom;
+    ep.partial = a.partial + (size_t)r * a.nblk;
+    ep.bmax = a.bmax + (size_t)r * a.nblk;
+    lines_block<N1, N2, L, kLineSum>(a.T + R.toff, R.ho, tw, R.fp, ep, blockIdx.x, buf, stw, smask);
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void k_all_reduce(AllRadii a) {
+    const int r = blockIdx.x;
+    const SumScaleArgs sa{a.scaled + r, a.fc_mean, a.deltac, a.r[r].denom, a.ncells, a.zeta, nullptr, nullptr, nullptr};
+    finish_box_sum<NT>(a.partial + (size_t)r * a.nblk, a.nblk, a.sums + r, sa);
+}
+
+template <int N1, int N2, int L>
+__global__ __launch_bounds__(L* N1) void k_all_thresholds(AllRadii a, const float2* __restrict__ tw) {
+    using C = LinesCore<N1, N2, L>;
+    constexpr int D = C::D, NT = C::NT, WORDS = C::WORDS;
+    __shared__ float2 buf[L * C::HP];
+    __shared__ float2 stw[D];
+    __shared__ unsigned long long smask[WORDS];
+    const int t = threadIdx.x, r = blockIdx.y, blk = blockIdx.x;
+    const AllRadius& R = a.r[r];
+    const ScaledThreshold sc = a.scaled[r];
+    unsigned* hit_flag = a.hits + (size_t)r * a.nblk + blk;
+    const size_t line0 = (size_t)blk * L;
+    // no cell of the group can reach the threshold (cells inside the band
+    // take the exact test, so the skip never drops a hit)
+    if (!a.linear && a.bmax[(size_t)r * a.nblk + blk] < sc.th.dstar - sc.th.band) {
+        if (t == 0) *hit_flag = 0u;
+        return;
+    }
+    float2 tmp[C::LOADS];
+    C::load(a.T + R.toff + line0 * R.ho, R.ho, R.fp.cmax + 1, tmp);
+    for (int q = t; q < D; q += NT) stw[q] = tw[q];
+    C::store(tmp, buf);
+    __syncthreads();
+    C::transform(buf, stw, R.fp.cmax + 1);
+    const float* xrf = reinterpret_cast<const float*>(buf);
+    const double inv_zeta = 1.0 / a.zeta;
+    unsigned long long any = 0ull;
+#pragma unroll 4
+    for (int q = 0; q < L * D / NT; ++q) {
+        const int f = t + q * NT;
+        const int i = f / D, c = f - i * D;
+        const unsigned long long bits = __ballot(
+            cell_hit(xrf[i * 2 * C::HP + c], sc.th, a.deltac, R.denom, !a.linear, sc.scale, inv_zeta));
+        if ((t & 63) == 0) smask[f >> 6] = bits;
+        any |= bits;
+    }
+    const bool hit = __syncthreads_or(any != 0ull);
+    if (t == 0) *hit_flag = hit ? 1u : 0u;
+    if (hit && t < WORDS) a.planes[((size_t)r * a.nblk + blk) * WORDS + t] = smask[t];
+}
+
+template <int N1, int N2, int L>
+__global__ __launch_bounds__(L* N1) void k_all_paint(AllRadii a, const float2* __restrict__ tw) {
+    using C = LinesCore<N1, N2, L>;
+    __shared__ float2 buf[L * C::HP];
+    __shared__ float2 stw[C::D];
+    __shared__ unsigned long long smask[C::WORDS];
+    const int t = threadIdx.x, blk = blockIdx.x, last = a.nr - 1;
+    const AllRadius& R = a.r[last];
+    // every wave reads the group's flags at once (last < 64) and ORs the flagged planes
+    const int lane = t & 63;
+    unsigned long long word = 0ull, flags = __ballot(lane < last && a.hits[(size_t)lane * a.nblk + blk]);
+    for (; flags; flags &= flags - 1) {
+        const int r = __ffsll((long long)flags) - 1;
+        if (t < C::WORDS) word |= a.planes[((size_t)r * a.nblk + blk) * C::WORDS + t];
+    }
+    LineEpilogue ep{};
+    ep.deltac = a.deltac;
+    ep.denom = R.denom;
+    ep.zeta = a.zeta;
+    ep.inv_zeta = 1.0 / a.zeta;
+    ep.out = a.out;
+    ep.th = a.scaled[last].th;
+    ep.scaled = a.linear ? nullptr : a.scaled + last;
+    ep.word = word;
+    lines_block<N1, N2, L, kLinePaint>(a.T + R.toff, R.ho, tw, R.fp, ep, blk, buf, stw, smask);
 }
 
 // Pruned r2c of the fused loop (three launches): only the modes that the
@@ -365,14 +525,49 @@ int launch_forward(const float* delta, float2* T0, float2* S, const float2* tw, 
     return CM21_OK;
 }
 
-// D, lines (N1, N2, L), radius (columns/rows D1, D2, W; lines N1, N2, L), forward
+template <int D1, int D2, int W, int N1, int N2, int L>
+int launch_all(const AllRadii& a, const float2* tw, hipStream_t st) {
+    constexpr int NT = W * D1;
+    auto timed = [&](int stage, auto&& launch, const char* name) {
+        const ProfToken t = prof_begin(stage, st);
+        launch();
+        CM21_LAUNCH_CHECK(name);
+        prof_end(t, st);
+        return (int)CM21_OK;
+    };
+    const dim3 groups(a.nblk, a.nr);
+    CM21_TRY(timed(CM21_STAGE_FUSED_COLUMNS, [&] {
+        k_all_columns<D1, D2, W, N1, N2, L><<<a.cblk[a.nr] + (a.linear ? 1 : 0), NT, 0, st>>>(a, tw);
+    }, "k_all_columns"));
+    CM21_TRY(timed(CM21_STAGE_FUSED_ROWS, [&] {
+        k_all_rows<D1, D2, W, N1, N2, L><<<a.rblk[a.nr], NT, 0, st>>>(a, tw);
+    }, "k_all_rows"));
+    if (!a.linear) {
+        CM21_TRY(timed(CM21_STAGE_FCOLL_SUM, [&] { k_all_sums<N1, N2, L><<<groups, NT, 0, st>>>(a, tw); }, "k_all_sums"));
+        k_all_reduce<NT><<<a.nr, NT, 0, st>>>(a);
+        CM21_LAUNCH_CHECK("k_all_reduce");
+    }
+    if (a.nr > 1)
+        CM21_TRY(timed(CM21_STAGE_FUSED_LINES_THRESHOLD, [&] {
+            k_all_thresholds<N1, N2, L><<<dim3(a.nblk, a.nr - 1), NT, 0, st>>>(a, tw);
+        }, "k_all_thresholds"));
+    return timed(CM21_STAGE_FUSED_LINES, [&] { k_all_paint<N1, N2, L><<<a.nblk, NT, 0, st>>>(a, tw); }, "k_all_paint");
+}
+
+// D, all radii, lines (N1, N2, L), radius (columns/rows D1, D2, W; lines N1, N2, L), forward
 const FusedShape kShapes[] = {
-    {64, launch_lines<4, 8, 64>, launch_radius<8, 8, 32, 4, 8, 64>, launch_forward<8, 8, 32, 4, 8, 64>, 32, 64},
-    {96, launch_lines<4, 12, 64>, launch_radius<8, 12, 32, 4, 12, 64>, launch_forward<8, 12, 32, 4, 12, 64>, 32, 64},
-    {128, launch_lines<8, 8, 32>, launch_radius<8, 16, 32, 8, 8, 32>, launch_forward<8, 16, 32, 8, 8, 32>, 32, 32},
-    {160, launch_lines<8, 10, 32>, launch_radius<16, 10, 16, 8, 10, 32>, launch_forward<16, 10, 16, 8, 10, 32>, 16, 32},
-    {256, launch_lines<16, 8, 16>, launch_radius<16, 16, 16, 16, 8, 16>, launch_forward<16, 16, 16, 16, 8, 16>, 16, 16},
-    {512, launch_lines<16, 16, 8>, launch_radius<16, 32, 8, 16, 16, 8>, launch_forward<16, 32, 8, 16, 16, 8>, 8, 8},
+    {64, launch_all<8, 8, 32, 4, 8, 64>, launch_lines<4, 8, 64>,
+     launch_radius<8, 8, 32, 4, 8, 64>, launch_forward<8, 8, 32, 4, 8, 64>, 32, 64},
+    {96, launch_all<8, 12, 32, 4, 12, 64>, launch_lines<4, 12, 64>,
+     launch_radius<8, 12, 32, 4, 12, 64>, launch_forward<8, 12, 32, 4, 12, 64>, 32, 64},
+    {128, launch_all<8, 16, 32, 8, 8, 32>, launch_lines<8, 8, 32>,
+     launch_radius<8, 16, 32, 8, 8, 32>, launch_forward<8, 16, 32, 8, 8, 32>, 32, 32},
+    {160, launch_all<16, 10, 16, 8, 10, 32>, launch_lines<8, 10, 32>,
+     launch_radius<16, 10, 16, 8, 10, 32>, launch_forward<16, 10, 16, 8, 10, 32>, 16, 32},
+    {256, nullptr, launch_lines<16, 8, 16>,
+     launch_radius<16, 16, 16, 16, 8, 16>, launch_forward<16, 16, 16, 16, 8, 16>, 16, 16},
+    {512, nullptr, launch_lines<16, 16, 8>,
+     launch_radius<16, 32, 8, 16, 16, 8>, launch_forward<16, 32, 8, 16, 16, 8>, 8, 8},
 };
 
 const FusedShape* fused_shape(int D) {
@@ -453,6 +648,37 @@ int fused_radius_launch(const FusedShape& sh, const RadiusRoles& a, const float2
     CM21_TRY(sh.radius(a, tw, st));
     prof_end(t, st);
     return CM21_OK;
+}
+
+size_t all_radii_table(const FusedShape& sh, float dk, const float* radii, const float* denoms, int n_radii,
+                       int filter_type, int ref_fallthrough, float scale, AllRadii* a) {
+    if (!sh.all || n_radii > kAllRadii) return 0;
+    const int D = sh.D;
+    size_t off = 0;
+    int nc = 0, nrow = 0;
+    a->nr = n_radii;
+    a->nblk = (int)fused_partials(D);
+    for (int r = 0; r < n_radii; ++r) {
+        AllRadius& R = a->r[r];
+        R.fp = fused_params(D, dk, radii[r], filter_type, ref_fallthrough, scale);
+        R.denom = denoms ? denoms[r] : 0.0f;
+        R.ho = padded_row(std::min(R.fp.cmax, D / 2) + 1);
+        R.toff = off;
+        off += (size_t)D * D * R.ho;
+        int nb = 0;
+        column_groups(sh, R.fp, &R.ncg, &nb);
+        a->cblk[r] = nc;
+        a->rblk[r] = nrow;
+        nc += R.ncg * nb;
+        nrow += R.ncg * D;
+    }
+    a->cblk[n_radii] = nc;
+    a->rblk[n_radii] = nrow;
+    return off;
+}
+
+int fused_all_radii(const FusedShape& sh, const AllRadii& a, const float2* tw, hipStream_t st) {
+    return sh.all(a, tw, st);
 }
 
 int fused_mask_clear(unsigned long long* mask, size_t words, hipStream_t st) {

@@ -51,6 +51,7 @@ struct LineEpilogue {
                                // blocks no cell of which can reach the threshold; or NULL
     DensityThreshold th;       // threshold when `scaled` is NULL (linear input)
     const ScaledThreshold* scaled;  // nonlinear input: scale and threshold of the radius
+    unsigned long long word;   // kLinePaint: the thread's mask word
     const int* active;         // threshold pass: the line groups to visit, or NULL (all)
     const int* nactive;        //   and their number
 };
@@ -92,13 +93,53 @@ struct RadiusRoles {
     LineEpilogue ep_sum;
 };
 
+// The all-radii form of the loop: every role of every radius in one launch
+// each (columns, rows, box sums, reductions, thresholds, paint) instead of one
+// launch per radius.  One entry per radius; up to kAllRadii of them travel as
+// kernel arguments.
+constexpr int kAllRadii = 48;  // (at most 64: the paint reads a group's flags with one ballot)
+struct AllRadius {
+    FusedParams fp;
+    int ho;                   // row stride of the radius' intermediate (padded to 16 modes)
+    unsigned long long toff;  // its offset (float2) in the intermediates
+    float denom;
+    int ncg;                  // column groups of its columns and rows blocks
+};
+struct AllRadii {
+    AllRadius r[kAllRadii];
+    int cblk[kAllRadii + 1];  // first columns / rows block of each radius
+    int rblk[kAllRadii + 1];
+    int nr, nblk;             // radii; line groups of the box
+    int linear;
+    float deltac, fc_mean;
+    double zeta, ncells;
+    float2* S;                   // spectrum, b-major
+    float2* T;                   // intermediates of every radius
+    double* partial;             // [nr][nblk] box-sum partials (nonlinear input)
+    float* bmax;                 // [nr][nblk] line group maxima
+    double* sums;                // [nr]
+    ScaledThreshold* scaled;     // [nr] box-mean scale (1 for linear input) and density threshold
+    unsigned* hits;              // [nr][nblk] whether a line group has a hit at a radius ...
+    unsigned long long* planes;  // [nr][N/64] ... and then its hit bits
+    float* out;
+};
+
 struct FusedShape {
     int D;
+    int (*all)(const AllRadii&, const float2* tw, hipStream_t);
     int (*lines)(int mode, const float2*, const float2*, const FusedParams&, const LineEpilogue&, hipStream_t);
     int (*radius)(const RadiusRoles&, const float2* tw, hipStream_t);
     int (*forward)(const float* delta, float2* T0, float2* S, const float2* tw, const FusedParams& fp, hipStream_t);
     int W, L;  // columns per column group, lines per line group
 };
+
+// Fills the radius table of the all-radii form (T offsets, blocks) and returns
+// the intermediates' size in float2, or 0 when it does not apply: more than
+// kAllRadii radii, or a side beyond 160, whose intermediates outgrow the caches
+// while one launch per radius already fills the chip.
+size_t all_radii_table(const FusedShape& sh, float dk, const float* radii, const float* denoms, int n_radii,
+                       int filter_type, int ref_fallthrough, float scale, AllRadii* a);
+int fused_all_radii(const FusedShape& sh, const AllRadii& a, const float2* tw, hipStream_t st);
 
 const FusedShape* fused_shape(int D);
 size_t fused_partials(int D);

@@ -22,7 +22,7 @@
 
 namespace cm21 {
 
-enum LineMode { kLineSum = 0, kLineThreshold = 1, kLineFinal = 2 };
+enum LineMode { kLineSum = 0, kLineThreshold = 1, kLineFinal = 2, kLinePaint = 3 };
 
 // Window of one mode from its integer |n|^2.  Inside the shell m2 >= m2lo the
 // reference's float32 cut test decides (find_bubbles.cu:22-35); the Gaussian
