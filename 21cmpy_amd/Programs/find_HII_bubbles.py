@@ -51,29 +51,33 @@ def radius_schedule(box_len, hii_dim, py2_int_scale=False, r_max=None, r_min=Non
         scale = float(cell)
     else:
         scale = (int(box_len) // int(hii_dim)) if py2_int_scale else float(box_len) / float(hii_dim)
-    R = float(r_max)
+    return np.array(_radii(float(r_max), r_min, fac, lf * scale), dtype=np.float32), scale
+
+
+@functools.lru_cache(maxsize=256)
+def _radii(R, r_min, fac, r_cell):
+    """The radii of radius_schedule: they depend on these four numbers alone."""
     radii = []
     while True:
-        final = (R / fac) <= lf * scale or (R / fac) <= r_min
-        R32 = np.float32(R)
+        final = (R / fac) <= r_cell or (R / fac) <= r_min
+        R32 = float(np.float32(R))
         radii.append(R32)
         if final:
-            break
-        R = float(R32) / fac
-    return np.array(radii, dtype=np.float32), scale
+            return tuple(radii)
+        R = R32 / fac
 
 
 def barrier_denominators(radii, sigma_min2, sig0_fn):
     """denom = float32(sqrt(2 (smin - float32(S(R))))) per radius
     (find_HII_bubbles.py:126-128); raises ValueError where smin <= S(R)."""
-    out = np.empty(len(radii), dtype=np.float32)
-    for i, R in enumerate(radii):
-        S0 = np.float32(sig0_fn(float(R)))
-        arg = 2.0 * (float(sigma_min2) - float(S0))
-        if not arg > 0.0:
-            raise ValueError(f"sigma_min^2={sigma_min2} <= S(R={float(R)})={float(S0)}: no barrier at this radius")
-        out[i] = np.float32(math.sqrt(arg))
-    return out
+    S0 = np.array([sig0_fn(R) for R in np.asarray(radii, dtype=np.float64).tolist()], dtype=np.float64)
+    S0 = S0.astype(np.float32).astype(np.float64)
+    arg = 2.0 * (float(sigma_min2) - S0)
+    bad = np.flatnonzero(~(arg > 0.0))
+    if bad.size:
+        i = int(bad[0])
+        raise ValueError(f"sigma_min^2={sigma_min2} <= S(R={float(radii[i])})={S0[i]}: no barrier at this radius")
+    return np.sqrt(arg).astype(np.float32)
 
 
 @functools.lru_cache(maxsize=16)
