@@ -234,15 +234,25 @@ extern "C" int cm21_update_sphere(float* ionized, const float* smoothed, int D, 
 
 // Workspace carve-up of the loop driver.
 namespace {
-// Pipelined fused loop: radius r uses intermediate r % kInter and the small
-// per-radius buffers r % kSlots; a launch touches radii r-2 .. r+2.
-constexpr int kInter = 5, kSlots = 3;
+// Pipelined fused loop: a radius uses one of loop_inter(D) intermediates in
+// turn and the small per-radius buffers r % kSlots; a launch touches radii
+// r-2 .. r+3.
+// From side 256 on the columns and rows of the first radii (neutral_radii: where
+// the bound of the rows pass may tell that the box stays neutral) run one launch
+// further ahead, so that the launch between the rows and the box sums of a
+// radius can decide it: one more intermediate, only then used.  Deciding
+// it in every box-sum block instead cost 5 us of each 31 us launch at 256^3;
+// running every radius ahead cost 3 to 8 % there, its intermediates outliving
+// the caches.  (Smaller sides take this loop only with the least workspace.)
+constexpr int kInterMax = 6, kSlots = 3;
+constexpr int kRowBounds = 4;  // bounds per plane (kBoundGroups of the rows pass)
+constexpr int loop_inter(int D) { return D >= 256 ? 6 : 5; }
 
 struct LoopWork {
     float2* spec;
     float2* filt;             // generic path: filtered spectrum
     float* smoothed;          // generic path: smoothed box
-    float2* inter[kInter];    // fused path: intermediates (inter[0] is filt,
+    float2* inter[kInterMax]; // fused path: intermediates (inter[0] is filt,
                               // inter[1] shares smoothed's region)
     double* partial;
     double* sums;
@@ -252,6 +262,7 @@ struct LoopWork {
     float* bmax[kSlots];      // per line group maxima
     int* active[kSlots];      // line groups the threshold pass visits, and their number
     int* nactive[kSlots];
+    float* bound[kSlots];     // bounds of the rows pass
     ScaledThreshold* scaled;  // per radius
     size_t bytes;
 };
@@ -273,8 +284,8 @@ LoopWork carve(void* base, int D, int n_radii, int update) {
     w.smoothed = (float*)(p + off);
     w.inter[1] = (float2*)(p + off);
     off = align_up(off + std::max(sizeof(float) * N, sizeof(float2) * Nt), 256);
-    // the fused path (update == 0 only) needs three more intermediates
-    for (int k = 2; k < kInter && !update; ++k) {
+    // the fused path (update == 0 only) needs three or four more intermediates
+    for (int k = 2; k < loop_inter(D) && !update; ++k) {
         w.inter[k] = (float2*)(p + off);
         off = align_up(off + sizeof(float2) * Nt, 256);
     }
@@ -295,6 +306,8 @@ LoopWork carve(void* base, int D, int n_radii, int update) {
         off = align_up(off + sizeof(int) * (fused_partials(D) + 1), 256);
         w.nactive[k] = (int*)(p + off);
         off = align_up(off + sizeof(int), 256);
+        w.bound[k] = (float*)(p + off);
+        off = align_up(off + sizeof(float) * kRowBounds * D, 256);
     }
     w.scaled = (ScaledThreshold*)(p + off);
     off = align_up(off + sizeof(ScaledThreshold) * (size_t)(n_radii > 0 ? n_radii : 1), 256);
@@ -342,6 +355,7 @@ AllWork carve_all(void* base, int D, const float* radii, const float* denoms, in
     // the forward transform passes through the intermediates' region
     a.T = (float2*)take(sizeof(float2) * std::max(nt, row));
     a.sums = (double*)take(sizeof(double) * n_radii);
+    a.bound = (float*)take(sizeof(float) * kRowBounds * D * n_radii);
     a.scaled = (ScaledThreshold*)take(sizeof(ScaledThreshold) * n_radii);
     a.hits = (unsigned*)take(sizeof(unsigned) * cells);
     a.planes = (unsigned long long*)take(sizeof(unsigned long long) * n_radii * (N / 64));
@@ -424,7 +438,7 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
     if (loop_is_fused(sh, prm)) {
         const float2* tw = plan_twiddles(plan);
         // the forward transform forms only the modes the widest window keeps,
-        // through the intermediate that radius 4 uses first
+        // through the intermediate that is used last
         FusedParams widest = fused_params(D, dk, radii[0], prm->filter_type, prm->ref_fallthrough, scale);
         for (int r = 1; r < n_radii; ++r) {
             const FusedParams f = fused_params(D, dk, radii[r], prm->filter_type, prm->ref_fallthrough, scale);
@@ -443,9 +457,9 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
             CM21_TRY(fused_forward(*sh, delta, a.T, a.S, tw, widest, st));
             return fused_all_radii(*sh, a, tw, st);
         }
-        CM21_TRY(fused_forward(*sh, delta, w.inter[kInter - 1], w.spec, tw, widest, st));
+        CM21_TRY(fused_forward(*sh, delta, w.inter[4], w.spec, tw, widest, st));
         CM21_TRY(fused_mask_clear(w.mask, (N + 63) / 64, st));
-        // One launch per radius on the caller's stream, each with up to five
+        // One launch per radius on the caller's stream, each with up to six
         // independent roles over neighbouring radii (k_fused_radius): launch
         // j holds the columns pass of radius j+2, the rows pass of radius j+1,
         // the box-sum pass of radius j, the box-sum reduction of radius j-1
@@ -463,76 +477,127 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
         auto params = [&](int r) {
             return fused_params(D, dk, radii[r], prm->filter_type, prm->ref_fallthrough, scale);
         };
-        auto threshold_epilogue = [&](int r) {
-            const int q = r % kSlots;
-            LineEpilogue e = line_epilogue(prm->deltac, denoms[r], prm->zeta, nl ? w.sums + r : nullptr,
-                                           prm->fc_mean, w.mask, ionized, w.lpart[q], (double)N,
-                                           nl ? w.bmax[q] : nullptr);
-            if (nl) {
-                e.scaled = w.scaled + r;
-                if (r < n_radii - 1) {
-                    e.active = w.active[q];
-                    e.nactive = w.nactive[q];
-                }
-            } else {
-                e.th = density_threshold_host(prm->deltac, denoms[r], prm->zeta, 1.0f);
-            }
-            return e;
-        };
+        std::vector<DensityThreshold> linear_th(nl ? 0 : n_radii);
+        for (size_t r = 0; r < linear_th.size(); ++r)
+            linear_th[r] = density_threshold_host(prm->deltac, denoms[r], prm->zeta, 1.0f);
         const int last = n_radii - 1;
+        // radii 0 .. ahead-1 run their columns and rows one launch further
+        // ahead and get a verdict (never the last radius, which is painted)
+        int ahead = 0;
+        if (D >= 256) {
+            std::vector<int> cmax(n_radii);
+            for (int r = 0; r < n_radii; ++r) cmax[r] = params(r).cmax;
+            ahead = neutral_radii(*prm, denoms, n_radii, cmax.data());
+        }
+        // the intermediate of each radius: a ring of six while radii run
+        // ahead, of five afterwards (the fewer, the more of them stay cached)
+        std::vector<int> inter_of(n_radii);
+        for (int r = 0; r < n_radii; ++r)
+            inter_of[r] = ahead > 0 && r <= ahead ? r % kInterMax : (r >= 5 ? inter_of[r - 5] : r);
+        auto inter = [&](int r) { return w.inter[inter_of[r]]; };
+        auto col_launch = [&](int r) { return r - (r < ahead ? 3 : 2); };
+        auto row_launch = [&](int r) { return r - (r < ahead ? 2 : 1); };
+        // the radius whose pass falls into launch j, or -1
+        auto radius_in = [&](auto&& launch_of, int j, int d) {
+            for (int r = j + d; r <= j + d + 1; ++r)
+                if (r >= 0 && r <= last && launch_of(r) == j) return r;
+            return -1;
+        };
         // launches j = -2 .. j_end-1: the last one holds the reduction of the
         // last radius and the threshold pass of the one before (nonlinear), or
         // the threshold pass of the radius before the last (linear)
         const int j_end = nl ? n_radii + 1 : n_radii - 1;
-        for (int j = -2; j < j_end; ++j) {
+        for (int j = ahead > 0 ? -3 : -2; j < j_end; ++j) {
             RadiusRoles a{};
-            if (j + 2 <= last) {
-                const int r = j + 2;
+            AskRoles q{};
+            a.deltac = prm->deltac;
+            a.zeta = prm->zeta;
+            if (const int r = radius_in(col_launch, j, 2); r >= 0) {
                 a.S = w.spec;
-                a.Tcols = w.inter[r % kInter];
+                a.Tcols = inter(r);
                 a.fp_cols = params(r);
                 int nb = 0;
                 column_groups(*sh, a.fp_cols, &a.ncg_cols, &nb);
                 a.n_cols = a.ncg_cols * nb;
             }
             a.n_mem = a.n_cols;
-            if (j + 1 >= 0 && j + 1 <= last) {
-                const int r = j + 1;
-                a.Trows = w.inter[r % kInter];
-                a.fp_rows = params(r);
+            if (const int r = radius_in(row_launch, j, 1); r >= 0) {
+                a.Trows = inter(r);
+                const FusedParams fp = params(r);
+                a.m2max_rows = fp.m2max;
+                a.cmax_rows = fp.cmax;
                 int nb = 0;
-                column_groups(*sh, a.fp_rows, &a.ncg_rows, &nb);
+                column_groups(*sh, fp, &a.ncg_rows, &nb);
                 a.n_mem += a.ncg_rows * D;
+                q.bound_rows = r < ahead && a.ncg_rows <= kRowBounds ? w.bound[r % kSlots] : nullptr;
+            }
+            if (j + 1 >= 0 && j + 1 < ahead) {
+                const int r = j + 1;
+                const FusedParams fp = params(r);
+                int ncg = 0, nb = 0;
+                column_groups(*sh, fp, &ncg, &nb);
+                q.n_ver = 1;
+                q.skip.bound = ncg <= kRowBounds ? w.bound[r % kSlots] : nullptr;
+                q.skip.S0 = w.spec;
+                q.skip.groups = ncg;
+                q.skip.linear = nl ? 0 : 1;
+                q.skip.deltac = prm->deltac;
+                q.skip.zeta_fc_mean = (float)(prm->zeta * (double)prm->fc_mean);
+                if (!nl) q.skip.th = linear_th[r];
+                q.skip_scale = fp.scale;
+                q.skip_denom = denoms[r];
+                q.verdict = w.scaled + r;
             }
             if (nl && j - 1 >= 0 && j - 1 <= last) {
-                const int r = j - 1, q = r % kSlots;
-                a.partial = w.lpart[q];
-                a.npart = nblk;
+                const int r = j - 1, s = r % kSlots;
+                a.partial = w.lpart[s];
                 a.total = w.sums + r;
-                a.sa = SumScaleArgs{w.scaled + r, prm->fc_mean, prm->deltac, denoms[r], (double)N, prm->zeta,
-                                    w.bmax[q], r < last ? w.active[q] : nullptr, r < last ? w.nactive[q] : nullptr};
+                a.scaled_red = w.scaled + r;
+                a.fc_mean = prm->fc_mean;
+                a.denom_red = denoms[r];
+                a.bmax_red = w.bmax[s];
+                a.active_red = r < last ? w.active[s] : nullptr;
+                a.nactive_red = r < last ? w.nactive[s] : nullptr;
+                if (r < ahead) q.state_red = w.scaled + r;
                 a.n_red = 1;
             }
             const int rt = nl ? j - 2 : j;  // the threshold pass (the last radius is painted below)
             if (rt >= 0 && rt < last) {
-                a.Uthr = w.inter[rt % kInter];
-                a.fp_thr = params(rt);
-                a.ep_thr = threshold_epilogue(rt);
+                a.Uthr = inter(rt);
+                a.cmax_thr = params(rt).cmax;
+                a.denom_thr = denoms[rt];
+                a.mask = w.mask;
+                if (nl) {
+                    a.scaled_thr = w.scaled + rt;
+                    a.bmax_thr = w.bmax[rt % kSlots];
+                    a.active_thr = w.active[rt % kSlots];
+                    a.nactive_thr = w.nactive[rt % kSlots];
+                } else {
+                    a.th = linear_th[rt];
+                }
                 a.n_thr = nblk;
+                if (!nl && rt < ahead) q.state_thr = w.scaled + rt;
             }
             if (nl && j >= 0 && j <= last) {
-                const int r = j, q = r % kSlots;
-                a.Usum = w.inter[r % kInter];
-                a.fp_sum = params(r);
-                a.ep_sum = line_epilogue(prm->deltac, denoms[r], prm->zeta, nullptr, prm->fc_mean, w.mask, ionized,
-                                         w.lpart[q], (double)N, w.bmax[q]);
+                const int r = j, s = r % kSlots;
+                a.Usum = inter(r);
+                a.cmax_sum = params(r).cmax;
+                a.denom_sum = denoms[r];
+                a.partial_sum = w.lpart[s];
+                a.bmax_sum = w.bmax[s];
+                if (r < ahead) q.state_sum = w.scaled + r;
                 a.n_sum = nblk;
             }
-            CM21_TRY(fused_radius_launch(*sh, a, tw, st));
+            q.any = q.n_ver || q.bound_rows || q.state_thr || q.state_sum || q.state_red;
+            CM21_TRY(fused_radius_launch(*sh, a, q, tw, st));
         }
         // mode 2: the final paint of the last radius
-        CM21_TRY(fused_lines(*sh, 2, w.inter[last % kInter], tw, params(last), threshold_epilogue(last), st,
-                             CM21_STAGE_FUSED_LINES_THRESHOLD));
+        LineEpilogue e = line_epilogue(prm->deltac, denoms[last], prm->zeta, w.mask, ionized);
+        if (nl)
+            e.scaled = w.scaled + last;
+        else
+            e.th = linear_th[last];
+        CM21_TRY(fused_lines(*sh, inter(last), tw, params(last), e, st, CM21_STAGE_FUSED_LINES_THRESHOLD));
         return CM21_OK;
     }
     {

@@ -38,8 +38,14 @@ namespace cm21 {
 // `active` the block lists the line groups whose maximum is not below
 // d* - band (the order of the list does not matter: each group writes only
 // its own mask words).
+// A radius at which no cell can be ionized has no box sums: its list is empty.
 template <int NT>
-__device__ void finish_box_sum(const double* partial, int n, double* out, const SumScaleArgs& sa) {
+__device__ void finish_box_sum(const double* partial, int n, double* out, const SumScaleArgs& sa,
+                               const ScaledThreshold* state = nullptr) {
+    if (state && state->neutral) {
+        if (threadIdx.x == 0 && sa.active) *sa.nactive = 0;
+        return;
+    }
     __shared__ double part[NT / 64];
     __shared__ DensityThreshold sth;
     __shared__ int count;
@@ -57,7 +63,7 @@ __device__ void finish_box_sum(const double* partial, int n, double* out, const 
             ScaledThreshold s;
             s.scale = scale;
             s.th = density_threshold(sa.deltac, sa.denom, sa.zeta, scale);
-            s.pad = 0.0f;
+            s.neutral = 0;
             *sa.scaled = s;
             sth = s.th;
         }
@@ -86,11 +92,11 @@ __device__ void finish_box_sum(const double* partial, int n, double* out, const 
 // final-paint block whose cells are all ionized writes 1 without transforming.
 // `blk` is the index of the L-line group the block works on.
 // `hs` is the line stride of U.  kLinePaint is kLineFinal with the block's mask
-// words in ep.word (thread t holds word t) instead of ep.mask.
+// words in `word` (thread t holds word t) instead of ep.mask.
 template <int N1, int N2, int L, int MODE_>
 __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs, const float2* __restrict__ tw,
-                                            const FusedParams& fp, const LineEpilogue& ep, int blk, float2* buf,
-                                            float2* stw, unsigned long long* smask) {
+                                            int cmax, const LineEpilogue& ep, int blk, float2* buf,
+                                            float2* stw, unsigned long long* smask, unsigned long long word = 0ull) {
     using C = LinesCore<N1, N2, L>;
     constexpr int D = C::D, NT = C::NT, WORDS = C::WORDS;
     constexpr int MODE = MODE_ == kLinePaint ? (int)kLineFinal : MODE_;
@@ -108,7 +114,7 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
             scale = s.scale;
             th = s.th;
         }
-        mword = t < WORDS ? (MODE_ == kLinePaint ? ep.word : ep.mask[word0 + t]) : ~0ull;
+        mword = t < WORDS ? (MODE_ == kLinePaint ? word : ep.mask[word0 + t]) : ~0ull;
         const bool all_ionized = __syncthreads_and(mword == ~0ull);
         if (all_ionized) {
             if (MODE == kLineFinal)
@@ -119,12 +125,12 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
     }
     // all global loads in flight before the first LDS store
     float2 tmp[C::LOADS];
-    C::load(U + line0 * hs, hs, fp.cmax + 1, tmp);
+    C::load(U + line0 * hs, hs, cmax + 1, tmp);
     for (int q = t; q < D; q += NT) stw[q] = tw[q];
     C::store(tmp, buf);
     if (MODE != kLineSum && t < WORDS) smask[t] = mword;
     __syncthreads();
-    C::transform(buf, stw, fp.cmax + 1);
+    C::transform(buf, stw, cmax + 1);
     double acc = 0.0;
     float vmax = -INFINITY;
     const int lane = t & 63;
@@ -144,12 +150,12 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
             vmax = fmaxf(vmax, delta);
         } else {
             const bool hit = cell_hit(delta, th, ep.deltac, ep.denom, use_scale, scale, ep.inv_zeta);
-            const unsigned long long word = smask[f >> 6];
+            const unsigned long long old = smask[f >> 6];
             if (MODE == kLineThreshold) {
                 const unsigned long long bits = __ballot(hit);
-                if (lane == 0) smask[f >> 6] = word | bits;
+                if (lane == 0) smask[f >> 6] = old | bits;
             } else {
-                const bool was = (word >> (f & 63)) & 1ull;
+                const bool was = (old >> (f & 63)) & 1ull;
                 float val = 1.0f;
                 if (!was && !hit) val = final_value(delta, ep.deltac, ep.denom, use_scale, scale, ep.zeta, ep.inv_zeta);
                 ep.out[cell0 + f] = val;
@@ -179,34 +185,29 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
     }
 }
 
-// With an active list (threshold pass after a box sum) block b works on the
-// b-th listed line group and the blocks past the end of the list return at
-// once, so line groups that cannot change cost one scalar load each and the
-// groups that can are spread over the first blocks of the dispatch;
-// otherwise block b works on line group b.
-template <int N1, int N2, int L, int MODE>
+// The final paint of the loop with a launch per radius.
+template <int N1, int N2, int L>
 __global__ __launch_bounds__(L* N1) void k_fused_lines(const float2* __restrict__ U, const float2* __restrict__ tw,
-                                                      FusedParams fp, LineEpilogue ep) {
+                                                      int cmax, LineEpilogue ep) {
     using C = LinesCore<N1, N2, L>;
     __shared__ float2 buf[L * C::HP];
     __shared__ float2 stw[C::D];
     __shared__ unsigned long long smask[C::WORDS];
-    int blk = blockIdx.x;
-    if (MODE == kLineThreshold && ep.active != nullptr) {
-        if (blk >= *ep.nactive) return;
-        blk = ep.active[blk];
-    }
-    lines_block<N1, N2, L, MODE>(U, C::HO, tw, fp, ep, blk, buf, stw, smask);
+    lines_block<N1, N2, L, kLineFinal>(U, C::HO, tw, cmax, ep, blockIdx.x, buf, stw, smask);
 }
 
-// One launch of the pipelined radius loop.  Its blocks take one of five
+// One launch of the pipelined radius loop.  Its blocks take one of six
 // roles: the columns pass of radius r+2 and the rows pass of radius r+1 (into
-// intermediates no other role of the launch touches), the one-block box-sum
-// reduction of radius r-1 (scale, threshold and active list), the threshold
-// pass of radius r-2 and the box-sum pass of radius r.  Every role reads only
-// what earlier launches wrote and writes buffers no other role of the launch
-// reads or writes, so the roles need no ordering among themselves; in-order
-// launches on one stream order the radii.
+// intermediates no other role of the launch touches; r+3 and r+2 for the
+// first radii), the one-block box-sum reduction of radius r-1 (scale,
+// threshold and active list), the one-block verdict whether the box stays
+// neutral at radius r+1 (the first radii), the threshold pass of radius r-2
+// and the box-sum pass of radius r.  A radius without a cell to ionize costs 10
+// us at 256^3 instead of 31 (box sums, nonlinear) and 25 us at 512^3 instead of
+// 220 (thresholds, linear).  Every role reads only what earlier launches wrote
+// and writes buffers no other role of the launch reads or writes, so the roles
+// need no ordering among themselves; in-order launches on one stream order the
+// radii.
 // Block order: the reduction, then for nonlinear input the box-sum blocks,
 // the columns/rows blocks and the threshold blocks (block i of these takes
 // the i-th listed line group; those past the end of the list return at
@@ -220,8 +221,10 @@ __global__ __launch_bounds__(L* N1) void k_fused_lines(const float2* __restrict_
 // The kernel asks for eight waves per SIMD, the box-sum role's full
 // occupancy (about 52 VGPRs, 19.5 KB of LDS at D = 256); the columns/rows
 // roles fit it without spilling through the re/im-staged transpose.
-template <int D1, int D2, int W, int N1, int N2, int L>
-__global__ __launch_bounds__(W* D1, 8) void k_fused_radius(RadiusRoles a, const float2* __restrict__ tw) {
+// ASK: the launch has a verdict, bounds or states to look at (launches of the
+// first radii); without it the kernel carries none of that.
+template <int D1, int D2, int W, int N1, int N2, int L, bool ASK>
+__device__ __forceinline__ void radius_roles(const RadiusRoles& a, const AskRoles& q, const float2* __restrict__ tw) {
     using C = LinesCore<N1, N2, L>;
     constexpr int D = D1 * D2, NT = W * D1;
     static_assert(C::D == D && C::NT == NT, "columns/rows and lines tiles must share D and the block size");
@@ -237,34 +240,71 @@ __global__ __launch_bounds__(W* D1, 8) void k_fused_radius(RadiusRoles a, const 
     unsigned long long* smask = reinterpret_cast<unsigned long long*>(lds + L * C::HP + D);
     int b = blockIdx.x;
     if (b < a.n_red) {
-        finish_box_sum<NT>(a.partial, a.npart, a.total, a.sa);
+        const SumScaleArgs sa{a.scaled_red,   a.fc_mean,    a.deltac,     a.denom_red,    (double)D * D * D,
+                              a.zeta,         a.bmax_red,   a.active_red, a.nactive_red};
+        finish_box_sum<NT>(a.partial, D * D / L, a.total, sa, ASK ? q.state_red : nullptr);
         return;
     }
     b -= a.n_red;
+    if (ASK && b < q.n_ver) {
+        const bool neutral = box_stays_neutral<NT, D>(q.skip, q.skip_scale, q.skip_denom);
+        if (threadIdx.x == 0) q.verdict->neutral = neutral ? 1 : 0;
+        return;
+    }
+    if (ASK) b -= q.n_ver;
     // nonlinear input: box sums, transposes, thresholds; linear input (no
     // box sums): thresholds, transposes
     const int thr0 = a.n_sum > 0 ? a.n_sum + a.n_mem : 0;
     if (b >= thr0 && b < thr0 + a.n_thr) {
         b -= thr0;
-        if (a.ep_thr.active != nullptr) {
-            if (b >= *a.ep_thr.nactive) return;
-            b = a.ep_thr.active[b];
+        if (a.active_thr != nullptr) {
+            if (b >= *a.nactive_thr) return;
+            b = a.active_thr[b];
         }
-        lines_block<N1, N2, L, kLineThreshold>(a.Uthr, C::HO, tw, a.fp_thr, a.ep_thr, b, buf, stw, smask);
+        if (ASK && q.state_thr && q.state_thr->neutral) return;
+        LineEpilogue ep{};
+        ep.deltac = a.deltac;
+        ep.denom = a.denom_thr;
+        ep.inv_zeta = 1.0 / a.zeta;
+        ep.mask = a.mask;
+        ep.bmax = const_cast<float*>(a.bmax_thr);
+        ep.th = a.th;
+        ep.scaled = a.scaled_thr;
+        lines_block<N1, N2, L, kLineThreshold>(a.Uthr, C::HO, tw, a.cmax_thr, ep, b, buf, stw, smask);
         return;
     }
     if (b >= thr0 + a.n_thr) b -= a.n_thr;
     const bool mem = b >= a.n_sum;
     int i = mem ? b - a.n_sum : b;
     if (!mem) {
-        lines_block<N1, N2, L, kLineSum>(a.Usum, C::HO, tw, a.fp_sum, a.ep_sum, i, buf, stw, smask);
+        if (ASK && q.state_sum && q.state_sum->neutral) return;
+        LineEpilogue ep{};
+        ep.deltac = a.deltac;
+        ep.denom = a.denom_sum;
+        ep.partial = a.partial_sum;
+        ep.bmax = a.bmax_sum;
+        lines_block<N1, N2, L, kLineSum>(a.Usum, C::HO, tw, a.cmax_sum, ep, i, buf, stw, smask);
     } else if (i < a.n_cols) {
         columns_body<D1, D2, W, kRounds, true>(a.S, a.Tcols, C::HO, tw, a.fp_cols, a.fp_cols.scale, i / a.ncg_cols,
                                 i % a.ncg_cols, lds);
     } else {
         i -= a.n_cols;
-        rows_body<D1, D2, W, kRounds>(a.Trows, C::HO, tw, a.fp_rows, i / a.ncg_rows, i % a.ncg_rows, lds);
+        FusedParams fp{};
+        fp.m2max = a.m2max_rows;
+        fp.cmax = a.cmax_rows;
+        rows_body<D1, D2, W, kRounds>(a.Trows, C::HO, tw, fp, i / a.ncg_rows, i % a.ncg_rows, lds,
+                                      ASK ? q.bound_rows : nullptr);
     }
+}
+
+template <int D1, int D2, int W, int N1, int N2, int L>
+__global__ __launch_bounds__(W* D1, 8) void k_fused_radius(RadiusRoles a, const float2* __restrict__ tw) {
+    radius_roles<D1, D2, W, N1, N2, L, false>(a, AskRoles{}, tw);
+}
+template <int D1, int D2, int W, int N1, int N2, int L>
+__global__ __launch_bounds__(W* D1, 8) void k_fused_radius_ask(RadiusRoles a, AskRoles q,
+                                                              const float2* __restrict__ tw) {
+    radius_roles<D1, D2, W, N1, N2, L, true>(a, q, tw);
 }
 
 // ------------------------------------------------------------------ all radii at once
@@ -276,10 +316,11 @@ __global__ __launch_bounds__(W* D1, 8) void k_fused_radius(RadiusRoles a, const 
 // the results are those of the launch per radius bit for bit.  What the loop
 // orders, the ionization mask, becomes one bit plane per radius: a group's
 // threshold block writes its hits where it has any, and the paint ORs the
-// flagged planes.  The thresholds of linear input are found by the columns
-// launch (one more block) instead of on the host.
-// A call of conv_bubbles takes 75 us at 64^3 (linear, 37 radii; 279 before)
-// and 247 us at 128^3 (nonlinear, 40 radii; 463), 130 of them the box sums.
+// flagged planes.  The thresholds of linear input are found on the device with
+// the verdicts on whole radii (box_stays_neutral).
+// A call of conv_bubbles takes 65 us at 64^3 (linear, 37 radii; 279 with a
+// launch per radius) and 210 us at 128^3 (nonlinear, 40 radii; 463), 90 of them
+// the box sums (VALU-bound; 130 without the verdicts).
 __device__ __forceinline__ int radius_of_block(const int* blk, int nr, int x) {
     int lo = 0, hi = nr - 1;  // last r with blk[r] <= x
     while (lo < hi) {
@@ -307,20 +348,13 @@ __global__ __launch_bounds__(W* D1) void k_all_columns(AllRadii a, const float2*
     using CT = ColumnTile<D1, D2, W, N1, N2, L>;
     __shared__ float2 lds[CT::kLdsCR];
     const int x = blockIdx.x;
-    if (x == a.cblk[a.nr]) {  // one more block: thresholds of linear input
-        const int r = threadIdx.x;
-        if (r < a.nr) {
-            ScaledThreshold s;
-            s.scale = 1.0f;
-            s.th = density_threshold(a.deltac, a.r[r].denom, a.zeta, 1.0f);
-            s.pad = 0.0f;
-            a.scaled[r] = s;
-        }
-        return;
-    }
     const int r = radius_of_block(a.cblk, a.nr, x), i = x - a.cblk[r];
     const AllRadius& R = a.r[r];
     columns_body<D1, D2, W, CT::kRounds, true>(a.S, a.T + R.toff, R.ho, tw, R.fp, R.fp.scale, i / R.ncg, i % R.ncg, lds);
+}
+
+__device__ __forceinline__ bool bounded(const AllRadius& R) {
+    return R.fp.cmax < kBoundModes && R.ncg <= kBoundGroups;
 }
 
 template <int D1, int D2, int W, int N1, int N2, int L>
@@ -330,7 +364,31 @@ __global__ __launch_bounds__(W* D1) void k_all_rows(AllRadii a, const float2* __
     const int x = blockIdx.x;
     const int r = radius_of_block(a.rblk, a.nr, x), i = x - a.rblk[r];
     const AllRadius& R = a.r[r];
-    rows_body<D1, D2, W, CT::kRounds>(a.T + R.toff, R.ho, tw, R.fp, i / R.ncg, i % R.ncg, lds);
+    rows_body<D1, D2, W, CT::kRounds>(a.T + R.toff, R.ho, tw, R.fp, i / R.ncg, i % R.ncg, lds,
+                                      bounded(R) ? a.bound + (size_t)r * CT::D * kBoundGroups : nullptr);
+}
+
+// One block per radius: the threshold of linear input, and whether the box
+// stays neutral there (never asked of the last radius, which is painted).
+template <int NT, int D>
+__global__ __launch_bounds__(NT) void k_all_verdicts(AllRadii a) {
+    const int r = blockIdx.x;
+    const AllRadius& R = a.r[r];
+    SkipArgs sk{};
+    ScaledThreshold s{};
+    s.scale = 1.0f;
+    if (a.linear) s.th = density_threshold(a.deltac, R.denom, a.zeta, 1.0f);
+    if (r < a.nr - 1 && bounded(R)) {
+        sk.bound = a.bound + (size_t)r * D * kBoundGroups;
+        sk.S0 = a.S;
+        sk.groups = R.ncg;
+        sk.linear = a.linear;
+        sk.deltac = a.deltac;
+        sk.zeta_fc_mean = (float)(a.zeta * (double)a.fc_mean);
+        sk.th = s.th;
+    }
+    s.neutral = box_stays_neutral<NT, D>(sk, R.fp.scale, R.denom) ? 1 : 0;
+    if (threadIdx.x == 0) a.scaled[r] = s;
 }
 
 template <int N1, int N2, int L>
@@ -341,19 +399,21 @@ __global__ __launch_bounds__(L* N1) void k_all_sums(AllRadii a, const float2* __
     __shared__ unsigned long long smask[C::WORDS];
     const int r = blockIdx.y;
     const AllRadius& R = a.r[r];
+    if (a.scaled[r].neutral) return;
     LineEpilogue ep{};
     ep.deltac = a.deltac;
     ep.denom = R.denom;
     ep.partial = a.partial + (size_t)r * a.nblk;
     ep.bmax = a.bmax + (size_t)r * a.nblk;
-    lines_block<N1, N2, L, kLineSum>(a.T + R.toff, R.ho, tw, R.fp, ep, blockIdx.x, buf, stw, smask);
+    lines_block<N1, N2, L, kLineSum>(a.T + R.toff, R.ho, tw, R.fp.cmax, ep, blockIdx.x, buf, stw, smask);
 }
 
 template <int NT>
 __global__ __launch_bounds__(NT) void k_all_reduce(AllRadii a) {
     const int r = blockIdx.x;
-    const SumScaleArgs sa{a.scaled + r, a.fc_mean, a.deltac, a.r[r].denom, a.ncells, a.zeta, nullptr, nullptr, nullptr};
-    finish_box_sum<NT>(a.partial + (size_t)r * a.nblk, a.nblk, a.sums + r, sa);
+    const SumScaleArgs sa{a.scaled + r, a.fc_mean, a.deltac, a.r[r].denom, a.ncells, a.zeta,
+                          nullptr,      nullptr,   nullptr};
+    finish_box_sum<NT>(a.partial + (size_t)r * a.nblk, a.nblk, a.sums + r, sa, a.scaled + r);
 }
 
 template <int N1, int N2, int L>
@@ -370,7 +430,9 @@ __global__ __launch_bounds__(L* N1) void k_all_thresholds(AllRadii a, const floa
     const size_t line0 = (size_t)blk * L;
     // no cell of the group can reach the threshold (cells inside the band
     // take the exact test, so the skip never drops a hit)
-    if (!a.linear && a.bmax[(size_t)r * a.nblk + blk] < sc.th.dstar - sc.th.band) {
+    const bool none =
+        sc.neutral || (!a.linear && a.bmax[(size_t)r * a.nblk + blk] < sc.th.dstar - sc.th.band);
+    if (none) {
         if (t == 0) *hit_flag = 0u;
         return;
     }
@@ -420,8 +482,7 @@ __global__ __launch_bounds__(L* N1) void k_all_paint(AllRadii a, const float2* _
     ep.out = a.out;
     ep.th = a.scaled[last].th;
     ep.scaled = a.linear ? nullptr : a.scaled + last;
-    ep.word = word;
-    lines_block<N1, N2, L, kLinePaint>(a.T + R.toff, R.ho, tw, R.fp, ep, blk, buf, stw, smask);
+    lines_block<N1, N2, L, kLinePaint>(a.T + R.toff, R.ho, tw, R.fp.cmax, ep, blk, buf, stw, smask, word);
 }
 
 // Pruned r2c of the fused loop (three launches): only the modes that the
@@ -485,25 +546,21 @@ __global__ void k_fill_u64(unsigned long long* __restrict__ p, size_t n) {
 // ------------------------------------------------------------------ host side
 
 template <int N1, int N2, int L>
-int launch_lines(int mode, const float2* U, const float2* tw, const FusedParams& fp, const LineEpilogue& ep,
-                 hipStream_t st) {
+int launch_lines(const float2* U, const float2* tw, int cmax, const LineEpilogue& ep, hipStream_t st) {
     constexpr int D = 2 * N1 * N2;
-    const unsigned blocks = (unsigned)((size_t)D * D / L);
-    if (mode == kLineSum)
-        k_fused_lines<N1, N2, L, kLineSum><<<blocks, L * N1, 0, st>>>(U, tw, fp, ep);
-    else if (mode == kLineThreshold)
-        k_fused_lines<N1, N2, L, kLineThreshold><<<blocks, L * N1, 0, st>>>(U, tw, fp, ep);
-    else
-        k_fused_lines<N1, N2, L, kLineFinal><<<blocks, L * N1, 0, st>>>(U, tw, fp, ep);
+    k_fused_lines<N1, N2, L><<<(unsigned)((size_t)D * D / L), L * N1, 0, st>>>(U, tw, cmax, ep);
     CM21_LAUNCH_CHECK("k_fused_lines");
     return CM21_OK;
 }
 
 template <int D1, int D2, int W, int N1, int N2, int L>
-int launch_radius(const RadiusRoles& a, const float2* tw, hipStream_t st) {
-    const int blocks = a.n_red + a.n_thr + a.n_mem + a.n_sum;
+int launch_radius(const RadiusRoles& a, const AskRoles& q, const float2* tw, hipStream_t st) {
+    const int blocks = a.n_red + q.n_ver + a.n_thr + a.n_mem + a.n_sum;
     if (blocks <= 0) return CM21_OK;
-    k_fused_radius<D1, D2, W, N1, N2, L><<<blocks, W * D1, 0, st>>>(a, tw);
+    if (q.any)
+        k_fused_radius_ask<D1, D2, W, N1, N2, L><<<blocks, W * D1, 0, st>>>(a, q, tw);
+    else
+        k_fused_radius<D1, D2, W, N1, N2, L><<<blocks, W * D1, 0, st>>>(a, tw);
     CM21_LAUNCH_CHECK("k_fused_radius");
     return CM21_OK;
 }
@@ -537,11 +594,13 @@ int launch_all(const AllRadii& a, const float2* tw, hipStream_t st) {
     };
     const dim3 groups(a.nblk, a.nr);
     CM21_TRY(timed(CM21_STAGE_FUSED_COLUMNS, [&] {
-        k_all_columns<D1, D2, W, N1, N2, L><<<a.cblk[a.nr] + (a.linear ? 1 : 0), NT, 0, st>>>(a, tw);
+        k_all_columns<D1, D2, W, N1, N2, L><<<a.cblk[a.nr], NT, 0, st>>>(a, tw);
     }, "k_all_columns"));
     CM21_TRY(timed(CM21_STAGE_FUSED_ROWS, [&] {
         k_all_rows<D1, D2, W, N1, N2, L><<<a.rblk[a.nr], NT, 0, st>>>(a, tw);
     }, "k_all_rows"));
+    k_all_verdicts<NT, D1 * D2><<<a.nr, NT, 0, st>>>(a);
+    CM21_LAUNCH_CHECK("k_all_verdicts");
     if (!a.linear) {
         CM21_TRY(timed(CM21_STAGE_FCOLL_SUM, [&] { k_all_sums<N1, N2, L><<<groups, NT, 0, st>>>(a, tw); }, "k_all_sums"));
         k_all_reduce<NT><<<a.nr, NT, 0, st>>>(a);
@@ -627,10 +686,10 @@ void column_groups(const FusedShape& sh, const FusedParams& fp, int* ncg, int* n
     *ncg = std::min(fp.cmax / sh.W + 1, ncg_all);
 }
 
-int fused_lines(const FusedShape& sh, int mode, const float2* U, const float2* tw, const FusedParams& fp,
+int fused_lines(const FusedShape& sh, const float2* U, const float2* tw, const FusedParams& fp,
                 const LineEpilogue& ep, hipStream_t st, int stage) {
     ProfToken t = prof_begin(stage, st);
-    CM21_TRY(sh.lines(mode, U, tw, fp, ep, st));
+    CM21_TRY(sh.lines(U, tw, fp.cmax, ep, st));
     prof_end(t, st);
     return CM21_OK;
 }
@@ -643,9 +702,10 @@ int fused_forward(const FusedShape& sh, const float* delta, float2* T0, float2* 
     return CM21_OK;
 }
 
-int fused_radius_launch(const FusedShape& sh, const RadiusRoles& a, const float2* tw, hipStream_t st) {
+int fused_radius_launch(const FusedShape& sh, const RadiusRoles& a, const AskRoles& q, const float2* tw,
+                        hipStream_t st) {
     ProfToken t = prof_begin(CM21_STAGE_FUSED_RADIUS, st);
-    CM21_TRY(sh.radius(a, tw, st));
+    CM21_TRY(sh.radius(a, q, tw, st));
     prof_end(t, st);
     return CM21_OK;
 }
@@ -702,6 +762,33 @@ static double erfcinv_host(double y) {
     return 0.5 * (lo + hi);
 }
 
+// The bound of the rows pass is the largest sum of moduli of a line's modes: on
+// Gaussian and lognormal boxes of this path's spectra 1.5 to 2.5 (mostly 1.7 to 2)
+// times sqrt(cmax + 1) standard deviations.  So a verdict can only come out neutral
+// where the threshold (of linear input, or with the box mean at its value for
+// mean density) is that many standard deviations away; sigma^2 = S(R) follows
+// from the denominators and sigma_min^2 from fc_mean, where it is given.  This
+// only decides whether to ask: boxes that would never pass keep the shorter
+// schedule (asking in vain costs 2 % at 256^3).  With it a 256^3 box takes 1664
+// us for 1822 (nonlinear, half ionized) and a 512^3 one 14.1 ms for 15.8 (linear).
+int neutral_radii(const cm21_bubble_params& prm, const float* denoms, int n_radii, const int* cmax) {
+    const double dc = prm.deltac, fc = prm.fc_mean;
+    double smin = 0.5 * (double)denoms[0] * denoms[0];  // S at the largest radius counted as 0
+    if (fc > 1e-30 && fc < 1.0) {
+        const double x = dc / erfcinv_host(fc);
+        if (0.5 * x * x > smin) smin = 0.5 * x * x;
+    }
+    int n = 0;
+    for (; n < n_radii - 1 && cmax[n] < kBoundModes; ++n) {
+        const double dn = denoms[n], s = smin - 0.5 * dn * dn;
+        double y = 1.0 / prm.zeta;
+        if (!prm.linear_input) y *= std::erfc(dc / dn) / fc;
+        if (!(y > 1e-30 && y < 1.999)) break;
+        if (dc - dn * erfcinv_host(y) < 1.7 * std::sqrt((cmax[n] + 1.0) * (s > 0.0 ? s : 0.0))) break;
+    }
+    return n < 4 ? 0 : n;  // the schedule's one launch more has to pay
+}
+
 DensityThreshold density_threshold_host(float deltac, float denom, double zeta, float scale) {
     const double y = 1.0 / (zeta * (double)scale);
     DensityThreshold t;
@@ -716,20 +803,14 @@ DensityThreshold density_threshold_host(float deltac, float denom, double zeta, 
     return t;
 }
 
-LineEpilogue line_epilogue(float deltac, float denom, double zeta, const double* sum, float fc_mean,
-                           unsigned long long* mask, float* out, double* partial, double ncells, float* bmax) {
+LineEpilogue line_epilogue(float deltac, float denom, double zeta, unsigned long long* mask, float* out) {
     LineEpilogue ep{};
-    ep.bmax = bmax;
     ep.deltac = deltac;
     ep.denom = denom;
     ep.zeta = zeta;
     ep.inv_zeta = 1.0 / zeta;
-    ep.sum = sum;
-    ep.fc_mean = fc_mean;
     ep.mask = mask;
     ep.out = out;
-    ep.partial = partial;
-    ep.ncells = ncells;
     return ep;
 }
 

@@ -31,7 +31,23 @@ struct DensityThreshold {
 struct ScaledThreshold {
     float scale;
     DensityThreshold th;
-    float pad;
+    int neutral;  // no cell of the box can be ionized at this radius (scale and th are then not set)
+};
+
+// Radii that keep at least this many modes a line get no bound: the sum of so
+// many moduli stays far above any threshold (simulated on Gaussian and
+// lognormal boxes, half and a fifth ionized: the last radius that it rules out
+// keeps 9 to 23).
+constexpr int kBoundModes = 32;
+
+// What box_stays_neutral decides from.
+struct SkipArgs {
+    const float* bound;  // [D][4] bounds of the rows pass, or NULL: not decided (no)
+    const float2* S0;    // the spectrum's k = 0 mode
+    int groups;          // column groups that the bounds have
+    int linear;
+    float deltac, zeta_fc_mean;  // nonlinear input
+    DensityThreshold th;  // linear input
 };
 
 // The threshold for linear input (scale 1), computed on the host.
@@ -40,20 +56,14 @@ DensityThreshold density_threshold_host(float deltac, float denom, double zeta, 
 struct LineEpilogue {
     float deltac, denom;
     double zeta, inv_zeta;
-    const double* sum;  // FP64 box sum of f_coll (nonlinear input), or NULL
-    float fc_mean;
     unsigned long long* mask;  // ionization state, one bit per cell
     float* out;                // final float box
     double* partial;           // per-block FP64 partial sums
-    double ncells;
     float* bmax;               // per-block maximum of the smoothed field: written by
                                // the box-sum pass, read by the threshold pass to skip
                                // blocks no cell of which can reach the threshold; or NULL
     DensityThreshold th;       // threshold when `scaled` is NULL (linear input)
     const ScaledThreshold* scaled;  // nonlinear input: scale and threshold of the radius
-    unsigned long long word;   // kLinePaint: the thread's mask word
-    const int* active;         // threshold pass: the line groups to visit, or NULL (all)
-    const int* nactive;        //   and their number
 };
 
 // Arguments of the box-sum reduction of one radius: the FP64 total, and for
@@ -69,28 +79,57 @@ struct SumScaleArgs {
 };
 
 // The roles of one launch of the pipelined radius loop (k_fused_radius) and
-// their block counts; a count of 0 is a role the launch does not have.
+// their block counts; a count of 0 is a role the launch does not have.  Only
+// what the roles read: kernel arguments are fetched anew for every launch, and
+// 130 bytes more of them (those of AskRoles) made the 33 launches of a linear
+// 256^3 box 0.5 us longer each.
 struct RadiusRoles {
     int n_red;               // box-sum reduction: 0 or 1 block
     int n_thr;               // threshold blocks (one line group each)
     int n_cols, n_mem;       // columns blocks; columns + rows blocks
     int n_sum;               // box-sum blocks (one line group each)
     int ncg_cols, ncg_rows;  // column groups of the columns and rows roles
+    float deltac;
+    double zeta;
     const float2* S;         // columns: pristine spectrum -> Tcols
     float2* Tcols;
     FusedParams fp_cols;
+    int m2max_rows, cmax_rows;
     float2* Trows;           // rows: in place
-    FusedParams fp_rows;
-    const double* partial;   // reduction: npart box-sum partials -> total
-    int npart;
+    const double* partial;   // reduction: one partial per line group -> total
     double* total;
-    SumScaleArgs sa;
+    ScaledThreshold* scaled_red;
+    float fc_mean, denom_red;
+    const float* bmax_red;
+    int* active_red;         // or NULL (the last radius has no list)
+    int* nactive_red;
     const float2* Uthr;      // threshold pass
-    FusedParams fp_thr;
-    LineEpilogue ep_thr;
+    int cmax_thr;
+    float denom_thr;
+    DensityThreshold th;     // linear input
+    unsigned long long* mask;
+    const ScaledThreshold* scaled_thr;  // nonlinear input
+    const float* bmax_thr;
+    const int* active_thr;
+    const int* nactive_thr;
     const float2* Usum;      // box-sum pass
-    FusedParams fp_sum;
-    LineEpilogue ep_sum;
+    int cmax_sum;
+    float denom_sum;
+    double* partial_sum;
+    float* bmax_sum;
+};
+
+// What a launch of the first radii has beside its roles.
+struct AskRoles {
+    int any;
+    int n_ver;               // verdict: 0 or 1 block, whether the box stays neutral at a radius
+    SkipArgs skip;
+    float skip_scale, skip_denom;
+    ScaledThreshold* verdict;
+    float* bound_rows;                 // rows: bounds of the radius, or NULL
+    const ScaledThreshold* state_thr;  // verdicts of the threshold blocks' (linear input), of
+    const ScaledThreshold* state_sum;  // the box sums' and of the reduction's radius, or NULL
+    const ScaledThreshold* state_red;
 };
 
 // The all-radii form of the loop: every role of every radius in one launch
@@ -118,6 +157,7 @@ struct AllRadii {
     double* partial;             // [nr][nblk] box-sum partials (nonlinear input)
     float* bmax;                 // [nr][nblk] line group maxima
     double* sums;                // [nr]
+    float* bound;                // [nr][D][4] bounds of the rows pass
     ScaledThreshold* scaled;     // [nr] box-mean scale (1 for linear input) and density threshold
     unsigned* hits;              // [nr][nblk] whether a line group has a hit at a radius ...
     unsigned long long* planes;  // [nr][N/64] ... and then its hit bits
@@ -127,8 +167,8 @@ struct AllRadii {
 struct FusedShape {
     int D;
     int (*all)(const AllRadii&, const float2* tw, hipStream_t);
-    int (*lines)(int mode, const float2*, const float2*, const FusedParams&, const LineEpilogue&, hipStream_t);
-    int (*radius)(const RadiusRoles&, const float2* tw, hipStream_t);
+    int (*lines)(const float2* U, const float2* tw, int cmax, const LineEpilogue&, hipStream_t);
+    int (*radius)(const RadiusRoles&, const AskRoles&, const float2* tw, hipStream_t);
     int (*forward)(const float* delta, float2* T0, float2* S, const float2* tw, const FusedParams& fp, hipStream_t);
     int W, L;  // columns per column group, lines per line group
 };
@@ -144,13 +184,14 @@ int fused_all_radii(const FusedShape& sh, const AllRadii& a, const float2* tw, h
 const FusedShape* fused_shape(int D);
 size_t fused_partials(int D);
 FusedParams fused_params(int D, float dk, float R, int filter_type, int ref_fallthrough, float scale);
-LineEpilogue line_epilogue(float deltac, float denom, double zeta, const double* sum, float fc_mean,
-                           unsigned long long* mask, float* out, double* partial, double ncells,
-                           float* bmax = nullptr);
+LineEpilogue line_epilogue(float deltac, float denom, double zeta, unsigned long long* mask, float* out);
 // Column groups and surviving b rows of the columns role at one radius
 // (the rows role uses the same column groups over all D rows p).
 void column_groups(const FusedShape& sh, const FusedParams& fp, int* ncg, int* nb);
-int fused_radius_launch(const FusedShape& sh, const RadiusRoles& a, const float2* tw, hipStream_t st);
+// Leading radii at which asking for a verdict (box_stays_neutral) can pay.
+int neutral_radii(const cm21_bubble_params& prm, const float* denoms, int n_radii, const int* cmax);
+int fused_radius_launch(const FusedShape& sh, const RadiusRoles& a, const AskRoles& q, const float2* tw,
+                        hipStream_t st);
 // The r2c of delta into the half spectrum S for the fused loop, stored
 // b-major (S[b][a][c]), formed only for the modes the widest window fp keeps
 // (|n|^2 <= fp.m2max), through the intermediate T0 (rows padded to 16
@@ -158,7 +199,8 @@ int fused_radius_launch(const FusedShape& sh, const RadiusRoles& a, const float2
 // them.
 int fused_forward(const FusedShape& sh, const float* delta, float2* T0, float2* S, const float2* tw,
                   const FusedParams& fp, hipStream_t st);
-int fused_lines(const FusedShape& sh, int mode, const float2* U, const float2* tw, const FusedParams& fp,
+// The final paint of the last radius from its intermediate U.
+int fused_lines(const FusedShape& sh, const float2* U, const float2* tw, const FusedParams& fp,
                 const LineEpilogue& ep, hipStream_t st, int stage = CM21_STAGE_FUSED_LINES);
 int fused_mask_clear(unsigned long long* mask, size_t words, hipStream_t st);
 

@@ -10,6 +10,7 @@
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "cm21_dft.hpp"
 #include "cm21_fused_api.hpp"
@@ -55,9 +56,14 @@ __device__ inline float2 fused_window(float2 x, int a, int b, int c, int m2, int
 // one-round tile, with no more registers live than in one round (the real
 // parts read back take the place of the real parts written).  The radius
 // kernel and the forward transform use it.
-template <int D1, int D2, int W, class Store>
+// done(u) is called with the D1 values of an item once they are stored.
+struct NoDone {
+    template <class U>
+    __device__ __forceinline__ void operator()(const U&) const {}
+};
+template <int D1, int D2, int W, class Store, class Done = NoDone>
 __device__ __forceinline__ void transpose_finish_reim(float2 (&v)[D2], const float2* __restrict__ tw, float* lds,
-                                                      Store store) {
+                                                      Store store, Done done = Done()) {
     constexpr int NT = W * D1, LD = D2 * D1 + 1;
     constexpr int ITEMS = (W * D2 + NT - 1) / NT;
     const int t = threadIdx.x;
@@ -92,15 +98,16 @@ __device__ __forceinline__ void transpose_finish_reim(float2 (&v)[D2], const flo
             dft<D1>(u[q]);
 #pragma unroll
             for (int k1 = 0; k1 < D1; ++k1) store(jj, k2, k1, u[q][k1]);
+            done(u[q]);
         }
     }
 }
 
-template <int D1, int D2, int W, int ROUNDS, class Store>
+template <int D1, int D2, int W, int ROUNDS, class Store, class Done = NoDone>
 __device__ __forceinline__ void transpose_finish(float2 (&v)[D2], const float2* __restrict__ tw, float2* lds,
-                                                 Store store) {
+                                                 Store store, Done done = Done()) {
     if constexpr (ROUNDS == 0) {
-        transpose_finish_reim<D1, D2, W>(v, tw, reinterpret_cast<float*>(lds), store);
+        transpose_finish_reim<D1, D2, W>(v, tw, reinterpret_cast<float*>(lds), store, done);
         return;
     }
     constexpr int NT = W * D1, K2R = D2 / (ROUNDS > 0 ? ROUNDS : 1), LD = K2R * D1 + 1;
@@ -124,6 +131,7 @@ __device__ __forceinline__ void transpose_finish(float2 (&v)[D2], const float2* 
             dft<D1>(u);
 #pragma unroll
             for (int k1 = 0; k1 < D1; ++k1) store(jj, h * K2R + kk, k1, u[k1]);
+            done(u);
         }
     }
 }
@@ -168,11 +176,33 @@ __device__ __forceinline__ void columns_body(const float2* __restrict__ S, float
     });
 }
 
+// Sum over the W consecutive lanes that share a row (W = 8, 16 or 32, aligned);
+// every lane gets it.
+template <int W>
+__device__ __forceinline__ float lane_group_sum(float v) {
+    static_assert(W == 8 || W == 16 || W == 32, "lane groups");
+    auto dpp = [](float x, auto ctrl) {
+        return __int_as_float(
+            __builtin_amdgcn_mov_dpp(__float_as_int(x), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    v += dpp(v, std::integral_constant<int, 0xB1>());   // lanes 1,0,3,2
+    v += dpp(v, std::integral_constant<int, 0x4E>());   // lanes 2,3,0,1
+    v += dpp(v, std::integral_constant<int, 0x141>());  // the other quad of eight lanes
+    if (W >= 16) v += dpp(v, std::integral_constant<int, 0x140>());  // the other half of sixteen
+    if (W >= 32) v += __shfl_xor(v, 16, 64);
+    return v;
+}
+
 // Rows pass of one block: inverse DFT along axis 1, in place, for the W
-// columns (p, c0..c0+W-1).  lds as for the columns pass.
+// columns (p, c0..c0+W-1).  lds as for the columns pass.  With `bound` the
+// block also stores in bound[p * kBoundGroups + cgroup] the largest sum of
+// moduli sum_c w_c |X_c| (w_0 = 1, else 2) of its columns over the lines of plane
+// p: the groups' sums together bound the modulus of the plane's real field.
+constexpr int kBoundGroups = 4;
 template <int D1, int D2, int W, int ROUNDS = 1>
 __device__ __forceinline__ void rows_body(float2* __restrict__ T, int ho, const float2* __restrict__ tw,
-                                          const FusedParams& fp, int p, int cgroup, float2* lds) {
+                                          const FusedParams& fp, int p, int cgroup, float2* lds,
+                                          float* bound = nullptr) {
     constexpr int D = D1 * D2, H = D / 2 + 1;
     const int t = threadIdx.x;
     const int j = t % W, n1 = t / W;
@@ -186,10 +216,64 @@ __device__ __forceinline__ void rows_body(float2* __restrict__ T, int ho, const 
         v[n2] = (c < H && bs * bs + c * c <= fp.m2max) ? T[((size_t)p * D + b) * ho + c] : make_float2(0.0f, 0.0f);
     }
     dft<D2>(v);
-    transpose_finish<D1, D2, W, ROUNDS>(v, tw, lds, [&](int jj, int k2, int k1, float2 u) {
-        const int cc = c0 + jj;
-        if (cc <= fp.cmax) T[((size_t)p * D + (k2 + D2 * k1)) * ho + cc] = u;
-    });
+    unsigned most = 0u;  // bits of a non-negative float (a NaN is larger than every number)
+    const float wc = c == 0 ? 1.0f : 2.0f;  // an item's column is the thread's own: j = t % W
+    transpose_finish<D1, D2, W, ROUNDS>(
+        v, tw, lds,
+        [&](int jj, int k2, int k1, float2 u) {
+            const int cc = c0 + jj;
+            if (cc <= fp.cmax) T[((size_t)p * D + (k2 + D2 * k1)) * ho + cc] = u;
+        },
+        [&](const auto& u) {
+            if (!bound) return;
+#pragma unroll
+            for (int k1 = 0; k1 < D1; ++k1) {
+                const float m = __builtin_amdgcn_sqrtf(u[k1].x * u[k1].x + u[k1].y * u[k1].y) * wc;
+                most = max(most, __float_as_uint(lane_group_sum<W>(m)) & 0x7fffffffu);
+            }
+        });
+    if (bound) {
+        __shared__ unsigned wmost[W * D1 / 64];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, off, 64));
+        if ((t & 63) == 0) wmost[t >> 6] = most;
+        __syncthreads();
+        if (t == 0) {
+            for (int w = 1; w < W * D1 / 64; ++w) most = max(most, wmost[w]);
+            bound[p * kBoundGroups + cgroup] = __uint_as_float(most);
+        }
+    }
+}
+
+// Whether no cell of the box can be ionized at a radius, from the rows pass'
+// bounds B_p on |delta| in each plane (one verdict by a block of NT threads):
+//   linear input: B < d* - band;
+//   nonlinear input: with every cell below deltac, erfc((deltac - delta)/denom)
+//   is convex in delta, so the box mean of f_coll is at least its value at the
+//   mean of delta (the k = 0 mode m), the scale is at most fc_mean / f(m), and
+//   zeta f scale < 1 everywhere when zeta fc_mean f(B) < f(m).
+// Margins of 1e-4 on the bound and 1e-3 on the comparison cover the float32
+// arithmetic of the transforms, of f_coll and of its mean; a NaN, an infinity or
+// an underflow of both sides says no.
+template <int NT, int D>
+__device__ __forceinline__ bool box_stays_neutral(const SkipArgs& sk, float scale, float denom) {
+    if (!sk.bound) return false;
+    const float m = sk.linear ? 0.0f : sk.S0->x * scale;
+    const float most = sk.linear ? 0.0f : (1.0f - 1e-3f) * erfcf((sk.deltac - m) / denom);
+    bool ok = true;
+    for (int p = threadIdx.x; p < D; p += NT) {
+        const float4 g = *reinterpret_cast<const float4*>(sk.bound + p * kBoundGroups);
+        float b = g.x;
+        if (sk.groups > 1) b += g.y;
+        if (sk.groups > 2) b += g.z;
+        if (sk.groups > 3) b += g.w;
+        b *= 1.0f + 1e-4f;
+        if (sk.linear)
+            ok = ok && b < sk.th.dstar - sk.th.band;
+        else
+            ok = ok && b <= sk.deltac && sk.zeta_fc_mean * erfcf((sk.deltac - b) / denom) < most;
+    }
+    return __syncthreads_and(ok) != 0;
 }
 
 // Forward DFT along a column axis for the pruned r2c: the inverse four-step
