@@ -18,19 +18,33 @@
 
 #include "cm21_internal.hpp"
 #include "cm21_window.hpp"
-#include "cm21_fused_api.hpp"
+#include "cm21_fused_dev.hpp"
 
 using namespace cm21;
 
 namespace {
 
+constexpr int kThreshCells = 4 * kThreads;  // cells per threshold block
+constexpr size_t kChunkAlign = kThreshCells;
+
+// W(kR) times the spectrum.  Bound by memory where modes survive (2 x 8 bytes a
+// mode); a mode that the cut surely takes (|k|R 0.1 % past it) is written as
+// zero without being read and without the FP64 root and the Gaussian of the
+// exact test.  The blocks run over the D*H modes of a plane in memory order (64
+// modes of a row to a block left 49 % of the lanes idle at H = 65 and 21 % at
+// H = 101); (i * row_magic) >> 32 is i / H there.  At 200^3, over the 37 radii of a
+// k-space top-hat, 22.5 -> 9.5 us a radius.
 __global__ void k_filter(float2* __restrict__ out, const float2* __restrict__ in, int D, WindowParams wp,
-                         float scale) {
-    const int H = D / 2 + 1;
-    const int c = blockIdx.x * kModeBlockX + threadIdx.x, b = blockIdx.y * kModeBlockY + threadIdx.y;
-    const int a = blockIdx.z;
-    if (c >= H || b >= D) return;
-    const size_t idx = ((size_t)a * D + b) * H + c;
+                         float scale, float ksq_cut, unsigned row_magic) {
+    const unsigned H = D / 2 + 1, i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= D * H) return;
+    const int a = blockIdx.y, b = (int)__umulhi(i, row_magic), c = (int)(i - b * H);
+    const size_t idx = (size_t)a * D * H + i;
+    const float ka = (float)mode_of(a, D) * wp.dk, kb = (float)mode_of(b, D) * wp.dk, kc = (float)c * wp.dk;
+    if (ka * ka + kb * kb + kc * kc > ksq_cut) {
+        out[idx] = make_float2(0.0f, 0.0f);
+        return;
+    }
     float w0, w2;
     bool cut;
     window_of(kmag_of(a, b, c, D, wp.dk, wp.korder), wp, w0, cut, w2);
@@ -42,144 +56,434 @@ __global__ void k_fill(float* __restrict__ p, size_t n, float v) {
     if (i < n) p[i] = v;
 }
 
-__device__ inline float fcoll_of(float smoothed, float deltac, float denom) {
-    return erfcf(__fdiv_rn(__fsub_rn(deltac, smoothed), denom));
-}
+// Cells per block of the f_coll sum: consecutive cells, so that the maximum a
+// block stores lets the threshold and the sphere paint pass its cells over.
+inline size_t sum_chunk(size_t N) { return align_up((N + kReduceBlocks - 1) / kReduceBlocks, kChunkAlign); }
 
-// Per-block FP64 partial sums of f_coll over a fixed grid of kReduceBlocks.
-__global__ void k_fcoll_partial(const float* __restrict__ sm, size_t N, float deltac, float denom,
-                                double* __restrict__ partial) {
+// FP64 partial sum of f_coll and maximum of the smoothed field of a chunk.
+// Bound by the VALU (erfcf and its divided argument).
+__global__ void k_fcoll_partial(const float* __restrict__ sm, size_t N, size_t chunk, float deltac, float denom,
+                                double* __restrict__ partial, float* __restrict__ cmax) {
+    const size_t p0 = (size_t)blockIdx.x * chunk, p1 = p0 + chunk < N ? p0 + chunk : N;
     double acc = 0.0;
-    for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += (size_t)gridDim.x * blockDim.x)
-        acc += (double)fcoll_of(sm[p], deltac, denom);
+    float most = -INFINITY;
+    for (size_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) {
+        const float d = sm[p];
+        acc += (double)fcoll_of(d, deltac, denom);
+        most = fmaxf(most, d);  // a NaN is no hit
+    }
     acc = block_sum(acc);
     if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+    if (cmax) {
+        __shared__ float part[kWaves];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) most = fmaxf(most, __shfl_xor(most, off, 64));
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = most;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < kWaves; ++w) most = fmaxf(most, part[w]);
+            cmax[blockIdx.x] = most;
+        }
+    }
 }
 
-// Sums `n` partials in a fixed order into *out (one block).
-__global__ void k_sum_partials(const double* __restrict__ partial, int n, double* __restrict__ out) {
+// The centre-pixel test of a radius on the generic path.
+struct CellTest {
+    float deltac, denom;
+    double zeta, inv_zeta;
+    const double* sum;              // nonlinear input: the f_coll sum ...
+    float fc_mean;
+    double ncells;
+    const ScaledThreshold* scaled;  // ... or what follows from it, or NULL
+    DensityThreshold th;            // linear input
+    const float* cmax;              // chunk maxima of the f_coll sum, or NULL
+    size_t chunk;
+};
+
+// The density threshold holds for f_coll falling with the argument; other
+// denominators leave every cell to the float32 test.
+__device__ __host__ inline bool plain_denom(float denom) { return denom > 0.0f && denom < INFINITY; }
+
+__device__ inline ScaledThreshold scaled_of_sum(double sum, double ncells, float fc_mean, float deltac, float denom,
+                                                double zeta) {
+    ScaledThreshold s;
+    s.scale = (float)((double)fc_mean / (sum / ncells));
+    s.th.dstar = 0.0f;
+    s.th.band = INFINITY;
+    if (plain_denom(denom)) s.th = density_threshold(deltac, denom, zeta, s.scale);
+    s.neutral = 0;
+    return s;
+}
+
+// Sums `n` partials in a fixed order into *out (one block); with `scaled` also
+// the box-mean scale and the density threshold of the radius, once for every
+// cell of the following pass (per cell they were two FP64 divisions).
+__global__ void k_sum_partials(const double* __restrict__ partial, int n, double* __restrict__ out, CellTest t,
+                               ScaledThreshold* __restrict__ scaled) {
     double acc = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) acc += partial[i];
     acc = block_sum(acc);
-    if (threadIdx.x == 0) *out = acc;
+    if (threadIdx.x == 0) {
+        *out = acc;
+        if (scaled) *scaled = scaled_of_sum(acc, t.ncells, t.fc_mean, t.deltac, t.denom, t.zeta);
+    }
 }
 
-__device__ inline float norm_scale(const double* sum, size_t N, float fc_mean) {
-    if (!sum) return 1.0f;
-    const double mean = *sum / (double)N;
-    return (float)((double)fc_mean / mean);
+// Scale and threshold of a block.  Without a prepared one (a call of the
+// threshold alone) only the scale: its cells take the float32 test.
+__device__ inline ScaledThreshold block_threshold(const CellTest& t) {
+    if (t.scaled) return *t.scaled;
+    ScaledThreshold s{1.0f, t.th, 0};
+    if (t.sum) {
+        s.scale = (float)((double)t.fc_mean / (*t.sum / t.ncells));
+        s.th.dstar = 0.0f;
+        s.th.band = INFINITY;
+    }
+    return s;
 }
 
-__global__ void k_threshold(float* __restrict__ ion, const float* __restrict__ sm, size_t N, float deltac,
-                            float denom, double zeta, double inv_zeta, const double* __restrict__ sum,
-                            float fc_mean, int final_step) {
-    const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    const float cur = ion[p];
-    if (cur == 1.0f) return;
-    float f = fcoll_of(sm[p], deltac, denom);
-    if (sum) f = __fmul_rn(f, norm_scale(sum, N, fc_mean));
-    if ((double)f >= inv_zeta)
-        ion[p] = 1.0f;
-    else if (final_step)
-        ion[p] = (float)((double)f * zeta);
+__device__ __forceinline__ bool cell_hits(float d, const CellTest& t, const ScaledThreshold& s) {
+    return cell_hit(d, s.th, t.deltac, t.denom, t.sum != nullptr, s.scale, t.inv_zeta);
 }
 
-// Sphere paint as a separable squared-distance transform.  d2 holds, per
-// cell, a squared distance to the nearest ionizing centre (kFar when none is
-// within range).  Only offsets with o^2 < R^2 matter, because the paint test
-// is d^2 < R^2 (Programs/find_bubbles.cu:97-98).
+// Threshold and final paint.  A block takes kThreshCells consecutive cells;
+// kThreshCells divides the chunk of the sum, so one maximum tells whether any of
+// them can be ionized.  Bound by memory: 22 us at 200^3 with the exact test
+// and two FP64 divisions per cell, 5.5 with the density threshold and the maxima.
+__global__ void k_threshold(float* __restrict__ ion, const float* __restrict__ sm, size_t N, CellTest t,
+                            int final_step) {
+    const size_t p0 = (size_t)blockIdx.x * kThreshCells;
+    const ScaledThreshold s = block_threshold(t);
+    if (!final_step && t.cmax && t.cmax[p0 / t.chunk] < s.th.dstar - s.th.band) return;
+#pragma unroll
+    for (int k = 0; k < kThreshCells / kThreads; ++k) {
+        const size_t p = p0 + k * kThreads + threadIdx.x;
+        if (p >= N) return;
+        if (ion[p] == 1.0f) continue;
+        const float d = sm[p];
+        if (cell_hits(d, t, s)) {
+            ion[p] = 1.0f;
+        } else if (final_step) {
+            float f = fcoll_of(d, t.deltac, t.denom);
+            if (t.sum) f = __fmul_rn(f, s.scale);
+            ion[p] = (float)((double)f * t.zeta);
+        }
+    }
+}
+
+// ------------------------------------------------------------------ sphere paint
+// A cell is painted when its squared distance to an ionizing centre is below
+// R^2 (Programs/find_bubbles.cu:97-98), in whole numbers: a separable squared
+// distance transform over the offsets with o^2 < R^2.
+//   rows:   the centres of a line of axis 2 as bits; the distance g to the
+//           nearest one along the line by bit scans (kNoCentre: none in reach);
+//   planes: h = min over o of g(b + o)^2 + o^2 along axis 1;
+//   paint:  whether h(a + o) + o^2 < R^2 for some o along axis 0.
+// The rows flag lines without a centre and the planes flag tiles without a
+// distance: nothing of those is written or read, and a tile of cells that are
+// all painted already is passed over.  Radii up to kNarrowReach cells (all
+// but boxes of very small cells) hold g^2 and h in 16 bits and take the tiles below:
+// saturating 16-bit adds and minima, two cells an instruction, against a column
+// of the tile in LDS, eight cells along the axis per thread, so that one LDS
+// read serves eight offsets and the squares stay in scalar registers.
+// Bound by those adds and minima, one instruction per cell and offset, and by
+// their launches: 4.9 + 3.5 + 4.3 us a radius at 128^3 (reach 0 to 30), for 8.4
+// (centres) + 3 x 29.6 (three 32-bit passes from global memory over all offsets) +
+// 5 (paint); the whole box 5.45 -> 2.29 ms.
+constexpr uint32_t kNoCentre = 0xFFFFu;
+constexpr int kNarrowReach = 190;  // the column of a tile stays below 64 KB of LDS
+constexpr int kTile = 64;          // cells along either side of a tile
+constexpr int kTileRun = 8;        // cells along the axis per thread
+static_assert(kTile / kTileRun * (kTile / 2) == kThreads, "one thread per run and pair of lines");
+
+// Position of the nearest set bit at or before x within `reach`, as a distance
+// (periodic: also across the line's start), or kNoCentre.
+__device__ __forceinline__ uint32_t reach_back(const unsigned long long* words, int nw, int D, int x, int reach,
+                                               int periodic) {
+    int w = x >> 6;
+    unsigned long long m = words[w] & (~0ull >> (63 - (x & 63)));
+    while (!m && --w >= 0 && x - (w * 64 + 63) <= reach) m = words[w];
+    if (m) return (uint32_t)(x - (w * 64 + 63 - __clzll((long long)m)));
+    if (!periodic) return kNoCentre;
+    for (w = nw - 1; w >= 0 && x + D - min(w * 64 + 63, D - 1) <= reach; --w)
+        if (words[w]) return (uint32_t)(x + D - (w * 64 + 63 - __clzll((long long)words[w])));
+    return kNoCentre;
+}
+
+__device__ __forceinline__ uint32_t reach_on(const unsigned long long* words, int nw, int D, int x, int reach,
+                                             int periodic) {
+    int w = x >> 6;
+    unsigned long long m = words[w] & (~0ull << (x & 63));
+    while (!m && ++w < nw && w * 64 - x <= reach) m = words[w];
+    if (m) return (uint32_t)(w * 64 + __ffsll(m) - 1 - x);
+    if (!periodic) return kNoCentre;
+    for (w = 0; w < nw && w * 64 + D - x <= reach; ++w)
+        if (words[w]) return (uint32_t)(w * 64 + __ffsll(words[w]) - 1 + D - x);
+    return kNoCentre;
+}
+
+// One wave per line of axis 2 (D^2 lines, a multiple of four).
+__global__ __launch_bounds__(kThreads) void k_sphere_rows(uint16_t* __restrict__ g, uint8_t* __restrict__ any_row,
+                                                          const float* __restrict__ sm, int D, CellTest t, int reach,
+                                                          int periodic) {
+    __shared__ unsigned long long bits[kWaves][32];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (D + 63) >> 6;
+    const size_t row = (size_t)blockIdx.x * kWaves + w, p0 = row * D;
+    const ScaledThreshold s = block_threshold(t);
+    bool quiet = false;
+    if (t.cmax) {  // a line lies in one or two chunks, or is longer than they are
+        quiet = true;
+        for (size_t c = p0 / t.chunk; c <= (p0 + D - 1) / t.chunk; ++c)
+            quiet = quiet && t.cmax[c] < s.th.dstar - s.th.band;
+    }
+    bool any = false;
+    for (int c = 0; c < nw && !quiet; ++c) {
+        const int x = c * 64 + lane;
+        const unsigned long long m = __ballot(x < D && cell_hits(sm[p0 + x], t, s));
+        if (lane == 0) bits[w][c] = m;
+        any = any || m;
+    }
+    if (lane == 0) any_row[row] = any;
+    __syncthreads();
+    if (!any) return;
+    for (int x = lane; x < D; x += 64) {
+        const uint32_t l = reach_back(bits[w], nw, D, x, reach, periodic);
+        const uint32_t r = reach_on(bits[w], nw, D, x, reach, periodic);
+        const uint32_t m = min(l, r);
+        g[p0 + x] = (uint16_t)(m <= (uint32_t)reach ? m : kNoCentre);
+    }
+}
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// Minimum over the offsets of the LDS column + o^2 for the thread's run of
+// cells.  col: the thread's pair of lines at the run's first cell less `reach`.
+// Offsets past the reach (the run's ends) have o^2 >= R^2 and change nothing.
+__device__ __forceinline__ void run_minimum(const u16x2* col, int reach, u16x2 best[kTileRun]) {
+#pragma unroll
+    for (int i = 0; i < kTileRun; ++i) best[i] = u16x2{0xFFFF, 0xFFFF};
+    u16x2 sq[kTileRun];  // sq[(j - i) % 8] = (j - i)^2 of the eight latest offsets
+#pragma unroll
+    for (int i = 1; i < kTileRun; ++i) {
+        const int o = -reach - i;
+        const unsigned short q = (unsigned short)min(o * o, 0xFFFF);
+        sq[(kTileRun - i) % kTileRun] = u16x2{q, q};
+    }
+    for (int j0 = 0; j0 < 2 * reach + kTileRun; j0 += kTileRun) {
+#pragma unroll
+        for (int u = 0; u < kTileRun; ++u) {
+            const int o = j0 + u - reach;
+            const unsigned short q = (unsigned short)min(o * o, 0xFFFF);
+            sq[u] = u16x2{q, q};
+            const u16x2 v = col[(j0 + u) * (kTile / 2)];
+#pragma unroll
+            for (int i = 0; i < kTileRun; ++i)
+                best[i] = __builtin_elementwise_min(
+                    best[i], __builtin_elementwise_add_sat(v, sq[(u - i + kTileRun) % kTileRun]));
+        }
+    }
+}
+
+// Rows of a tile's LDS column: the tile, the reach on both sides and the run's
+// rounding up.
+inline size_t tile_lds(int reach) { return sizeof(u16x2) * (kTile / 2) * (size_t)(kTile + 2 * reach + kTileRun); }
+
+// Position along the axis of column row r of the tile that starts at x0, or -1.
+__device__ __forceinline__ int tile_position(int x0, int r, int reach, int D, int periodic) {
+    int q = x0 + r - reach;
+    if (periodic) {
+        q %= D;
+        return q < 0 ? q + D : q;
+    }
+    return q < 0 || q >= D ? -1 : q;
+}
+
+// PAINT: axis 0, from h into `ion`; otherwise axis 1, from g into h.  `from`
+// flags what was written of the input, `any_tile` what is written of h.
+template <bool PAINT>
+__global__ __launch_bounds__(kThreads) void k_sphere_tile(const uint16_t* __restrict__ in,
+                                                          const uint8_t* __restrict__ from, uint16_t* __restrict__ h,
+                                                          uint8_t* __restrict__ any_tile, float* __restrict__ ion,
+                                                          int D, int reach, int periodic, float R2) {
+    extern __shared__ u16x2 col[];
+    const int t = threadIdx.x, pair = t & 31, run = t >> 5;
+    const int x = blockIdx.x * kTile + 2 * pair;       // axis 2 (D is even: a pair is inside or outside)
+    const int s0 = blockIdx.y * kTile;                 // first cell of the tile along the axis
+    const int other = blockIdx.z;                      // the third axis
+    const int nt = gridDim.y, nx = gridDim.x;
+    const size_t stride = PAINT ? (size_t)D * D : (size_t)D;
+    const size_t base = PAINT ? (size_t)other * D : (size_t)other * D * D;
+    const int rows = kTile + 2 * reach + kTileRun;
+    bool todo = false;
+    for (int r = t; r < rows && !todo; r += kThreads) {
+        const int q = tile_position(s0, r, reach, D, periodic);
+        if (q >= 0) todo = PAINT ? from[((size_t)q * nt + other / kTile) * nx + blockIdx.x]
+                                 : from[(size_t)other * D + q];
+    }
+    todo = __syncthreads_or(todo);
+    if (PAINT && todo) {
+        bool open = false;
+        for (int i = 0; i < kTileRun; ++i) {
+            const int q = s0 + run * kTileRun + i;
+            if (x < D && q < D) {
+                const size_t p = base + (size_t)q * stride + x;
+                open = open || ion[p] != 1.0f || ion[p + 1] != 1.0f;
+            }
+        }
+        todo = __syncthreads_or(open);
+    }
+    if (!PAINT && t == 0) any_tile[((size_t)other * nt + blockIdx.y) * nx + blockIdx.x] = todo;
+    if (!todo) return;
+    for (int r = run; r < rows; r += kThreads / 32) {
+        const int q = tile_position(s0, r, reach, D, periodic);
+        u16x2 v{0xFFFF, 0xFFFF};
+        if (q >= 0 && x < D &&
+            (PAINT ? from[((size_t)q * nt + other / kTile) * nx + blockIdx.x] : from[(size_t)other * D + q])) {
+            const size_t p = base + (size_t)q * stride + x;
+            v = *reinterpret_cast<const u16x2*>(in + p);
+            if (!PAINT) {
+                v.x = v.x == kNoCentre ? v.x : (unsigned short)(v.x * v.x);
+                v.y = v.y == kNoCentre ? v.y : (unsigned short)(v.y * v.y);
+            }
+        }
+        col[r * (kTile / 2) + pair] = v;
+    }
+    __syncthreads();
+    u16x2 best[kTileRun];
+    run_minimum(col + run * kTileRun * (kTile / 2) + pair, reach, best);
+    if (x >= D) return;
+#pragma unroll
+    for (int i = 0; i < kTileRun; ++i) {
+        const int q = s0 + run * kTileRun + i;
+        if (q >= D) return;
+        const size_t p = base + (size_t)q * stride + x;
+        if (PAINT) {
+            if ((float)best[i].x < R2) ion[p] = 1.0f;
+            if ((float)best[i].y < R2) ion[p + 1] = 1.0f;
+        } else {
+            *reinterpret_cast<u16x2*>(h + p) = best[i];
+        }
+    }
+}
+
+// The planes and the paint for a reach beyond kNarrowReach: 32-bit, a thread
+// per cell, from offset 0 outwards until none can be nearer.
 constexpr uint32_t kFar = 0x3FFFFFFFu;
 
-__global__ void k_sphere_seed(uint32_t* __restrict__ d2, const float* __restrict__ sm, size_t N, float deltac,
-                              float denom, double inv_zeta, const double* __restrict__ sum, float fc_mean) {
+template <bool PAINT>
+__global__ void k_sphere_far(const uint16_t* __restrict__ g, const uint8_t* __restrict__ any_row,
+                             uint32_t* __restrict__ h, float* __restrict__ ion, int D, int reach, int periodic,
+                             float R2) {
     const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    float f = fcoll_of(sm[p], deltac, denom);
-    if (sum) f = __fmul_rn(f, norm_scale(sum, N, fc_mean));
-    d2[p] = ((double)f >= inv_zeta) ? 0u : kFar;
-}
-
-__global__ void k_sphere_pass(uint32_t* __restrict__ out, const uint32_t* __restrict__ in, int D, int axis,
-                              int omax, int periodic) {
-    const size_t N = (size_t)D * D * D;
-    const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    const size_t stride = axis == 2 ? 1 : (axis == 1 ? (size_t)D : (size_t)D * D);
+    if (p >= (size_t)D * D * D) return;
+    if (PAINT && ion[p] == 1.0f) return;
+    const size_t stride = PAINT ? (size_t)D * D : (size_t)D;
     const int pos = (int)((p / stride) % D);
     const size_t base = p - (size_t)pos * stride;
     uint32_t best = kFar;
-    for (int o = -omax; o <= omax; ++o) {
-        int q = pos + o;
-        if (periodic) {
-            q %= D;
-            if (q < 0) q += D;
-        } else if (q < 0 || q >= D) {
-            continue;
+    for (int o = 0; o <= reach && (uint32_t)(o * o) < best; ++o) {
+        for (int side = 0; side < 2; ++side) {
+            int q = side ? pos + o : pos - o;
+            if (periodic)
+                q = q < 0 ? q + D : (q >= D ? q - D : q);  // (the reach is below D)
+            if (q < 0 || q >= D) continue;
+            const size_t at = base + (size_t)q * stride;
+            uint32_t v = kFar;
+            if (PAINT)
+                v = h[at];
+            else if (any_row[at / D] && g[at] != kNoCentre)
+                v = (uint32_t)g[at] * g[at];
+            if (v < kFar) best = min(best, v + (uint32_t)(o * o));
         }
-        const uint32_t v = in[base + (size_t)q * stride];
-        if (v < kFar) {
-            const uint32_t c = v + (uint32_t)(o * o);
-            best = c < best ? c : best;
-        }
+        if (PAINT && (float)best < R2) break;
     }
-    out[p] = best;
-}
-
-__global__ void k_sphere_apply(float* __restrict__ ion, const uint32_t* __restrict__ d2, size_t N, float R2) {
-    const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    const uint32_t v = d2[p];
-    if (v < kFar && (float)v < R2) ion[p] = 1.0f;
+    if (!PAINT)
+        h[p] = best;
+    else if ((float)best < R2)
+        ion[p] = 1.0f;
 }
 
 int launch_filter(void* spec_out, const void* spec_in, int D, const WindowParams& wp, float scale,
                   hipStream_t st) {
-    k_filter<<<mode_grid(D, D / 2 + 1), mode_block(), 0, st>>>((float2*)spec_out, (const float2*)spec_in, D, wp,
-                                                               scale);
+    // |k|^2 past which the cut of window_of takes every mode
+    float ksq_cut = INFINITY;
+    if (wp.filter_type == 1 || (wp.filter_type == 0 && wp.ref_fallthrough)) {
+        const double k = 1.001 / (0.413566994 * (double)wp.R);
+        if (wp.R > 0.0f) ksq_cut = (float)(k * k);
+    }
+    // ceil(2^32 / H): exact for i < D*H <= 2^21 + 2^11, i * H < 2^32
+    const unsigned H = D / 2 + 1, magic = (unsigned)(((1ull << 32) + H - 1) / H);
+    k_filter<<<dim3(grid_for((size_t)D * H), D), kThreads, 0, st>>>((float2*)spec_out, (const float2*)spec_in, D, wp,
+                                                                    scale, ksq_cut, magic);
     CM21_LAUNCH_CHECK("k_filter");
     return CM21_OK;
 }
 
+// The f_coll sum; with t and scaled also the radius' scale and threshold, and
+// the chunk maxima.
 int launch_fcoll_sum(const float* sm, int D, float deltac, float denom, double* dev_sum, void* work,
-                     hipStream_t st) {
+                     hipStream_t st, const CellTest* t = nullptr, float* cmax = nullptr,
+                     ScaledThreshold* scaled = nullptr) {
     const size_t N = (size_t)D * D * D;
     double* partial = (double*)work;
-    k_fcoll_partial<<<kReduceBlocks, kThreads, 0, st>>>(sm, N, deltac, denom, partial);
+    k_fcoll_partial<<<kReduceBlocks, kThreads, 0, st>>>(sm, N, sum_chunk(N), deltac, denom, partial, cmax);
     CM21_LAUNCH_CHECK("k_fcoll_partial");
-    k_sum_partials<<<1, kThreads, 0, st>>>(partial, kReduceBlocks, dev_sum);
+    k_sum_partials<<<1, kThreads, 0, st>>>(partial, kReduceBlocks, dev_sum, t ? *t : CellTest{}, scaled);
     CM21_LAUNCH_CHECK("k_sum_partials");
     return CM21_OK;
 }
 
-int launch_threshold(float* ion, const float* sm, int D, float deltac, float denom, double zeta,
-                     const double* sum, float fc_mean, int final_step, hipStream_t st) {
+CellTest cell_test(int D, float deltac, float denom, double zeta, const double* sum, float fc_mean) {
+    CellTest t{};
+    t.deltac = deltac;
+    t.denom = denom;
+    t.zeta = zeta;
+    t.inv_zeta = 1.0 / zeta;
+    t.sum = sum;
+    t.fc_mean = fc_mean;
+    t.ncells = (double)((size_t)D * D * D);
+    t.th.dstar = 0.0f;
+    t.th.band = INFINITY;
+    if (!sum && plain_denom(denom)) t.th = density_threshold_host(deltac, denom, zeta, 1.0f);
+    return t;
+}
+
+int launch_threshold(float* ion, const float* sm, int D, const CellTest& t, int final_step, hipStream_t st) {
     const size_t N = (size_t)D * D * D;
-    k_threshold<<<grid_for(N), kThreads, 0, st>>>(ion, sm, N, deltac, denom, zeta, 1.0 / zeta, sum, fc_mean,
-                                                  final_step);
+    k_threshold<<<grid_for(N, kThreshCells), kThreads, 0, st>>>(ion, sm, N, t, final_step);
     CM21_LAUNCH_CHECK("k_threshold");
     return CM21_OK;
 }
 
-int launch_sphere(float* ion, const float* sm, int D, float deltac, float denom, double zeta, const double* sum,
-                  float fc_mean, float R_cells, int periodic, void* work, hipStream_t st) {
+int launch_sphere(float* ion, const float* sm, int D, const CellTest& test, float R_cells, int periodic, void* work,
+                  hipStream_t st) {
     const size_t N = (size_t)D * D * D;
-    uint32_t* a = (uint32_t*)work;
-    uint32_t* b = a + N;
     const float R2 = R_cells * R_cells;  // float32(R*R), find_bubbles.cu:98
-    int omax = (int)std::ceil((double)R_cells);
-    while (omax > 0 && (float)(omax * omax) >= R2) --omax;  // largest o with o^2 < R^2
-    if (omax >= D) omax = periodic ? D / 2 : D - 1;
-    k_sphere_seed<<<grid_for(N), kThreads, 0, st>>>(a, sm, N, deltac, denom, 1.0 / zeta, sum, fc_mean);
-    CM21_LAUNCH_CHECK("k_sphere_seed");
-    k_sphere_pass<<<grid_for(N), kThreads, 0, st>>>(b, a, D, 2, omax, periodic);
-    CM21_LAUNCH_CHECK("k_sphere_pass");
-    k_sphere_pass<<<grid_for(N), kThreads, 0, st>>>(a, b, D, 1, omax, periodic);
-    CM21_LAUNCH_CHECK("k_sphere_pass");
-    k_sphere_pass<<<grid_for(N), kThreads, 0, st>>>(b, a, D, 0, omax, periodic);
-    CM21_LAUNCH_CHECK("k_sphere_pass");
-    k_sphere_apply<<<grid_for(N), kThreads, 0, st>>>(ion, b, N, R2);
-    CM21_LAUNCH_CHECK("k_sphere_apply");
+    int reach = (int)std::ceil((double)R_cells);
+    while (reach > 0 && (float)(reach * reach) >= R2) --reach;  // largest o with o^2 < R^2
+    if (reach >= D) reach = periodic ? D / 2 : D - 1;
+    // of the 8 N bytes: h (4 N, or 2 N in 16 bits), g (2 N), the flags (2 N)
+    uint16_t* g = (uint16_t*)((char*)work + 4 * N);
+    uint8_t* any_row = (uint8_t*)work + 6 * N;
+    uint8_t* any_tile = any_row + (size_t)D * D;
+    k_sphere_rows<<<(unsigned)((size_t)D * D / kWaves), kThreads, 0, st>>>(g, any_row, sm, D, test, reach, periodic);
+    CM21_LAUNCH_CHECK("k_sphere_rows");
+    if (reach <= kNarrowReach) {
+        const unsigned n = (unsigned)((D + kTile - 1) / kTile);
+        uint16_t* h = (uint16_t*)work;
+        k_sphere_tile<false><<<dim3(n, n, D), kThreads, tile_lds(reach), st>>>(g, any_row, h, any_tile, nullptr, D,
+                                                                              reach, periodic, R2);
+        CM21_LAUNCH_CHECK("k_sphere_tile");
+        k_sphere_tile<true><<<dim3(n, n, D), kThreads, tile_lds(reach), st>>>(h, any_tile, nullptr, nullptr, ion, D,
+                                                                             reach, periodic, R2);
+        CM21_LAUNCH_CHECK("k_sphere_tile");
+        return CM21_OK;
+    }
+    uint32_t* h = (uint32_t*)work;
+    k_sphere_far<false><<<grid_for(N), kThreads, 0, st>>>(g, any_row, h, nullptr, D, reach, periodic, R2);
+    CM21_LAUNCH_CHECK("k_sphere_far");
+    k_sphere_far<true><<<grid_for(N), kThreads, 0, st>>>(nullptr, nullptr, h, ion, D, reach, periodic, R2);
+    CM21_LAUNCH_CHECK("k_sphere_far");
     return CM21_OK;
 }
 
@@ -212,7 +516,7 @@ extern "C" int cm21_fcoll_threshold(float* ionized, const float* smoothed, int D
     CM21_REQUIRE(ionized && smoothed, "cm21_fcoll_threshold: NULL argument");
     CM21_REQUIRE(valid_dim(D), "cm21_fcoll_threshold: D=%d must be even in [2,2048]", D);
     CM21_REQUIRE(zeta > 0.0, "cm21_fcoll_threshold: zeta must be positive");
-    return launch_threshold(ionized, smoothed, D, deltac, denom, zeta, dev_sum, fc_mean, final_step,
+    return launch_threshold(ionized, smoothed, D, cell_test(D, deltac, denom, zeta, dev_sum, fc_mean), final_step,
                             (hipStream_t)stream);
 }
 
@@ -228,8 +532,8 @@ extern "C" int cm21_update_sphere(float* ionized, const float* smoothed, int D, 
     CM21_REQUIRE(zeta > 0.0, "cm21_update_sphere: zeta must be positive");
     CM21_REQUIRE(R_cells >= 0.0f && R_cells <= 1024.0f, "cm21_update_sphere: R_cells=%g not in [0,1024]",
                  (double)R_cells);
-    return launch_sphere(ionized, smoothed, D, deltac, denom, zeta, dev_sum, fc_mean, R_cells, periodic ? 1 : 0,
-                         work, (hipStream_t)stream);
+    return launch_sphere(ionized, smoothed, D, cell_test(D, deltac, denom, zeta, dev_sum, fc_mean), R_cells,
+                         periodic ? 1 : 0, work, (hipStream_t)stream);
 }
 
 // Workspace carve-up of the loop driver.
@@ -255,6 +559,7 @@ struct LoopWork {
     float2* inter[kInterMax]; // fused path: intermediates (inter[0] is filt,
                               // inter[1] shares smoothed's region)
     double* partial;
+    float* cmax;              // generic path: chunk maxima of the f_coll sum
     double* sums;
     void* sphere;
     unsigned long long* mask;
@@ -291,6 +596,8 @@ LoopWork carve(void* base, int D, int n_radii, int update) {
     }
     w.partial = (double*)(p + off);
     off = align_up(off + cm21_reduce_workspace_bytes(), 256);
+    w.cmax = (float*)(p + off);
+    off = align_up(off + sizeof(float) * kReduceBlocks, 256);
     w.sums = (double*)(p + off);
     off = align_up(off + sizeof(double) * (size_t)(n_radii > 0 ? n_radii : 1), 256);
     w.sphere = update ? (void*)(p + off) : nullptr;
@@ -616,22 +923,25 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
         t = prof_begin(CM21_STAGE_C2R, st);
         CM21_TRY(cm21_c2r(plan, w.filt, w.smoothed, stream));
         prof_end(t, st);
-        const double* sum = nullptr;
+        CellTest test = cell_test(D, prm->deltac, denoms[r], prm->zeta, prm->linear_input ? nullptr : w.sums + r,
+                                  prm->fc_mean);
         if (!prm->linear_input) {
             t = prof_begin(CM21_STAGE_FCOLL_SUM, st);
-            CM21_TRY(launch_fcoll_sum(w.smoothed, D, prm->deltac, denoms[r], w.sums + r, w.partial, st));
+            CM21_TRY(launch_fcoll_sum(w.smoothed, D, prm->deltac, denoms[r], w.sums + r, w.partial, st, &test, w.cmax,
+                                      w.scaled + r));
             prof_end(t, st);
-            sum = w.sums + r;
+            test.scaled = w.scaled + r;
+            test.cmax = w.cmax;
+            test.chunk = sum_chunk(N);
         }
         if (prm->update && !final_step) {
             t = prof_begin(CM21_STAGE_SPHERE, st);
-            CM21_TRY(launch_sphere(ionized, w.smoothed, D, prm->deltac, denoms[r], prm->zeta, sum, prm->fc_mean,
-                                   radii[r] * prm->sphere_r_scale, prm->sphere_periodic, w.sphere, st));
+            CM21_TRY(launch_sphere(ionized, w.smoothed, D, test, radii[r] * prm->sphere_r_scale,
+                                   prm->sphere_periodic, w.sphere, st));
             prof_end(t, st);
         } else {
             t = prof_begin(CM21_STAGE_THRESHOLD, st);
-            CM21_TRY(launch_threshold(ionized, w.smoothed, D, prm->deltac, denoms[r], prm->zeta, sum, prm->fc_mean,
-                                      final_step ? 1 : 0, st));
+            CM21_TRY(launch_threshold(ionized, w.smoothed, D, test, final_step ? 1 : 0, st));
             prof_end(t, st);
         }
     }
