@@ -40,7 +40,8 @@ def power_spectrum(field, box_len, edges, field_sum=None, dimensional=None):
     """(K, k_ave, ps_ave, counts) as NumPy arrays, delta_T.py:87-103."""
     dim = P.DIMENSIONAL_T_POWER_SPEC if dimensional is None else dimensional
     ps, ks, cnt = gpu.power_spectrum(field, box_len, edges, field_sum=field_sum, dimensional=dim)
-    ps, ks, cnt = ps.cpu().numpy(), ks.cpu().numpy(), cnt.cpu().numpy()
+    ps, ks, cnt = torch.stack((ps, ks, cnt.view(torch.float64))).cpu().numpy()
+    cnt = cnt.view(np.int64)
     with np.errstate(invalid="ignore", divide="ignore"):
         k_ave = np.where(cnt > 0, ks / np.maximum(cnt, 1), 0.0)
         ps_ave = np.where(cnt > 0, ps / np.maximum(cnt, 1), 0.0)

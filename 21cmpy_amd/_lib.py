@@ -129,6 +129,7 @@ SIGNATURES = {
     "cm21_move_mass": (I, [VP, VP, VP, VP, VP, I, I, F, F, I, VP]),
     "cm21_delta_T": (I, [VP, VP, VP, I, F, VP, VP, VP]),
     "cm21_pk_workspace_bytes": (SZ, [I, I]),
+    "cm21_bin_lut": (I, [VP, I, I, D, VP, VP]),
     "cm21_power_spectrum": (I, [VP, VP, VP, I, D, VP, I, I, VP, VP, VP, VP, SZ, VP]),
     "cm21_profile_enable": (I, [I]),
     "cm21_profile_collect": (I, [c_double_p, ctypes.POINTER(ctypes.c_int64), I]),

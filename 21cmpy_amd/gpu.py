@@ -214,6 +214,18 @@ def bin_lut(D, box_len, edges):
     return b
 
 
+def _device_bin_lut(D, box_len, edges):
+    """``bin_lut`` as a device tensor; for ascending edges made there."""
+    e = np.ascontiguousarray(edges, dtype=np.float64)
+    if not (e.ndim == 1 and 1 <= e.size <= 512 and D % 2 == 0 and np.all(e[1:] >= e[:-1])):
+        return torch.from_numpy(bin_lut(D, box_len, edges)).to(_DEV)
+    lut = torch.empty(3 * (D // 2) ** 2 + 1, dtype=torch.int32, device=_DEV)
+    dev = torch.from_numpy(e).to(_DEV)
+    _lib.call("cm21_bin_lut", _lib.ptr(dev), e.size, D, 2.0 * np.pi / float(box_len), _lib.ptr(lut),
+              _lib.stream_handle())
+    return lut
+
+
 def power_spectrum(field, box_len, edges, field_sum=None, dimensional=False, lut=None):
     """(ps_sum, k_sum, counts) device tensors for the spherically binned
     Delta^2(k) of (field/mean - 1)."""
@@ -223,14 +235,14 @@ def power_spectrum(field, box_len, edges, field_sum=None, dimensional=False, lut
     if field_sum is None:
         field_sum = field.double().sum().reshape(1)
     if lut is None:
-        lut = torch.from_numpy(bin_lut(D, box_len, edges)).to(_DEV)
+        lut = _device_bin_lut(D, box_len, edges)
     if lut.dtype != torch.int32 or lut.numel() != 3 * (D // 2) ** 2 + 1 or not lut.is_cuda:
         raise ValueError(f"bin LUT must be a CUDA int32 tensor of {3 * (D // 2) ** 2 + 1} entries")
     if not 1 <= nb <= 512:
         raise ValueError("1 <= number of bins <= 512")
-    ps = torch.empty(nb, dtype=torch.float64, device=_DEV)
-    ks = torch.empty(nb, dtype=torch.float64, device=_DEV)
-    cnt = torch.empty(nb, dtype=torch.int64, device=_DEV)
+    # one buffer, so that a caller can fetch the three in one copy
+    ps, ks, cnt = torch.empty((3, nb), dtype=torch.float64, device=_DEV).unbind(0)
+    cnt = cnt.view(torch.int64)
     nbytes = _lib.query("cm21_pk_workspace_bytes", D, nb)
     work = torch.empty(nbytes, dtype=torch.uint8, device=_DEV)
     _lib.call("cm21_power_spectrum", _lib.plan(D).handle, _lib.ptr(field), _lib.ptr(field_sum), D, float(box_len),

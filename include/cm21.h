@@ -231,6 +231,10 @@ int cm21_delta_T(float* dT, const float* xH, const float* delta, int D,
  * the device, deterministically.  1 <= nbins <= 512.  field_sum is the FP64 device sum of field.
  * `work` holds at least cm21_pk_workspace_bytes(D, nbins) bytes. */
 size_t cm21_pk_workspace_bytes(int D, int nbins);
+/* lut[m2], m2 = 0 .. 3(D/2)^2: the first of the nbins ascending upper edges (on
+ * the device) that is not below dk sqrt(m2); nbins past the last, -1 for m2 = 0. */
+int cm21_bin_lut(const double* edges, int nbins, int D, double dk, int32_t* lut,
+                 void* stream);
 int cm21_power_spectrum(cm21_plan* plan, const float* field,
                         const double* field_sum, int D, double box_len,
                         const int32_t* bin_lut, int nbins, int dimensional,
