@@ -74,7 +74,7 @@ def init(DIM=None, HII_DIM=None, BOX_LEN=None, seed=0, box_id=0, pspec="planck",
             raise ValueError(f"pspec must be 'planck', 'powerlaw' or a spectrum object, not {pspec!r}")
         table = pk_table(DIM, L, None if isinstance(pspec, str) else pspec)
         spec = gpu.grf_init_table(DIM, L, table[0], table[1], seed, box_id)
-    deltax = gpu.c2r(spec)                                   # initialize.py:79-82
+    deltax = gpu.inverse(spec)                                 # initialize.py:79-82
     R = smoothing_radius(L, HII_DIM)
     # initialize.py:86-109: the smoothed box and the displacement boxes, picked to HII_DIM
     smoothed, *vs = gpu.smoothed_fields(spec, L, HII_DIM, R, displacements=with_velocity)

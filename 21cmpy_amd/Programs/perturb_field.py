@@ -124,9 +124,9 @@ def velocities_at(z, deltax, HII_DIM=None, box_len=None, ddt_over_d=None, save=F
     if DIM % HII:
         raise ValueError(f"HII_DIM={HII} must divide DIM={DIM}")
     f = planck.ddt_growth_over_growth(float(z)) if ddt_over_d is None else float(ddt_over_d)
-    spec = gpu.r2c(deltax)  # DIM^3 times the c2r-ready spectrum
     R = initialize.smoothing_radius(L, HII)
-    vs = gpu.smoothed_fields(spec, L, HII, R, smoothed=False, scale=np.float32(f / float(DIM) ** 3))
+    # the spectrum is DIM^3 times the c2r-ready one
+    vs = gpu.box_fields(deltax, L, HII, R, smoothed=False, scale=np.float32(f / float(DIM) ** 3))
     if save:
         d = os.path.join(out_dir or P.IO_DIR, "Boxes")
         os.makedirs(d, exist_ok=True)

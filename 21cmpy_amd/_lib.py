@@ -126,6 +126,10 @@ SIGNATURES = {
     "cm21_subsample": (I, [VP, VP, I, I, F, VP]),
     "cm21_velocity": (I, [VP, VP, I, F, I, I, F, VP]),
     "cm21_fold_fields": (I, [VP, VP, I, I, F, F, F, I, I, VP]),
+    "cm21_fold_box_workspace_bytes": (SZ, [I]),
+    "cm21_fold_box": (I, [VP, VP, VP, I, I, F, F, F, I, I, VP, SZ, VP]),
+    "cm21_inverse_workspace_bytes": (SZ, [I]),
+    "cm21_inverse": (I, [VP, VP, VP, VP, SZ, VP]),
     "cm21_move_mass": (I, [VP, VP, VP, VP, VP, I, I, F, F, I, VP]),
     "cm21_delta_T": (I, [VP, VP, VP, I, F, VP, VP, VP]),
     "cm21_pk_workspace_bytes": (SZ, [I, I]),

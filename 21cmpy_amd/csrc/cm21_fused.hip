@@ -537,6 +537,83 @@ __global__ __launch_bounds__(W* D1, 6) void k_fwd_columns(const float2* __restri
                                    reinterpret_cast<float2*>(lds));
 }
 
+// Whole c2r of a half spectrum S[a][b][c] (no window): columns along a into the
+// padded rows T[p][b][c], rows along b in place, lines along c into the box.
+// Bound by memory, three passes over the half box: 261 + 231 + 278 us at 512^3, at
+// 4.1 to 4.9 TB/s, where a large copy runs at 4.7 (the library's transform, which
+// overwrites its input, 1460 us and 200 for a copy of it); 79 us at 256^3 (152 and
+// 22).  A block has 16 columns or more, 128 bytes of a line.
+template <int D1, int D2, int W>
+struct InverseTile {
+    static constexpr int D = D1 * D2, H = D / 2 + 1, HO = padded_row(H), NCG = (H + W - 1) / W;
+    static_assert(D % 8 == 0, "whole lines per XCD");
+    // The column groups of a line follow each other on one XCD, so that a 128-byte
+    // line of S that two groups share is fetched into one L2: blocks go to
+    // the eight XCDs in turn.
+    __device__ static __forceinline__ void of_block(int x, int* line, int* group) {
+        const int i = x >> 3;
+        *line = (x & 7) + 8 * (i / NCG);
+        *group = i % NCG;
+    }
+};
+
+template <int D1, int D2, int W>
+__global__ __launch_bounds__(W* D1) void k_inv_columns(const float2* __restrict__ S, float2* __restrict__ T,
+                                                      const float2* __restrict__ tw) {
+    using I = InverseTile<D1, D2, W>;
+    constexpr int D = I::D, H = I::H;
+    __shared__ float lds[W * (D + 1)];
+    int b, group;
+    I::of_block(blockIdx.x, &b, &group);
+    const int t = threadIdx.x, n1 = t / W, c0 = group * W, c = c0 + t % W;
+    float2 v[D2];
+#pragma unroll
+    for (int n2 = 0; n2 < D2; ++n2)
+        v[n2] = c < H ? S[((size_t)(n1 + D1 * n2) * D + b) * H + c] : make_float2(0.0f, 0.0f);
+    dft<D2>(v);
+    transpose_finish<D1, D2, W, 0>(v, tw, reinterpret_cast<float2*>(lds), [&](int jj, int k2, int k1, float2 u) {
+        if (c0 + jj < H) T[((size_t)(k2 + D2 * k1) * D + b) * I::HO + c0 + jj] = u;
+    });
+}
+
+template <int D1, int D2, int W>
+__global__ __launch_bounds__(W* D1) void k_inv_rows(float2* __restrict__ T, const float2* __restrict__ tw) {
+    using I = InverseTile<D1, D2, W>;
+    constexpr int D = I::D, H = I::H;
+    __shared__ float lds[W * (D + 1)];
+    int p, group;
+    I::of_block(blockIdx.x, &p, &group);
+    const int t = threadIdx.x, n1 = t / W, c0 = group * W, c = c0 + t % W;
+    float2 v[D2];
+#pragma unroll
+    for (int n2 = 0; n2 < D2; ++n2)
+        v[n2] = c < H ? T[((size_t)p * D + n1 + D1 * n2) * I::HO + c] : make_float2(0.0f, 0.0f);
+    dft<D2>(v);
+    transpose_finish<D1, D2, W, 0>(v, tw, reinterpret_cast<float2*>(lds), [&](int jj, int k2, int k1, float2 u) {
+        if (c0 + jj < H) T[((size_t)p * D + k2 + D2 * k1) * I::HO + c0 + jj] = u;
+    });
+}
+
+template <int N1, int N2, int L>
+__global__ __launch_bounds__(L* N1) void k_inv_lines(const float2* __restrict__ T, float2* __restrict__ out,
+                                                    const float2* __restrict__ tw) {
+    using C = LinesCore<N1, N2, L>;
+    __shared__ float2 buf[L * C::HP];
+    __shared__ float2 stw[C::D];
+    const int t = threadIdx.x;
+    const size_t line0 = (size_t)blockIdx.x * L;
+    float2 tmp[C::LOADS];
+    C::load(T + line0 * C::HO, C::HO, C::H, tmp);
+    for (int q = t; q < C::D; q += C::NT) stw[q] = tw[q];
+    C::store(tmp, buf);
+    __syncthreads();
+    C::transform(buf, stw);
+    for (int f = t; f < L * C::N; f += C::NT) {
+        const int i = f / C::N, m = f - i * C::N;
+        out[line0 * C::N + f] = buf[i * C::HP + m];
+    }
+}
+
 __global__ void k_fill_u64(unsigned long long* __restrict__ p, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0ull;
@@ -583,6 +660,18 @@ int launch_forward(const float* delta, float2* T0, float2* S, const float2* tw, 
 }
 
 template <int D1, int D2, int W, int N1, int N2, int L>
+int launch_inverse(const float2* S, float2* T, float* out, const float2* tw, hipStream_t st) {
+    using I = InverseTile<D1, D2, W>;
+    k_inv_columns<D1, D2, W><<<I::D * I::NCG, W * D1, 0, st>>>(S, T, tw);
+    CM21_LAUNCH_CHECK("k_inv_columns");
+    k_inv_rows<D1, D2, W><<<I::D * I::NCG, W * D1, 0, st>>>(T, tw);
+    CM21_LAUNCH_CHECK("k_inv_rows");
+    k_inv_lines<N1, N2, L><<<I::D * I::D / L, L * N1, 0, st>>>(T, reinterpret_cast<float2*>(out), tw);
+    CM21_LAUNCH_CHECK("k_inv_lines");
+    return CM21_OK;
+}
+
+template <int D1, int D2, int W, int N1, int N2, int L>
 int launch_all(const AllRadii& a, const float2* tw, hipStream_t st) {
     constexpr int NT = W * D1;
     auto timed = [&](int stage, auto&& launch, const char* name) {
@@ -613,20 +702,26 @@ int launch_all(const AllRadii& a, const float2* tw, hipStream_t st) {
     return timed(CM21_STAGE_FUSED_LINES, [&] { k_all_paint<N1, N2, L><<<a.nblk, NT, 0, st>>>(a, tw); }, "k_all_paint");
 }
 
-// D, all radii, lines (N1, N2, L), radius (columns/rows D1, D2, W; lines N1, N2, L), forward
+// D, all radii, lines (N1, N2, L), radius (columns/rows D1, D2, W; lines N1, N2, L), forward, inverse
 const FusedShape kShapes[] = {
     {64, launch_all<8, 8, 32, 4, 8, 64>, launch_lines<4, 8, 64>,
-     launch_radius<8, 8, 32, 4, 8, 64>, launch_forward<8, 8, 32, 4, 8, 64>, 32, 64},
+     launch_radius<8, 8, 32, 4, 8, 64>, launch_forward<8, 8, 32, 4, 8, 64>, launch_inverse<8, 8, 32, 4, 8, 64>,
+     32, 64},
     {96, launch_all<8, 12, 32, 4, 12, 64>, launch_lines<4, 12, 64>,
-     launch_radius<8, 12, 32, 4, 12, 64>, launch_forward<8, 12, 32, 4, 12, 64>, 32, 64},
+     launch_radius<8, 12, 32, 4, 12, 64>, launch_forward<8, 12, 32, 4, 12, 64>, launch_inverse<8, 12, 32, 4, 12, 64>,
+     32, 64},
     {128, launch_all<8, 16, 32, 8, 8, 32>, launch_lines<8, 8, 32>,
-     launch_radius<8, 16, 32, 8, 8, 32>, launch_forward<8, 16, 32, 8, 8, 32>, 32, 32},
+     launch_radius<8, 16, 32, 8, 8, 32>, launch_forward<8, 16, 32, 8, 8, 32>, launch_inverse<8, 16, 32, 8, 8, 32>,
+     32, 32},
     {160, launch_all<16, 10, 16, 8, 10, 32>, launch_lines<8, 10, 32>,
-     launch_radius<16, 10, 16, 8, 10, 32>, launch_forward<16, 10, 16, 8, 10, 32>, 16, 32},
+     launch_radius<16, 10, 16, 8, 10, 32>, launch_forward<16, 10, 16, 8, 10, 32>, launch_inverse<16, 10, 16, 8, 10, 32>,
+     16, 32},
     {256, nullptr, launch_lines<16, 8, 16>,
-     launch_radius<16, 16, 16, 16, 8, 16>, launch_forward<16, 16, 16, 16, 8, 16>, 16, 16},
+     launch_radius<16, 16, 16, 16, 8, 16>, launch_forward<16, 16, 16, 16, 8, 16>, launch_inverse<16, 16, 16, 16, 8, 16>,
+     16, 16},
     {512, nullptr, launch_lines<16, 16, 8>,
-     launch_radius<16, 32, 8, 16, 16, 8>, launch_forward<16, 32, 8, 16, 16, 8>, 8, 8},
+     launch_radius<16, 32, 8, 16, 16, 8>, launch_forward<16, 32, 8, 16, 16, 8>, launch_inverse<16, 32, 16, 16, 16, 8>,
+     8, 8},
 };
 
 const FusedShape* fused_shape(int D) {

@@ -170,6 +170,7 @@ struct FusedShape {
     int (*lines)(const float2* U, const float2* tw, int cmax, const LineEpilogue&, hipStream_t);
     int (*radius)(const RadiusRoles&, const AskRoles&, const float2* tw, hipStream_t);
     int (*forward)(const float* delta, float2* T0, float2* S, const float2* tw, const FusedParams& fp, hipStream_t);
+    int (*inverse)(const float2* S, float2* T, float* out, const float2* tw, hipStream_t);
     int W, L;  // columns per column group, lines per line group
 };
 

@@ -9,6 +9,7 @@
 
 #include "cm21_internal.hpp"
 #include "cm21_window.hpp"
+#include "cm21_fused_api.hpp"
 
 using namespace cm21;
 
@@ -228,12 +229,15 @@ __global__ void k_velocity(float2* __restrict__ out, const float2* __restrict__ 
 // What bounds it: the writes of the small spectra (four of 68 MB at d = 256)
 // and the FP64 sine and cosine of the window, 8.4 M modes instead of the 67 M
 // of the 512^3 spectrum.  At 512 -> 256 it takes 216 us and the four 256^3
-// inverse transforms 600 us, for a filter (585 us), three displacement passes
+// inverse transforms 316 us, for a filter (585 us), three displacement passes
 // (3 x 500), four 512^3 transforms (4 x 1450) and four picks (4 x 50):
-// initial conditions 10.2 -> 3.0 ms, velocity boxes at z 7.4 -> 2.1 ms.
+// initial conditions 10.2 -> 1.89 ms with the transform of the whole box at 775,
+// perturbed density and velocity boxes 9.6 -> 1.37 ms with the pruned forward
+// transform.  The strides are those of the spectrum's first two axes.
 __global__ void k_fold_fields(float2* __restrict__ out, const float2* __restrict__ in, int D, int d, WindowParams wp,
-                              float scale, int bm, long m2max, int smoothed, int velocity) {
-    const int H = D / 2 + 1, h = d / 2 + 1;
+                              float scale, int bm, long m2max, int smoothed, int velocity, size_t stride_a,
+                              size_t stride_b) {
+    const int h = d / 2 + 1;
     const int mc = blockIdx.x * kModeBlockX + threadIdx.x, mb = blockIdx.y * kModeBlockY + threadIdx.y;
     const int ma = blockIdx.z;
     if (mc >= h || mb >= d) return;
@@ -260,7 +264,7 @@ __global__ void k_fold_fields(float2* __restrict__ out, const float2* __restrict
                 bool cut;
                 window_of(sqrt_rn(ksq), wp, w0, cut, w2);
                 if (cut) continue;
-                float2 v = in[((size_t)a * D + b) * H + c];
+                float2 v = in[a * stride_a + b * stride_b + c];
                 const float sgn = neg ? -1.0f : 1.0f;
                 if (smoothed) {
                     const float2 r = apply_window(v, w0, false, w2, scale);
@@ -353,23 +357,83 @@ extern "C" int cm21_velocity(void* spec_out, const void* spec_in, int D, float d
     return CM21_OK;
 }
 
-extern "C" int cm21_fold_fields(void* spec_out, const void* spec_in, int D, int sw, float delta_k, float R,
-                                float scale, int smoothed, int velocity, void* stream) {
-    CM21_REQUIRE(spec_out && spec_in, "cm21_fold_fields: NULL spectrum");
-    CM21_REQUIRE(valid_dim(D), "cm21_fold_fields: D=%d must be even in [2,2048]", D);
-    CM21_REQUIRE(valid_dim(sw) && sw <= D && D % sw == 0, "cm21_fold_fields: sw=%d must be even and divide D=%d", sw, D);
-    CM21_REQUIRE(smoothed || velocity, "cm21_fold_fields: no field asked for");
-    CM21_REQUIRE(delta_k > 0.0f, "cm21_fold_fields: delta_k must be positive");
-    // the type-0 window cuts kR > 1/0.413566994 (the kernel's float32 test
-    // decides inside a shell of 1e-5)
+namespace {
+// The type-0 window cuts kR > 1/0.413566994 (the kernel's float32 test decides
+// inside a shell of 1e-5): the largest |n|^2 and |n| it can keep.
+void fold_reach(int D, float delta_k, float R, long* m2max, int* bm) {
     const int hd = D / 2;
     const double all = 3.0 * hd * hd, kcut = 1.0 / (0.413566994 * (double)delta_k * (double)R);
     const double m2 = std::floor(kcut * kcut * (1.0 + 1e-5));
-    const long m2max = (R > 0.0f && m2 < all) ? (long)m2 : (long)all;
-    const int bm = (int)std::min<double>(std::sqrt((double)m2max) + 1.0, (double)hd);
+    *m2max = (R > 0.0f && m2 < all) ? (long)m2 : (long)all;
+    *bm = (int)std::min<double>(std::sqrt((double)*m2max) + 1.0, (double)hd);
+}
+
+int fold(float2* out, const float2* in, int D, int sw, float delta_k, float R, float scale, int smoothed, int velocity,
+         size_t stride_a, size_t stride_b, hipStream_t st) {
+    long m2max;
+    int bm;
+    fold_reach(D, delta_k, R, &m2max, &bm);
     WindowParams wp{delta_k, R, 0, 1, 1};
-    k_fold_fields<<<mode_grid(sw, sw / 2 + 1), mode_block(), 0, (hipStream_t)stream>>>(
-        (float2*)spec_out, (const float2*)spec_in, D, sw, wp, scale, bm, m2max, smoothed ? 1 : 0, velocity ? 1 : 0);
+    k_fold_fields<<<mode_grid(sw, sw / 2 + 1), mode_block(), 0, st>>>(out, in, D, sw, wp, scale, bm, m2max,
+                                                                     smoothed ? 1 : 0, velocity ? 1 : 0, stride_a,
+                                                                     stride_b);
     CM21_LAUNCH_CHECK("k_fold_fields");
     return CM21_OK;
+}
+
+int check_fold(const char* fn, const void* out, const void* in, int D, int sw, float delta_k, int smoothed,
+               int velocity) {
+    CM21_REQUIRE(out && in, "%s: NULL argument", fn);
+    CM21_REQUIRE(valid_dim(D), "%s: D=%d must be even in [2,2048]", fn, D);
+    CM21_REQUIRE(valid_dim(sw) && sw <= D && D % sw == 0, "%s: sw=%d must be even and divide D=%d", fn, sw, D);
+    CM21_REQUIRE(smoothed || velocity, "%s: no field asked for", fn);
+    CM21_REQUIRE(delta_k > 0.0f, "%s: delta_k must be positive", fn);
+    return CM21_OK;
+}
+
+size_t padded_spectrum_bytes(int D) { return align_up(sizeof(float2) * D * D * padded_row(D / 2 + 1), 256); }
+}  // namespace
+
+extern "C" int cm21_fold_fields(void* spec_out, const void* spec_in, int D, int sw, float delta_k, float R,
+                                float scale, int smoothed, int velocity, void* stream) {
+    CM21_TRY(check_fold("cm21_fold_fields", spec_out, spec_in, D, sw, delta_k, smoothed, velocity));
+    const size_t H = D / 2 + 1;
+    return fold((float2*)spec_out, (const float2*)spec_in, D, sw, delta_k, R, scale, smoothed, velocity, D * H, H,
+                (hipStream_t)stream);
+}
+
+extern "C" size_t cm21_fold_box_workspace_bytes(int D) { return fused_shape(D) ? 2 * padded_spectrum_bytes(D) : 0; }
+
+extern "C" int cm21_fold_box(cm21_plan* plan, void* spec_out, const float* box, int D, int sw, float delta_k, float R,
+                             float scale, int smoothed, int velocity, void* work, size_t work_bytes, void* stream) {
+    CM21_TRY(check_fold("cm21_fold_box", spec_out, box, D, sw, delta_k, smoothed, velocity));
+    const FusedShape* sh = fused_shape(D);
+    CM21_REQUIRE(plan && plan_dim(plan) == D && sh, "cm21_fold_box: no transform of D=%d", D);
+    CM21_REQUIRE(work && work_bytes >= cm21_fold_box_workspace_bytes(D) && ((uintptr_t)box & 7) == 0,
+                 "cm21_fold_box: workspace %zu bytes < required %zu, or a box not aligned to 8 bytes", work_bytes,
+                 cm21_fold_box_workspace_bytes(D));
+    float2* T = (float2*)work;
+    float2* S = (float2*)((char*)work + padded_spectrum_bytes(D));
+    long m2max;
+    FusedParams fp{};
+    fold_reach(D, delta_k, R, &m2max, &fp.bm);
+    fp.m2max = (int)m2max;
+    fp.cmax = fp.bm;
+    CM21_TRY(fused_forward(*sh, box, T, S, plan_twiddles(plan), fp, (hipStream_t)stream));
+    const size_t row = padded_row(D / 2 + 1);  // S is b-major
+    return fold((float2*)spec_out, S, D, sw, delta_k, R, scale, smoothed, velocity, row, D * row, (hipStream_t)stream);
+}
+
+extern "C" size_t cm21_inverse_workspace_bytes(int D) { return fused_shape(D) ? padded_spectrum_bytes(D) : 0; }
+
+extern "C" int cm21_inverse(cm21_plan* plan, const void* spec, float* out, void* work, size_t work_bytes,
+                            void* stream) {
+    CM21_REQUIRE(plan && spec && out && work, "cm21_inverse: NULL argument");
+    const int D = plan_dim(plan);
+    const FusedShape* sh = fused_shape(D);
+    CM21_REQUIRE(sh, "cm21_inverse: no transform of D=%d", D);
+    CM21_REQUIRE(work_bytes >= cm21_inverse_workspace_bytes(D) && (((uintptr_t)out | (uintptr_t)spec) & 7) == 0,
+                 "cm21_inverse: workspace %zu bytes < required %zu, or an operand not aligned to 8 bytes", work_bytes,
+                 cm21_inverse_workspace_bytes(D));
+    return sh->inverse((const float2*)spec, (float2*)work, out, plan_twiddles(plan), (hipStream_t)stream);
 }

@@ -70,6 +70,22 @@ def hii_filter(spec, box_len, R, filter_type=1, ref_fallthrough=True, korder=0, 
     return out
 
 
+def inverse(spec, work=None):
+    """``c2r`` of a Hermitian spectrum, which stays as it is, into a new box.  For the sides
+    of the library's own transforms (64, 96, 128, 160, 256, 512) those, through
+    ``work`` (uint8, cm21_inverse_workspace_bytes(D)) or a buffer of the call."""
+    D = spec.shape[0]
+    _check_spec(spec, D, "spec")
+    nbytes = _lib.query("cm21_inverse_workspace_bytes", D)
+    if not nbytes or spec.data_ptr() % 8:
+        return c2r(spec)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=spec.device) if work is None else work
+    out = torch.empty((D, D, D), dtype=torch.float32, device=spec.device)
+    _lib.call("cm21_inverse", _lib.plan(D).handle, _lib.ptr(spec), _lib.ptr(out), _lib.ptr(work), work.numel(),
+              _lib.stream_handle())
+    return out
+
+
 def fcoll_sum(smoothed, deltac, denom):
     D = smoothed.shape[0]
     _check_box(smoothed, D, "smoothed")
@@ -175,7 +191,30 @@ def smoothed_fields(spec, box_len, sw, R, smoothed=True, displacements=True, sca
     fold = torch.empty((n, sw, sw, sw // 2 + 1), dtype=torch.complex64, device=spec.device)
     _lib.call("cm21_fold_fields", _lib.ptr(fold), _lib.ptr(spec), D, int(sw), delta_k(box_len), float(R), float(scale),
               1 if smoothed else 0, 1 if displacements else 0, _lib.stream_handle())
-    return [c2r(f, preserve_input=False) for f in fold]
+    return _inverse_all(fold)
+
+
+def _inverse_all(specs):
+    nbytes = _lib.query("cm21_inverse_workspace_bytes", specs.shape[1])
+    work = torch.empty(nbytes, dtype=torch.uint8, device=specs.device) if nbytes else None
+    return [inverse(f, work) for f in specs]
+
+
+def box_fields(box, box_len, sw, R, smoothed=True, displacements=True, scale=1.0):
+    """``smoothed_fields`` of a real box (its spectrum is cm21_r2c's)."""
+    D = box.shape[0]
+    _check_box(box, D, "box")
+    nbytes = _lib.query("cm21_fold_box_workspace_bytes", D) if sw >= 2 and sw % 2 == 0 and D % sw == 0 else 0
+    if not nbytes or box.data_ptr() % 8:
+        return smoothed_fields(r2c(box), box_len, sw, R, smoothed, displacements, scale)
+    n = int(bool(smoothed)) + 3 * int(bool(displacements))
+    fold = torch.empty((n, sw, sw, sw // 2 + 1), dtype=torch.complex64, device=box.device)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=box.device)
+    _lib.call("cm21_fold_box", _lib.plan(D).handle, _lib.ptr(fold), _lib.ptr(box), D, int(sw), delta_k(box_len),
+              float(R), float(scale), 1 if smoothed else 0, 1 if displacements else 0, _lib.ptr(work), nbytes,
+              _lib.stream_handle())
+    del work
+    return _inverse_all(fold)
 
 
 def move_mass(deltax, vx, vy, vz, disp_scale, growth_init, scheme="cic", out=None):

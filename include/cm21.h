@@ -206,6 +206,17 @@ int cm21_velocity(void* spec_out, const void* spec_in, int D, float delta_k,
 int cm21_fold_fields(void* spec_out, const void* spec_in, int D, int sw, float delta_k, float R, float scale,
                      int smoothed, int velocity, void* stream);
 
+/* cm21_r2c of a real box followed by cm21_fold_fields, with a transform that
+ * forms only the modes the window keeps, and the unnormalised inverse transform
+ * of a half spectrum that leaves it as it is (of a Hermitian spectrum; otherwise like
+ * cm21_c2r).  Both for the sides whose workspace query is not 0 (64, 96, 128,
+ * 160, 256, 512); `work` holds at least that many bytes. */
+size_t cm21_fold_box_workspace_bytes(int D);
+int cm21_fold_box(cm21_plan* plan, void* spec_out, const float* box, int D, int sw, float delta_k, float R,
+                  float scale, int smoothed, int velocity, void* work, size_t work_bytes, void* stream);
+size_t cm21_inverse_workspace_bytes(int D);
+int cm21_inverse(cm21_plan* plan, const void* spec, float* out, void* work, size_t work_bytes, void* stream);
+
 /* ------------------------------------------------------------------ perturb
  * Replaces move_mass + the renormalisation (Programs/perturb_field.cu:90-133;
  * perturb_field.py:93-105): the DIM^3 particles at cell centres move by
