@@ -24,44 +24,40 @@ __device__ inline uint4 philox4x32_10(uint4 c, uint2 k) {
             k.x += 0x9E3779B9u;
             k.y += 0xBB67AE85u;
         }
-        const uint32_t hi0 = __umulhi(0xD2511F53u, c.x), lo0 = 0xD2511F53u * c.x;
-        const uint32_t hi1 = __umulhi(0xCD9E8D57u, c.z), lo1 = 0xCD9E8D57u * c.z;
-        c = make_uint4(hi1 ^ c.y ^ k.x, lo1, hi0 ^ c.w ^ k.y, lo0);
+        // one 64-bit product instruction for both halves (they run at a quarter of
+        // the rate of an add: with the ten rounds' halves apart, most of k_grf)
+        const uint64_t p0 = (uint64_t)0xD2511F53u * c.x, p1 = (uint64_t)0xCD9E8D57u * c.z;
+        c = make_uint4((uint32_t)(p1 >> 32) ^ c.y ^ k.x, (uint32_t)p1, (uint32_t)(p0 >> 32) ^ c.w ^ k.y, (uint32_t)p0);
     }
     return c;
 }
 
 // Box-Muller in float32, r = sqrt(-2 ln a), theta = 2 pi b, with the
 // uniforms a = ((u0 >> 8) + 0.5) 2^-24 and b likewise, handled so that no
-// argument is rounded: a = m 2^-25 with m = 2 (u0 >> 8) + 1 is an exact float
-// when a <= 1/2, and 1 - a is one otherwise (ln a = log1p(-(1 - a))); 2b =
-// m' 2^-24 is exact below 1, and 2b - 1 is exact above (sin and cos change
+// argument is rounded: a = m 2^-25 with m = 2 (u0 >> 8) + 1 is its nearest float f
+// and an exact remainder d, ln a = ln f + d/f (the next term is below 2^-26 of it);
+// 2b = m' 2^-24 is exact below 1, and 2b - 1 is exact above (sin and cos change
 // sign), so sincospi sees an exact argument.  Each result is within a few
 // float32 ulp of the FP64 values.
 __device__ inline void box_muller(uint32_t u0, uint32_t u1, float& g1, float& g2) {
     const uint32_t m0 = 2u * (u0 >> 8) + 1u;
-    const float lna = m0 < (1u << 24) ? logf(ldexpf((float)m0, -25))
-                                      : log1pf(-ldexpf((float)((1u << 25) - m0), -25));
+    const float f = (float)m0, d = (float)(int)(m0 - (uint32_t)f);
+    const float lna = fmaf(d, __builtin_amdgcn_rcpf(f), logf(f * 0x1p-25f));
     const float r = sqrtf(-2.0f * lna);
     const uint32_t m1 = 2u * (u1 >> 8) + 1u;
+    const uint32_t half = m1 & (1u << 24);
     float s, c;
-    if (m1 < (1u << 24)) {
-        sincospif(ldexpf((float)m1, -24), &s, &c);
-    } else {
-        sincospif(ldexpf((float)(m1 - (1u << 24)), -24), &s, &c);
-        s = -s;
-        c = -c;
-    }
-    g1 = r * c;
-    g2 = r * s;
+    sincospif((float)(m1 ^ half) * 0x1p-24f, &s, &c);
+    g1 = r * (half ? -c : c);
+    g2 = r * (half ? -s : s);
 }
 
 struct GrfParams {
-    float dkf;              // 2 pi / box_len
-    float amp_over_volume;  // P(k) normalisation / box_len^3
-    float n_indexf;         // spectral slope
-    float inv_k_cut;        // 1 / Gaussian cut-off scale
-    float inv_volume;       // 1 / box_len^3
+    float dkf;          // 2 pi / box_len
+    float norm;         // power law: sqrt(P(k) normalisation / box_len^3 * dk^n), and the
+    float quarter_n;    // exponents of the amplitude norm * exp2(quarter_n log2 |n|^2
+    float half_cut;     //   - half_cut |n|^2)
+    float inv_volume;   // 1 / box_len^3
     uint32_t seed, box_id;
     const float* ktab;  // tabulated P(k): increasing K (NULL = power law)
     const float* ptab;
@@ -105,6 +101,7 @@ __device__ inline float table_pk(float k, const float* K, const float* Pt, int n
 }
 
 // One mode: its Philox draw, amplitude and Hermitian placement.
+template <bool TABLE>
 __device__ __forceinline__ void grf_mode(float2* __restrict__ spec, int D, int a, int b, int c, const GrfParams& gp,
                                          const float* sK, const float* sP, const TableGuess& tg) {
     const int H = D / 2 + 1;
@@ -116,27 +113,32 @@ __device__ __forceinline__ void grf_mode(float2* __restrict__ spec, int D, int a
     // Modes on the c = 0 and c = D/2 planes pair with (-a, -b) in the same
     // plane; the pair shares the random numbers of its lower linear index.
     const bool edge = (c == 0) || (c == D / 2);
-    const int ma = (D - a) % D, mb = (D - b) % D;
-    const long lin_self = (long)a * D + b, lin_mirror = (long)ma * D + mb;
+    const int ma = a ? D - a : 0, mb = b ? D - b : 0;
+    const int lin_self = a * D + b, lin_mirror = ma * D + mb;  // below 2^22
     const bool use_mirror = edge && lin_mirror < lin_self;
-    const bool selfconj = edge && ma == a && mb == b;
-    const long ra = use_mirror ? ma : a, rb = use_mirror ? mb : b;
-    const unsigned long long rep = ((unsigned long long)(ra * D + rb)) * (unsigned long long)H + (unsigned long long)c;
+    const bool selfconj = edge && lin_mirror == lin_self;
+    const uint64_t rep = (uint64_t)(uint32_t)(use_mirror ? lin_mirror : lin_self) * (uint32_t)H + (uint32_t)c;
     const uint4 u = philox4x32_10(make_uint4((uint32_t)rep, (uint32_t)(rep >> 32), 0u, 0u), make_uint2(gp.seed, gp.box_id));
     float g1, g2;
     box_muller(u.x, u.y, g1, g2);
 
-    // |n|^2 is an exact integer; k and the amplitude in float32
+    // |n|^2 is an exact integer (and an exact float); the amplitude in float32
     const int na = mode_of(a, D), nb = mode_of(b, D);
-    const float k = gp.dkf * sqrtf((float)(na * na + nb * nb + c * c));
+    const float m2 = (float)(na * na + nb * nb + c * c);
     float amp;
-    if (gp.ntab > 0) {
-        amp = sqrtf(table_pk(k, sK, sP, gp.ntab, tg) * gp.inv_volume);
+    if (TABLE) {
+        amp = sqrtf(table_pk(gp.dkf * sqrtf(m2), sK, sP, gp.ntab, tg) * gp.inv_volume);
     } else {
-        const float x = k * gp.inv_k_cut;
-        // k^n as exp2(n log2 k) (k > 0 here): about 1e-6 relative, a third of
-        // the instructions of powf
-        amp = sqrtf(gp.amp_over_volume * (exp2f(gp.n_indexf * log2f(k)) * expf(-(x * x))));
+        // sqrt(k^n exp(-(k/k_cut)^2)) by one log2 and one exp2 of the hardware (1 ulp
+        // each).  With |n|^2 = f 2^e, f in [1, 2), the power of 2^e goes into the result's
+        // exponent and the logarithm stays below 1: 9e-8 rms of the mode (1.5e-7
+        // with exp2f(n log2f(k)), expf and sqrtf, twice the instructions)
+        const int e = __builtin_amdgcn_frexp_expf(m2) - 1;
+        const float f = 2.0f * __builtin_amdgcn_frexp_mantf(m2);
+        const float whole = rintf(gp.quarter_n * (float)e);
+        const float x = fmaf(gp.quarter_n, (float)e, -whole) +
+                        fmaf(gp.quarter_n, __builtin_amdgcn_logf(f), -gp.half_cut * m2);
+        amp = ldexpf(gp.norm * __builtin_amdgcn_exp2f(x), (int)whole);
     }
     if (selfconj) {
         spec[idx] = make_float2(amp * g1, 0.0f);
@@ -146,30 +148,39 @@ __device__ __forceinline__ void grf_mode(float2* __restrict__ spec, int D, int a
     }
 }
 
-// Blocks of 64 x 4 threads; block (0, y, z) covers a = z and the kGrfRows
-// rows b from y * kGrfRows, its 256 threads walking the rows' modes as one
-// run (no lane idles at the end of each row of D/2+1 modes), so the P(k)
-// table is loaded into LDS once per kGrfRows * H modes.
+// Block (0, y, z) covers a = z and the kGrfRows rows b from y * kGrfRows, its 256
+// threads walking the rows' modes as one run (no lane idles at the end of each
+// row of D/2+1 modes), so the P(k) table is loaded into LDS once per
+// kGrfRows * H modes.  Bound by the VALU (the integer products of the ten rounds
+// first): 335 us at 512^3, 630 with the halves of the products apart, logarithm
+// and sincos twice over and a modulo in each mode; its writes alone take 115.
 constexpr int kGrfRows = 16;
 
-__global__ __launch_bounds__(kModeBlockX* kModeBlockY) void k_grf(float2* __restrict__ spec, int D, GrfParams gp) {
-    __shared__ float sK[kMaxTable], sP[kMaxTable];
-    if (gp.ntab > 0) {
-        const int t = threadIdx.y * kModeBlockX + threadIdx.x;
-        for (int i = t; i < gp.ntab; i += kModeBlockX * kModeBlockY) {
+template <bool TABLE>
+__global__ __launch_bounds__(kThreads) void k_grf(float2* __restrict__ spec, int D, GrfParams gp) {
+    __shared__ float sK[TABLE ? kMaxTable : 1], sP[TABLE ? kMaxTable : 1];
+    if (TABLE) {
+        for (int i = threadIdx.x; i < gp.ntab; i += kThreads) {
             sK[i] = gp.ktab[i];
             sP[i] = gp.ptab[i];
         }
         __syncthreads();
     }
-    const TableGuess tg = gp.ntab > 0 ? table_guess(sK, gp.ntab) : TableGuess{0.0f, 0.0f};
+    const TableGuess tg = TABLE ? table_guess(sK, gp.ntab) : TableGuess{0.0f, 0.0f};
     const int H = D / 2 + 1;
     const int a = blockIdx.z;
     const int b0 = blockIdx.y * kGrfRows;
-    const int n = (min(D, b0 + kGrfRows) - b0) * H;  // the block's modes, rows b0.. of plane a
-    for (int q = threadIdx.y * kModeBlockX + threadIdx.x; q < n; q += kModeBlockX * kModeBlockY) {
-        const int rb = q / H;
-        grf_mode(spec, D, a, b0 + rb, q - rb * H, gp, sK, sP, tg);
+    const int rows = min(D, b0 + kGrfRows) - b0;
+    const int dr = kThreads / H, dc = kThreads - dr * H;
+    int row = threadIdx.x / H, c = threadIdx.x - row * H;
+    while (row < rows) {
+        grf_mode<TABLE>(spec, D, a, b0 + row, c, gp, sK, sP, tg);
+        row += dr;
+        c += dc;
+        if (c >= H) {
+            c -= H;
+            ++row;
+        }
     }
 }
 
@@ -310,10 +321,11 @@ extern "C" int cm21_grf_init(void* spec_out, int D, double box_len, double amp, 
     CM21_REQUIRE(spec_out, "cm21_grf_init: NULL spectrum");
     CM21_REQUIRE(valid_dim(D), "cm21_grf_init: D=%d must be even in [2,2048]", D);
     CM21_REQUIRE(box_len > 0.0 && k_cut > 0.0 && amp >= 0.0, "cm21_grf_init: box_len, k_cut must be > 0, amp >= 0");
-    const double vol = box_len * box_len * box_len;
-    GrfParams gp{(float)(2.0 * M_PI / box_len), (float)(amp / vol), (float)n_index, (float)(1.0 / k_cut),
-                 (float)(1.0 / vol), seed, box_id, nullptr, nullptr, 0};
-    k_grf<<<grf_grid(D), mode_block(), 0, (hipStream_t)stream>>>((float2*)spec_out, D, gp);
+    const double vol = box_len * box_len * box_len, dk = 2.0 * M_PI / box_len, log2e = 1.4426950408889634;
+    GrfParams gp{(float)dk, (float)std::sqrt(amp / vol * std::pow(dk, n_index)), (float)(0.25 * n_index),
+                 (float)(0.5 * log2e * dk * dk / (k_cut * k_cut)), (float)(1.0 / vol), seed, box_id, nullptr, nullptr,
+                 0};
+    k_grf<false><<<grf_grid(D), kThreads, 0, (hipStream_t)stream>>>((float2*)spec_out, D, gp);
     CM21_LAUNCH_CHECK("k_grf");
     return CM21_OK;
 }
@@ -326,9 +338,9 @@ extern "C" int cm21_grf_init_table(void* spec_out, int D, double box_len, const 
     CM21_REQUIRE(box_len > 0.0, "cm21_grf_init_table: box_len must be > 0");
     CM21_REQUIRE(n_table >= 2 && n_table <= kMaxTable, "cm21_grf_init_table: n_table=%d not in [2,%d]", n_table,
                  kMaxTable);
-    GrfParams gp{(float)(2.0 * M_PI / box_len), 0.0f, 0.0f, 1.0f, (float)(1.0 / (box_len * box_len * box_len)),
+    GrfParams gp{(float)(2.0 * M_PI / box_len), 0.0f, 0.0f, 0.0f, (float)(1.0 / (box_len * box_len * box_len)),
                  seed, box_id, k_table, p_table, n_table};
-    k_grf<<<grf_grid(D), mode_block(), 0, (hipStream_t)stream>>>((float2*)spec_out, D, gp);
+    k_grf<true><<<grf_grid(D), kThreads, 0, (hipStream_t)stream>>>((float2*)spec_out, D, gp);
     CM21_LAUNCH_CHECK("k_grf");
     return CM21_OK;
 }
