@@ -228,39 +228,80 @@ __global__ void k_velocity(float2* __restrict__ out, const float2* __restrict__ 
     out[idx] = r;
 }
 
+// window_of's type-0 fall-through window inside its cut (kR <= 2.4181) with the
+// sine and cosine from their Taylor series in FP64 (the next terms are below 3e-15;
+// both are rounded to float32 as there) and the Gaussian from the hardware's exp2:
+// gauss = -(0.413566994 0.643)^2 log2(e) / 2.
+__device__ __forceinline__ float window_inside(float kR, float gauss) {
+    const double x = (double)kR, u = x * x;
+    float w0 = 1.0f;
+    double s = -3.86817017063068413e-23, c = -8.89679139245057408e-22;
+    s = fma(s, u, 1.95729410633912626e-20);
+    c = fma(c, u, 4.11031762331216484e-19);
+    s = fma(s, u, -8.22063524662432950e-18);
+    c = fma(c, u, -1.56192069685862253e-16);
+    s = fma(s, u, 2.81145725434552060e-15);
+    c = fma(c, u, 4.77947733238738525e-14);
+    s = fma(s, u, -7.64716373181981641e-13);
+    c = fma(c, u, -1.14707455977297245e-11);
+    s = fma(s, u, 1.60590438368216133e-10);
+    c = fma(c, u, 2.08767569878681002e-09);
+    s = fma(s, u, -2.50521083854417202e-08);
+    c = fma(c, u, -2.75573192239858883e-07);
+    s = fma(s, u, 2.75573192239858925e-06);
+    c = fma(c, u, 2.48015873015873016e-05);
+    s = fma(s, u, -1.98412698412698413e-04);
+    c = fma(c, u, -1.38888888888888894e-03);
+    s = fma(s, u, 8.33333333333333322e-03);
+    c = fma(c, u, 4.16666666666666644e-02);
+    s = fma(s, u, -1.66666666666666657e-01);
+    c = fma(c, u, -5.00000000000000000e-01);
+    s = fma(s, u, 1.0);
+    c = fma(c, u, 1.0);
+    const float p3 = (float)(u * x), p2 = (float)u;
+    const float inner = __fsub_rn(__fdiv_rn((float)(s * x), p3), __fdiv_rn((float)c, p2));
+    if (x > 1e-4) w0 = (float)(3.0 * (double)inner);
+    return w0 * __builtin_amdgcn_exp2f(gauss * p2);
+}
+
 // Spectra of boxes that are only read on every q-th cell (q = D/d): a field
 // of the D^3 grid picked at multiples of q is the inverse transform on the
 // d^3 grid of its spectrum folded modulo d, Y[m] = sum of W(n) X[n] over n = m
 // (mod d).  One thread per mode m of the small half spectrum adds the one to
 // eight modes n inside the window's cut (|n|^2 <= m2max; negative n_c through
 // the conjugate of -n), in a fixed order, and forms the smoothed spectrum and
-// the three displacement spectra i k/k^2 W X from one read of X, in the
-// arithmetic of k_filter and k_velocity.
+// the three displacement spectra i k/k^2 W X from one read of X.  The threads
+// take a plane's modes in memory order.
 //
-// What bounds it: the writes of the small spectra (four of 68 MB at d = 256)
-// and the FP64 sine and cosine of the window, 8.4 M modes instead of the 67 M
-// of the 512^3 spectrum.  At 512 -> 256 it takes 216 us and the four 256^3
-// inverse transforms 316 us, for a filter (585 us), three displacement passes
-// (3 x 500), four 512^3 transforms (4 x 1450) and four picks (4 x 50):
-// initial conditions 10.2 -> 1.89 ms with the transform of the whole box at 775,
-// perturbed density and velocity boxes 9.6 -> 1.37 ms with the pruned forward
-// transform.  The strides are those of the spectrum's first two axes.
+// What bounds it: the writes of the small spectra (four of 68 MB at d = 256) and
+// the FP64 window, of 8.4 M modes instead of the 67 M of the 512^3 spectrum.  At
+// 512 -> 256 it takes 110 us (216 with window_of and its library functions, 185
+// with those in memory order) and the four 256^3 inverse transforms 316 us, for a
+// filter (585 us), three displacement passes (3 x 500), four 512^3 transforms
+// (4 x 1450) and four picks (4 x 50): initial conditions 10.2 -> 1.52 ms with the
+// transform of the whole box at 775 and the field at 335, perturbed density and
+// velocity boxes 9.6 -> 1.11 ms with the pruned forward transform.  The strides are
+// those of the spectrum's first two axes.
 __global__ void k_fold_fields(float2* __restrict__ out, const float2* __restrict__ in, int D, int d, WindowParams wp,
-                              float scale, int bm, long m2max, int smoothed, int velocity, size_t stride_a,
-                              size_t stride_b) {
+                              float scale, int bm, int m2max, int smoothed, int velocity, size_t stride_a,
+                              size_t stride_b, float gauss) {
     const int h = d / 2 + 1;
-    const int mc = blockIdx.x * kModeBlockX + threadIdx.x, mb = blockIdx.y * kModeBlockY + threadIdx.y;
-    const int ma = blockIdx.z;
-    if (mc >= h || mb >= d) return;
+    const int i = blockIdx.x * kThreads + threadIdx.x, ma = blockIdx.y;  // a plane's modes in memory order
+    if (i >= d * h) return;
+    const int mb = i / h, mc = i - mb * h;
     const int lo = -min(bm, D / 2 - 1), hi = min(bm, D / 2);  // index D/2 is the mode +D/2
     float2 y[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) y[q] = make_float2(0.0f, 0.0f);
     // the largest n <= hi with n = m (mod d), then down to lo
-    for (int na = ma + (hi - ma >= 0 ? (hi - ma) / d : -((ma - hi + d - 1) / d)) * d; na >= lo; na -= d) {
-        for (int nb = mb + (hi - mb >= 0 ? (hi - mb) / d : -((mb - hi + d - 1) / d)) * d; nb >= lo; nb -= d) {
-            for (int nc = mc + (hi - mc >= 0 ? (hi - mc) / d : -((mc - hi + d - 1) / d)) * d; nc >= lo; nc -= d) {
-                if ((long)na * na + (long)nb * nb + (long)nc * nc > m2max) continue;
+    auto first = [&](int m) { return m + (hi - m >= 0 ? (hi - m) / d : -((m - hi + d - 1) / d)) * d; };
+    const int fa = first(ma), fb = first(mb), fc = first(mc);
+    for (int na = fa; na >= lo; na -= d) {
+        for (int nb = fb; nb >= lo; nb -= d) {
+            const int left = m2max - na * na - nb * nb;
+            if (left < 0) continue;
+            for (int nc = fc; nc >= lo; nc -= d) {
+                if (nc * nc > left) continue;
                 // the stored mode: n, or -n for negative n_c
                 const bool neg = nc < 0;
                 int a = neg ? -na : na, b = neg ? -nb : nb;
@@ -271,35 +312,32 @@ __global__ void k_fold_fields(float2* __restrict__ out, const float2* __restrict
                 const float k1 = __fmul_rn((float)mode_of(b, D), wp.dk);
                 const float k2 = __fmul_rn((float)c, wp.dk);
                 const float ksq = __fadd_rn(__fadd_rn(__fmul_rn(k0, k0), __fmul_rn(k1, k1)), __fmul_rn(k2, k2));
-                float w0, w2;
-                bool cut;
-                window_of(sqrt_rn(ksq), wp, w0, cut, w2);
-                if (cut) continue;
+                const float kR = __fmul_rn(sqrt_rn(ksq), wp.R);
+                if ((float)((double)kR * 0.413566994) > 1.0f) continue;  // cut
                 float2 v = in[a * stride_a + b * stride_b + c];
-                const float sgn = neg ? -1.0f : 1.0f;
-                if (smoothed) {
-                    const float2 r = apply_window(v, w0, false, w2, scale);
-                    y[0].x += r.x;
-                    y[0].y += sgn * r.y;
-                }
+                const float w = window_inside(kR, gauss) * scale;
+                v.x *= w;
+                v.y *= neg ? -w : w;
+                y[0].x += v.x;
+                y[0].y += v.y;
                 if (velocity && ksq != 0.0f) {
+                    // i k/k^2 times the stored mode; of -n the conjugate, where k changes sign
+                    const float f = (neg ? -1.0f : 1.0f) / ksq;
                     const float kk[3] = {k0, k1, k2};
                     const int idx[3] = {a, b, c};
 #pragma unroll
                     for (int q = 0; q < 3; ++q) {
                         if (idx[q] == D / 2) continue;
-                        const float f = __fdiv_rn(kk[q], ksq);
-                        float2 r = make_float2(-__fmul_rn(f, v.y), __fmul_rn(f, v.x));  // (i f) * v
-                        r = apply_window(r, w0, false, w2, scale);
-                        y[q + 1].x += r.x;
-                        y[q + 1].y += sgn * r.y;
+                        const float g = f * kk[q];
+                        y[q + 1].x -= g * v.y;
+                        y[q + 1].y += g * v.x;
                     }
                 }
             }
         }
     }
-    const size_t nc = (size_t)d * d * h, idx = ((size_t)ma * d + mb) * h + mc;
-    float2* o = out + idx;
+    const size_t nc = (size_t)d * d * h;
+    float2* o = out + (size_t)ma * d * h + i;
     if (smoothed) {
         *o = y[0];
         o += nc;
@@ -386,9 +424,11 @@ int fold(float2* out, const float2* in, int D, int sw, float delta_k, float R, f
     int bm;
     fold_reach(D, delta_k, R, &m2max, &bm);
     WindowParams wp{delta_k, R, 0, 1, 1};
-    k_fold_fields<<<mode_grid(sw, sw / 2 + 1), mode_block(), 0, st>>>(out, in, D, sw, wp, scale, bm, m2max,
+    const double g = 0.413566994 * 0.643;
+    const float gauss = (float)(-0.5 * g * g * std::log((double)kE) / std::log(2.0));
+    k_fold_fields<<<dim3(grid_for((size_t)sw * (sw / 2 + 1)), sw), kThreads, 0, st>>>(out, in, D, sw, wp, scale, bm, (int)m2max,
                                                                      smoothed ? 1 : 0, velocity ? 1 : 0, stride_a,
-                                                                     stride_b);
+                                                                     stride_b, gauss);
     CM21_LAUNCH_CHECK("k_fold_fields");
     return CM21_OK;
 }
