@@ -233,6 +233,178 @@ __global__ __launch_bounds__(L* N1) void k_batch_lines(BatchLaunch a) {
     }
 }
 
+// ------------------------------------------------------------------ planes
+// Rows and lines of one plane p of a box in one block, where the half spectrum of a
+// plane fits LDS (up to 160): the rows pass leaves its plane there and the lines
+// work on it in place, so an intermediate is written once (columns) and read
+// once, where rows and lines of their own write it twice and read it twice.  The
+// four-step factors D1 x D2 and N1 x N2 are those of the tiles, whose arithmetic this
+// is.  A group of LG = NT/N1 lines is passed over when its cells are all ionized, or
+// when on each of its lines the sum of moduli of the modes, which bounds the field, is
+// below the threshold: asked while few modes survive and as long as it was of use at
+// the radius before.
+// 21 boxes: 64^3 0.82 -> 0.59 ms, 128^3 4.55 -> 3.69, 160^3 9.29 -> 9.00; the 64 boxes
+// of 96^3 to 160^3 14.99 -> 13.87 ms.  Bound by the VALU and, at 160^3, by the one block
+// of ten waves that fits a CU (halves of a plane per block, the first step along b
+// done twice: 10.1 ms).  Nonlinear input, whose sum needs the rows a second time, lost
+// (28 ms for 22 on those 64 boxes).
+template <int D1, int D2, int N1, int N2, int NT>
+struct Plane {
+    static constexpr int LG = NT / N1;  // lines per group
+    using C = LinesCore<N1, N2, LG>;
+    static constexpr int D = C::D, H = C::H, HP = C::HP, GROUPS = D / LG, WORDS = C::WORDS;
+    static_assert(C::NT == NT && D1 * D2 == D && GROUPS * LG == D, "whole groups");
+    struct Lds {
+        float2 P[D * HP];
+        float2 tw[D];
+        unsigned long long mask[GROUPS * WORDS];
+        float part[NT];
+    };
+
+    // P: the half lines of plane p (modes c < hs, zeros beyond), followed by a barrier.
+    __device__ static __forceinline__ void rows(const float2* __restrict__ T, const BatchRadius& R, int p, Lds& s) {
+        constexpr int ITEMS = (H * D2 + NT - 1) / NT;
+        const int t = threadIdx.x, hs = R.hs, m2max = R.fp.m2max;
+        const float2* src = T + (size_t)p * D * hs;
+        for (int it = t; it < hs * D1; it += NT) {
+            const int n1 = it / hs, c = it - n1 * hs;
+            float2 v[D2];
+#pragma unroll
+            for (int n2 = 0; n2 < D2; ++n2) {
+                const int bs = mode_of(n1 + D1 * n2, D);
+                v[n2] = bs * bs + c * c <= m2max ? src[D1 * n2 * hs + it] : make_float2(0.0f, 0.0f);
+            }
+            dft<D2>(v);
+#pragma unroll
+            for (int k2 = 0; k2 < D2; ++k2)
+                s.P[(k2 * D1 + n1) * HP + c] = (n1 * k2 == 0) ? v[k2] : cmul(v[k2], s.tw[n1 * k2]);
+        }
+        __syncthreads();
+        float2 u[ITEMS][D1];
+#pragma unroll
+        for (int q = 0; q < ITEMS; ++q) {
+            const int it = t + q * NT, k2 = it / hs, c = it - k2 * hs;
+            if (it < hs * D2) {
+#pragma unroll
+                for (int n = 0; n < D1; ++n) u[q][n] = s.P[(k2 * D1 + n) * HP + c];
+                dft<D1>(u[q]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < ITEMS; ++q) {
+            const int it = t + q * NT, k2 = it / hs, c = it - k2 * hs;
+            if (it < hs * D2) {
+#pragma unroll
+                for (int k1 = 0; k1 < D1; ++k1) s.P[(k2 + D2 * k1) * HP + c] = u[q][k1];
+            }
+        }
+        const int rest = H - hs;
+        for (int it = t; it < D * rest; it += NT) {
+            const int i = it / rest, c = hs + it - i * rest;
+            s.P[i * HP + c] = make_float2(0.0f, 0.0f);
+        }
+        __syncthreads();
+    }
+
+    // Whether every cell of the group's lines is below `lim` (uniform).
+    __device__ static __forceinline__ bool quiet(const float2* buf, int hs, float lim, float* part) {
+        const int t = threadIdx.x, i = t % LG;
+        float sum = 0.0f;
+        for (int c = t / LG; c < hs; c += N1) {
+            const float2 x = buf[i * HP + c];
+            sum += (c == 0 ? 1.0f : 2.0f) * __builtin_amdgcn_sqrtf(x.x * x.x + x.y * x.y);
+        }
+        part[t] = sum;
+        __syncthreads();
+        bool ok = true;
+        if (t < LG) {
+            for (int k = 1; k < N1; ++k) sum += part[t + k * LG];
+            ok = sum * (1.0f + 1e-4f) < lim;
+        }
+        return __syncthreads_and(ok) != 0;
+    }
+};
+
+// Threshold pass of linear input: grid (D, nbox); a block walks all radii of its
+// plane with the ionization mask of the cells in LDS.
+template <int D1, int D2, int N1, int N2, int NT, int WAVES>
+__global__ __launch_bounds__(NT, WAVES) void k_batch_planes(BatchLaunch a) {
+    using P = Plane<D1, D2, N1, N2, NT>;
+    using C = typename P::C;
+    constexpr int D = P::D, LG = P::LG, CELLS = LG * D;
+    __shared__ typename P::Lds s;
+    const int t = threadIdx.x, lane = t & 63;
+    const int p = blockIdx.x, box = blockIdx.y;
+    const float2* Tb = a.T + box * a.tbox;
+    const BatchCell* cb = a.cells + (size_t)box * a.nr;
+    float* ob = a.out + ((size_t)box * D + p) * D * D;
+    for (int q = t; q < D; q += NT) s.tw[q] = a.tw[q];
+    for (int q = t; q < P::GROUPS * P::WORDS; q += NT) s.mask[q] = 0ull;
+    __syncthreads();
+    bool ask = true;
+    unsigned done = 0;  // groups whose cells are all ionized
+    for (int r = 0; r < a.nr - 1; ++r) {
+        const BatchRadius& R = a.rad[r];
+        P::rows(Tb + R.toff, R, p, s);
+        const BatchCell& cell = cb[r];
+        const bool use_scale = cell.use_scale != 0;
+        bool of_use = false;
+        for (int g = 0; g < P::GROUPS; ++g) {
+            if (done >> g & 1u) continue;
+            float2* buf = s.P + g * LG * P::HP;
+            unsigned long long* mask = s.mask + g * P::WORDS;
+            if (ask && R.hs <= kBoundModes && P::quiet(buf, R.hs, cell.th.dstar - cell.th.band, s.part)) {
+                of_use = true;
+                continue;
+            }
+            C::transform(buf, s.tw);
+            const float* x = reinterpret_cast<const float*>(buf);
+#pragma unroll 4
+            for (int f = t; f < CELLS; f += NT) {
+                const int i = f / D, rr = f - i * D;
+                const bool hit = cell_hit(x[i * 2 * P::HP + rr], cell.th, cell.deltac, cell.denom, use_scale,
+                                          cell.scale, cell.inv_zeta);
+                const unsigned long long bits = __ballot(hit);
+                if (lane == 0) mask[f >> 6] |= bits;
+            }
+            __syncthreads();
+            bool full = true;
+            for (int q = t; q < P::WORDS; q += NT) full = full && mask[q] == ~0ull;
+            if (__syncthreads_and(full)) done |= 1u << g;
+        }
+        ask = of_use;
+        if (done == (1u << P::GROUPS) - 1u) {  // the final paint is 1 everywhere
+            for (int f = t; f < D * D; f += NT) ob[f] = 1.0f;
+            return;
+        }
+        __syncthreads();
+    }
+    const int r = a.nr - 1;
+    P::rows(Tb + a.rad[r].toff, a.rad[r], p, s);
+    const BatchCell& cell = cb[r];
+    const bool use_scale = cell.use_scale != 0;
+    for (int g = 0; g < P::GROUPS; ++g) {
+        float2* buf = s.P + g * LG * P::HP;
+        if (done >> g & 1u) {
+            for (int f = t; f < CELLS; f += NT) ob[g * CELLS + f] = 1.0f;
+            continue;
+        }
+        C::transform(buf, s.tw);
+        const float* x = reinterpret_cast<const float*>(buf);
+#pragma unroll 4
+        for (int f = t; f < CELLS; f += NT) {
+            const int i = f / D, rr = f - i * D;
+            const float delta = x[i * 2 * P::HP + rr];
+            const bool was = (s.mask[g * P::WORDS + (f >> 6)] >> (f & 63)) & 1ull;
+            float val = 1.0f;
+            if (!was && !cell_hit(delta, cell.th, cell.deltac, cell.denom, use_scale, cell.scale, cell.inv_zeta))
+                val = final_value(delta, cell.deltac, cell.denom, use_scale, cell.scale, cell.zeta, cell.inv_zeta);
+            ob[g * CELLS + f] = val;
+        }
+    }
+}
+
 // ------------------------------------------------------------------ tiles
 
 using LaunchFn = int (*)(const BatchLaunch&, hipStream_t);
@@ -264,13 +436,20 @@ int launch_bsum(const BatchLaunch& a, hipStream_t st) {
     return CM21_OK;
 }
 
+template <int D1, int D2, int N1, int N2, int NT, int WAVES>
+int launch_bplanes(const BatchLaunch& a, hipStream_t st) {
+    k_batch_planes<D1, D2, N1, N2, NT, WAVES><<<dim3(D1 * D2, a.nbox), NT, 0, st>>>(a);
+    CM21_LAUNCH_CHECK("k_batch_planes");
+    return CM21_OK;
+}
+
 struct ColTile {
-    int W;
+    int W, factor;  // D1
     LaunchFn cols, rows;
     const char* name;
 };
 struct LineTile {
-    int L;
+    int L, factor;  // N1
     LaunchFn lines, sum;
     const char* name;
 };
@@ -280,24 +459,30 @@ struct BatchShape {
     int ncols;
     LineTile lines[4];
     int nlines;
+    LaunchFn planes;  // rows and lines in one, with the factors of the first tiles, or NULL
+    int planes_from;  // boxes from which on it is the faster way
 };
 
-#define CM21_COL(D1, D2, W) {W, launch_bcols<D1, D2, W>, launch_brows<D1, D2, W>, #D1 "x" #D2 "/W" #W}
-#define CM21_LINE(N1, N2, L) {L, launch_blines<N1, N2, L>, launch_bsum<N1, N2, L>, #N1 "x" #N2 "/L" #L}
+#define CM21_COL(D1, D2, W) {W, D1, launch_bcols<D1, D2, W>, launch_brows<D1, D2, W>, #D1 "x" #D2 "/W" #W}
+#define CM21_LINE(N1, N2, L) {L, N1, launch_blines<N1, N2, L>, launch_bsum<N1, N2, L>, #N1 "x" #N2 "/L" #L}
 
 // Candidate tiles per D; the first of each list is the default (the shape of
 // the single-box loop, so that defaults reproduce it exactly).
 const BatchShape kBatchShapes[] = {
     {64, {CM21_COL(8, 8, 32), CM21_COL(8, 8, 16), CM21_COL(16, 4, 16)}, 3,
-     {CM21_LINE(4, 8, 64), CM21_LINE(8, 4, 32), CM21_LINE(4, 8, 32)}, 3},
+     {CM21_LINE(4, 8, 64), CM21_LINE(8, 4, 32), CM21_LINE(4, 8, 32)}, 3,
+     launch_bplanes<8, 8, 4, 8, 256, 8>, 12},
     {96, {CM21_COL(8, 12, 32), CM21_COL(8, 12, 16), CM21_COL(16, 6, 16)}, 3,
-     {CM21_LINE(4, 12, 64), CM21_LINE(8, 6, 32), CM21_LINE(4, 12, 32), CM21_LINE(6, 8, 32)}, 4},
+     {CM21_LINE(4, 12, 64), CM21_LINE(8, 6, 32), CM21_LINE(4, 12, 32), CM21_LINE(6, 8, 32)}, 4,
+     launch_bplanes<8, 12, 4, 12, 384, 5>, 8},
     {128, {CM21_COL(8, 16, 32), CM21_COL(16, 8, 16), CM21_COL(8, 16, 16)}, 3,
-     {CM21_LINE(8, 8, 32), CM21_LINE(4, 16, 64), CM21_LINE(8, 8, 16), CM21_LINE(16, 4, 16)}, 4},
+     {CM21_LINE(8, 8, 32), CM21_LINE(4, 16, 64), CM21_LINE(8, 8, 16), CM21_LINE(16, 4, 16)}, 4,
+     launch_bplanes<8, 16, 8, 8, 512, 4>, 4},
     {160, {CM21_COL(16, 10, 16), CM21_COL(8, 20, 32), CM21_COL(16, 10, 8)}, 3,
-     {CM21_LINE(8, 10, 32), CM21_LINE(4, 20, 64), CM21_LINE(8, 10, 16), CM21_LINE(16, 5, 16)}, 4},
-    {256, {CM21_COL(16, 16, 16), CM21_COL(16, 16, 8)}, 2, {CM21_LINE(16, 8, 16), CM21_LINE(8, 16, 32)}, 2},
-    {512, {CM21_COL(16, 32, 8)}, 1, {CM21_LINE(16, 16, 8)}, 1},
+     {CM21_LINE(8, 10, 32), CM21_LINE(4, 20, 64), CM21_LINE(8, 10, 16), CM21_LINE(16, 5, 16)}, 4,
+     launch_bplanes<16, 10, 8, 10, 640, 3>, 12},
+    {256, {CM21_COL(16, 16, 16), CM21_COL(16, 16, 8)}, 2, {CM21_LINE(16, 8, 16), CM21_LINE(8, 16, 32)}, 2, nullptr, 0},
+    {512, {CM21_COL(16, 32, 8)}, 1, {CM21_LINE(16, 16, 8)}, 1, nullptr, 0},
 };
 
 #undef CM21_COL
@@ -307,6 +492,16 @@ const BatchShape* batch_shape(int D) {
     for (const auto& s : kBatchShapes)
         if (s.D == D) return &s;
     return nullptr;
+}
+
+// Whether a group runs as planes: linear input, tiles of the planes' factors, and
+// enough boxes for the longer blocks to fill the chip.  Planes against rows and lines
+// apart: 64^3 0.96 times as fast with 8 boxes, 1.13 with 12, 1.39 with 21; 96^3 0.94 with
+// 6, 1.12 with 8, 1.00 with 21, 1.16 with 24; 128^3 0.92 with 2, 1.10 with 4, 1.05 with 5,
+// 1.26 with 17; 160^3 0.95 with 4, 1.00 with 9, 1.02 with 13.
+bool as_planes(const BatchShape& s, int nbox, int col_tile, int line_tile, const cm21_bubble_params* prm) {
+    return s.planes && prm->linear_input && nbox >= s.planes_from && s.cols[col_tile].factor == s.cols[0].factor &&
+           s.lines[line_tile].factor == s.lines[0].factor;
 }
 
 int min_lines_per_block(const BatchShape& s) {
@@ -504,19 +699,20 @@ int run_forward(const GroupHost& h, hipStream_t st, char* work) {
     return cm21_r2c(h.g->plan, h.g->delta, work + h.o_S, (void*)st);
 }
 
-int run_transforms(const GroupHost& h, const BatchLaunch& a, int col_tile, hipStream_t st) {
+int run_transforms(const GroupHost& h, const BatchLaunch& a, int col_tile, bool planes, hipStream_t st) {
     const ColTile& ct = h.shape->cols[col_tile];
     ProfToken t = prof_begin(CM21_STAGE_FUSED_COLUMNS, st);
     CM21_TRY(ct.cols(a, st));
     prof_end(t, st);
+    if (planes) return CM21_OK;
     t = prof_begin(CM21_STAGE_FUSED_ROWS, st);
     CM21_TRY(ct.rows(a, st));
     prof_end(t, st);
     return CM21_OK;
 }
 
-int run_threshold(const GroupHost& h, const BatchLaunch& a, int line_tile, const cm21_bubble_params* prm,
-                  hipStream_t st) {
+int run_threshold(const GroupHost& h, const BatchLaunch& a, int line_tile, bool planes,
+                  const cm21_bubble_params* prm, hipStream_t st) {
     const LineTile& lt = h.shape->lines[line_tile];
     if (!prm->linear_input) {
         ProfToken t = prof_begin(CM21_STAGE_FCOLL_SUM, st);
@@ -529,7 +725,7 @@ int run_threshold(const GroupHost& h, const BatchLaunch& a, int line_tile, const
     k_batch_thresholds<<<(n + 63) / 64, 64, 0, st>>>(a, (double)h.N);
     CM21_LAUNCH_CHECK("k_batch_thresholds");
     ProfToken t = prof_begin(CM21_STAGE_FUSED_LINES, st);
-    CM21_TRY(lt.lines(a, st));
+    CM21_TRY((planes ? h.shape->planes : lt.lines)(a, st));
     prof_end(t, st);
     return CM21_OK;
 }
@@ -539,6 +735,7 @@ struct Prepared {
     std::vector<char> blob;
     std::vector<BatchLaunch> launches;
     std::vector<int> col_tile, line_tile;
+    std::vector<char> planes;
 };
 
 int prepare(const cm21_batch_group* groups, int ngroups, const cm21_bubble_params* prm, void* work,
@@ -552,12 +749,15 @@ int prepare(const cm21_batch_group* groups, int ngroups, const cm21_bubble_param
     p.launches.clear();
     p.col_tile.clear();
     p.line_tile.clear();
+    p.planes.clear();
     for (const auto& h : p.lay.groups) {
         const int ct = tile_or_default(h.g->tile_columns);
         const int lt = tile_or_default(h.g->tile_lines);
         int cb = 0, rb = 0;
         fill_tables(h, prm, ct, p.blob, &cb, &rb);
+        const bool planes = as_planes(*h.shape, h.nbox, ct, lt, prm);
         p.launches.push_back(make_launch(h, (char*)work, cb, rb, h.D * h.D / h.shape->lines[lt].L));
+        p.planes.push_back(planes);
         p.col_tile.push_back(ct);
         p.line_tile.push_back(lt);
     }
@@ -574,8 +774,8 @@ int run_group(const Prepared& p, size_t i, const cm21_bubble_params* prm, void* 
     ProfToken t = prof_begin(CM21_STAGE_R2C, gs);
     CM21_TRY(run_forward(h, gs, (char*)work));
     prof_end(t, gs);
-    CM21_TRY(run_transforms(h, p.launches[i], p.col_tile[i], gs));
-    CM21_TRY(run_threshold(h, p.launches[i], p.line_tile[i], prm, gs));
+    CM21_TRY(run_transforms(h, p.launches[i], p.col_tile[i], p.planes[i], gs));
+    CM21_TRY(run_threshold(h, p.launches[i], p.line_tile[i], p.planes[i], prm, gs));
     return CM21_OK;
 }
 
@@ -748,17 +948,17 @@ extern "C" int cm21_batch_autotune(cm21_batch_group* groups, int ngroups, const 
         rc = upload(p, work, st);
         if (rc == CM21_OK) rc = run_forward(h, st, (char*)work);
         // columns/rows candidates (idempotent: S -> T)
-        double best = 1e300;
+        double best = 1e300, apart = 0.0;
         int best_c = 0;
         for (int c = 0; c < h.shape->ncols && rc == CM21_OK; ++c) {
             int cb = 0, rb = 0;
             fill_tables(h, params, c, p.blob, &cb, &rb);
             BatchLaunch a = make_launch(h, (char*)work, cb, rb, p.launches[0].nblk);
             rc = upload(p, work, st);
-            if (rc == CM21_OK) rc = run_transforms(h, a, c, st);  // warm
+            if (rc == CM21_OK) rc = run_transforms(h, a, c, false, st);  // warm
             if (rc != CM21_OK) break;
             if (hipEventRecord(e0, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
-            for (int i = 0; i < reps && rc == CM21_OK; ++i) rc = run_transforms(h, a, c, st);
+            for (int i = 0; i < reps && rc == CM21_OK; ++i) rc = run_transforms(h, a, c, false, st);
             if (rc == CM21_OK && hipEventRecord(e1, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
             float ms = 0.0f;
             if (rc == CM21_OK) rc = elapsed(&ms);
@@ -769,20 +969,21 @@ extern "C" int cm21_batch_autotune(cm21_batch_group* groups, int ngroups, const 
             }
         }
         if (rc != CM21_OK) break;
+        apart = best;
         // leave T from the chosen columns tile, then time the threshold stage
         int cb = 0, rb = 0;
         fill_tables(h, params, best_c, p.blob, &cb, &rb);
         rc = upload(p, work, st);
         BatchLaunch a = make_launch(h, (char*)work, cb, rb, p.launches[0].nblk);
-        if (rc == CM21_OK) rc = run_transforms(h, a, best_c, st);
+        if (rc == CM21_OK) rc = run_transforms(h, a, best_c, false, st);
         best = 1e300;
         int best_l = 0;
         for (int l = 0; l < h.shape->nlines && rc == CM21_OK; ++l) {
             a.nblk = h.D * h.D / h.shape->lines[l].L;
-            rc = run_threshold(h, a, l, params, st);  // warm
+            rc = run_threshold(h, a, l, false, params, st);  // warm
             if (rc != CM21_OK) break;
             if (hipEventRecord(e0, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
-            for (int i = 0; i < reps && rc == CM21_OK; ++i) rc = run_threshold(h, a, l, params, st);
+            for (int i = 0; i < reps && rc == CM21_OK; ++i) rc = run_threshold(h, a, l, false, params, st);
             if (rc == CM21_OK && hipEventRecord(e1, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
             float ms = 0.0f;
             if (rc == CM21_OK) rc = elapsed(&ms);
@@ -791,6 +992,24 @@ extern "C" int cm21_batch_autotune(cm21_batch_group* groups, int ngroups, const 
                 best = ms;
                 best_l = l;
             }
+        }
+        apart += best;
+        if (rc == CM21_OK && as_planes(*h.shape, h.nbox, 0, 0, params)) {
+            // rows and lines in one, against the best of both apart
+            fill_tables(h, params, 0, p.blob, &cb, &rb);
+            rc = upload(p, work, st);
+            a = make_launch(h, (char*)work, cb, rb, 0);
+            auto run = [&] {
+                const int e = run_transforms(h, a, 0, true, st);
+                return e == CM21_OK ? run_threshold(h, a, 0, true, params, st) : e;
+            };
+            if (rc == CM21_OK) rc = run();  // warm
+            if (rc == CM21_OK && hipEventRecord(e0, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
+            for (int i = 0; i < reps && rc == CM21_OK; ++i) rc = run();
+            if (rc == CM21_OK && hipEventRecord(e1, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
+            float ms = 0.0f;
+            if (rc == CM21_OK) rc = elapsed(&ms);
+            if (rc == CM21_OK && ms < apart) best_c = best_l = 0;
         }
         if (rc == CM21_OK) {
             groups[gi].tile_columns = best_c;
