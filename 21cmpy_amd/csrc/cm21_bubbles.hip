@@ -779,7 +779,7 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
         // The threshold pass recomputes the last-axis transform in the line
         // groups whose maximum can reach the threshold rather than storing and
         // re-reading the smoothed field; the final paint is one more launch.
-        const int nblk = (int)fused_partials(D);
+        const int nblk = D * D / sh->L;
         const bool nl = !prm->linear_input;
         auto params = [&](int r) {
             return fused_params(D, dk, radii[r], prm->filter_type, prm->ref_fallthrough, scale);

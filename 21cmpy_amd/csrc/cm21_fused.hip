@@ -40,7 +40,7 @@ namespace cm21 {
 // its own mask words).
 // A radius at which no cell can be ionized has no box sums: its list is empty.
 template <int NT>
-__device__ void finish_box_sum(const double* partial, int n, double* out, const SumScaleArgs& sa,
+__device__ void finish_box_sum(const double* partial, int n, int nblk, double* out, const SumScaleArgs& sa,
                                const ScaledThreshold* state = nullptr) {
     if (state && state->neutral) {
         if (threadIdx.x == 0 && sa.active) *sa.nactive = 0;
@@ -72,7 +72,7 @@ __device__ void finish_box_sum(const double* partial, int n, double* out, const 
     if (!sa.scaled || !sa.active) return;
     __syncthreads();
     const float lim = sth.dstar - sth.band;
-    for (int i = threadIdx.x; i < n; i += NT)
+    for (int i = threadIdx.x; i < nblk; i += NT)
         if (!(sa.bmax[i] < lim)) sa.active[atomicAdd(&count, 1)] = i;
     __syncthreads();
     if (threadIdx.x == 0) *sa.nactive = count;
@@ -100,6 +100,8 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
     using C = LinesCore<N1, N2, L>;
     constexpr int D = C::D, NT = C::NT, WORDS = C::WORDS;
     constexpr int MODE = MODE_ == kLinePaint ? (int)kLineFinal : MODE_;
+    // the lines and threads of a box-sum partial
+    constexpr int SL = sum_lines(D, L), SNT = NT / (L / SL);
     const int t = threadIdx.x;
     const size_t line0 = (size_t)blk * L;
     const size_t word0 = line0 * D / 64;
@@ -142,7 +144,7 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
     float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 4
     for (int q = 0; q < L * D / NT; ++q) {
-        const int f = t + q * NT;
+        const int f = MODE == kLineSum && SNT != NT ? t / SNT * SL * D + t % SNT + q * SNT : t + q * NT;
         const int i = f / D, r = f - i * D;
         const float delta = xrf[i * 2 * C::HP + r];
         if (MODE == kLineSum) {
@@ -176,8 +178,20 @@ __device__ __forceinline__ void lines_block(const float2* __restrict__ U, int hs
                 ep.bmax[blk] = m;
             }
         }
-        acc = block_sum(acc);
-        if (t == 0) ep.partial[blk] = acc;
+        if (SNT == NT) {
+            acc = block_sum(acc);
+            if (t == 0) ep.partial[blk] = acc;
+        } else {
+            __shared__ double wsum[NT / 64];
+            acc = wave_sum(acc);
+            if (lane == 0) wsum[t >> 6] = acc;
+            __syncthreads();
+            if (t % SNT == 0) {
+                double sum = 0.0;
+                for (int w = 0; w < SNT / 64; ++w) sum += wsum[(t >> 6) + w];
+                ep.partial[blk * (L / SL) + t / SNT] = sum;
+            }
+        }
     }
     if (MODE == kLineThreshold) {
         __syncthreads();
@@ -242,7 +256,7 @@ __device__ __forceinline__ void radius_roles(const RadiusRoles& a, const AskRole
     if (b < a.n_red) {
         const SumScaleArgs sa{a.scaled_red,   a.fc_mean,    a.deltac,     a.denom_red,    (double)D * D * D,
                               a.zeta,         a.bmax_red,   a.active_red, a.nactive_red};
-        finish_box_sum<NT>(a.partial, D * D / L, a.total, sa, ASK ? q.state_red : nullptr);
+        finish_box_sum<NT>(a.partial, D * D / sum_lines(D, L), D * D / L, a.total, sa, ASK ? q.state_red : nullptr);
         return;
     }
     b -= a.n_red;
@@ -413,7 +427,7 @@ __global__ __launch_bounds__(NT) void k_all_reduce(AllRadii a) {
     const int r = blockIdx.x;
     const SumScaleArgs sa{a.scaled + r, a.fc_mean, a.deltac, a.r[r].denom, a.ncells, a.zeta,
                           nullptr,      nullptr,   nullptr};
-    finish_box_sum<NT>(a.partial + (size_t)r * a.nblk, a.nblk, a.sums + r, sa, a.scaled + r);
+    finish_box_sum<NT>(a.partial + (size_t)r * a.nblk, a.nblk, a.nblk, a.sums + r, sa, a.scaled + r);
 }
 
 template <int N1, int N2, int L>
@@ -710,6 +724,9 @@ int launch_all(const AllRadii& a, const float2* tw, hipStream_t st) {
     return timed(CM21_STAGE_FUSED_LINES, [&] { k_all_paint<N1, N2, L><<<a.nblk, NT, 0, st>>>(a, tw); }, "k_all_paint");
 }
 
+// At 512^3 blocks of 256 threads on 16 columns (128 bytes) and 16 lines: 11.0 ms a box
+// with linear input and 14.3 with nonlinear, against 14.1 and 17.4 with blocks of 128 on
+// eight, whose 64-byte pieces fetched a line's halves into two L2s.
 // D, all radii, lines (N1, N2, L), radius (columns/rows D1, D2, W; lines N1, N2, L), forward, inverse
 const FusedShape kShapes[] = {
     {64, launch_all<8, 8, 32, 4, 8, 64>, launch_lines<4, 8, 64>,
@@ -727,9 +744,9 @@ const FusedShape kShapes[] = {
     {256, nullptr, launch_lines<16, 8, 16>,
      launch_radius<16, 16, 16, 16, 8, 16>, launch_forward<16, 16, 16, 16, 8, 16>, launch_inverse<16, 16, 16, 16, 8, 16>,
      16, 16},
-    {512, nullptr, launch_lines<16, 16, 8>,
-     launch_radius<16, 32, 8, 16, 16, 8>, launch_forward<16, 32, 16, 16, 16, 8>, launch_inverse<16, 32, 16, 16, 16, 8>,
-     8, 8},
+    {512, nullptr, launch_lines<16, 16, 16>,
+     launch_radius<16, 32, 16, 16, 16, 16>, launch_forward<16, 32, 16, 16, 16, 8>, launch_inverse<16, 32, 16, 16, 16, 8>,
+     16, 16},
 };
 
 const FusedShape* fused_shape(int D) {
@@ -740,7 +757,7 @@ const FusedShape* fused_shape(int D) {
 
 size_t fused_partials(int D) {
     const FusedShape* s = fused_shape(D);
-    return s ? (size_t)D * D / s->L : 0;
+    return s ? (size_t)D * D / sum_lines(D, s->L) : 0;
 }
 
 // Per-radius bounds of the pruned transforms.
@@ -873,7 +890,7 @@ static double erfcinv_host(double y) {
 // from the denominators and sigma_min^2 from fc_mean, where it is given.  This
 // only decides whether to ask: boxes that would never pass keep the shorter
 // schedule (asking in vain costs 2 % at 256^3).  With it a 256^3 box takes 1664
-// us for 1822 (nonlinear, half ionized) and a 512^3 one 14.1 ms for 15.8 (linear).
+// us for 1822 (nonlinear, half ionized) and a 512^3 one (blocks of eight columns) 14.1 ms for 15.8 (linear).
 int neutral_radii(const cm21_bubble_params& prm, const float* denoms, int n_radii, const int* cmax) {
     const double dc = prm.deltac, fc = prm.fc_mean;
     double smin = 0.5 * (double)denoms[0] * denoms[0];  // S at the largest radius counted as 0

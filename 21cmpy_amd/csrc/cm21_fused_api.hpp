@@ -164,6 +164,10 @@ struct AllRadii {
     float* out;
 };
 
+// Lines of a box-sum partial: those of a line group, but eight at side 512, where
+// a group has 16 (the float32 sums of a thread cover the cells of eight lines).
+__host__ __device__ constexpr int sum_lines(int D, int L) { return D == 512 && L > 8 ? 8 : L; }
+
 struct FusedShape {
     int D;
     int (*all)(const AllRadii&, const float2* tw, hipStream_t);
