@@ -29,7 +29,8 @@
 //   Input layer (density plus two constant conditioning channels, the
 //   latter folded into a per-sample bias): 3^3 taps on the fp32 matrix cores
 //   (v_mfma_f32_16x16x4f32), forward and weight gradient.
-//   2x2x2 stride-2 transposed convolution: bf16 matrix cores.
+//   2x2x2 stride-2 transposed convolution: bf16 matrix cores forward and
+//   input gradient, fp32 matrix cores (K = 4 voxels) weight gradient.
 //   2x2x2 average pooling, the 1^3 head with sigmoid + binary cross entropy
 //   (fused into the last convolution for inference), and AdamW: fp32 VALU.
 #include <cmath>
@@ -74,6 +75,7 @@ __device__ __forceinline__ u32x4 mask8(u32x4 x, u32x4 m) {
     return r;
 }
 
+__device__ __forceinline__ bool pos_bf(bf16_t m) { return m != 0 && !(m & 0x8000u); }
 
 // ------------------------------------------------------------------ 3^3 conv (MFMA)
 
@@ -900,6 +902,67 @@ __global__ __launch_bounds__(256) void k_sum_blocks(const float* __restrict__ pa
 }
 inline unsigned sum_blocks_grid(int n) { return (unsigned)((n + kSumOut - 1) / kSumOut); }
 
+// Per-sample channel sums of a (masked) gradient over a chunk of one
+// sample's voxels per block: partial[b][blk][c].  Each thread reads 16-byte
+// vectors of 8 channels; lanes with the same vector slot are added in a
+// fixed order at the end.
+__global__ __launch_bounds__(256) void k_channel_partials(const bf16_t* __restrict__ g,
+                                                          const bf16_t* __restrict__ mask, int C,
+                                                          size_t vox_per_sample, float* __restrict__ partial) {
+    __shared__ float red[256 * 8];
+    const int b = blockIdx.y;
+    const int vc = C / 8;  // 16-byte vectors per voxel (C in {16, 32, 64})
+    const int t = threadIdx.x;
+    const int cv = t % vc, lanes = 256 / vc, l = t / vc;
+    const size_t per = (vox_per_sample + gridDim.x - 1) / gridDim.x;
+    const size_t v0 = (size_t)blockIdx.x * per;
+    const size_t v1 = v0 + per < vox_per_sample ? v0 + per : vox_per_sample;
+    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (size_t v = v0 + l; v < v1; v += lanes) {
+        const size_t idx = ((size_t)b * vox_per_sample + v) * C + cv * 8;
+        u32x4 q = *(const u32x4*)(g + idx);
+        if (mask) q = mask8(q, *(const u32x4*)(mask + idx));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            s[2 * k] += __uint_as_float(q[k] << 16);
+            s[2 * k + 1] += __uint_as_float(q[k] & 0xffff0000u);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) red[t * 8 + k] = s[k];
+    __syncthreads();
+    if (t < C) {
+        const int c8 = t / 8, k = t % 8;
+        float acc = 0.0f;
+        for (int q = 0; q < lanes; ++q) acc += red[(q * vc + c8) * 8 + k];
+        partial[((size_t)b * gridDim.x + blockIdx.x) * C + t] = acc;
+    }
+}
+
+// per_sample[b][c] = sum_blk partial[b][blk][c]; total[c] = sum_b per_sample[b][c]
+// (either output may be NULL).
+// One block per channel, one thread per partial block (nblk <= 128): for each
+// sample the 128 partials are added by a fixed butterfly within each wave and
+// the two wave sums in order; the samples in order.
+__global__ __launch_bounds__(128) void k_channel_final(const float* __restrict__ partial, int B, int nblk, int C,
+                                                       float* __restrict__ per_sample, float* __restrict__ total) {
+    __shared__ float ws[2];
+    const int c = blockIdx.x, k = threadIdx.x, lane = k & 63, w = k >> 6;
+    float tot = 0.0f;
+    for (int b = 0; b < B; ++b) {
+        float v = k < nblk ? partial[((size_t)b * nblk + k) * C + c] : 0.0f;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        if (lane == 0) ws[w] = v;
+        __syncthreads();
+        const float s = ws[0] + ws[1];
+        __syncthreads();
+        if (k == 0 && per_sample) per_sample[b * C + c] = s;
+        tot += s;
+    }
+    if (k == 0 && total) total[c] = tot;
+}
+
 // ------------------------------------------------------------------ pooling
 
 // One thread per (output voxel, 8 channels): eight 16-byte loads, the mean
@@ -929,44 +992,7 @@ __global__ __launch_bounds__(64) void k_pool_fwd(const bf16_t* __restrict__ x, b
     *(u32x4*)(y + ((((size_t)b * Dh + oz) * Dh + oy) * Dh + ox) * C + cc) = o;
 }
 
-// dx += dy / 8 (or =): a thread owns 8 channels of the four voxels of an x
-// column under one pooled (z, y), so the lanes of a wave cover whole x-lines of
-// dx with 16-byte accesses and dy is read once per column.  Bound by HBM (dx
-// read and written): 268 MB of dx at 128^3, batch 4, take 80 us (383 with
-// one thread per element).  Channel counts that are no multiple of 8 keep the
-// form per element.
-__global__ __launch_bounds__(256) void k_pool_bwd(const bf16_t* __restrict__ dy, bf16_t* __restrict__ dx, int D, int C,
-                                                  int add) {
-    const int Dh = D / 2, C8 = C / 8;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= D * C8) return;
-    const int x = i / C8, cc = (i - x * C8) * 8;
-    const int yh = blockIdx.y, zh = blockIdx.z % Dh, b = blockIdx.z / Dh;
-    const u32x4 g = *(const u32x4*)(dy + ((((size_t)b * Dh + zh) * Dh + yh) * Dh + x / 2) * C + cc);
-    bf16_t* p = dx + ((((size_t)b * D + 2 * zh) * D + 2 * yh) * D + x) * C + cc;
-    const size_t sy = (size_t)D * C, sz = sy * D;
-    u32x4 v[4];
-    if (add) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = *(const u32x4*)(p + (q >> 1) * sz + (q & 1) * sy);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        u32x4 o;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float lo = __uint_as_float(g[k] << 16) * 0.125f, hi = __uint_as_float(g[k] & 0xffff0000u) * 0.125f;
-            if (add) {
-                lo += __uint_as_float(v[q][k] << 16);
-                hi += __uint_as_float(v[q][k] & 0xffff0000u);
-            }
-            o[k] = f2bf2(lo, hi);
-        }
-        *(u32x4*)(p + (q >> 1) * sz + (q & 1) * sy) = o;
-    }
-}
-
-__global__ void k_pool_bwd_any(const bf16_t* __restrict__ dy, bf16_t* __restrict__ dx, int B, int D, int C, int add) {
+__global__ void k_pool_bwd(const bf16_t* __restrict__ dy, bf16_t* __restrict__ dx, int B, int D, int C, int add) {
     const int Dh = D / 2;
     const size_t n = (size_t)B * D * D * D * C;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
@@ -1114,137 +1140,143 @@ __global__ void k_pack_up(const float* __restrict__ w, bf16_t* __restrict__ wn, 
     wk[(size_t)ci * 8 * cout + k] = h;
 }
 
-// Weight and bias gradients of the transposed conv on
-// v_mfma_f32_16x16x32_bf16: dW[co][s][ci] = sum_v dy[2v+s][co] x[v][ci],
-// db[co] = sum_u dy[u][co].  A tile is four input x-lines (of any y, z and
-// sample) of 16 voxels and the 4 x 32 output voxels under each, channels-last
-// in LDS (16-channel chunks, 40 bytes a voxel); K = 32 input voxels, two lines.
-// Wave (sz, sy) forms its two sub-positions: fragments come from lane pairs as
-// in the 3^3 weight gradient, dy's at every other voxel; the bias is one more
-// product against ones, its waves added with the blocks.  Lines past the last
-// and voxels past the side are zeros, so every side is taken.
-//
-// What bounds it: HBM (dy and x once: 335 MB for 32 -> 16 at 64^3 -> 128^3,
-// batch 4).  68 us there, bias included; the fp32 form that loaded both
-// operands two bytes a lane took 271 us and the channel sums of dy 65.
-template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void k_up_wgrad(const bf16_t* __restrict__ x, const bf16_t* __restrict__ dy,
-                                                  float* __restrict__ partial, int B, int D, int tiles_per_block) {
-    constexpr int NTI = CIN / 16, NTC = COUT / 16, VS = 20, TL = 4;
-    constexpr int XPL = TL * 16 * VS, GPL = TL * 4 * 32 * VS;  // one chunk: x lines, dy rows (line, sz, sy)
-    constexpr int NPX = TL * 16 * (CIN / 8) / 256, NPG = TL * 4 * 32 * (COUT / 8) / 256;
-    static_assert(TL * 16 * (CIN / 8) % 256 == 0 && TL * 4 * 32 * (COUT / 8) % 256 == 0, "whole rounds");
-    __shared__ __attribute__((aligned(16))) bf16_t xs[NTI * XPL];
-    __shared__ __attribute__((aligned(16))) bf16_t gs[NTC * GPL];
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // 2 sz + sy
+// dW[co][s][ci] = sum_v dy[2v+s][co] x[v][ci]: block partials over voxel
+// ranges; each thread owns 4 x 4 (co, ci) for all 8 s; sets split voxels.
+// Matrix-core weight gradient of the transposed conv on
+// v_mfma_f32_16x16x4f32: dW[co][s][ci] = sum_v dy[2v+s][co] x[v][ci].  K = 4
+// voxels per product, one per lane group, so both operands come straight
+// from the channels-last tensors (bf16 -> fp32 is exact): lane (row, grp)
+// supplies dy[out(voxel grp, s)][16 cot + row] and x[voxel grp][16 cit + row].
+// Grid: (blocks over x-lines, groups of SPW sub-positions); wave w takes the
+// 4-voxel steps 4 w, 4 w + 16, ... of each line and keeps SPW x cout/16 x
+// cin/16 accumulator tiles; the waves are added in a fixed order at the end.
+template <int CIN, int COUT, int SPW>
+__global__ __launch_bounds__(256) void k_up_wgrad_mfma(const bf16_t* __restrict__ x, const bf16_t* __restrict__ dy,
+                                                       float* __restrict__ partial, int B, int D,
+                                                       int lines_per_block) {
+    constexpr int NTC = COUT / 16, NTI = CIN / 16;
+    static_assert(CIN % 16 == 0 && COUT % 16 == 0 && 8 % SPW == 0, "shapes");
+    __shared__ floatx4 red[3][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, grp = lane >> 4;
-    const unsigned sel = (row & 1) ? 0x03020706u : 0x05040100u;
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-    const int nlines = B * D * D, nx = (D + 15) / 16, ntiles = (nlines + TL - 1) / TL * nx;
+    const int s0 = blockIdx.y * SPW;
     const size_t D2 = 2 * (size_t)D;
-    floatx4 acc[2][NTC][NTI], accb[NTC];
+    floatx4 acc[SPW][NTC][NTI];
 #pragma unroll
-    for (int n = 0; n < NTC; ++n) {
-        accb[n] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int m = 0; m < NTI; ++m) acc[h][n][m] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    bf16x8 ones;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
-    u32x4 px[NPX], pg[NPG];
-    auto fetch = [&](int tile) {
-        const int x0 = tile % nx * 16, L0 = tile / nx * TL;
-#pragma unroll
-        for (int q = 0; q < NPX; ++q) {
-            const int i = t + q * 256;
-            const int ch = i % (CIN / 8) * 8, v = i / (CIN / 8), L = L0 + v / 16, xx = x0 + v % 16;
-            px[q] = L < nlines && xx < D ? *(const u32x4*)(x + ((size_t)L * D + xx) * CIN + ch) : zero;
-        }
-#pragma unroll
-        for (int q = 0; q < NPG; ++q) {
-            const int i = t + q * 256;
-            const int ch = i % (COUT / 8) * 8, v = i / (COUT / 8);
-            const int L = L0 + v / 128, sr = v / 32 & 3, xx = 2 * x0 + v % 32;
-            const int yy = L % D, zz = L / D % D, b = L / (D * D);
-            const size_t u = ((b * D2 + 2 * zz + (sr >> 1)) * D2 + 2 * yy + (sr & 1)) * D2 + xx;
-            pg[q] = L < nlines && xx < 2 * D ? *(const u32x4*)(dy + u * COUT + ch) : zero;
-        }
-    };
-    const int t0 = blockIdx.x * tiles_per_block, t1 = min(t0 + tiles_per_block, ntiles);
-    if (t0 < t1) fetch(t0);
-    for (int tile = t0; tile < t1; ++tile) {
-        __syncthreads();  // the previous tile is consumed
-#pragma unroll
-        for (int q = 0; q < NPX; ++q) {
-            const int i = t + q * 256, ch = i % (CIN / 8) * 8;
-            bf16_t* p = xs + ch / 16 * XPL + i / (CIN / 8) * VS + ch % 16;
-            *(u32x2*)p = u32x2{px[q][0], px[q][1]};
-            *(u32x2*)(p + 4) = u32x2{px[q][2], px[q][3]};
-        }
-#pragma unroll
-        for (int q = 0; q < NPG; ++q) {
-            const int i = t + q * 256, ch = i % (COUT / 8) * 8;
-            bf16_t* p = gs + ch / 16 * GPL + i / (COUT / 8) * VS + ch % 16;
-            *(u32x2*)p = u32x2{pg[q][0], pg[q][1]};
-            *(u32x2*)(p + 4) = u32x2{pg[q][2], pg[q][3]};
-        }
-        __syncthreads();
-        if (tile + 1 < t1) fetch(tile + 1);
-#pragma unroll
-        for (int k = 0; k < TL / 2; ++k) {
-            // this lane's eight voxels: line 2 k + grp / 2, x = 8 (grp % 2) + 0 .. 7
-            const int l = 2 * k + (grp >> 1), xv = (grp & 1) * 8 + (row & 1);
-            bf16x8 bx[NTI];
-#pragma unroll
-            for (int m = 0; m < NTI; ++m) {
-                u32x4 v;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    v[i] = voxel_pair(xs + m * XPL + (l * 16 + xv + 2 * i) * VS + (row >> 1) * 2, sel);
-                bx[m] = __builtin_bit_cast(bf16x8, v);
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int n = 0; n < NTC; ++n) {
-                    u32x4 v;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        v[i] = voxel_pair(
-                            gs + n * GPL + ((l * 4 + wave) * 32 + 2 * (xv + 2 * i) + h) * VS + (row >> 1) * 2, sel);
-                    const bf16x8 ga = __builtin_bit_cast(bf16x8, v);
-                    accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, ones, accb[n], 0, 0, 0);
-#pragma unroll
-                    for (int m = 0; m < NTI; ++m)
-                        acc[h][n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, bx[m], acc[h][n][m], 0, 0, 0);
-                }
-        }
-    }
-    // lane: co = 16 n + 4 grp + i, ci = 16 m + row; sub-position 2 wave + h
-    float* out = partial + (size_t)blockIdx.x * (COUT * 8 * CIN + COUT);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int a = 0; a < SPW; ++a)
 #pragma unroll
         for (int n = 0; n < NTC; ++n)
 #pragma unroll
-            for (int m = 0; m < NTI; ++m)
+            for (int m = 0; m < NTI; ++m) acc[a][n][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int nlines = B * D * D;
+    const int L0 = blockIdx.x * lines_per_block;
+    const int L1 = L0 + lines_per_block < nlines ? L0 + lines_per_block : nlines;
+    for (int L = L0; L < L1; ++L) {
+        const size_t yy = L % D, zz = (L / D) % D, b = L / (D * D);
+        size_t ob[SPW];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    out[((size_t)(n * 16 + grp * 4 + i) * 8 + 2 * wave + h) * CIN + m * 16 + row] = acc[h][n][m][i];
-    // the four waves' bias sums, in order
-    __shared__ floatx4 red[4][NTC][4];
+        for (int a = 0; a < SPW; ++a) {
+            const int s = s0 + a;
+            ob[a] = ((b * D2 + 2 * zz + (s >> 2)) * D2 + 2 * yy + ((s >> 1) & 1)) * D2 + (s & 1);
+        }
+        for (int xb = 4 * wave; xb < D; xb += 16) {
+            const int xx = xb + grp;
+            float bx[NTI];
 #pragma unroll
-    for (int n = 0; n < NTC; ++n)
-        if (row == 0) red[wave][n][grp] = accb[n];
-    __syncthreads();
-    if (t < NTC * 4) {
-        const int n = t / 4, q = t % 4;
-        *(floatx4*)(out + COUT * 8 * CIN + n * 16 + q * 4) =
-            ((red[0][n][q] + red[1][n][q]) + red[2][n][q]) + red[3][n][q];
+            for (int m = 0; m < NTI; ++m) bx[m] = bf2f(x[((size_t)L * D + xx) * CIN + m * 16 + row]);
+#pragma unroll
+            for (int a = 0; a < SPW; ++a) {
+                const size_t u = ob[a] + 2 * (size_t)xx;
+#pragma unroll
+                for (int n = 0; n < NTC; ++n) {
+                    const float av = bf2f(dy[u * COUT + n * 16 + row]);
+#pragma unroll
+                    for (int m = 0; m < NTI; ++m)
+                        acc[a][n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bx[m], acc[a][n][m], 0, 0, 0);
+                }
+            }
+        }
+    }
+    float* out = partial + (size_t)blockIdx.x * COUT * 8 * CIN;
+#pragma unroll
+    for (int a = 0; a < SPW; ++a)
+#pragma unroll
+        for (int n = 0; n < NTC; ++n)
+#pragma unroll
+            for (int m = 0; m < NTI; ++m) {
+                __syncthreads();
+                if (wave > 0) red[wave - 1][lane] = acc[a][n][m];
+                __syncthreads();
+                if (wave == 0) {
+                    floatx4 sum = acc[a][n][m];
+#pragma unroll
+                    for (int w = 0; w < 3; ++w) sum += red[w][lane];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        out[((size_t)(n * 16 + grp * 4 + i) * 8 + s0 + a) * CIN + m * 16 + row] = sum[i];
+                }
+            }
+}
+
+template <int CIN, int COUT>
+__global__ __launch_bounds__(256) void k_up_wgrad(const bf16_t* __restrict__ x, const bf16_t* __restrict__ dy,
+                                                  float* __restrict__ partial, int B, int D, int vox_per_block) {
+    constexpr int PAIRS = (COUT / 4) * (CIN / 4);
+    constexpr int SETS = 256 / PAIRS;
+    static_assert(PAIRS <= 256 && 256 % PAIRS == 0, "pairs per block");
+    __shared__ float red[(SETS > 1 ? 256 : 1) * 16];
+    const int t = threadIdx.x;
+    const int pair = t % PAIRS, set = t / PAIRS;
+    const int co0 = (pair % (COUT / 4)) * 4, ci0 = (pair / (COUT / 4)) * 4;
+    const size_t nv = (size_t)B * D * D * D;
+    const size_t v0 = (size_t)blockIdx.x * vox_per_block;
+    const size_t v1 = v0 + vox_per_block < nv ? v0 + vox_per_block : nv;
+    const int D2 = 2 * D;
+    float* out = partial + (size_t)blockIdx.x * COUT * 8 * CIN;
+    for (int s = 0; s < 8; ++s) {
+        float acc[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+        for (size_t v = v0 + set; v < v1; v += SETS) {
+            const int xx = v % D, yy = (v / D) % D, zz = (v / ((size_t)D * D)) % D;
+            const int b = v / ((size_t)D * D * D);
+            const size_t u =
+                (((size_t)b * D2 + 2 * zz + (s >> 2)) * D2 + 2 * yy + ((s >> 1) & 1)) * D2 + 2 * xx + (s & 1);
+            // 4 consecutive bf16 = one 8-byte load each
+            const uint2 gq = *(const uint2*)(dy + u * COUT + co0);
+            const uint2 xq = *(const uint2*)(x + v * CIN + ci0);
+            const float gv[4] = {__uint_as_float(gq.x << 16), __uint_as_float(gq.x & 0xffff0000u),
+                                 __uint_as_float(gq.y << 16), __uint_as_float(gq.y & 0xffff0000u)};
+            const float xv[4] = {__uint_as_float(xq.x << 16), __uint_as_float(xq.x & 0xffff0000u),
+                                 __uint_as_float(xq.y << 16), __uint_as_float(xq.y & 0xffff0000u)};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(gv[i], xv[j], acc[i][j]);
+        }
+        if (SETS > 1) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) red[t * 16 + i * 4 + j] = acc[i][j];
+            __syncthreads();
+            if (set == 0)
+                for (int s2 = 1; s2 < SETS; ++s2)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[i][j] += red[(s2 * PAIRS + pair) * 16 + i * 4 + j];
+        }
+        if (set == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) out[((size_t)(co0 + i) * 8 + s) * CIN + ci0 + j] = acc[i][j];
+        }
     }
 }
 
@@ -1336,91 +1368,54 @@ __global__ __launch_bounds__(256) void k_in_fwd(const float* __restrict__ delta,
     }
 }
 
-// Input-layer weight gradient on the fp32 matrix cores
-// (v_mfma_f32_16x16x4f32): dwd[co][t] = sum_v g'[v][co] scale delta[v + off(t)]
-// (g' = g where the layer's output is positive), and as tap 27 the sums of g'
-// alone, per sample.  A block walks tiles of 4 x 4 lines of 16 voxels of one
-// sample: g' channels-last in LDS (40 bytes a voxel, so the dword of a channel
-// pair falls on distinct banks) and the scaled density with its halo; the next
-// tile is fetched into registers meanwhile.  Each wave owns the four lines of
-// a z-plane: K = 4 voxels per product, one per lane group, two column tiles for
-// the 28 taps; the waves are added in a fixed order at the end.
-//
-// What bounds it: HBM (g and y once: 537 MB at 128^3, batch 4) beside 55 us of
-// fp32 products.  179 us there, with the sums that the bias and the
-// conditioning need; the form that loaded each operand from memory two bytes
-// a lane took 865 us, the channel sums 75 more.
-constexpr int kInTaps = 28;
-__global__ __launch_bounds__(256) void k_in_wgrad(const float* __restrict__ delta, const bf16_t* __restrict__ g,
-                                                  const bf16_t* __restrict__ y, float* __restrict__ partial, int D,
-                                                  float scale, int tiles_per_block) {
-    constexpr int HY = 6, HX = 18, NH = 6 * HY * HX, NPD = (NH + 255) / 256, VS = 20;
-    __shared__ float ds[NH];
-    __shared__ __attribute__((aligned(16))) bf16_t gs[256 * VS];
+// Input-layer weight gradient of the density channel on the fp32 matrix
+// cores (v_mfma_f32_16x16x4f32): dwd[co][t] = sum_v g'[v][co] scale
+// delta[v + off(t)] (g' = g where the layer's output is positive).  K = 4
+// voxels per product, one per lane group, so both operands come straight from
+// memory: lane (row, grp) supplies g'[voxel grp][channel row] and the scaled
+// density at voxel grp shifted by tap 16 j + row (two N tiles cover the 27
+// taps; tap rows fetched per x-line).  Grid: blocks over x-lines; wave w takes
+// the 4-voxel steps 4 w, 4 w + 16, ... of each line; the waves are added in a
+// fixed order at the end.
+__global__ __launch_bounds__(256) void k_in_wgrad_mfma(const float* __restrict__ delta, const bf16_t* __restrict__ g,
+                                                       const bf16_t* __restrict__ y, float* __restrict__ partial, int B,
+                                                       int D, float scale, int lines_per_block) {
     __shared__ floatx4 red[3][2][64];
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, grp = lane >> 4;
-    const int b = blockIdx.y, nx = D / 16, ny = D / 4, ntiles = nx * ny * ny;
-    const size_t vb = (size_t)b * D * D * D;
-    // density offset of this lane's taps 16 j + row from the voxel's halo cell
-    int toff[2];
+    int tdz[2], tdy[2], tdx[2];
+    bool tok[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int tp = 16 * j + row;
-        toff[j] = tp < 27 ? tap_off<HY, HX, 1>(tp) : 0;
+        const int t = 16 * j + row;
+        tok[j] = t < 27;
+        const int tt = tok[j] ? t : 0;
+        tdz[j] = tt / 9 - 1;
+        tdy[j] = (tt / 3) % 3 - 1;
+        tdx[j] = tt % 3 - 1;
     }
-    const bool count = 16 + row == 27, pad = 16 + row > 27;  // of the second column tile
-    const bool odd = row & 1;
     floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
-    float hd[NPD];
-    u32x4 hg[2];
-    auto fetch = [&](int tile) {
-        const int x0 = tile % nx * 16, y0 = tile / nx % ny * 4, z0 = tile / (nx * ny) * 4;
+    const int nlines = B * D * D;
+    const int L0 = blockIdx.x * lines_per_block;
+    const int L1 = L0 + lines_per_block < nlines ? L0 + lines_per_block : nlines;
+    for (int L = L0; L < L1; ++L) {
+        const int yy = L % D, zz = (L / D) % D, b = L / (D * D);
+        const float* drow[2];
 #pragma unroll
-        for (int q = 0; q < NPD; ++q) {
-            const int i = t + q * 256;
-            const int hx = i % HX, hy = i / HX % HY, hz = i / (HX * HY);
-            if (i < NH)
-                hd[q] = scale * delta[vb + ((size_t)wrap(z0 + hz - 1, D) * D + wrap(y0 + hy - 1, D)) * D +
-                                      wrap(x0 + hx - 1, D)];
-        }
+        for (int j = 0; j < 2; ++j)
+            drow[j] = delta + (((size_t)b * D + wrap(zz + tdz[j], D)) * D + wrap(yy + tdy[j], D)) * D;
+        const size_t lbase = (size_t)L * D;
+        for (int xb = 4 * wave; xb < D; xb += 16) {
+            const int xx = xb + grp;
+            const size_t idx = (lbase + xx) * 16 + row;
+            const float av = pos_bf(y[idx]) ? bf2f(g[idx]) : 0.0f;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int i = t + q * 256, v = i >> 1;  // 8 channels of voxel v = (lz, ly, lx)
-            const size_t idx =
-                (vb + ((size_t)(z0 + (v >> 6)) * D + y0 + (v >> 4 & 3)) * D + x0 + (v & 15)) * 16 + (i & 1) * 8;
-            hg[q] = mask8(*(const u32x4*)(g + idx), *(const u32x4*)(y + idx));
-        }
-    };
-    const int t0 = blockIdx.x * tiles_per_block, t1 = min(t0 + tiles_per_block, ntiles);
-    if (t0 < t1) fetch(t0);
-    for (int tile = t0; tile < t1; ++tile) {
-        __syncthreads();  // the previous tile is consumed
-#pragma unroll
-        for (int q = 0; q < NPD; ++q)
-            if (t + q * 256 < NH) ds[t + q * 256] = hd[q];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int i = t + q * 256;
-            bf16_t* p = gs + (i >> 1) * VS + (i & 1) * 8;
-            *(u32x2*)p = u32x2{hg[q][0], hg[q][1]};
-            *(u32x2*)(p + 4) = u32x2{hg[q][2], hg[q][3]};
-        }
-        __syncthreads();
-        if (tile + 1 < t1) fetch(tile + 1);
-#pragma unroll
-        for (int l = 0; l < 4; ++l)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int v = ((wave * 4 + l) << 4) + 4 * k + grp;
-                const unsigned w = *(const unsigned*)(gs + v * VS + (row >> 1) * 2);
-                const float av = __uint_as_float(odd ? w & 0xffff0000u : w << 16);
-                const float* dp = ds + (wave * HY + l) * HX + 4 * k + grp;
-                const float d1 = dp[toff[1]];
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, dp[toff[0]], acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, count ? 1.0f : (pad ? 0.0f : d1), acc[1], 0, 0, 0);
+            for (int j = 0; j < 2; ++j) {
+                const float bv = tok[j] ? scale * drow[j][wrap(xx + tdx[j], D)] : 0.0f;
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[j], 0, 0, 0);
             }
+        }
     }
     if (wave > 0) {
 #pragma unroll
@@ -1428,43 +1423,40 @@ __global__ __launch_bounds__(256) void k_in_wgrad(const float* __restrict__ delt
     }
     __syncthreads();
     if (wave == 0) {
-        float* out = partial + ((size_t)blockIdx.x * gridDim.y + b) * 16 * kInTaps;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             floatx4 sum = acc[j];
 #pragma unroll
             for (int w = 0; w < 3; ++w) sum += red[w][j][lane];
             const int tap = 16 * j + row;
-            if (tap < kInTaps) {
+            if (tap < 27) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) out[(grp * 4 + i) * kInTaps + tap] = sum[i];
+                for (int i = 0; i < 4; ++i) partial[(size_t)blockIdx.x * 16 * 27 + (grp * 4 + i) * 27 + tap] = sum[i];
             }
         }
     }
 }
 
 // Full input-layer weight gradient [co][t][3] and bias gradient from the
-// per-sample sums s[b][co][28] of k_in_wgrad: the conditioning channels are
-// constant, so their gradient is the same for every tap, sum_b cond[b][k]
-// gsum[b][co] with gsum tap 27 of s.
-__global__ void k_in_finish(const float* __restrict__ s, const float* __restrict__ cond, float* __restrict__ dw,
-                            float* __restrict__ db, int B, int COUT) {
+// density part (dwd[co][t]) and the per-sample gradient sums gsum[b][co]:
+// the conditioning channels are constant, so their gradient is the same for
+// every tap: sum_b cond[b][k] gsum[b][co].
+__global__ void k_in_finish(const float* __restrict__ dwd, const float* __restrict__ gsum,
+                            const float* __restrict__ cond, float* __restrict__ dw, float* __restrict__ db, int B,
+                            int COUT) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= COUT * 27) return;
-    const int co = i / 27, tap = i % 27;
-    float d = 0.0f, s1 = 0.0f, s2 = 0.0f, s0 = 0.0f;
+    const int co = i / 27;
+    float s1 = 0.0f, s2 = 0.0f, s0 = 0.0f;
     for (int b = 0; b < B; ++b) {
-        const float* p = s + ((size_t)b * COUT + co) * kInTaps;
-        const float gsum = p[27];
-        d += p[tap];
-        s0 += gsum;
-        s1 += cond[b * 2 + 0] * gsum;
-        s2 += cond[b * 2 + 1] * gsum;
+        s0 += gsum[b * COUT + co];
+        s1 += cond[b * 2 + 0] * gsum[b * COUT + co];
+        s2 += cond[b * 2 + 1] * gsum[b * COUT + co];
     }
-    dw[i * 3 + 0] = d;
+    dw[i * 3 + 0] = dwd[i];
     dw[i * 3 + 1] = s1;
     dw[i * 3 + 2] = s2;
-    if (tap == 0) db[co] = s0;
+    if (i % 27 == 0) db[co] = s0;
 }
 
 // ------------------------------------------------------------------ head: 1^3 conv, sigmoid, BCE
@@ -1651,10 +1643,20 @@ const WgradShape* wgrad_shape(int cin, int cout) {
     return nullptr;
 }
 
+constexpr int kChanBlocks = 128;    // per-sample blocks of the channel sums
+
+int channel_sums(const void* g, const void* mask, int C, size_t vps, int B, float* cpart, float* total,
+                 float* per_sample, hipStream_t st) {
+    k_channel_partials<<<dim3(kChanBlocks, B), 256, 0, st>>>((const bf16_t*)g, (const bf16_t*)mask, C, vps, cpart);
+    CM21_LAUNCH_CHECK("k_channel_partials");
+    static_assert(kChanBlocks <= 128, "one thread per partial block");
+    k_channel_final<<<C, 128, 0, st>>>(cpart, B, kChanBlocks, C, per_sample, total);
+    CM21_LAUNCH_CHECK("k_channel_final");
+    return CM21_OK;
+}
 constexpr int kHeadBlocks = 1024;
-// blocks of the transposed-conv weight gradient (partials of 16 KB a block at 32 -> 16, 66 KB at 64 -> 32)
-constexpr int up_blocks(int cin) { return cin < 64 ? 1024 : 512; }
-constexpr int kInBlocks = 1024;     // blocks of the input-layer weight gradient over all samples
+constexpr int kUpBlocksMax = 1024;  // line blocks of the transposed-conv weight gradient
+constexpr int kInBlocks = 1024;     // line blocks of the input-layer weight gradient
 
 bool valid_unet_dim(int D) { return D >= 16 && D <= 1024 && D % 16 == 0; }
 
@@ -1783,14 +1785,9 @@ extern "C" int cm21_unet_pool_fwd(const void* x, void* y, int B, int D, int C, v
 
 extern "C" int cm21_unet_pool_bwd(const void* dy, void* dx, int B, int D, int C, int accumulate, void* stream) {
     CM21_REQUIRE(dy && dx && B >= 1 && D >= 2 && D % 2 == 0 && C >= 1, "cm21_unet_pool_bwd: bad arguments");
-    if (C % 8 == 0 && (size_t)B * (D / 2) < 65536 && D / 2 < 65536) {
-        k_pool_bwd<<<dim3((D * (C / 8) + 255) / 256, D / 2, B * (D / 2)), 256, 0, (hipStream_t)stream>>>(
-            (const bf16_t*)dy, (bf16_t*)dx, D, C, accumulate ? 1 : 0);
-    } else {
-        const size_t n = (size_t)B * D * D * D * C;
-        k_pool_bwd_any<<<grid_for(n), kThreads, 0, (hipStream_t)stream>>>((const bf16_t*)dy, (bf16_t*)dx, B, D, C,
-                                                                          accumulate ? 1 : 0);
-    }
+    const size_t n = (size_t)B * D * D * D * C;
+    k_pool_bwd<<<grid_for(n), kThreads, 0, (hipStream_t)stream>>>((const bf16_t*)dy, (bf16_t*)dx, B, D, C,
+                                                                    accumulate ? 1 : 0);
     CM21_LAUNCH_CHECK("k_pool_bwd");
     return CM21_OK;
 }
@@ -1806,20 +1803,33 @@ int up_fwd_t(const void* x, const void* wn, const float* b, void* y, int B, int 
 }
 template <int CIN, int COUT>
 int up_bwd_t(const void* x, const void* dy, const void* wk, void* dx, float* dw, float* db, int B, int D, float* part,
-             hipStream_t st) {
+             float* cpart, hipStream_t st) {
     const size_t nv = (size_t)B * D * D * D;
     if (dx) {
         k_up_bwd_mfma<CIN, COUT><<<(unsigned)((nv / 16 + 3) / 4), 256, 0, st>>>((const bf16_t*)dy, (const bf16_t*)wk,
                                                                                (bf16_t*)dx, B, D);
         CM21_LAUNCH_CHECK("k_up_bwd_mfma");
     }
-    const int tiles = (B * D * D + 3) / 4 * ((D + 15) / 16), tpb = (tiles + up_blocks(CIN) - 1) / up_blocks(CIN);
-    const int nblk = (tiles + tpb - 1) / tpb;
-    k_up_wgrad<CIN, COUT><<<nblk, 256, 0, st>>>((const bf16_t*)x, (const bf16_t*)dy, part, B, D, tpb);
+    int nblk;
+    if (D % 4 == 0) {
+        // matrix cores; SPW sub-positions per block keep 64 accumulator registers
+        constexpr int SPW = (COUT / 16) * (CIN / 16) <= 2 ? 8 : 2;
+        const int nlines = B * D * D;
+        const int lpb = (nlines + kUpBlocksMax - 1) / kUpBlocksMax;
+        nblk = (nlines + lpb - 1) / lpb;
+        k_up_wgrad_mfma<CIN, COUT, SPW><<<dim3(nblk, 8 / SPW), 256, 0, st>>>((const bf16_t*)x, (const bf16_t*)dy,
+                                                                             part, B, D, lpb);
+    } else {
+        const int vpb = (int)((nv + kUpBlocksMax - 1) / kUpBlocksMax);
+        nblk = (int)((nv + vpb - 1) / vpb);
+        k_up_wgrad<CIN, COUT><<<nblk, 256, 0, st>>>((const bf16_t*)x, (const bf16_t*)dy, part, B, D, vpb);
+    }
     CM21_LAUNCH_CHECK("k_up_wgrad");
-    const int n0 = COUT * 8 * CIN, n = n0 + COUT;
-    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(part, nblk, n, dw, n0, db);
+    const int n = COUT * 8 * CIN;
+    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(part, nblk, n, dw, n, nullptr);
     CM21_LAUNCH_CHECK("k_sum_blocks");
+    const size_t vps = (size_t)8 * D * D * D;
+    CM21_TRY(channel_sums(dy, nullptr, COUT, vps, B, cpart, db, nullptr, st));
     return CM21_OK;
 }
 }  // namespace
@@ -1837,7 +1847,8 @@ extern "C" int cm21_unet_up_fwd(const void* x, const void* wn, const float* bias
 
 extern "C" size_t cm21_unet_up_workspace_bytes(int B, int D, int cin, int cout) {
     if (B < 1 || D < 2 || cin < 1 || cout < 1) return 0;
-    return align_up((size_t)up_blocks(cin) * ((size_t)cout * 8 * cin + cout) * sizeof(float), 256);
+    return align_up((size_t)kUpBlocksMax * cout * 8 * cin * sizeof(float), 256) +
+           align_up((size_t)B * kChanBlocks * cout * sizeof(float), 256);
 }
 
 extern "C" int cm21_unet_up_bwd(const void* x, const void* dy, const void* wk, void* dx, float* dw, float* db, int B,
@@ -1848,9 +1859,10 @@ extern "C" int cm21_unet_up_bwd(const void* x, const void* dy, const void* wk, v
     const size_t need = cm21_unet_up_workspace_bytes(B, D, cin, cout);
     if (work_bytes < need) return fail(CM21_ERR_NOMEM, "cm21_unet_up_bwd: workspace %zu < %zu", work_bytes, need);
     float* part = (float*)work;
+    float* cpart = (float*)((char*)work + align_up((size_t)kUpBlocksMax * cout * 8 * cin * sizeof(float), 256));
     hipStream_t st = (hipStream_t)stream;
-    if (cin == 64 && cout == 32) return up_bwd_t<64, 32>(x, dy, wk, dx, dw, db, B, D, part, st);
-    if (cin == 32 && cout == 16) return up_bwd_t<32, 16>(x, dy, wk, dx, dw, db, B, D, part, st);
+    if (cin == 64 && cout == 32) return up_bwd_t<64, 32>(x, dy, wk, dx, dw, db, B, D, part, cpart, st);
+    if (cin == 32 && cout == 16) return up_bwd_t<32, 16>(x, dy, wk, dx, dw, db, B, D, part, cpart, st);
     return fail(CM21_ERR_INVALID, "cm21_unet_up_bwd: no kernel for cin=%d cout=%d", cin, cout);
 }
 
@@ -1874,40 +1886,38 @@ extern "C" int cm21_unet_in_fwd(const float* delta, const float* cond, const flo
     return CM21_OK;
 }
 
-namespace {
-// Blocks per sample of the input-layer weight gradient, and tiles per block.
-void in_blocks(int B, int D, int* nblk, int* tpb) {
-    const int tiles = (D / 16) * (D / 4) * (D / 4), want = B < kInBlocks ? kInBlocks / B : 1;
-    *tpb = (tiles + want - 1) / want;
-    *nblk = (tiles + *tpb - 1) / *tpb;
-}
-}  // namespace
-
 extern "C" size_t cm21_unet_in_workspace_bytes(int B, int D) {
     if (B < 1 || !valid_unet_dim(D)) return 0;
-    int nblk, tpb;
-    in_blocks(B, D, &nblk, &tpb);
-    return align_up((size_t)(nblk + 1) * B * 16 * kInTaps * sizeof(float), 256);
+    return align_up((size_t)kInBlocks * 16 * 27 * sizeof(float), 256) +
+           align_up((size_t)B * kChanBlocks * 16 * sizeof(float), 256) + align_up((size_t)B * 16 * sizeof(float), 256) +
+           align_up((size_t)16 * 27 * sizeof(float), 256);
 }
 
 extern "C" int cm21_unet_in_wgrad(const float* delta, const float* cond, const void* g, const void* y, float* dw,
                                   float* db, int B, int D, float delta_scale, void* work, size_t work_bytes,
                                   void* stream) {
-    CM21_REQUIRE(delta && cond && g && y && dw && db && work && B >= 1 && B < 65536 && valid_unet_dim(D),
+    CM21_REQUIRE(delta && cond && g && y && dw && db && work && B >= 1 && valid_unet_dim(D),
                  "cm21_unet_in_wgrad: bad arguments");
     const size_t need = cm21_unet_in_workspace_bytes(B, D);
     if (work_bytes < need) return fail(CM21_ERR_NOMEM, "cm21_unet_in_wgrad: workspace %zu < %zu", work_bytes, need);
     hipStream_t st = (hipStream_t)stream;
-    int nblk, tpb;
-    in_blocks(B, D, &nblk, &tpb);
-    const int n = B * 16 * kInTaps;
-    float* sums = (float*)work;
-    float* part = sums + n;
-    k_in_wgrad<<<dim3(nblk, B), 256, 0, st>>>(delta, (const bf16_t*)g, (const bf16_t*)y, part, D, delta_scale, tpb);
-    CM21_LAUNCH_CHECK("k_in_wgrad");
-    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(part, nblk, n, sums, n, nullptr);
+    char* p = (char*)work;
+    float* part = (float*)p;
+    p += align_up((size_t)kInBlocks * 16 * 27 * sizeof(float), 256);
+    float* cpart = (float*)p;
+    p += align_up((size_t)B * kChanBlocks * 16 * sizeof(float), 256);
+    float* gsum = (float*)p;
+    p += align_up((size_t)B * 16 * sizeof(float), 256);
+    float* dwd = (float*)p;
+    const int nlines = B * D * D;
+    const int lpb = (nlines + kInBlocks - 1) / kInBlocks;
+    const int nblk = (nlines + lpb - 1) / lpb;
+    k_in_wgrad_mfma<<<nblk, 256, 0, st>>>(delta, (const bf16_t*)g, (const bf16_t*)y, part, B, D, delta_scale, lpb);
+    CM21_LAUNCH_CHECK("k_in_wgrad_mfma");
+    k_sum_blocks<<<sum_blocks_grid(16 * 27), 256, 0, st>>>(part, nblk, 16 * 27, dwd, 16 * 27, nullptr);
     CM21_LAUNCH_CHECK("k_sum_blocks");
-    k_in_finish<<<(16 * 27 + 255) / 256, 256, 0, st>>>(sums, cond, dw, db, B, 16);
+    CM21_TRY(channel_sums(g, y, 16, (size_t)D * D * D, B, cpart, nullptr, gsum, st));
+    k_in_finish<<<(16 * 27 + 255) / 256, 256, 0, st>>>(dwd, gsum, cond, dw, db, B, 16);
     CM21_LAUNCH_CHECK("k_in_finish");
     return CM21_OK;
 }

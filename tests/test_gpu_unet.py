@@ -547,54 +547,3 @@ def test_wgrad_edges(gpu, D, B, cin, cout, c0, masked):
     _close_f32(dw, ref, "dw")
     _close_f32(db, gf.sum(0), "db")
     assert torch.equal(dw, dw2)
-
-
-@pytest.mark.parametrize("D,B,C", [(2, 1, 8), (6, 2, 24), (16, 1, 64), (34, 1, 16), (4, 3, 5), (6, 1, 20)])
-@pytest.mark.parametrize("add", [0, 1])
-def test_pool_bwd_edges(gpu, D, B, C, add):
-    """Every channel count and side; exact in fp32, rounded once to bf16."""
-    dy, dx = _bf((B, D // 2, D // 2, D // 2, C), seed=D), _bf((B, D, D, D, C), seed=C)
-    up = dy
-    for a in (1, 2, 3):
-        up = up.repeat_interleave(2, dim=a)
-    want = (up.float() * 0.125 + (dx.float() if add else 0.0)).to(torch.bfloat16)
-    gpu.call("cm21_unet_pool_bwd", _vp(dy), _vp(dx), B, D, C, add, gpu.stream_handle())
-    assert torch.equal(dx, want)
-
-
-@pytest.mark.parametrize("D,B", [(2, 2), (6, 2), (10, 2), (12, 1), (16, 3), (20, 1), (24, 2)])
-@pytest.mark.parametrize("cin,cout", [(64, 32), (32, 16)])
-def test_up_wgrad_edges(gpu, D, B, cin, cout):
-    """Weight and bias gradients of the transposed conv at sides that leave
-    lines and voxels over.  fp32 sums: 1e-3 of the largest entry."""
-    x, dy = _bf((B, D, D, D, cin), seed=D), _bf((B, 2 * D, 2 * D, 2 * D, cout), seed=D + 1)
-    dw, db = torch.full((cout, 8, cin), 7.0, device="cuda"), torch.full((cout,), 7.0, device="cuda")
-    work = torch.empty(gpu.query("cm21_unet_up_workspace_bytes", B, D, cin, cout), dtype=torch.uint8, device="cuda")
-    gpu.call("cm21_unet_up_bwd", _vp(x), _vp(dy), None, None, _fp(dw), _fp(db), B, D, cin, cout, _vp(work),
-             work.numel(), gpu.stream_handle())
-    xd, gd = _d(x).reshape(-1, cin), _d(dy)
-    ref = torch.stack([gd[:, s >> 2::2, s >> 1 & 1::2, s & 1::2].reshape(-1, cout).T @ xd for s in range(8)], 1)
-    _close_f32(dw, ref, "dw")
-    _close_f32(db, gd.reshape(-1, cout).sum(0), "db")
-
-
-@pytest.mark.parametrize("D,B", [(16, 1), (16, 3), (48, 2), (80, 1)])
-def test_in_wgrad_edges(gpu, D, B):
-    """Input-layer gradients at sides with few tiles and odd batches."""
-    delta, cond = _f((B, D, D, D), seed=1), _f((B, 2), seed=2)
-    g, y = _bf((B, D, D, D, 16), seed=3), _bf((B, D, D, D, 16), seed=4)
-    dw, db = torch.full((16, 27, 3), 7.0, device="cuda"), torch.full((16,), 7.0, device="cuda")
-    work = torch.empty(gpu.query("cm21_unet_in_workspace_bytes", B, D), dtype=torch.uint8, device="cuda")
-    gpu.call("cm21_unet_in_wgrad", _fp(delta), _fp(cond), _vp(g), _vp(y), _fp(dw), _fp(db), B, D, ctypes.c_float(0.5),
-             _vp(work), work.numel(), gpu.stream_handle())
-    gd = (_d(g) * (_d(y) > 0))
-    dd = _d(delta) * 0.5
-    gsum = gd.sum((1, 2, 3))
-    ref = torch.empty((16, 27, 3), dtype=torch.float64)
-    for t in range(27):
-        sh = torch.roll(dd, (1 - t // 9, 1 - t // 3 % 3, 1 - t % 3), (1, 2, 3))
-        ref[:, t, 0] = gd.reshape(-1, 16).T @ sh.reshape(-1)
-    ref[:, :, 1:] = (gsum.T @ _d(cond))[:, None, :]
-    _close_f32(dw[..., 0], ref[..., 0], "dw")
-    _close_f32(dw[..., 1:], ref[..., 1:], "dw cond")
-    _close_f32(db, gsum.sum(0), "db")
