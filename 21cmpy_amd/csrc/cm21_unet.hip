@@ -23,9 +23,10 @@
 //     (masked by the ReLU of the forward output) with the weights transposed
 //     and spatially flipped.
 //   3^3 convolution, weight gradient: v_mfma_f32_16x16x32_bf16 with K = 32
-//     voxels, the masked output gradient and a ring of input planes in LDS
-//     channels-last, fragments put together from lane pairs.  Per-block
-//     partials reduced in a fixed order.
+//     voxels of an x-line, the masked output gradient and the input written
+//     to LDS channel-major (the input in three dx-shifted copies) so that
+//     every fragment is one aligned 16-byte read; fp32 VALU for boxes of
+//     side 16.  Per-block partials reduced in a fixed order.
 //   Input layer (density plus two constant conditioning channels, the
 //   latter folded into a per-sample bias): 3^3 taps on the fp32 matrix cores
 //   (v_mfma_f32_16x16x4f32), forward and weight gradient.
@@ -651,253 +652,255 @@ struct WgradArgs {
     const bf16_t* x1;
     const bf16_t* g;
     const bf16_t* mask;
-    float* partial;  // [gridDim.x][cout][27][cin] + [cout]: weights, then bias
-    int nz;          // z-planes of a unit
-    int units, units_per_block;
+    float* partial;  // [gridDim.x][cout][27][cin]
+    int tiles_per_block;
 };
 
-// Eight (or ten) consecutive voxels of one channel from channels-last LDS
-// rows.  Lane pairs (2p, 2p + 1) own channels 2p and 2p + 1 of a 16-channel
-// chunk: the even lane reads the dword of both channels at voxel 2i, the odd
-// lane at voxel 2i + 1, they swap dwords (DPP), and each keeps its own
-// channel's halves: one LDS read per two voxels, and no transposed copy.
-__device__ __forceinline__ unsigned voxel_pair(const bf16_t* p, unsigned sel) {
-    const unsigned own = *(const unsigned*)p;
-    const unsigned nb = (unsigned)__builtin_amdgcn_mov_dpp((int)own, 0xB1, 0xF, 0xF, true);  // quad_perm 1,0,3,2
-    return __builtin_amdgcn_perm(nb, own, sel);
-}
-
-// threads of a weight-gradient block: three waves (dz) per 16 input channels, at most 32 of them
-constexpr int wgrad_threads(int cin) { return 192 * ((cin < 32 ? cin : 32) / 16); }
-
-// Weight gradient dW[co][tap][ci] = sum_v g'[v][co] x[v + off(tap)][ci] (g' =
-// g where the forward output is positive) and bias gradient db[co] = sum_v
-// g'[v][co], on v_mfma_f32_16x16x32_bf16 with K = 32 voxels: an x-line of 32,
-// or two lines of 16 (XT = 16, sides that are no multiple of 32).
-//
-// A block owns TY lines x XT voxels of at most 32 input and 32 output channels
-// (grid y: the parts of wider layers) and walks nz z-planes with a ring of three
-// input planes (with halo) and the masked gradient plane in LDS, channels-last
-// as in memory (16-channel chunks, 40 bytes a voxel: 16-byte loads, 8-byte
-// LDS writes, and dword reads that fall on distinct banks but for two).  The
-// next plane is fetched into registers while one computes.  Wave (dz, ci
-// chunk) holds the 9 (dy, dx) x cout/16 accumulator tiles of its dz for the
-// whole launch: an input row's three dx-shifted fragments come from five LDS
-// reads and serve the three output lines that it touches, and no two waves
-// share an output, so partials need no sum within the block.  The bias is one
-// more product per gradient fragment, against ones.  Blocks are added in a
-// fixed order by k_sum_blocks.
-//
-// What bounds it: HBM at 16 channels (x, g and the mask once, x with a halo of
-// 1.6, mostly in L2), the matrix cores and LDS above.  It replaces a form that
-// wrote transposed copies, three of the input, to LDS two bytes at a time,
-// read g and the mask once per (dz, chunk) and left the bias to two more
-// passes over g.  Per launch at batch 4 (before, without the bias sums of 52
-// us each -> now): 16 -> 16 at 128^3 939 -> 310 us, 32 -> 16 at 128^3 1914 ->
-// 615, 32 -> 32 at 64^3 383 -> 120, 64 -> 32 at 64^3 807 -> 227.
-template <int CIN, int COUT, int XT>
-__global__ __launch_bounds__(wgrad_threads(CIN)) void k_conv3_wgrad(WgradArgs a) {
-    constexpr int CIB = CIN < 32 ? CIN : 32, COB = COUT < 32 ? COUT : 32;  // channels of a block
-    constexpr int NTI = CIB / 16, NTC = COB / 16, NT = wgrad_threads(CIN);
-    constexpr int TY = 4, HY = TY + 2, HX = XT + 2, VS = 20;  // VS: bf16 per voxel and chunk
-    constexpr int LG = 32 / XT;                               // lines per K slice
-    constexpr int XPL = HY * HX * VS, GPL = TY * XT * VS;     // one chunk of an input / gradient plane
-    constexpr int XC = HY * HX * (CIB / 8), GC = TY * XT * (COB / 8);  // 16-byte pieces per plane
-    constexpr int NPX = (XC + NT - 1) / NT, NPG = (GC + NT - 1) / NT;
-    static_assert(XT == 32 || XT == 16, "K = 32 voxels");
-    __shared__ __attribute__((aligned(16))) bf16_t xs[3 * NTI * XPL];
-    __shared__ __attribute__((aligned(16))) bf16_t gs[NTC * GPL];
-    const int D = a.D, t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int row = lane & 15, grp = lane >> 4;
-    const int dz = wave % 3, cit = wave / 3;
-    const int c0 = a.c0, c1 = CIN - c0;
-    const int ci0 = blockIdx.y % (CIN / CIB) * CIB, co0 = blockIdx.y / (CIN / CIB) * COB;
-    const unsigned sel = (row & 1) ? 0x03020706u : 0x05040100u;
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-    const int nx = D / XT, ny = D / TY, nzc = D / a.nz;
-    floatx4 acc[9][NTC], accb[NTC];
+// Voxel tile 2 x 2 x 16 (64 voxels); taps in groups of 3 (grid.y = 9).  Each
+// thread owns 4 output x 4 input channels for the group's 3 taps; thread sets
+// split the voxels and are added in LDS at the end.
+template <int CIN, int COUT>
+__global__ __launch_bounds__(256) void k_conv3_wgrad(WgradArgs a) {
+    constexpr int TZ = 2, TY = 2, HZ = 4, HY = 4, HX = 18, NV = TZ * TY * 16;
+    constexpr int PAIRS = (COUT / 4) * (CIN / 4);
+    constexpr int SETS = 256 / PAIRS;
+    static_assert(PAIRS <= 256 && 256 % PAIRS == 0, "pairs per block");
+    __shared__ __attribute__((aligned(16))) bf16_t xt[HZ * HY * HX * CIN];
+    __shared__ float gt[NV * COUT];
+    __shared__ float red[(SETS > 1 ? 256 : 1) * 16];
+    const int D = a.D;
+    const int tg = blockIdx.y;  // taps 3*tg .. 3*tg+2
+    const int t = threadIdx.x;
+    const int pair = t % PAIRS, set = t / PAIRS;
+    const int co0 = (pair % (COUT / 4)) * 4, ci0 = (pair / (COUT / 4)) * 4;
+    const int c1 = CIN - a.c0;
+    const int nx = D / 16, ny = D / TY, nz = D / TZ;
+    const int ntiles = a.B * nz * ny * nx;
+    float acc[3][4][4];
 #pragma unroll
-    for (int n = 0; n < NTC; ++n) {
-        accb[n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int q = 0; q < 3; ++q)
 #pragma unroll
-        for (int q = 0; q < 9; ++q) acc[q][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    bf16x8 ones;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
-    // this lane's voxel inside a K slice: line grp / (XT / 8), voxel 8 (grp % (XT / 8)) + (row & 1)
-    const int kl = grp / (XT / 8), kx = grp % (XT / 8) * 8 + (row & 1);
-    const bf16_t* xlane = xs + cit * XPL + (kl * HX + kx) * VS + (row >> 1) * 2;
-    const bf16_t* glane = gs + (kl * XT + kx) * VS + (row >> 1) * 2;
-
-    for (int u = blockIdx.x * a.units_per_block; u < (int)(blockIdx.x + 1) * a.units_per_block && u < a.units; ++u) {
-        const int x0 = (u % nx) * XT, y0 = (u / nx % ny) * TY, z0 = (u / (nx * ny) % nzc) * a.nz;
-        const size_t vb = (size_t)(u / (nx * ny * nzc)) * D * D * D;
-        auto fetch_x = [&](int gz, u32x4 (&pf)[NPX]) {
-            const size_t pz = vb + (size_t)wrap(gz, D) * D * D;
-#pragma unroll
-            for (int q = 0; q < NPX; ++q) {
-                const int i = t + q * NT;
-                const int ch = ci0 + i % (CIB / 8) * 8, v = i / (CIB / 8), hx = v % HX, hy = v / HX;
-                u32x4 r = zero;
-                if (i < XC) {
-                    const size_t gv = pz + (size_t)wrap(y0 + hy - 1, D) * D + wrap(x0 + hx - 1, D);
-                    r = ch < c0 ? *(const u32x4*)(a.x0 + gv * c0 + ch) : *(const u32x4*)(a.x1 + gv * c1 + (ch - c0));
-                }
-                pf[q] = r;
-            }
-        };
-        auto store_x = [&](int slot, const u32x4 (&pf)[NPX]) {
-#pragma unroll
-            for (int q = 0; q < NPX; ++q) {
-                const int i = t + q * NT;
-                const int ch = i % (CIB / 8) * 8, v = i / (CIB / 8);
-                if (i < XC) {
-                    bf16_t* p = xs + (slot * NTI + ch / 16) * XPL + v * VS + ch % 16;
-                    *(u32x2*)p = u32x2{pf[q][0], pf[q][1]};
-                    *(u32x2*)(p + 4) = u32x2{pf[q][2], pf[q][3]};
-                }
-            }
-        };
-        u32x4 px[NPX], pg[NPG];
-        auto fetch_g = [&](int gz) {
-            const size_t pz = vb + (size_t)gz * D * D;
-#pragma unroll
-            for (int q = 0; q < NPG; ++q) {
-                const int i = t + q * NT;
-                const int ch = i % (COB / 8) * 8, v = i / (COB / 8);
-                u32x4 r = zero;
-                if (i < GC) {
-                    const size_t gv = (pz + (size_t)(y0 + v / XT) * D + x0 + v % XT) * COUT + co0 + ch;
-                    r = *(const u32x4*)(a.g + gv);
-                    if (a.mask) r = mask8(r, *(const u32x4*)(a.mask + gv));
-                }
-                pg[q] = r;
-            }
-        };
-        auto store_g = [&]() {
-#pragma unroll
-            for (int q = 0; q < NPG; ++q) {
-                const int i = t + q * NT;
-                const int ch = i % (COB / 8) * 8, v = i / (COB / 8);
-                if (i < GC) {
-                    bf16_t* p = gs + ch / 16 * GPL + v * VS + ch % 16;
-                    *(u32x2*)p = u32x2{pg[q][0], pg[q][1]};
-                    *(u32x2*)(p + 4) = u32x2{pg[q][2], pg[q][3]};
-                }
-            }
-        };
-        // planes z0 - 1, z0, z0 + 1 in slots 0, 1, 2 and the first gradient plane
-        __syncthreads();  // the previous unit is consumed
-        for (int s = 0; s < 3; ++s) {
-            fetch_x(z0 - 1 + s, px);
-            store_x(s, px);
+            for (int j = 0; j < 4; ++j) acc[q][i][j] = 0.0f;
+    for (int s = 0; s < a.tiles_per_block; ++s) {
+        const int tile = blockIdx.x * a.tiles_per_block + s;
+        if (tile >= ntiles) break;  // uniform
+        const int xt0 = (tile % nx) * 16;
+        const int yt0 = ((tile / nx) % ny) * TY;
+        const int zt0 = ((tile / (nx * ny)) % nz) * TZ;
+        const int b = tile / (nx * ny * nz);
+        __syncthreads();  // previous tile fully consumed
+        for (int i = t; i < HZ * HY * HX * (CIN / 8); i += 256) {
+            const int ch = (i % (CIN / 8)) * 8;
+            const int vox = i / (CIN / 8);
+            const int hx = vox % HX, hy = (vox / HX) % HY, hz = vox / (HX * HY);
+            const size_t g = (((size_t)b * D + wrap(zt0 + hz - 1, D)) * D + wrap(yt0 + hy - 1, D)) * D +
+                             wrap(xt0 + hx - 1, D);
+            const u32x4 v = ch < a.c0 ? *(const u32x4*)(a.x0 + g * a.c0 + ch)
+                                      : *(const u32x4*)(a.x1 + g * c1 + (ch - a.c0));
+            *(u32x4*)(xt + vox * CIN + ch) = v;
         }
-        fetch_g(z0);
-        store_g();
-        int slot = dz;  // of this wave's input plane, z + dz - 1
+        for (int i = t; i < NV * COUT; i += 256) {
+            const int co = i % COUT, v = i / COUT;
+            const int lx = v % 16, ly = (v / 16) % TY, lz = v / (16 * TY);
+            const size_t g = (((size_t)b * D + zt0 + lz) * D + yt0 + ly) * D + xt0 + lx;
+            float gv = bf2f(a.g[g * COUT + co]);
+            if (a.mask && !pos_bf(a.mask[g * COUT + co])) gv = 0.0f;
+            gt[i] = gv;
+        }
         __syncthreads();
-        for (int z = 0; z < a.nz; ++z) {
-            const bool more = z + 1 < a.nz;
-            if (more) {
-                fetch_x(z0 + z + 2, px);
-                fetch_g(z0 + z + 1);
+        for (int v = set; v < NV; v += SETS) {
+            const int lx = v % 16, ly = (v / 16) % TY, lz = v / (16 * TY);
+            float gv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) gv[i] = gt[v * COUT + co0 + i];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const int tap = tg * 3 + q;
+                const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
+                const bf16_t* xp = xt + (((lz + dz) * HY + (ly + dy)) * HX + (lx + dx)) * CIN + ci0;
+                float xv[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) xv[j] = bf2f(xp[j]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[q][i][j] = fmaf(gv[i], xv[j], acc[q][i][j]);
             }
-            const bf16_t* xp = xlane + slot * NTI * XPL;
-            bf16x8 ga[TY / LG][NTC];
-#pragma unroll
-            for (int r = 0; r + LG <= HY; ++r) {
-                // gradient fragments of the lines that row r is the first to touch
-                if (r % LG == 0 && r + LG <= TY) {
-#pragma unroll
-                    for (int n = 0; n < NTC; ++n) {
-                        u32x4 v;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) v[i] = voxel_pair(glane + n * GPL + (r * XT + 2 * i) * VS, sel);
-                        ga[r / LG][n] = __builtin_bit_cast(bf16x8, v);
-                        if (dz == 1 && cit == 0)  // (blocks of ci0 > 0 form it too, and do not store it)
-                            accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[r / LG][n], ones, accb[n], 0, 0, 0);
-                    }
-                }
-                unsigned pr[5];
-#pragma unroll
-                for (int i = 0; i < 5; ++i) pr[i] = voxel_pair(xp + (r * HX + 2 * i) * VS, sel);
-                u32x4 w[3];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    w[0][i] = pr[i];
-                    w[1][i] = __builtin_amdgcn_alignbit(pr[i + 1], pr[i], 16);
-                    w[2][i] = pr[i + 1];
-                }
-#pragma unroll
-                for (int dy = 0; dy < 3; ++dy) {
-                    const int l = r - dy;
-                    if (l >= 0 && l % LG == 0 && l + LG <= TY) {
-#pragma unroll
-                        for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-                            for (int n = 0; n < NTC; ++n)
-                                acc[dy * 3 + dx][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                    ga[l / LG][n], __builtin_bit_cast(bf16x8, w[dx]), acc[dy * 3 + dx][n], 0, 0, 0);
-                    }
-                }
-            }
-            if (more) {
-                __syncthreads();  // every wave is done with plane z - 1 and the gradient
-                store_x(z % 3, px);
-                store_g();
-                __syncthreads();
-            }
-            slot = slot == 2 ? 0 : slot + 1;
         }
     }
-    // lane: co = co0 + 16 n + 4 grp + i, ci = ci0 + 16 cit + row
-    float* out = a.partial + (size_t)blockIdx.x * (COUT * 27 * CIN + COUT);
+    // add the sets (fixed order) and write this block's partial
+    float* out = a.partial + (size_t)blockIdx.x * COUT * 27 * CIN;
 #pragma unroll
-    for (int n = 0; n < NTC; ++n) {
-        const int co = co0 + n * 16 + grp * 4;
-#pragma unroll
-        for (int q = 0; q < 9; ++q)
+    for (int q = 0; q < 3; ++q) {
+        const int tap = tg * 3 + q;
+        if (SETS > 1) {
+            __syncthreads();
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                out[((size_t)(co + i) * 27 + dz * 9 + q) * CIN + ci0 + cit * 16 + row] = acc[q][n][i];
-        if (dz == 1 && ci0 + cit == 0 && row == 0) *(floatx4*)(out + COUT * 27 * CIN + co) = accb[n];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) red[t * 16 + i * 4 + j] = acc[q][i][j];
+            __syncthreads();
+            if (set == 0) {
+                for (int s2 = 1; s2 < SETS; ++s2)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[q][i][j] += red[(s2 * PAIRS + pair) * 16 + i * 4 + j];
+            }
+        }
+        if (set == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) out[((size_t)(co0 + i) * 27 + tap) * CIN + ci0 + j] = acc[q][i][j];
+        }
+    }
+}
+
+// Matrix-core weight gradient, dW[co][tap][ci] = sum_v g'[v][co] x[v + off(tap)][ci]
+// (g' = g where the forward output is positive), on v_mfma_f32_16x16x32_bf16
+// with K = 32 voxels of an x-line.  Grid: (voxel-slab blocks, 16-input-channel
+// chunk x dz).  Voxel tiles of 2 x 2 lines of 32 voxels; the masked gradient
+// (all cout channels) and the chunk's input (the 2 planes at dz, 4 rows, 34
+// voxels) are written to LDS channel-major, the input in three copies shifted
+// by dx = 0, 1, 2, so that every fragment (8 consecutive voxels of one
+// channel) is one aligned 16-byte read.  Wave w owns line w of every tile and
+// keeps the 9 (dy, dx) taps x cout/16 accumulator tiles over all of the
+// block's tiles; the four waves are added in a fixed order at the end, and
+// the blocks by k_sum_blocks.
+template <int CIN, int COUT>
+__global__ __launch_bounds__(256) void k_conv3_wgrad_mfma(WgradArgs a) {
+    constexpr int NTC = COUT / 16, NTI = CIN / 16, XT = 32, XH = XT + 2, HY = 4;
+    constexpr int GS = 4 * XT + 8;           // gs channel stride (bf16), padded against bank conflicts
+    constexpr int XS = 2 * HY * XT + 8;      // xs channel stride
+    static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts");
+    __shared__ __attribute__((aligned(16))) bf16_t xs[3 * 16 * XS];
+    __shared__ __attribute__((aligned(16))) bf16_t gs[COUT * GS];
+    const int D = a.D;
+    const int cit = blockIdx.y % NTI, dz = blockIdx.y / NTI;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int row = lane & 15, grp = lane >> 4;
+    const int lz = wave >> 1, ly = wave & 1;
+    const int nx = D / XT, ny = D / 2, nz = D / 2;
+    const int ntiles = a.B * nz * ny * nx;
+    // the chunk's channels come from x0 or x1 (c0 is a multiple of 16)
+    const int cb = cit * 16;
+    const bool from0 = cb < a.c0;
+    const bf16_t* xsrc = from0 ? a.x0 : a.x1;
+    const int xstride = from0 ? a.c0 : CIN - a.c0;
+    const int xoff = from0 ? cb : cb - a.c0;
+    floatx4 acc[9][NTC];
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+#pragma unroll
+        for (int n = 0; n < NTC; ++n) acc[q][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0; s < a.tiles_per_block; ++s) {
+        const int tile = blockIdx.x * a.tiles_per_block + s;
+        if (tile >= ntiles) break;  // uniform
+        const int x0 = (tile % nx) * XT;
+        const int y0 = ((tile / nx) % ny) * 2;
+        const int z0 = ((tile / (nx * ny)) % nz) * 2;
+        const int b = tile / (nx * ny * nz);
+        const size_t vb = (size_t)b * D * D * D;
+        __syncthreads();  // the previous tile is consumed
+        // masked output gradient: gs[co][line][x], line = 2 lz + ly
+        for (int i = t; i < 4 * XT * (COUT / 8); i += 256) {
+            const int ch = (i % (COUT / 8)) * 8, v = i / (COUT / 8);
+            const int x = v % XT, l = v / XT;
+            const size_t g = vb + ((size_t)(z0 + (l >> 1)) * D + (y0 + (l & 1))) * D + x0 + x;
+            u32x4 q = *(const u32x4*)(a.g + g * COUT + ch);
+            if (a.mask) q = mask8(q, *(const u32x4*)(a.mask + g * COUT + ch));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                gs[(ch + 2 * k) * GS + l * XT + x] = (bf16_t)(q[k] & 0xffffu);
+                gs[(ch + 2 * k + 1) * GS + l * XT + x] = (bf16_t)(q[k] >> 16);
+            }
+        }
+        // the chunk's input: xs[dx][ci][pz][hy][xd] = x(z0 + pz + dz - 1, y0 + hy - 1, x0 + xd + dx - 1)
+        for (int i = t; i < 2 * HY * XH * 2; i += 256) {
+            const int half = i & 1, v = i >> 1;
+            const int xi = v % XH, r = v / XH;
+            const int pz = r / HY, hy = r % HY;
+            const size_t g =
+                vb + ((size_t)wrap(z0 + pz + dz - 1, D) * D + wrap(y0 + hy - 1, D)) * D + wrap(x0 + xi - 1, D);
+            const u32x4 q = *(const u32x4*)(xsrc + g * xstride + xoff + half * 8);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int xd = xi - c;
+                if (xd >= 0 && xd < XT) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int ci = half * 8 + 2 * k;
+                        xs[(c * 16 + ci) * XS + r * XT + xd] = (bf16_t)(q[k] & 0xffffu);
+                        xs[(c * 16 + ci + 1) * XS + r * XT + xd] = (bf16_t)(q[k] >> 16);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        bf16x8 ga[NTC];
+#pragma unroll
+        for (int n = 0; n < NTC; ++n)
+            ga[n] = __builtin_bit_cast(bf16x8, *(const u32x4*)(gs + (n * 16 + row) * GS + wave * XT + grp * 8));
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) {
+                const bf16x8 xb = __builtin_bit_cast(
+                    bf16x8, *(const u32x4*)(xs + (dx * 16 + row) * XS + (lz * HY + ly + dy) * XT + grp * 8));
+#pragma unroll
+                for (int n = 0; n < NTC; ++n)
+                    acc[dy * 3 + dx][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[n], xb, acc[dy * 3 + dx][n], 0, 0, 0);
+            }
+    }
+    // fixed-order sum of the four waves, one tap at a time, into this block's
+    // partial (lane: co = 16 n + 4 grp + i, ci = cb + row)
+    float* red = (float*)xs;
+    float* out = a.partial + (size_t)blockIdx.x * COUT * 27 * CIN;
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        __syncthreads();
+        if (wave > 0) {
+#pragma unroll
+            for (int n = 0; n < NTC; ++n) *(floatx4*)(red + (((wave - 1) * NTC + n) * 64 + lane) * 4) = acc[q][n];
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int tap = dz * 9 + q;
+#pragma unroll
+            for (int n = 0; n < NTC; ++n) {
+                floatx4 sum = acc[q][n];
+#pragma unroll
+                for (int w = 0; w < 3; ++w) sum += *(const floatx4*)(red + ((w * NTC + n) * 64 + lane) * 4);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) out[((size_t)(n * 16 + grp * 4 + i) * 27 + tap) * CIN + cb + row] = sum[i];
+            }
+        }
     }
 }
 
 // Fixed-order sum over blocks of n-float partials: out[i] = sum_b partial[b][i].
 // A block of 256 threads covers 32 outputs; thread group g (of 8) adds the
-// partials b = g, g + 8, ... in turn, four loads in flight, then the 8 group
-// sums are added in order (deterministic, and 8 short dependent chains instead
-// of one long one).  Entries from n0 on go to out1 (weights, then bias).
+// partials b = g, g + 8, ... in turn, then the 8 group sums are added in
+// order (deterministic, and 8 short dependent chains instead of one long one).
 constexpr int kSumOut = 32;
 __global__ __launch_bounds__(256) void k_sum_blocks(const float* __restrict__ partial, int nblk, int n,
-                                                    float* __restrict__ out, int n0, float* __restrict__ out1) {
+                                                    float* __restrict__ out) {
     __shared__ float red[8][kSumOut];
     const int j = threadIdx.x % kSumOut, g = threadIdx.x / kSumOut;
     const int i = blockIdx.x * kSumOut + j;
     float s = 0.0f;
-    if (i < n) {
-        int b = g;
-        for (; b + 24 < nblk; b += 32) {
-            float v[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = partial[(size_t)(b + 8 * q) * n + i];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) s += v[q];
-        }
-        for (; b < nblk; b += 8) s += partial[(size_t)b * n + i];
-    }
+    if (i < n)
+        for (int b = g; b < nblk; b += 8) s += partial[(size_t)b * n + i];
     red[g][j] = s;
     __syncthreads();
     if (g == 0 && i < n) {
         float r = red[0][j];
         for (int q = 1; q < 8; ++q) r += red[q][j];
-        if (i < n0)
-            out[i] = r;
-        else if (out1)
-            out1[i - n0] = r;
+        out[i] = r;
     }
 }
 inline unsigned sum_blocks_grid(int n) { return (unsigned)((n + kSumOut - 1) / kSumOut); }
@@ -1615,23 +1618,21 @@ const ConvShape* conv_shape(int cin, int cout) {
     return nullptr;
 }
 
-// Blocks of the weight gradient along x: as many as stay resident (LDS 30 to 59
-// KB, 124 to 240 registers), over the parts of grid y.
-constexpr int wgrad_blocks(int cin, int cout) {
-    return cin == 16 ? 768 : 512 / (((cin + 31) / 32) * ((cout + 31) / 32));
-}
-
 using WgradFn = void (*)(const WgradArgs&, int nblk, hipStream_t);
-template <int CIN, int COUT, int XT>
+template <int CIN, int COUT>
 void launch_wgrad(const WgradArgs& a, int nblk, hipStream_t st) {
-    const int parts = ((CIN + 31) / 32) * ((COUT + 31) / 32);
-    k_conv3_wgrad<CIN, COUT, XT><<<dim3(nblk, parts), wgrad_threads(CIN), 0, st>>>(a);
+    k_conv3_wgrad<CIN, COUT><<<dim3(nblk, 9), 256, 0, st>>>(a);
+}
+template <int CIN, int COUT>
+void launch_wgrad_mfma(const WgradArgs& a, int nblk, hipStream_t st) {
+    k_conv3_wgrad_mfma<CIN, COUT><<<dim3(nblk, 3 * (CIN / 16)), 256, 0, st>>>(a);
 }
 struct WgradShape {
     int cin, cout;
-    WgradFn x32, x16;  // sides that are a multiple of 32, and the others
+    WgradFn fn;    // fp32 VALU, voxel tiles 2 x 2 x 16 (any D)
+    WgradFn mfma;  // matrix cores, voxel tiles 2 x 2 x 32 (D a multiple of 32, c0 a multiple of 16)
 };
-#define CM21_WGRAD(CI, CO) {CI, CO, launch_wgrad<CI, CO, 32>, launch_wgrad<CI, CO, 16>}
+#define CM21_WGRAD(CI, CO) {CI, CO, launch_wgrad<CI, CO>, launch_wgrad_mfma<CI, CO>}
 const WgradShape kWgradShapes[] = {
     CM21_WGRAD(16, 16), CM21_WGRAD(16, 32), CM21_WGRAD(32, 16), CM21_WGRAD(32, 32),
     CM21_WGRAD(32, 64), CM21_WGRAD(64, 32), CM21_WGRAD(64, 64),
@@ -1642,6 +1643,8 @@ const WgradShape* wgrad_shape(int cin, int cout) {
         if (s.cin == cin && s.cout == cout) return &s;
     return nullptr;
 }
+
+constexpr int kWgradBlocks = 256;   // voxel-slab blocks of the weight gradient
 
 constexpr int kChanBlocks = 128;    // per-sample blocks of the channel sums
 
@@ -1735,7 +1738,9 @@ extern "C" int cm21_unet_conv3_fwd(const cm21_unet_conv* c, void* stream) {
 
 extern "C" size_t cm21_unet_wgrad_workspace_bytes(int B, int D, int cin, int cout) {
     if (B < 1 || !valid_unet_dim(D) || cin < 1 || cout < 1) return 0;
-    return align_up((size_t)wgrad_blocks(cin, cout) * ((size_t)cout * 27 * cin + cout) * sizeof(float), 256);
+    const size_t w = (size_t)kWgradBlocks * cout * 27 * cin * sizeof(float);
+    const size_t c = (size_t)B * kChanBlocks * cout * sizeof(float);
+    return align_up(w, 256) + align_up(c, 256);
 }
 
 extern "C" int cm21_unet_conv3_wgrad(const cm21_unet_wgrad* w, void* stream) {
@@ -1750,12 +1755,14 @@ extern "C" int cm21_unet_conv3_wgrad(const cm21_unet_wgrad* w, void* stream) {
     if (w->work_bytes < need)
         return fail(CM21_ERR_NOMEM, "cm21_unet_conv3_wgrad: workspace %zu < %zu", w->work_bytes, need);
     hipStream_t st = (hipStream_t)stream;
-    // z-planes per unit: the longest walk (fewest re-read halo planes) that
-    // still gives every block a unit
-    const int xt = w->D % 32 == 0 ? 32 : 16, cap = wgrad_blocks(w->cin, w->cout);
-    const int columns = w->B * (w->D / xt) * (w->D / 4);
-    int nz = 16;
-    while (nz > 2 && columns * (w->D / nz) < cap) nz /= 2;
+    float* partial = (float*)w->work;
+    float* cpart = (float*)((char*)w->work + align_up((size_t)kWgradBlocks * w->cout * 27 * w->cin * sizeof(float), 256));
+    // the matrix-core form needs x-lines of 32 voxels and whole 16-channel
+    // chunks per input tensor; the VALU form takes the rest
+    const bool mfma = w->D % 32 == 0 && w->c0 % 16 == 0;
+    const int ntiles = w->B * (w->D / 2) * (w->D / 2) * (w->D / (mfma ? 32 : 16));
+    const int tpb = (ntiles + kWgradBlocks - 1) / kWgradBlocks;
+    const int nblk = (ntiles + tpb - 1) / tpb;
     WgradArgs a{};
     a.B = w->B;
     a.D = w->D;
@@ -1764,16 +1771,14 @@ extern "C" int cm21_unet_conv3_wgrad(const cm21_unet_wgrad* w, void* stream) {
     a.x1 = (const bf16_t*)w->x1;
     a.g = (const bf16_t*)w->g;
     a.mask = (const bf16_t*)w->mask;
-    a.partial = (float*)w->work;
-    a.nz = nz;
-    a.units = columns * (w->D / nz);
-    a.units_per_block = (a.units + cap - 1) / cap;
-    const int nblk = (a.units + a.units_per_block - 1) / a.units_per_block;
-    (xt == 32 ? s->x32 : s->x16)(a, nblk, st);
+    a.partial = partial;
+    a.tiles_per_block = tpb;
+    (mfma ? s->mfma : s->fn)(a, nblk, st);
     CM21_LAUNCH_CHECK("k_conv3_wgrad");
-    const int n0 = w->cout * 27 * w->cin, n = n0 + w->cout;
-    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(a.partial, nblk, n, w->dw, n0, w->db);
+    const int n = w->cout * 27 * w->cin;
+    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(partial, nblk, n, w->dw);
     CM21_LAUNCH_CHECK("k_sum_blocks");
+    if (w->db) CM21_TRY(channel_sums(w->g, w->mask, w->cout, (size_t)w->D * w->D * w->D, w->B, cpart, w->db, nullptr, st));
     return CM21_OK;
 }
 
@@ -1826,7 +1831,7 @@ int up_bwd_t(const void* x, const void* dy, const void* wk, void* dx, float* dw,
     }
     CM21_LAUNCH_CHECK("k_up_wgrad");
     const int n = COUT * 8 * CIN;
-    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(part, nblk, n, dw, n, nullptr);
+    k_sum_blocks<<<sum_blocks_grid(n), 256, 0, st>>>(part, nblk, n, dw);
     CM21_LAUNCH_CHECK("k_sum_blocks");
     const size_t vps = (size_t)8 * D * D * D;
     CM21_TRY(channel_sums(dy, nullptr, COUT, vps, B, cpart, db, nullptr, st));
@@ -1914,7 +1919,7 @@ extern "C" int cm21_unet_in_wgrad(const float* delta, const float* cond, const v
     const int nblk = (nlines + lpb - 1) / lpb;
     k_in_wgrad_mfma<<<nblk, 256, 0, st>>>(delta, (const bf16_t*)g, (const bf16_t*)y, part, B, D, delta_scale, lpb);
     CM21_LAUNCH_CHECK("k_in_wgrad_mfma");
-    k_sum_blocks<<<sum_blocks_grid(16 * 27), 256, 0, st>>>(part, nblk, 16 * 27, dwd, 16 * 27, nullptr);
+    k_sum_blocks<<<sum_blocks_grid(16 * 27), 256, 0, st>>>(part, nblk, 16 * 27, dwd);
     CM21_LAUNCH_CHECK("k_sum_blocks");
     CM21_TRY(channel_sums(g, y, 16, (size_t)D * D * D, B, cpart, nullptr, gsum, st));
     k_in_finish<<<(16 * 27 + 255) / 256, 256, 0, st>>>(dwd, gsum, cond, dw, db, B, 16);
@@ -1941,7 +1946,7 @@ extern "C" int cm21_unet_head(const void* x, const float* w, const float* bias, 
                                             (float)(1.0 / (double)nv));
     CM21_LAUNCH_CHECK("k_head");
     if (target) {
-        k_sum_blocks<<<sum_blocks_grid(17), 256, 0, st>>>(part, kHeadBlocks, 17, dwb, 17, nullptr);
+        k_sum_blocks<<<sum_blocks_grid(17), 256, 0, st>>>(part, kHeadBlocks, 17, dwb);
         CM21_LAUNCH_CHECK("k_sum_blocks");
         k_sum_f64<<<1, 256, 0, st>>>(lpart, kHeadBlocks, 1.0 / (double)nv, loss);
         CM21_LAUNCH_CHECK("k_sum_f64");

@@ -518,32 +518,3 @@ def test_conv_pool_output_matches_pool_kernel(gpu, D):
                      head=_fp(bias), prob=_fp(bias))
     with pytest.raises(RuntimeError):
         lib.call("cm21_unet_conv3_fwd", ctypes.byref(c), st)
-
-
-@pytest.mark.parametrize("D,B,cin,cout,c0", [(16, 1, 16, 16, 16), (16, 3, 64, 64, 64), (16, 2, 32, 64, 8),
-                                             (32, 1, 64, 32, 24), (48, 1, 32, 16, 16), (48, 2, 16, 32, 8),
-                                             (64, 1, 32, 32, 32)])
-@pytest.mark.parametrize("masked", [True, False])
-def test_wgrad_edges(gpu, D, B, cin, cout, c0, masked):
-    """Weight and bias gradients at the smallest sides, both line widths, split
-    inputs whose halves are no multiple of 16 channels, with and without the
-    ReLU mask; db may be NULL.  fp32 sums: 1e-3 of the largest entry."""
-    lib = pkg("_lib")
-    x = _bf((B, D, D, D, cin), seed=D + cin)
-    g = _bf((B, D, D, D, cout), seed=D + cout)
-    m = _bf((B, D, D, D, cout), seed=7) if masked else None
-    x0, x1 = x[..., :c0].contiguous(), x[..., c0:].contiguous() if c0 < cin else None
-    work = torch.empty(lib.query("cm21_unet_wgrad_workspace_bytes", B, D, cin, cout), dtype=torch.uint8, device="cuda")
-    dw, db = torch.full((cout, 27, cin), 7.0, device="cuda"), torch.full((cout,), 7.0, device="cuda")
-    dw2 = torch.empty_like(dw)
-    for w, b in ((dw, db), (dw2, None)):
-        a = lib.UnetWgrad(B=B, D=D, cin=cin, cout=cout, c0=c0, x0=_vp(x0), x1=_vp(x1), g=_vp(g), mask=_vp(m), dw=_fp(w),
-                          db=_fp(b), work=_vp(work), work_bytes=work.numel())
-        lib.call("cm21_unet_conv3_wgrad", ctypes.byref(a), lib.stream_handle())
-    gd = _d(g) * ((_d(m) > 0) if masked else 1.0)
-    xd, gf = _d(x), gd.reshape(-1, cout)
-    ref = torch.stack([gf.T @ torch.roll(xd, (1 - t // 9, 1 - t // 3 % 3, 1 - t % 3), (1, 2, 3)).reshape(-1, cin)
-                       for t in range(27)], 1)
-    _close_f32(dw, ref, "dw")
-    _close_f32(db, gf.sum(0), "db")
-    assert torch.equal(dw, dw2)
