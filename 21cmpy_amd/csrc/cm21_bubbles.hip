@@ -181,8 +181,10 @@ __global__ void k_threshold(float* __restrict__ ion, const float* __restrict__ s
 //   paint:  whether h(a + o) + o^2 < R^2 for some o along axis 0.
 // The rows flag lines without a centre and the planes flag tiles without a
 // distance: nothing of those is written or read, and a tile of cells that are
-// all painted already is passed over.  Radii up to kNarrowReach cells (all
-// but boxes of very small cells) hold g^2 and h in 16 bits and take the tiles below:
+// all painted already is passed over.  Reaches up to kNarrowReach cells (all
+// but boxes of very small cells) hold g^2 and h in 16 bits, where sums saturate at
+// kNarrowMax, and take the tiles below (a reach that the side cuts short can come
+// with an R^2 beyond that, which only the 32-bit form can compare with):
 // saturating 16-bit adds and minima, two cells an instruction, against a column
 // of the tile in LDS, eight cells along the axis per thread, so that one LDS
 // read serves eight offsets and the squares stay in scalar registers.
@@ -192,6 +194,7 @@ __global__ void k_threshold(float* __restrict__ ion, const float* __restrict__ s
 // 5 (paint); the whole box 5.45 -> 2.29 ms.
 constexpr uint32_t kNoCentre = 0xFFFFu;
 constexpr int kNarrowReach = 190;  // the column of a tile stays below 64 KB of LDS
+constexpr float kNarrowMax = 65535.0f;
 constexpr int kTile = 64;          // cells along either side of a tile
 constexpr int kTileRun = 8;        // cells along the axis per thread
 static_assert(kTile / kTileRun * (kTile / 2) == kThreads, "one thread per run and pair of lines");
@@ -258,7 +261,8 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // Minimum over the offsets of the LDS column + o^2 for the thread's run of
 // cells.  col: the thread's pair of lines at the run's first cell less `reach`.
-// Offsets past the reach (the run's ends) have o^2 >= R^2 and change nothing.
+// Offsets past the reach (the run's ends) change nothing: they have o^2 >= R^2 or,
+// where the side cut the reach short, no cell or one that a nearer offset has too.
 __device__ __forceinline__ void run_minimum(const u16x2* col, int reach, u16x2 best[kTileRun]) {
 #pragma unroll
     for (int i = 0; i < kTileRun; ++i) best[i] = u16x2{0xFFFF, 0xFFFF};
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(kThreads) void k_sphere_tile(const uint16_t* __rest
     }
 }
 
-// The planes and the paint for a reach beyond kNarrowReach: 32-bit, a thread
+// The planes and the paint for a reach or an R^2 beyond the tiles': 32-bit, a thread
 // per cell, from offset 0 outwards until none can be nearer.
 constexpr uint32_t kFar = 0x3FFFFFFFu;
 
@@ -468,7 +472,7 @@ int launch_sphere(float* ion, const float* sm, int D, const CellTest& test, floa
     uint8_t* any_tile = any_row + (size_t)D * D;
     k_sphere_rows<<<(unsigned)((size_t)D * D / kWaves), kThreads, 0, st>>>(g, any_row, sm, D, test, reach, periodic);
     CM21_LAUNCH_CHECK("k_sphere_rows");
-    if (reach <= kNarrowReach) {
+    if (reach <= kNarrowReach && R2 <= kNarrowMax) {
         const unsigned n = (unsigned)((D + kTile - 1) / kTile);
         uint16_t* h = (uint16_t*)work;
         k_sphere_tile<false><<<dim3(n, n, D), kThreads, tile_lds(reach), st>>>(g, any_row, h, any_tile, nullptr, D,

@@ -60,3 +60,17 @@ def test_threshold_forms(gpu, D, denom, final):
     got = ion.cpu().numpy()
     assert np.array_equal((got == 1)[~near], (want == 1)[~near])
     assert np.allclose(got[~near], want[~near], rtol=1e-5, atol=1e-7, equal_nan=True)
+
+
+@pytest.mark.parametrize("D,R", [(150, 256.0), (150, 257.0), (160, 270.0), (180, 256.5), (180, 300.0), (190, 327.0),
+                                 (190, 1024.0)])
+def test_sphere_paint_radius_past_the_box(gpu, D, R):
+    """A clipped sphere of more cells than the side: the reach along an axis ends
+    at the box, the squared radius does not, and past 65535 it is beyond what 16
+    bits hold."""
+    centers = np.zeros((D, D, D), bool)
+    centers[0, 0, D - 1] = True
+    sm = np.where(centers, 2.0, -1.0).astype(np.float32)
+    ion = torch.zeros((D, D, D), device="cuda")
+    pkg("gpu").update_sphere(ion, torch.from_numpy(sm).cuda(), DELTAC, DENOM, ZETA, R, False)
+    assert np.array_equal(ion.cpu().numpy(), bubbles.paint_spheres(np.zeros_like(sm), centers, np.float32(R), False))
