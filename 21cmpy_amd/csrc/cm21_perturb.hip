@@ -3,11 +3,13 @@
 // Reference: Programs/perturb_field.cu:90-133 (move_mass) and
 // Programs/perturb_field.py:93-105, in the reference's float32 position
 // arithmetic.  NGP deposits the whole mass in the truncated cell (bit-exact
-// indices); CIC shares it over the 8 nearest cell centres.  Deposits are float atomics: the summation order varies from run
-// to run at the 1e-7 relative level, the target cells never do.
+// indices); CIC shares it over the 8 nearest cell centres.  Deposits are float
+// atomics: the summation order varies from run to run at the 1e-7 relative level,
+// the target cells never do.
 //
 // The particles of one HII cell share their displacement and deposit
-// together (k_move_cells), through an LDS tile around their block's patch.
+// together (k_move_cells, k_move_waves), through an LDS tile around their block's patch.
+#include <algorithm>
 #include <cmath>
 
 #include "cm21_internal.hpp"
@@ -81,8 +83,15 @@ __device__ inline float particle_mass(float delta, float growth_init) {
 constexpr int kHalo = 4, kReach = 2 * kHalo;  // tile side: patch side + kReach
 constexpr int kNY = 16, kNZ = 16, kWalk = 8, kMoveThreads = 512;
 
+__device__ __forceinline__ int wrapped(int x, int sw) {
+    x %= sw;
+    return x < 0 ? x + sw : x;
+}
+__device__ __forceinline__ void add_global(float* acc, int sw, int x, int y, int z, float w) {
+    atomicAdd(&acc[((size_t)wrapped(x, sw) * sw + wrapped(y, sw)) * sw + wrapped(z, sw)], w);
+}
+
 struct Tile {
-    float* acc;
     int ox, oy, oz, Tx, Ty, Tz, sw;
     bool use;
 
@@ -90,13 +99,6 @@ struct Tile {
         int l = x - o;
         l += l < 0 ? sw : 0;
         return l >= sw ? l - sw : l;
-    }
-    __device__ __forceinline__ static int cell(int x, int sw) {
-        x %= sw;
-        return x < 0 ? x + sw : x;
-    }
-    __device__ __forceinline__ void add_global(int x, int y, int z, float w) const {
-        atomicAdd(&acc[((size_t)cell(x, sw) * sw + cell(y, sw)) * sw + cell(z, sw)], w);
     }
 };
 
@@ -138,8 +140,33 @@ struct AxisWeights {
     }
 };
 
+// Deposits of one particle.
+template <int SCHEME>
+__device__ __forceinline__ void move_particle(float* __restrict__ acc, float delta, int i, int j, int k,
+                                              const float (&pv)[3], const MoveParams& mp) {
+    const int at[3] = {i, j, k};
+    AxisWeights<SCHEME, 0> o[3];
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        float f;
+        if (!particle_coord(particle_start(at[ax], mp.DIM), pv[ax], mp, f)) return;
+        o[ax].place(f);
+    }
+    const float mass = particle_mass(delta, mp.growth_init);
+    for (int c = 0; c < (SCHEME == 0 ? 1 : 8); ++c) {
+        const int a = c >> 2, b = (c >> 1) & 1, e = c & 1;
+        float wt = mass;
+        if (SCHEME == 1) {
+            wt = __fmul_rn(wt, a ? o[0].t : __fsub_rn(1.0f, o[0].t));
+            wt = __fmul_rn(wt, b ? o[1].t : __fsub_rn(1.0f, o[1].t));
+            wt = __fmul_rn(wt, e ? o[2].t : __fsub_rn(1.0f, o[2].t));
+        }
+        if (wt != 0.0f) add_global(acc, mp.sw, o[0].cell + a, o[1].cell + b, o[2].cell + e, wt);
+    }
+}
+
 // Q: DIM/sw when it is 1 to 4 (the weights of every plane stay in registers),
-// or 0 for a larger ratio (formed again per row).
+// or 0 for a larger ratio (formed again per row; few of them, see by_waves).
 template <int SCHEME, int Q>
 __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__ acc, const float* __restrict__ delta,
                                                     const float* __restrict__ vx, const float* __restrict__ vy,
@@ -155,7 +182,7 @@ __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__
     const int t = threadIdx.x;
     const int hy = y0 + t / kNZ % kNY, hz = z0 + t % kNZ;
     const int half = t / (kNY * kNZ), xa = x0 + half * (PX / 2);  // this thread's part of the walk
-    const Tile tl{acc, x0 - kHalo, y0 - kHalo, z0 - kHalo, Tx, Ty, Tz, sw, sw >= Tx && sw >= Ty && sw >= Tz};
+    const Tile tl{x0 - kHalo, y0 - kHalo, z0 - kHalo, Tx, Ty, Tz, sw, sw >= Tx && sw >= Ty && sw >= Tz};
     if (tl.use)
         for (int c = t; c < Tx * Ty * Tz; c += kMoveThreads) tile[c] = 0.0;
     if (t < kWalk * NQ) startx[t] = particle_start(x0 * NQ + t, DIM);
@@ -288,25 +315,7 @@ __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__
         if (!(ok && isfinite(total))) {
             for (int p = 0; p < q * q * q; ++p) {
                 const int i = p / (q * q), j = p / q % q, k = p % q;
-                W o[3];
-                float f[3];
-                if (!(particle_coord(particle_start(i0 + i, DIM), pv[0], mp, f[0]) &&
-                      particle_coord(particle_start(j0 + j, DIM), pv[1], mp, f[1]) &&
-                      particle_coord(particle_start(k0 + k, DIM), pv[2], mp, f[2])))
-                    continue;
-                const float mass = particle_mass(dp[((size_t)i * DIM + j) * DIM + k], mp.growth_init);
-#pragma unroll
-                for (int ax = 0; ax < 3; ++ax) o[ax].place(f[ax]);
-                for (int c = 0; c < (SCHEME == 0 ? 1 : 8); ++c) {
-                    const int a = c >> 2, b = (c >> 1) & 1, e = c & 1;
-                    float wt = mass;
-                    if (SCHEME == 1) {
-                        wt = __fmul_rn(wt, a ? o[0].t : __fsub_rn(1.0f, o[0].t));
-                        wt = __fmul_rn(wt, b ? o[1].t : __fsub_rn(1.0f, o[1].t));
-                        wt = __fmul_rn(wt, e ? o[2].t : __fsub_rn(1.0f, o[2].t));
-                    }
-                    if (wt != 0.0f) tl.add_global(o[0].cell + a, o[1].cell + b, o[2].cell + e, wt);
-                }
+                move_particle<SCHEME>(acc, dp[((size_t)i * DIM + j) * DIM + k], i0 + i, j0 + j, k0 + k, pv, mp);
             }
             continue;
         }
@@ -326,7 +335,7 @@ __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__
                 for (int b = 0; b < C; ++b)
 #pragma unroll
                     for (int c = 0; c < C; ++c)
-                        if (s[a][b][c] != 0.0f) tl.add_global(base[0] + a, base[1] + b, base[2] + c, s[a][b][c]);
+                        if (s[a][b][c] != 0.0f) add_global(acc, sw, base[0] + a, base[1] + b, base[2] + c, s[a][b][c]);
         }
     }
     if (!tl.use) return;
@@ -345,9 +354,205 @@ __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__
     }
 }
 
+// Larger ratios: a wavefront per displacement cell, or per share of one, where a
+// thread per cell leaves the chip idle (8 blocks at 512 -> 16).  A share is `len` of the
+// cell's planes along x and one of `parts` shares of a plane's q^2 columns.  A lane
+// sums its columns along x against the C weights of the planes, which the lanes
+// hold one plane each, then with the column's own weights into C^3 sums; these
+// are added over the lanes, half of them handed over at each step, after which lane l
+// has one sum.  A block takes a patch of P^3 cells (P = 1: up to eight shares of one)
+// and adds the sums up in an FP64 LDS tile around where its first cell goes, because
+// a global atomic per sum is 0.2 ns each and was the bound (512 -> 64: 1.7 ms).
+// CIC, against a thread per cell and a thread per 16 particles of a 16^3 patch:
+// 512 -> 16 108 us (9700, 943; 5 TB/s), 512 -> 32 138 (1282, 985), 512 -> 8 116 (66700,
+// 129600), 256 -> 32 57 (172, 168), 128 -> 16 22 (146, 42).  Bound by memory from q = 16
+// on, below by the sums' 31 exchanges a cell, and by the three launches up to 128^3.
+constexpr int kShareLen = 32;     // planes of a share (a lane each, up to 64 - kAhead)
+constexpr int kAhead = 8;         // planes whose loads are in flight together
+constexpr int kFillWaves = 8192;  // wavefronts wanted, eight per SIMD
+constexpr int kTileEdge = 10;     // P = 4, two cells on both sides and the CIC neighbours
+
+struct WaveSplit {
+    int P, halo;             // cells along a patch, tile cells on its sides
+    int len, chunks, parts;  // planes of a share, shares along x and of a plane
+    int shares;              // shares of a cell in a block
+};
+
+template <int SCHEME>
+__global__ __launch_bounds__(kMoveThreads, 6) void k_move_waves(float* __restrict__ acc, const float* __restrict__ delta,
+                                                             const float* __restrict__ vx, const float* __restrict__ vy,
+                                                             const float* __restrict__ vz, MoveParams mp, WaveSplit ws) {
+    using W = AxisWeights<SCHEME, 0>;
+    constexpr int C = W::C, C3 = C * C * C, CP = SCHEME == 0 ? 8 : 32;
+    __shared__ double tile[kTileEdge * kTileEdge * kTileEdge];
+    const int DIM = mp.DIM, sw = mp.sw, q = mp.q, lane = threadIdx.x & 63;
+    const int P = ws.P, T = P + C - 1 + 2 * ws.halo, np = (sw + P - 1) / P;
+    for (int c = threadIdx.x; c < T * T * T; c += kMoveThreads) tile[c] = 0.0;
+    const int x0 = (int)(blockIdx.x / (np * np)) * P, y0 = (int)(blockIdx.x / np % np) * P, z0 = (int)(blockIdx.x % np) * P;
+    int org[3];  // the tile's first cell
+    {
+        const size_t h = ((size_t)x0 * sw + y0) * sw + z0;
+        const float pv[3] = {vx[h], vy[h], vz[h]};
+        const int first[3] = {x0 * q, y0 * q, z0 * q};
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            float f;
+            W o;
+            o.place(particle_coord(particle_start(first[ax], DIM), pv[ax], mp, f) ? f : 0.0f);
+            org[ax] = o.cell - ws.halo;
+        }
+    }
+    __syncthreads();
+    const int cells = P * P * P;
+    for (int u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < cells * ws.shares; u += kMoveThreads / 64) {
+        const int pc = u % cells, share = blockIdx.y * ws.shares + u / cells;
+        const int hx = x0 + pc / (P * P), hy = y0 + pc / P % P, hz = z0 + pc % P;
+        if (hx >= sw || hy >= sw || hz >= sw || share >= ws.chunks * ws.parts) continue;
+        const int chunk = share / ws.parts, part = share % ws.parts, len = ws.len, parts = ws.parts;
+        const size_t h = ((size_t)hx * sw + hy) * sw + hz;
+        const float pv[3] = {vx[h], vy[h], vz[h]};
+        const int first[3] = {hx * q, hy * q, hz * q};
+        const int i0 = first[0] + chunk * len, ni = min(len, q - chunk * len);
+        const float* dp = delta + ((size_t)i0 * DIM + first[1]) * DIM + first[2];
+        int base[3];
+        bool ok = true;
+        auto weigh = [&](int ax, int p, W& o) {
+            float f;
+            ok = particle_coord(particle_start(p, DIM), pv[ax], mp, f) && ok;
+            o.place(f);
+            ok = o.weigh(base[ax], sw) && ok;
+        };
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            float f;
+            W o;
+            ok = particle_coord(particle_start(first[ax], DIM), pv[ax], mp, f) && ok;
+            o.place(f);
+            base[ax] = o.cell;
+        }
+        W wx;  // of plane `lane` of the share, nothing past its end
+        weigh(0, i0 + min(lane, ni - 1), wx);
+#pragma unroll
+        for (int a = 0; a < C; ++a)
+            if (lane >= ni) wx.w[a] = 0.0f;
+        float s[CP];
+#pragma unroll
+        for (int c = 0; c < CP; ++c) s[c] = 0.0f;
+        float total = 0.0f;
+        const int cols = q * q, dj = parts * 64 / q, dk = parts * 64 - dj * q;
+        int col = part * 64 + lane, j = col / q, k = col - j * q;
+        for (int c0 = part * 64; c0 < cols; c0 += parts * 64) {
+            const bool in = col < cols;  // the last lanes of a plane read its first column
+            const float* p = in ? dp + (size_t)j * DIM + k : dp;
+            float m[C];
+#pragma unroll
+            for (int a = 0; a < C; ++a) m[a] = 0.0f;
+            for (int i = 0; i < ni; i += kAhead) {
+                float d[kAhead];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) d[u] = p[(size_t)min(i + u, ni - 1) * DIM * DIM];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) {
+                    const float mass = particle_mass(d[u], mp.growth_init);
+                    total += mass;
+#pragma unroll
+                    for (int a = 0; a < C; ++a)
+                        m[a] = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(wx.w[a]), i + u)), mass, m[a]);
+                }
+            }
+            W wy, wz;
+            weigh(1, first[1] + (in ? j : 0), wy);
+            weigh(2, first[2] + (in ? k : 0), wz);
+#pragma unroll
+            for (int a = 0; a < C; ++a)
+#pragma unroll
+                for (int b = 0; b < C; ++b) {
+                    const float w = in ? m[a] * wy.w[b] : 0.0f;
+#pragma unroll
+                    for (int c = 0; c < C; ++c) s[(a * C + b) * C + c] = fmaf(w, wz.w[c], s[(a * C + b) * C + c]);
+                }
+            col += parts * 64;
+            j += dj;
+            k += dk;
+            if (k >= q) {
+                k -= q;
+                ++j;
+            }
+        }
+        if (!__all(ok && isfinite(total))) {
+            for (int p = part * 64 + lane; p < ni * cols; p += parts * 64) {
+                const int i = p / cols, y = p / q % q, z = p % q;
+                move_particle<SCHEME>(acc, dp[((size_t)i * DIM + y) * DIM + z], i0 + i, first[1] + y, first[2] + z, pv, mp);
+            }
+            continue;
+        }
+        // lane l ends with sum number (bits of l reversed)
+#pragma unroll
+        for (int n = CP / 2, bit = 1; n > 0; n >>= 1, bit <<= 1) {
+            const bool up = lane & bit;
+#pragma unroll
+            for (int c = 0; c < n; ++c) {
+                const float give = up ? s[c] : s[c + n];
+                s[c] = (up ? s[c + n] : s[c]) + __shfl_xor(give, bit, 64);
+            }
+        }
+#pragma unroll
+        for (int bit = CP; bit < 64; bit <<= 1) s[0] += __shfl_xor(s[0], bit, 64);
+        const int n = (int)(__brev((unsigned)lane) >> (SCHEME == 0 ? 29 : 27));
+        if (lane < CP && n < C3 && s[0] != 0.0f) {
+            const int lx = wrapped(base[0] - org[0], sw), ly = wrapped(base[1] - org[1], sw);
+            const int lz = wrapped(base[2] - org[2], sw);
+            const int a = n / (C * C), b = n / C % C, c = n % C;
+            if (lx <= T - C && ly <= T - C && lz <= T - C)
+                atomicAdd(&tile[((lx + a) * T + ly + b) * T + lz + c], (double)s[0]);
+            else
+                add_global(acc, sw, base[0] + a, base[1] + b, base[2] + c, s[0]);
+        }
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < T * T * T; c += kMoveThreads) {
+        const float v = (float)tile[c];
+        if (v != 0.0f) add_global(acc, sw, org[0] + c / (T * T), org[1] + c / T % T, org[2] + c % T, v);
+    }
+}
+
+// Whether the cells go to a wavefront each.  Time of a thread per cell over that,
+// CIC: q = 5 2.0 at sw = 16, 0.9 at 32, 0.3 at 64 and 80; q = 6 2.9 at 16, 1.5 at 32,
+// 0.97 at 40, 0.6 at 48 and 56; q = 8 3.0 at 32, 1.3 at 48, 1.5 at 56, 1.1 at 64 and 128;
+// q = 9 0.9 at 64, 80 and 128; q = 10 1.6 at 48, 1.2 at 64, 1.1 at 80; q = 12 1.5 at 64;
+// q = 16 3.2 at 64.  Up to q = 4 the thread has its weights in registers and is never
+// slower by more than the launches.
+bool by_waves(const MoveParams& mp) { return mp.q >= 10 || (mp.q >= 5 && mp.sw < (mp.q < 8 ? 40 : 64)); }
+
+int patches(int sw, int P) {
+    const int n = (sw + P - 1) / P;
+    return n * n * n;
+}
+
+// The largest patch with two blocks to a CU, and shares that fill the chip.
+WaveSplit wave_split(const MoveParams& mp) {
+    WaveSplit ws;
+    ws.P = patches(mp.sw, 4) >= 512 ? 4 : (patches(mp.sw, 2) >= 512 ? 2 : 1);
+    ws.halo = ws.P > 1 ? 2 : 0;
+    ws.len = std::min(mp.q, kShareLen);
+    ws.chunks = (mp.q + ws.len - 1) / ws.len;
+    const long waves = (long)mp.sw * mp.sw * mp.sw * ws.chunks, most = ((long)mp.q * mp.q + 63) / 64;
+    ws.parts = (int)std::min((kFillWaves + waves - 1) / waves, most);
+    ws.shares = ws.P > 1 ? ws.chunks * ws.parts : std::min(ws.chunks * ws.parts, kMoveThreads / 64);
+    return ws;
+}
+
 template <int SCHEME>
 int launch_move(float* acc, const float* delta, const float* vx, const float* vy, const float* vz, const MoveParams& mp,
                 hipStream_t st) {
+    if (by_waves(mp)) {
+        const WaveSplit ws = wave_split(mp);
+        const int all = ws.chunks * ws.parts;
+        k_move_waves<SCHEME><<<dim3(patches(mp.sw, ws.P), (all + ws.shares - 1) / ws.shares), kMoveThreads, 0, st>>>(
+            acc, delta, vx, vy, vz, mp, ws);
+        CM21_LAUNCH_CHECK("k_move_waves");
+        return CM21_OK;
+    }
     auto blocks = [&](int n) { return (unsigned)((mp.sw + n - 1) / n); };
     // a walk of kWalk cells, or of 2 where that would leave CUs without a block
     const int PX = blocks(kWalk) * blocks(kNY) * blocks(kNZ) >= 512 ? kWalk : 2;

@@ -60,3 +60,55 @@ def test_move_mass_keeps_bad_particles_apart(gpu):
         assert np.isfinite(got).all()
         # 16 particles of 64^3 are gone; cells hold (mass / 8) - 1
         assert abs((got.astype(np.float64) + 1.0).sum() * 8 - (DIM ** 3 - 16)) < 0.05
+
+
+@pytest.mark.parametrize("DIM,sw", [(48, 3), (96, 2), (128, 1), (128, 2), (160, 10), (176, 16), (208, 26), (272, 34)])
+@pytest.mark.parametrize("amp", [0.0, 3.0, 200.0])
+def test_move_mass_large_ratios(gpu, DIM, sw, amp):
+    """A wavefront per displacement cell: shares of one cell, of its planes and
+    columns, patches of 1, 2 and 4 cells that the side does not fill, and cells
+    that leave their patch's tile."""
+    test_move_mass_edges(gpu, DIM, sw, amp)
+
+
+def test_move_mass_large_ratio_keeps_bad_particles_apart(gpu):
+    g = pkg("gpu")
+    DIM, sw, L = 96, 6, 60.0
+    rng = np.random.default_rng(6)
+    delta = np.zeros((DIM,) * 3, np.float32)
+    v = [(3.0 * rng.standard_normal((sw,) * 3)).astype(np.float32) for _ in range(3)]
+    s = pkg("Programs.perturb_field").displacement_scale(0.12, 0.0036, L)
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    delta[10, 20, 31] = np.nan
+    delta[40, 41, 42] = np.inf
+    for scheme, most in (("ngp", 1), ("cic", 8)):
+        got = g.move_mass(dev(delta), *[dev(a) for a in v], s, 0.0036, scheme).cpu().numpy()
+        assert 1 <= np.isnan(got).sum() <= most and 1 <= np.isinf(got).sum() <= most
+    delta[:] = 0.0
+    v[0][0, 0, 0] = np.nan  # a patch's first cell
+    v[2][4, 5, 3] = np.inf
+    for scheme in ("ngp", "cic"):
+        got = g.move_mass(dev(delta), *[dev(a) for a in v], s, 0.0036, scheme).cpu().numpy()
+        assert np.isfinite(got).all()
+        assert abs((got.astype(np.float64) + 1.0).sum() * 16 ** 3 - (DIM ** 3 - 2 * 16 ** 3)) < 2.0
+
+
+def test_move_mass_time_does_not_grow_with_the_ratio(gpu):
+    """The same 256^3 particles on fewer cells: nowhere near the 31 times of a
+    thread per cell between 32^3 and 8^3 cells (both take about 50 us)."""
+    g = pkg("gpu")
+    delta = torch.zeros((256,) * 3, device="cuda")
+
+    def best(sw):
+        v = [torch.zeros((sw,) * 3, device="cuda") for _ in range(3)]
+        times = []
+        for _ in range(6):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            g.move_mass(delta, *v, 1e-4, 0.0036, "cic")
+            e[1].record()
+            torch.cuda.synchronize()
+            times.append(e[0].elapsed_time(e[1]))
+        return min(times)
+
+    assert best(8) < 6.0 * best(32)
