@@ -74,3 +74,16 @@ def test_sphere_paint_radius_past_the_box(gpu, D, R):
     ion = torch.zeros((D, D, D), device="cuda")
     pkg("gpu").update_sphere(ion, torch.from_numpy(sm).cuda(), DELTAC, DENOM, ZETA, R, False)
     assert np.array_equal(ion.cpu().numpy(), bubbles.paint_spheres(np.zeros_like(sm), centers, np.float32(R), False))
+
+
+@pytest.mark.parametrize("D,R,centre,periodic", [(128, 300.0, True, True), (128, 300.0, False, True), (130, 257.0, True, True),
+                                                 (380, 381.0, True, True), (190, 327.5, True, False), (190, 1024.0, False, False),
+                                                 (148, 256.0, True, False)])
+def test_sphere_paint_radius_past_every_cell(gpu, D, R, centre, periodic):
+    """No cell as far as R, R^2 past 16 bits: one centre paints the whole box, none paints nothing."""
+    sm = torch.full((D, D, D), -1.0, device="cuda")
+    if centre:
+        sm[0, D - 1, D - 1] = 2.0
+    ion = torch.zeros_like(sm)
+    pkg("gpu").update_sphere(ion, sm, DELTAC, DENOM, ZETA, R, periodic)
+    assert bool((ion == (1.0 if centre else 0.0)).all())
