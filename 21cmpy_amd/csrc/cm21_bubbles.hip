@@ -465,7 +465,8 @@ int launch_threshold(float* ion, const float* sm, int D, const CellTest& t, int 
 int launch_sphere(float* ion, const float* sm, int D, const CellTest& test, float R_cells, int periodic, void* work,
                   hipStream_t st) {
     const size_t N = (size_t)D * D * D;
-    const float R2 = R_cells * R_cells;  // float32(R*R), find_bubbles.cu:98
+    if (!(R_cells > 0.0f)) return CM21_OK;  // (a negative sphere scale) no offset is inside
+    const float R2 = R_cells * R_cells;     // float32(R*R), find_bubbles.cu:98
     int reach = (int)std::ceil((double)R_cells);
     while (reach > 0 && (float)(reach * reach) >= R2) --reach;  // largest o with o^2 < R^2
     if (reach >= D) reach = periodic ? D / 2 : D - 1;

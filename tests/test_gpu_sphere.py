@@ -87,3 +87,27 @@ def test_sphere_paint_radius_past_every_cell(gpu, D, R, centre, periodic):
     ion = torch.zeros_like(sm)
     pkg("gpu").update_sphere(ion, sm, DELTAC, DENOM, ZETA, R, periodic)
     assert bool((ion == (1.0 if centre else 0.0)).all())
+
+
+@pytest.mark.parametrize("scale", [-0.1, -1.0, -30.0])
+def test_sphere_paint_negative_scale_paints_nothing(gpu, scale):
+    """A negative sphere radius has no offset inside it: every radius but the
+    last (threshold and partial values) leaves the box as it is, so the list of
+    radii and its last one alone give the same."""
+    lib = pkg("_lib")
+    D, L = 32, 48.0
+    delta = torch.randn((D,) * 3, generator=torch.Generator().manual_seed(1)).cuda()
+    radii = np.array([9.0, 5.0, 1.2], np.float32)
+    den = np.full(3, 1.0, np.float32)
+    prm = lib.BubbleParams(box_len=L, deltac=1.686, zeta=30.0, growth_inv=1.0, fc_mean=0.1, linear_input=1, filter_type=1,
+                           ref_fallthrough=1, update=1, sphere_periodic=0, sphere_r_scale=scale, fused=0)
+    work = torch.empty(lib.query("cm21_find_bubbles_workspace_bytes", D, 3, 1), dtype=torch.uint8, device="cuda")
+
+    def run(r, d):
+        out = torch.empty_like(delta)
+        lib.call("cm21_find_bubbles", lib.plan(D, 1).handle, lib.ptr(delta), lib.ptr(out),
+                 r.ctypes.data_as(lib.c_float_p), d.ctypes.data_as(lib.c_float_p), len(r), prm, lib.ptr(work),
+                 work.numel(), lib.stream_handle())
+        return out
+
+    assert torch.equal(run(radii, den), run(radii[2:], den[2:]))
