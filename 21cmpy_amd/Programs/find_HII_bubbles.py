@@ -195,18 +195,19 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
 
 # Graph replay needs the captured buffers to stay alive.  One entry is kept per
 # (box side, stream), the granularity at which the library keeps graphs: a new
-# input address replaces the entry (and its buffers) of its shape and stream.
+# input address or a larger workspace (its size depends on the radii and the
+# filter) replaces the entry (and its buffers) of its shape and stream.
 _graph_cache = {}
 
 
 def _graph_buffers(d, nbytes, stream):
     """Output and workspace kept alive for graph replay of the input `d`."""
-    slot = (tuple(d.shape), nbytes, stream.cuda_stream)
+    slot = (tuple(d.shape), stream.cuda_stream)
     cur = _graph_cache.get(slot)
-    if cur is None or cur[0] != d.data_ptr():
-        _graph_cache[slot] = (d.data_ptr(), torch.empty_like(d),
-                              torch.empty(nbytes, dtype=torch.uint8, device=d.device))
-    return _graph_cache[slot][1], _graph_cache[slot][2]
+    if cur is None or cur[0] != d.data_ptr() or cur[2].numel() < nbytes:
+        cur = _graph_cache[slot] = (d.data_ptr(), torch.empty_like(d),
+                                    torch.empty(nbytes, dtype=torch.uint8, device=d.device))
+    return cur[1], cur[2]
 
 
 def xH_filename(Z, nf, fil, dim, box_size):
