@@ -120,6 +120,11 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
     separate filter and threshold kernels.
     graph: capture the loop into a HIP graph and replay it when called again
     with the same tensors and parameters (needs a non-default stream).
+
+    Memory: the fused loop of sides up to 160 keeps every radius' transform, 30 MB
+    at 64^3 to 0.32 GB at 160^3 with filter 1 and 67 MB to 0.85 GB with filter 2 (41
+    radii); where that does not fit, the loop with a launch per radius takes 9 to
+    119 MB.
     """
     if visualize:
         raise ValueError("visualize is not supported by the GPU path")
@@ -167,7 +172,8 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
     plan = _lib.plan(D, 1)
     r = np.ascontiguousarray(radii, dtype=np.float32)
     dn = np.ascontiguousarray(denoms, dtype=np.float32)
-    nbytes = _lib.query("cm21_find_bubbles_full_workspace_bytes", D, r.ctypes.data_as(_lib.c_float_p), len(r), prm)
+    full = _lib.query("cm21_find_bubbles_full_workspace_bytes", D, r.ctypes.data_as(_lib.c_float_p), len(r), prm)
+    least = _lib.query("cm21_find_bubbles_workspace_bytes", D, len(r), int(update))
     # Everything runs on `s`, ordered after the caller's pending work and
     # before the caller's later work: the input upload, the loop, the read-back.
     if s != caller:
@@ -177,10 +183,11 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
         d = d.to(dev, dtype=torch.float32).contiguous()
         if graph:
             # a replayed graph reuses the captured addresses: keep the buffers
-            ion, work = _graph_buffers(d, nbytes, s)
+            ion, work = _graph_buffers(d, full, s, least)
         else:
             ion = torch.empty_like(d)
-            work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            work = _workspace(full, least, dev)
+        nbytes = min(work.numel(), full)
         _lib.call("cm21_find_bubbles", plan.handle, _lib.ptr(d), _lib.ptr(ion),
                   r.ctypes.data_as(_lib.c_float_p), dn.ctypes.data_as(_lib.c_float_p), len(radii),
                   prm, _lib.ptr(work), nbytes, _lib.stream_handle(s))
@@ -193,6 +200,17 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
     return out if is_tensor else host
 
 
+def _workspace(full, least, device):
+    """`full` bytes, or `least` where the memory does not hold those (the loop
+    then takes a launch per radius, with the same result)."""
+    try:
+        return torch.empty(full, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        if least >= full:
+            raise
+    return torch.empty(least, dtype=torch.uint8, device=device)
+
+
 # Graph replay needs the captured buffers to stay alive.  One entry is kept per
 # (box side, stream), the granularity at which the library keeps graphs: a new
 # input address or a larger workspace (its size depends on the radii and the
@@ -200,14 +218,14 @@ def conv_bubbles(deltax, param_dict, Z=None, scale=None, fil=1, update=0, LE=Fal
 _graph_cache = {}
 
 
-def _graph_buffers(d, nbytes, stream):
+def _graph_buffers(d, nbytes, stream, least=None):
     """Output and workspace kept alive for graph replay of the input `d`."""
     slot = (tuple(d.shape), stream.cuda_stream)
     cur = _graph_cache.get(slot)
-    if cur is None or cur[0] != d.data_ptr() or cur[2].numel() < nbytes:
-        cur = _graph_cache[slot] = (d.data_ptr(), torch.empty_like(d),
-                                    torch.empty(nbytes, dtype=torch.uint8, device=d.device))
-    return cur[1], cur[2]
+    if cur is None or cur[0] != d.data_ptr() or cur[1] < nbytes:
+        cur = _graph_cache[slot] = (d.data_ptr(), nbytes, torch.empty_like(d),
+                                    _workspace(nbytes, nbytes if least is None else least, d.device))
+    return cur[2], cur[3]
 
 
 def xH_filename(Z, nf, fil, dim, box_size):

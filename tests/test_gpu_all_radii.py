@@ -82,3 +82,33 @@ def test_sides_without_the_form_ask_for_the_least(gpu):
                                fused=fused)
         assert lib.query("cm21_find_bubbles_full_workspace_bytes", D, rp, 2, prm) == \
             lib.query("cm21_find_bubbles_workspace_bytes", D, 2, upd)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_conv_bubbles_without_room_for_every_radius(gpu, graph):
+    """Where the memory holds the workspace of the launch per radius but not that
+    of every radius at once, the call still runs, with the same box."""
+    fb, g = pkg("Programs.find_HII_bubbles"), pkg("gpu")
+    D, L = 160, 160.0
+    sp = pkg("cosmo_files.sigmas").PowerLawSpectrum(D, L)
+    delta = g.c2r(g.grf_init(D, L, sp.amp, 5)).contiguous()
+    from scipy.special import erfcinv
+    dc = 1.686 / 0.12
+    kw = dict(fil=2, LE=True, quiet=True, deltac=dc, sigma_min2=(dc / float(erfcinv(0.5 / 30.0))) ** 2 / 2.0, zeta=30.0,
+              sig0=sp.sig0_discrete)
+    want = fb.conv_bubbles(delta, {"BoxSize": L, "HIIdim": D}, **kw)
+    fb._graph_cache.clear()
+    stream = torch.cuda.Stream() if graph else None
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + (400 << 20)
+    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        for _ in range(2):
+            got = fb.conv_bubbles(delta, {"BoxSize": L, "HIIdim": D}, graph=graph, stream=stream, **kw)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        fb._graph_cache.clear()
+    assert (want == 1).any() and want.unique().numel() > 1000  # ionized cells and partial values
