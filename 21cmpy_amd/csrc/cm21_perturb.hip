@@ -166,7 +166,8 @@ __device__ __forceinline__ void move_particle(float* __restrict__ acc, float del
 }
 
 // Q: DIM/sw when it is 1 to 4 (the weights of every plane stay in registers),
-// or 0 for a larger ratio (formed again per row; few of them, see by_waves).
+// or 0 (formed again per row) for a larger ratio, few of them (by_waves), and
+// for masses that are not aligned.
 template <int SCHEME, int Q>
 __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__ acc, const float* __restrict__ delta,
                                                     const float* __restrict__ vx, const float* __restrict__ vy,
@@ -200,7 +201,8 @@ __global__ __launch_bounds__(kMoveThreads) void k_move_cells(float* __restrict__
 #pragma unroll
                 for (int j = 0; j < NQ; ++j) {
                     const float* row = dp + ((size_t)i * DIM + j) * DIM;
-                    // rows start at multiples of q floats and DIM is a multiple of 8
+                    // rows start at multiples of q floats from `delta`, which the launch
+                    // found aligned to q of them, and DIM is a multiple of 8
                     if constexpr (Q == 2) {
                         const float2 d = *(const float2*)row;
                         m[i][j][0] = d.x, m[i][j][1] = d.y;
@@ -559,10 +561,14 @@ int launch_move(float* acc, const float* delta, const float* vx, const float* vy
     const int Tx = PX + kReach, Ty = kNY + kReach, Tz = kNZ + kReach;
     const unsigned grid = blocks(PX) * blocks(kNY) * blocks(kNZ);
     const size_t lds = sizeof(double) * Tx * Ty * Tz;  // 72 KB, two blocks a CU (45 KB for the short walk)
-    auto* k = mp.q == 1 ? k_move_cells<SCHEME, 1>
-                        : (mp.q == 2 ? k_move_cells<SCHEME, 2>
-                                     : (mp.q == 3 ? k_move_cells<SCHEME, 3>
-                                                  : (mp.q == 4 ? k_move_cells<SCHEME, 4> : k_move_cells<SCHEME, 0>)));
+    // two and four masses of a row are one load; a view that does not start at a
+    // multiple of them takes the kernel that loads them one by one
+    const bool aligned = (uintptr_t)delta % (sizeof(float) * mp.q) == 0;
+    auto* k = mp.q == 1              ? k_move_cells<SCHEME, 1>
+              : mp.q == 2 && aligned ? k_move_cells<SCHEME, 2>
+              : mp.q == 3            ? k_move_cells<SCHEME, 3>
+              : mp.q == 4 && aligned ? k_move_cells<SCHEME, 4>
+                                     : k_move_cells<SCHEME, 0>;
     k<<<grid, kMoveThreads, lds, st>>>(acc, delta, vx, vy, vz, mp, PX, Tx, Ty, Tz);
     CM21_LAUNCH_CHECK("k_move_cells");
     return CM21_OK;

@@ -112,3 +112,24 @@ def test_move_mass_time_does_not_grow_with_the_ratio(gpu):
         return min(times)
 
     assert best(8) < 6.0 * best(32)
+
+
+@pytest.mark.parametrize("DIM,sw", [(64, 64), (64, 32), (48, 16), (64, 16), (160, 32), (64, 8)])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_move_mass_of_an_unaligned_view(gpu, DIM, sw, offset):
+    """Density and displacements that start in the middle of an allocation."""
+    g = pkg("gpu")
+    L = 60.0
+    rng = np.random.default_rng(DIM + sw)
+    delta = rng.standard_normal((DIM,) * 3).astype(np.float32)
+    v = [(3.0 * rng.standard_normal((sw,) * 3)).astype(np.float32) for _ in range(3)]
+    s = pkg("Programs.perturb_field").displacement_scale(0.12, 0.0036, L)
+
+    def view(a):
+        t = torch.empty(a.size + offset, device="cuda")[offset:].view(a.shape)
+        return t.copy_(torch.from_numpy(a))
+
+    got = g.move_mass(view(delta), *[view(a) for a in v], s, 0.0036, "cic").cpu().numpy()
+    assert np.allclose(got, perturb.move_mass_cic(delta, *v, 0.12, 0.0036, L), rtol=1e-5, atol=2e-6)
+    got = g.move_mass(view(delta), *[view(a) for a in v], s, 0.0036, "ngp").cpu().numpy()
+    assert np.allclose(got, perturb.move_mass_ngp(delta, *v, 0.12, 0.0036, L), rtol=1e-5, atol=2e-6)
