@@ -494,14 +494,19 @@ const BatchShape* batch_shape(int D) {
     return nullptr;
 }
 
-// Whether a group runs as planes: linear input, tiles of the planes' factors, and
-// enough boxes for the longer blocks to fill the chip.  Planes against rows and lines
+// The planes are the lines candidate after the tiles, of the sides that have them.
+int lines_candidates(const BatchShape& s) { return s.nlines + (s.planes ? 1 : 0); }
+
+// Whether a group runs as planes: where its lines candidate says so or, without a
+// choice (-1), for linear input, a columns tile of the planes' factors and enough
+// boxes for the longer blocks to fill the chip.  Planes against rows and lines
 // apart: 64^3 0.96 times as fast with 8 boxes, 1.13 with 12, 1.39 with 21; 96^3 0.94 with
 // 6, 1.12 with 8, 1.00 with 21, 1.16 with 24; 128^3 0.92 with 2, 1.10 with 4, 1.05 with 5,
 // 1.26 with 17; 160^3 0.95 with 4, 1.00 with 9, 1.02 with 13.
-bool as_planes(const BatchShape& s, int nbox, int col_tile, int line_tile, const cm21_bubble_params* prm) {
-    return s.planes && prm->linear_input && nbox >= s.planes_from && s.cols[col_tile].factor == s.cols[0].factor &&
-           s.lines[line_tile].factor == s.lines[0].factor;
+bool as_planes(const BatchShape& s, int nbox, int tile_columns, int tile_lines, const cm21_bubble_params* prm) {
+    if (!s.planes || !prm->linear_input) return false;
+    if (tile_lines >= 0) return tile_lines == s.nlines;
+    return nbox >= s.planes_from && (tile_columns < 0 || s.cols[tile_columns].factor == s.cols[0].factor);
 }
 
 int min_lines_per_block(const BatchShape& s) {
@@ -555,7 +560,8 @@ int build_layout(const cm21_batch_group* groups, int ngroups, const cm21_bubble_
         CM21_REQUIRE(g.radii, "cm21_find_bubbles_batched: group %d: radii is NULL", gi);
         CM21_REQUIRE(g.tile_columns >= -1 && g.tile_columns < h.shape->ncols,
                      "cm21_find_bubbles_batched: group %d: tile_columns=%d out of range", gi, g.tile_columns);
-        CM21_REQUIRE(g.tile_lines >= -1 && g.tile_lines < h.shape->nlines,
+        CM21_REQUIRE(g.tile_lines >= -1 &&
+                         g.tile_lines < (prm->linear_input ? lines_candidates(*h.shape) : h.shape->nlines),
                      "cm21_find_bubbles_batched: group %d: tile_lines=%d out of range", gi, g.tile_lines);
         if (check_arrays) {
             CM21_REQUIRE(g.delta && g.ionized && g.denoms && g.boxes && g.plan,
@@ -751,11 +757,11 @@ int prepare(const cm21_batch_group* groups, int ngroups, const cm21_bubble_param
     p.line_tile.clear();
     p.planes.clear();
     for (const auto& h : p.lay.groups) {
+        const bool planes = as_planes(*h.shape, h.nbox, h.g->tile_columns, h.g->tile_lines, prm);
         const int ct = tile_or_default(h.g->tile_columns);
-        const int lt = tile_or_default(h.g->tile_lines);
+        const int lt = planes ? 0 : tile_or_default(h.g->tile_lines);
         int cb = 0, rb = 0;
         fill_tables(h, prm, ct, p.blob, &cb, &rb);
-        const bool planes = as_planes(*h.shape, h.nbox, ct, lt, prm);
         p.launches.push_back(make_launch(h, (char*)work, cb, rb, h.D * h.D / h.shape->lines[lt].L));
         p.planes.push_back(planes);
         p.col_tile.push_back(ct);
@@ -910,13 +916,14 @@ extern "C" int cm21_find_bubbles_batched(const cm21_batch_group* groups, int ngr
 extern "C" int cm21_batch_tile_count(int D, int stage) {
     const BatchShape* s = batch_shape(D);
     if (!s || stage < 0 || stage > 1) return -1;
-    return stage == 0 ? s->ncols : s->nlines;
+    return stage == 0 ? s->ncols : lines_candidates(*s);
 }
 
 extern "C" const char* cm21_batch_tile_name(int D, int stage, int index) {
     const BatchShape* s = batch_shape(D);
     if (!s || stage < 0 || stage > 1) return nullptr;
     if (stage == 0) return (index >= 0 && index < s->ncols) ? s->cols[index].name : nullptr;
+    if (s->planes && index == s->nlines) return "planes";
     return (index >= 0 && index < s->nlines) ? s->lines[index].name : nullptr;
 }
 
@@ -994,8 +1001,9 @@ extern "C" int cm21_batch_autotune(cm21_batch_group* groups, int ngroups, const 
             }
         }
         apart += best;
-        if (rc == CM21_OK && as_planes(*h.shape, h.nbox, 0, 0, params)) {
-            // rows and lines in one, against the best of both apart
+        if (rc == CM21_OK && h.shape->planes && !params->linear_input && ms_out) ms_out[slot++] = 0.0;
+        if (rc == CM21_OK && h.shape->planes && params->linear_input) {
+            // columns, rows and lines in one, against the best of both apart
             fill_tables(h, params, 0, p.blob, &cb, &rb);
             rc = upload(p, work, st);
             a = make_launch(h, (char*)work, cb, rb, 0);
@@ -1009,7 +1017,11 @@ extern "C" int cm21_batch_autotune(cm21_batch_group* groups, int ngroups, const 
             if (rc == CM21_OK && hipEventRecord(e1, st) != hipSuccess) rc = fail(CM21_ERR_HIP, "hipEventRecord failed");
             float ms = 0.0f;
             if (rc == CM21_OK) rc = elapsed(&ms);
-            if (rc == CM21_OK && ms < apart) best_c = best_l = 0;
+            if (ms_out) ms_out[slot++] = ms / reps;
+            if (rc == CM21_OK && ms < apart) {
+                best_c = 0;
+                best_l = h.shape->nlines;
+            }
         }
         if (rc == CM21_OK) {
             groups[gi].tile_columns = best_c;

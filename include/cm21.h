@@ -317,7 +317,10 @@ size_t cm21_find_bubbles_batched_workspace_bytes(const cm21_batch_group* groups,
 int cm21_find_bubbles_batched(const cm21_batch_group* groups, int ngroups, const cm21_bubble_params* params,
                               void* work, size_t work_bytes, void* stream);
 
-/* Tile candidates per D: stage 0 = columns/rows passes, 1 = lines pass.
+/* Tile candidates per D: stage 0 = columns/rows passes, 1 = lines pass.  The last
+ * lines candidate of sides up to 160 is "planes", rows and lines of a plane in one
+ * block (linear input only); the other lines candidates run the two apart, and
+ * without a choice (tile_lines = -1) the number of boxes decides.
  * cm21_batch_tile_count returns -1 for an unsupported D. */
 int cm21_batch_tile_count(int D, int stage);
 const char* cm21_batch_tile_name(int D, int stage, int index);
@@ -325,8 +328,9 @@ const char* cm21_batch_tile_name(int D, int stage, int index);
 /* Times every candidate of both stages on the caller's data (reps timed runs
  * each, after one warm run) and writes the fastest into each group's
  * tile_columns / tile_lines.  ms_out (optional) receives the mean time of
- * each candidate, group by group, columns candidates first.  Leaves the
- * outputs unspecified; synchronises the stream. */
+ * each candidate, group by group, columns candidates first; that of the planes
+ * holds the columns pass too, and is 0 for nonlinear input.  Leaves the outputs
+ * unspecified; synchronises the stream. */
 int cm21_batch_autotune(cm21_batch_group* groups, int ngroups, const cm21_bubble_params* params, void* work,
                         size_t work_bytes, int reps, double* ms_out, void* stream);
 

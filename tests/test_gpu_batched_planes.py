@@ -37,3 +37,60 @@ def test_planes_equal_rows_and_lines(gpu, D, nbox, fil):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)), i
     ion = [float((x == 1).double().mean()) for x in together]
     assert ion[0] < 0.05 and ion[1] > 0.95 and all(0.02 < x < 0.98 for x in ion[3:])
+
+
+def _batch(D, nbox, linear=True, **kw):
+    g, bm = pkg("gpu"), pkg("Programs.find_HII_bubbles_batched")
+    L = 1.5625 * D
+    spectrum = pkg("cosmo_files.sigmas").PowerLawSpectrum(D, L)
+    specs = [{"D": D, "box_len": L, "zeta": 12.0 + i, "deltac": 1.686 if linear else 14.05, "sigma_min2": 0.5 if linear else 40.0,
+              "sig0": lambda R: sigma.sig0_discrete(R, D, L)} for i in range(nbox)]
+    bb = bm.BatchedBubbles(specs, fil=1, LE=linear, graph=False, tiles=None, **kw)
+    bb.set_deltas([g.c2r(g.grf_init(D, L, spectrum.amp, i)) * (1.0 if linear else 0.12) for i in range(nbox)])
+    return bb
+
+
+def _stage_calls(bb):
+    """Launches of (rows, lines) passes of one run."""
+    lib = pkg("_lib")
+    lib.profile_enable(True)
+    try:
+        bb.run()
+        torch.cuda.synchronize()
+        counts = lib.profile_collect()
+    finally:
+        lib.profile_enable(False)
+    return counts.get("fused_rows", (0, 0))[1], counts["fused_lines"][1]
+
+
+@pytest.mark.parametrize("D,nbox", [(64, 16), (128, 2)])
+def test_a_choice_of_lines_is_kept(gpu, D, nbox):
+    """A tile that is asked for runs rows and lines apart, "planes" runs them
+    together, whatever the number of boxes would choose by itself; a tuned
+    group runs what was written into it."""
+    bb = _batch(D, nbox)
+    lib = pkg("_lib").load()
+    key, = bb.tiles()
+    n = lib.cm21_batch_tile_count(D, 1)
+    assert lib.cm21_batch_tile_name(D, 1, n - 1) == b"planes" and lib.cm21_batch_tile_name(D, 1, n) is None
+    assert _stage_calls(bb)[0] == (0 if nbox == 16 else 1)
+    for l in range(n):
+        bb.set_tiles({key: (0, l)})
+        assert _stage_calls(bb) == ((0, 1) if l == n - 1 else (1, 1)), l
+    bb.stream = torch.cuda.Stream()
+    res = bb.autotune(reps=2)[key]
+    assert res["chosen"][1] == res["names"][-n:][res["lines"]]
+    assert _stage_calls(bb)[0] == (0 if res["chosen"][1] == "planes" else 1)
+
+
+def test_planes_are_for_linear_input(gpu):
+    lib = pkg("_lib")
+    bb = _batch(64, 12, linear=False)
+    key, = bb.tiles()
+    assert _stage_calls(bb)[0] == 1
+    bb.set_tiles({key: (0, lib.load().cm21_batch_tile_count(64, 1) - 1)})
+    with pytest.raises(lib.CM21Error):
+        bb.run()
+    bb.set_tiles({key: (-1, -1)})
+    bb.stream = torch.cuda.Stream()
+    assert bb.autotune(reps=1)[key]["chosen"][1] != "planes"
