@@ -51,10 +51,13 @@ def radius_schedule(box_len, hii_dim, py2_int_scale=False, r_max=None, r_min=Non
         scale = float(cell)
     else:
         scale = (int(box_len) // int(hii_dim)) if py2_int_scale else float(box_len) / float(hii_dim)
-    return np.array(_radii(float(r_max), r_min, fac, lf * scale), dtype=np.float32), scale
+    args = (float(r_max), r_min, fac, lf * scale)
+    # kept for plain numbers only: arrays have no value to look up by, and a tensor's
+    # identity or a float32 equal to a float64 would find another schedule
+    radii = _radii_of_numbers if all(type(a) in (int, float) for a in args) else _radii
+    return np.array(radii(*args), dtype=np.float32), scale
 
 
-@functools.lru_cache(maxsize=256)
 def _radii(R, r_min, fac, r_cell):
     """The radii of radius_schedule: they depend on these four numbers alone."""
     radii = []
@@ -65,6 +68,9 @@ def _radii(R, r_min, fac, r_cell):
         if final:
             return tuple(radii)
         R = R32 / fac
+
+
+_radii_of_numbers = functools.lru_cache(maxsize=256)(_radii)
 
 
 def barrier_denominators(radii, sigma_min2, sig0_fn):
