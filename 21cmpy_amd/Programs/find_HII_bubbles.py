@@ -54,7 +54,8 @@ def radius_schedule(box_len, hii_dim, py2_int_scale=False, r_max=None, r_min=Non
     args = (float(r_max), r_min, fac, lf * scale)
     # kept for plain numbers only: arrays have no value to look up by, and a tensor's
     # identity or a float32 equal to a float64 would find another schedule
-    radii = _radii_of_numbers if all(type(a) in (int, float) for a in args) else _radii
+    plain = type(r_min) in (int, float) and type(fac) in (int, float)
+    radii = _radii_of_numbers if plain else _radii
     return np.array(radii(*args), dtype=np.float32), scale
 
 
@@ -76,13 +77,19 @@ _radii_of_numbers = functools.lru_cache(maxsize=256)(_radii)
 def barrier_denominators(radii, sigma_min2, sig0_fn):
     """denom = float32(sqrt(2 (smin - float32(S(R))))) per radius
     (find_HII_bubbles.py:126-128); raises ValueError where smin <= S(R)."""
-    S0 = np.array([sig0_fn(R) for R in np.asarray(radii, dtype=np.float64).tolist()], dtype=np.float64)
-    S0 = S0.astype(np.float32).astype(np.float64)
+    R, S0, error = np.asarray(radii, dtype=np.float64).tolist(), [], None
+    try:
+        S0 += map(sig0_fn, R)
+    except Exception as e:  # a larger radius without a barrier is named first
+        error = e
+    S0 = np.array(S0, dtype=np.float64).reshape(len(S0)).astype(np.float32).astype(np.float64)
     arg = 2.0 * (float(sigma_min2) - S0)
     bad = np.flatnonzero(~(arg > 0.0))
     if bad.size:
         i = int(bad[0])
-        raise ValueError(f"sigma_min^2={sigma_min2} <= S(R={float(radii[i])})={S0[i]}: no barrier at this radius")
+        raise ValueError(f"sigma_min^2={sigma_min2} <= S(R={R[i]})={S0[i]}: no barrier at this radius")
+    if error is not None:
+        raise error
     return np.sqrt(arg).astype(np.float32)
 
 

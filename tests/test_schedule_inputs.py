@@ -32,3 +32,31 @@ def test_radius_schedule_follows_its_arguments():
             break
         R = float(np.float32(R)) / np.float32(1.125)
     assert np.array_equal(narrow, np.array(want, np.float32)) and len(wide) == len(narrow)
+
+
+@pytest.mark.parametrize("kind", [float, np.float32, np.array, lambda v: torch.tensor(v, dtype=torch.float64)])
+def test_barrier_takes_any_scalar_of_sigma(kind):
+    fb = pkg("Programs.find_HII_bubbles")
+    radii = np.array([5.0, 2.0], np.float32)
+    got = fb.barrier_denominators(radii, 2.0, lambda R: kind(0.5 / R))
+    assert got.shape == (2,) and got.dtype == np.float32
+    assert np.array_equal(got, np.sqrt([2.0 * (2.0 - float(np.float32(0.5 / R))) for R in (5.0, 2.0)]).astype(np.float32))
+
+
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")
+def test_barrier_of_one_element_arrays_and_the_first_radius_without_one():
+    """S(R) as an array of one element, and the first radius that has no
+    barrier named also where S fails at a smaller one."""
+    fb = pkg("Programs.find_HII_bubbles")
+    radii = np.array([5.0, 2.0], np.float32)
+    assert fb.barrier_denominators(radii, 2.0, lambda R: np.array([0.5 / R])).shape == (2,)
+
+    def sigma(R):
+        if R < 3.0:
+            raise KeyError(R)
+        return 5.0
+
+    with pytest.raises(ValueError, match=r"S\(R=5.0\)=5.0"):
+        fb.barrier_denominators(radii, 2.0, sigma)
+    with pytest.raises(KeyError):
+        fb.barrier_denominators(radii, 20.0, sigma)
