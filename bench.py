@@ -291,11 +291,11 @@ def plain_rate(torch, delta, L, deltac, smin, zeta, steps, linear=True, fused=Tr
                            linear_input=1 if linear else 0, filter_type=1, ref_fallthrough=1, update=0,
                            sphere_periodic=0, sphere_r_scale=1.0, fused=1 if fused else 0, graph=1 if graph else 0)
     plan = lib.plan(D, 1)
-    nbytes = lib.query("cm21_find_bubbles_workspace_bytes", D, len(radii), 0)
-    work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
     ion = torch.empty_like(delta)
     r_arr = np.ascontiguousarray(radii, np.float32)
     d_arr = np.ascontiguousarray(denoms, np.float32)
+    nbytes = lib.query("cm21_find_bubbles_full_workspace_bytes", D, r_arr.ctypes.data_as(lib.c_float_p), len(radii), prm)
+    work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
     stream = torch.cuda.Stream()
     stream.wait_stream(torch.cuda.current_stream())
 
@@ -535,11 +535,11 @@ def main():
                            filter_type=1, ref_fallthrough=1, update=0, sphere_periodic=0, sphere_r_scale=1.0,
                            fused=0 if args.generic else 1, graph=0 if args.no_graph else 1)
     plan = lib.plan(D, 1)
-    nbytes = lib.query("cm21_find_bubbles_workspace_bytes", D, len(radii), 0)
-    work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
     ion = torch.empty_like(upd)
     r_arr = np.ascontiguousarray(radii, np.float32)
     d_arr = np.ascontiguousarray(denoms, np.float32)
+    nbytes = lib.query("cm21_find_bubbles_full_workspace_bytes", D, r_arr.ctypes.data_as(lib.c_float_p), len(radii), prm)
+    work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
     torch.cuda.synchronize()
     stream = torch.cuda.Stream()  # graph capture needs a non-default stream
 

@@ -266,13 +266,13 @@ int cm21_power_spectrum(cm21_plan* plan, const float* field,
 #define CM21_STAGE_FCOLL_SUM 3
 #define CM21_STAGE_THRESHOLD 4
 #define CM21_STAGE_SPHERE 5
-#define CM21_STAGE_FUSED_COLUMNS 6         /* batched: columns pass of every (radius, box) */
-#define CM21_STAGE_FUSED_ROWS 7            /* batched: rows pass */
-#define CM21_STAGE_FUSED_LINES 8           /* batched: persistent lines pass */
-#define CM21_STAGE_FUSED_LINES_THRESHOLD 9 /* single box: the final paint */
-#define CM21_STAGE_FUSED_RADIUS 10         /* single box: one launch per radius (columns, rows,
-                                              box sum, reduction and threshold roles of
-                                              neighbouring radii) */
+/* "every radius": the single box whose workspace holds every radius' transform */
+#define CM21_STAGE_FUSED_COLUMNS 6         /* batched, every radius: columns pass */
+#define CM21_STAGE_FUSED_ROWS 7            /* batched, every radius: rows pass */
+#define CM21_STAGE_FUSED_LINES 8           /* batched: persistent lines pass; every radius: the final paint */
+#define CM21_STAGE_FUSED_LINES_THRESHOLD 9 /* launch per radius: the final paint; every radius: thresholds */
+#define CM21_STAGE_FUSED_RADIUS 10         /* launch per radius (columns, rows, box sum, reduction, verdict
+                                              and threshold roles of neighbouring radii) */
 #define CM21_NSTAGES 11
 int cm21_profile_enable(int stage_mask);
 int cm21_profile_collect(double* ms, int64_t* count, int nstages);
