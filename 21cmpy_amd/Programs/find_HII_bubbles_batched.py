@@ -68,6 +68,14 @@ def _tile_key(D, box_len, nbox, fil, LE):
     return f"D{int(D)}_L{float(box_len):g}_B{int(nbox)}_f{int(fil)}_{'lin' if LE else 'nl'}"
 
 
+def _tile_lines(entry):
+    """Lines tile of a stored choice.  "or_planes" marks a tile that was the fastest
+    of those that run rows and lines apart, on boxes that say nothing about the
+    caller's: whether they run together is then left to the library."""
+    lines = int(entry.get("lines", -1))
+    return -2 - lines if entry.get("or_planes") and lines >= 0 else lines
+
+
 def load_tiles(path=TILES):
     if os.path.exists(path):
         with open(path) as f:
@@ -155,7 +163,7 @@ class BatchedBubbles:
                 D=g["D"], nbox=len(g["idx"]), box_len=g["L"], n_radii=len(g["radii"]),
                 radii=g["radii"].ctypes.data_as(_lib.c_float_p), denoms=g["denoms"].ctypes.data_as(_lib.c_float_p),
                 boxes=g["boxes"], delta=g["delta"].data_ptr(), ionized=g["ion"].data_ptr(), plan=g["plan"].handle,
-                tile_columns=int(t.get("columns", -1)), tile_lines=int(t.get("lines", -1)))
+                tile_columns=int(t.get("columns", -1)), tile_lines=_tile_lines(t))
         nbytes = _lib.query("cm21_find_bubbles_batched_workspace_bytes", self._garr, len(self._groups), self.prm)
         if nbytes == 0:
             raise ValueError("cm21_find_bubbles_batched_workspace_bytes rejected the groups")
@@ -173,7 +181,8 @@ class BatchedBubbles:
                 for k, g in enumerate(self._groups)}
 
     def set_tiles(self, choice):
-        """choice: {key: (columns, lines)}; -1 = default."""
+        """choice: {key: (columns, lines)}; -1 = default, lines -2 - i = tile i with
+        the choice of "planes" left open."""
         for k, g in enumerate(self._groups):
             if g["key"] in choice:
                 c, l = choice[g["key"]]

@@ -32,6 +32,7 @@
 // table per D; cm21_batch_autotune times the candidates on the caller's data
 // and returns the fastest.
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <mutex>
 #include <unordered_map>
@@ -459,8 +460,10 @@ struct BatchShape {
     int ncols;
     LineTile lines[4];
     int nlines;
-    LaunchFn planes;  // rows and lines in one, with the factors of the first tiles, or NULL
-    int planes_from;  // boxes from which on it is the faster way
+    LaunchFn planes;       // rows and lines in one, with the factors of the first tiles, or NULL
+    int planes_from;       // boxes from which on it is the faster way where the expected ionized
+    double planes_limit;   // fraction is at most this, and
+    int planes_always;     // from which on it is whatever the fraction
 };
 
 #define CM21_COL(D1, D2, W) {W, D1, launch_bcols<D1, D2, W>, launch_brows<D1, D2, W>, #D1 "x" #D2 "/W" #W}
@@ -471,18 +474,18 @@ struct BatchShape {
 const BatchShape kBatchShapes[] = {
     {64, {CM21_COL(8, 8, 32), CM21_COL(8, 8, 16), CM21_COL(16, 4, 16)}, 3,
      {CM21_LINE(4, 8, 64), CM21_LINE(8, 4, 32), CM21_LINE(4, 8, 32)}, 3,
-     launch_bplanes<8, 8, 4, 8, 256, 8>, 12},
+     launch_bplanes<8, 8, 4, 8, 256, 8>, 12, 0.75, 16},
     {96, {CM21_COL(8, 12, 32), CM21_COL(8, 12, 16), CM21_COL(16, 6, 16)}, 3,
      {CM21_LINE(4, 12, 64), CM21_LINE(8, 6, 32), CM21_LINE(4, 12, 32), CM21_LINE(6, 8, 32)}, 4,
-     launch_bplanes<8, 12, 4, 12, 384, 5>, 8},
+     launch_bplanes<8, 12, 4, 12, 384, 5>, 8, 0.65, INT_MAX},
     {128, {CM21_COL(8, 16, 32), CM21_COL(16, 8, 16), CM21_COL(8, 16, 16)}, 3,
      {CM21_LINE(8, 8, 32), CM21_LINE(4, 16, 64), CM21_LINE(8, 8, 16), CM21_LINE(16, 4, 16)}, 4,
-     launch_bplanes<8, 16, 8, 8, 512, 4>, 4},
+     launch_bplanes<8, 16, 8, 8, 512, 4>, 4, 1.0, 4},
     {160, {CM21_COL(16, 10, 16), CM21_COL(8, 20, 32), CM21_COL(16, 10, 8)}, 3,
      {CM21_LINE(8, 10, 32), CM21_LINE(4, 20, 64), CM21_LINE(8, 10, 16), CM21_LINE(16, 5, 16)}, 4,
-     launch_bplanes<16, 10, 8, 10, 640, 3>, 12},
-    {256, {CM21_COL(16, 16, 16), CM21_COL(16, 16, 8)}, 2, {CM21_LINE(16, 8, 16), CM21_LINE(8, 16, 32)}, 2, nullptr, 0},
-    {512, {CM21_COL(16, 32, 8)}, 1, {CM21_LINE(16, 16, 8)}, 1, nullptr, 0},
+     launch_bplanes<16, 10, 8, 10, 640, 3>, 12, 0.52, INT_MAX},
+    {256, {CM21_COL(16, 16, 16), CM21_COL(16, 16, 8)}, 2, {CM21_LINE(16, 8, 16), CM21_LINE(8, 16, 32)}, 2, nullptr, 0, 0.0, 0},
+    {512, {CM21_COL(16, 32, 8)}, 1, {CM21_LINE(16, 16, 8)}, 1, nullptr, 0, 0.0, 0},
 };
 
 #undef CM21_COL
@@ -497,16 +500,34 @@ const BatchShape* batch_shape(int D) {
 // The planes are the lines candidate after the tiles, of the sides that have them.
 int lines_candidates(const BatchShape& s) { return s.nlines + (s.planes ? 1 : 0); }
 
-// Whether a group runs as planes: where its lines candidate says so or, without a
-// choice (-1), for linear input, a columns tile of the planes' factors and enough
-// boxes for the longer blocks to fill the chip.  Planes against rows and lines
-// apart: 64^3 0.96 times as fast with 8 boxes, 1.13 with 12, 1.39 with 21; 96^3 0.94 with
-// 6, 1.12 with 8, 1.00 with 21, 1.16 with 24; 128^3 0.92 with 2, 1.10 with 4, 1.05 with 5,
-// 1.26 with 17; 160^3 0.95 with 4, 1.00 with 9, 1.02 with 13.
-bool as_planes(const BatchShape& s, int nbox, int tile_columns, int tile_lines, const cm21_bubble_params* prm) {
+// The lines tile of a group that runs rows and lines apart.
+int lines_tile(int tile_lines) { return tile_lines >= 0 ? tile_lines : (tile_lines == -1 ? 0 : -2 - tile_lines); }
+
+// Whether a group runs as planes: where its lines candidate says so; where the choice is
+// left open (tile_lines < 0), for linear input, enough boxes for the longer blocks to
+// fill the chip and, where the planes lose on boxes that are ionized late, a small
+// enough expected ionized fraction zeta erfc(deltac / sqrt(2 sigma_min^2)) (S at the
+// largest radius counted as 0).  A default columns tile has the planes' factors, so that
+// both ways give the same bits.
+// Rows and lines apart over planes, by that fraction 0.05 / 0.3 / 0.5 / 0.7 / 0.95:
+//   64^3, 8 boxes   1.36 1.17 1.07 0.99 0.92    12  1.46 1.22 1.13 1.01 0.94
+//         16        1.52 1.32 1.21 1.11 1.01    28  2.09 1.77 1.62 1.50 1.38
+//   96^3, 6         1.19 1.02 0.91 0.81 0.70     8  1.55 1.35 1.21 1.06 0.98
+//         12        1.34 1.22 1.08 0.95 0.84    28  1.43 1.27 1.13 1.01 0.90
+//   128^3, 2        1.12 0.96 0.85 0.75 0.74     4  1.62 1.48 1.35 1.19 1.12
+//         6         1.45 1.23 1.10 0.97 0.99    25  1.51 1.37 1.25 1.12 1.02
+//   160^3, 4        1.24 1.14 1.01 0.88 0.76    12  1.24 1.14 1.02 0.89 0.79
+//         18        1.24 1.12 0.99 0.87 0.79    26  1.22 1.11 1.00 0.88 0.79
+bool as_planes(const BatchShape& s, const cm21_batch_group& g, const cm21_bubble_params* prm) {
     if (!s.planes || !prm->linear_input) return false;
-    if (tile_lines >= 0) return tile_lines == s.nlines;
-    return nbox >= s.planes_from && (tile_columns < 0 || s.cols[tile_columns].factor == s.cols[0].factor);
+    if (g.tile_lines >= 0) return g.tile_lines == s.nlines;
+    if (g.nbox < s.planes_from) return false;
+    if (g.tile_lines == -1 && g.tile_columns >= 0 && s.cols[g.tile_columns].factor != s.cols[0].factor) return false;
+    if (g.nbox >= s.planes_always) return true;
+    double ionized = 0.0;
+    for (int b = 0; b < g.nbox; ++b)
+        ionized += std::min(1.0, g.boxes[b].zeta * std::erfc((double)g.boxes[b].deltac / (double)g.denoms[(size_t)b * g.n_radii]));
+    return ionized <= s.planes_limit * g.nbox;
 }
 
 int min_lines_per_block(const BatchShape& s) {
@@ -560,7 +581,7 @@ int build_layout(const cm21_batch_group* groups, int ngroups, const cm21_bubble_
         CM21_REQUIRE(g.radii, "cm21_find_bubbles_batched: group %d: radii is NULL", gi);
         CM21_REQUIRE(g.tile_columns >= -1 && g.tile_columns < h.shape->ncols,
                      "cm21_find_bubbles_batched: group %d: tile_columns=%d out of range", gi, g.tile_columns);
-        CM21_REQUIRE(g.tile_lines >= -1 &&
+        CM21_REQUIRE(g.tile_lines >= -1 - h.shape->nlines &&
                          g.tile_lines < (prm->linear_input ? lines_candidates(*h.shape) : h.shape->nlines),
                      "cm21_find_bubbles_batched: group %d: tile_lines=%d out of range", gi, g.tile_lines);
         if (check_arrays) {
@@ -757,9 +778,9 @@ int prepare(const cm21_batch_group* groups, int ngroups, const cm21_bubble_param
     p.line_tile.clear();
     p.planes.clear();
     for (const auto& h : p.lay.groups) {
-        const bool planes = as_planes(*h.shape, h.nbox, h.g->tile_columns, h.g->tile_lines, prm);
+        const bool planes = as_planes(*h.shape, *h.g, prm);
         const int ct = tile_or_default(h.g->tile_columns);
-        const int lt = planes ? 0 : tile_or_default(h.g->tile_lines);
+        const int lt = planes ? 0 : lines_tile(h.g->tile_lines);
         int cb = 0, rb = 0;
         fill_tables(h, prm, ct, p.blob, &cb, &rb);
         p.launches.push_back(make_launch(h, (char*)work, cb, rb, h.D * h.D / h.shape->lines[lt].L));

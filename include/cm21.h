@@ -304,7 +304,8 @@ typedef struct cm21_batch_group {
     float* ionized;              /* device, nbox boxes */
     cm21_plan* plan;             /* cm21_plan_create(&p, D, nbox) */
     int tile_columns;            /* candidate index, -1 = default */
-    int tile_lines;              /* candidate index, -1 = default */
+    int tile_lines;              /* candidate index, or with the choice of "planes" (below) left open:
+                                    -1 the default tile, -2 - i tile i */
 } cm21_batch_group;
 
 /* params: filter_type, ref_fallthrough, linear_input, update (must be 0) and
@@ -319,8 +320,9 @@ int cm21_find_bubbles_batched(const cm21_batch_group* groups, int ngroups, const
 
 /* Tile candidates per D: stage 0 = columns/rows passes, 1 = lines pass.  The last
  * lines candidate of sides up to 160 is "planes", rows and lines of a plane in one
- * block (linear input only); the other lines candidates run the two apart, and
- * without a choice (tile_lines = -1) the number of boxes decides.
+ * block (linear input only); the other lines candidates run the two apart, and where
+ * the choice is left open (tile_lines < 0) the number of boxes and their expected
+ * ionized fraction decide.
  * cm21_batch_tile_count returns -1 for an unsupported D. */
 int cm21_batch_tile_count(int D, int stage);
 const char* cm21_batch_tile_name(int D, int stage, int index);

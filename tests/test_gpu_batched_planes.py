@@ -2,6 +2,8 @@
 boxes two at a time, which run them apart: the same transforms in the same order,
 so the ionized boxes are equal bit for bit.  Among them a box that stays
 neutral, one that is ionized throughout and one that holds a NaN."""
+import math
+
 import pytest
 import torch
 
@@ -77,6 +79,9 @@ def test_a_choice_of_lines_is_kept(gpu, D, nbox):
     for l in range(n):
         bb.set_tiles({key: (0, l)})
         assert _stage_calls(bb) == ((0, 1) if l == n - 1 else (1, 1)), l
+        if l < n - 1:  # the same tile with the choice left open
+            bb.set_tiles({key: (0, -2 - l)})
+            assert _stage_calls(bb) == ((0, 1) if nbox == 16 else (1, 1)), l
     bb.stream = torch.cuda.Stream()
     res = bb.autotune(reps=2)[key]
     assert res["chosen"][1] == res["names"][-n:][res["lines"]]
@@ -94,3 +99,37 @@ def test_planes_are_for_linear_input(gpu):
     bb.set_tiles({key: (-1, -1)})
     bb.stream = torch.cuda.Stream()
     assert bb.autotune(reps=1)[key]["chosen"][1] != "planes"
+
+
+@pytest.mark.parametrize("D,nbox,late", [(64, 12, True), (64, 16, False), (96, 8, True), (128, 4, False), (160, 12, True)])
+def test_planes_where_boxes_are_ionized_late(gpu, D, nbox, late):
+    """Without a choice: planes for boxes that stay neutral, and for boxes that are
+    ionized late only where the planes do not lose on them."""
+    lib = pkg("_lib")
+    bb = _batch(D, nbox)
+    g = bb._garr[0]
+    for j in range(nbox):
+        # zeta erfc(deltac / denom) of 0.1, then of 0.9 in every box
+        g.boxes[j].zeta = 0.1 / math.erfc(g.boxes[j].deltac / g.denoms[j * g.n_radii])
+    assert _stage_calls(bb)[0] == 0
+    for j in range(nbox):
+        g.boxes[j].zeta *= 9.0
+    assert _stage_calls(bb)[0] == (1 if late else 0)
+    n = lib.load().cm21_batch_tile_count(D, 1)
+    bb.set_tiles({list(bb.tiles())[0]: (-1, -1 - n)})  # past the last tile
+    with pytest.raises(lib.CM21Error):
+        bb.run()
+
+
+@pytest.mark.parametrize("D,nbox", [(64, 3), (96, 2), (128, 2), (160, 3)])
+def test_forced_planes_equal_rows_and_lines(gpu, D, nbox):
+    """Both ways on the same boxes, with tiles of the same factors: equal bit for bit."""
+    bb = _batch(D, nbox)
+    key, = bb.tiles()
+    out = []
+    for l in (0, pkg("_lib").load().cm21_batch_tile_count(D, 1) - 1):
+        bb.set_tiles({key: (0, l)})
+        bb.run()
+        out.append([bb.ionized(i).clone() for i in range(nbox)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b) and 0.01 < float((a == 1).double().mean()) < 0.99
