@@ -245,8 +245,9 @@ __global__ __launch_bounds__(L* N1) void k_batch_lines(BatchLaunch a) {
 // below the threshold: asked while few modes survive and as long as it was of use at
 // the radius before.
 // 21 boxes: 64^3 0.82 -> 0.59 ms, 128^3 4.55 -> 3.69, 160^3 9.29 -> 9.00; the 64 boxes
-// of 96^3 to 160^3 14.99 -> 13.87 ms.  Bound by the VALU and, at 160^3, by the one block
-// of ten waves that fits a CU (halves of a plane per block, the first step along b
+// of 96^3 to 160^3 14.99 -> 13.87 ms.  0.5 to 0.6 of the VALU rate and 0.4 to 0.6 TB/s at 2.3
+// to 3.6 waves per SIMD: few waves between the barriers, at 160^3 the one block of ten
+// that fits a CU (halves of a plane per block, the first step along b
 // done twice: 10.1 ms).  Nonlinear input, whose sum needs the rows a second time, lost
 // (28 ms for 22 on those 64 boxes).
 template <int D1, int D2, int N1, int N2, int NT>

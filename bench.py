@@ -633,9 +633,10 @@ def main():
                      "traffic_frac": (traffic / (dom_ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if traffic else None,
                      "alg_bytes_per_launch": ab[dom], "ms_per_launch": dom_ms,
                      "note": "achieved credits the unpruned algorithm's bytes; the pruned launch moves "
-                             "`traffic` bytes (traffic_frac of peak) and is bound by VALU issue (valu_roofline)"},
-        # what bounds the kernel: VALU issue (counter-measured instructions per
-        # launch over this run's launch time)
+                             "`traffic` bytes (traffic_frac of peak) and is bound by VALU issue where it has box "
+                             "sums (valu_roofline, a mean that includes the launches of radii passed over)"},
+        # what bounds the launches with box sums: VALU issue (counter-measured
+        # instructions per launch over this run's launch time)
         "valu_roofline": ({"achieved": valu / (dom_ms * 1e-3) / 1e9, "peak": VALU_PEAK_G,
                            "unit": "G wave64-instructions/s", "frac": valu / (dom_ms * 1e-3) / 1e9 / VALU_PEAK_G,
                            "valu_per_launch": valu,
