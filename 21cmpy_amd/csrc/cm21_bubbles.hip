@@ -649,11 +649,23 @@ float loop_scale(int D, const cm21_bubble_params* prm) {
 
 float loop_delta_k(const cm21_bubble_params* prm) { return (float)(2.0 * M_PI / (double)prm->box_len); }
 
+// Whether the launch per radius is the faster form for a side that has both: with the
+// Gaussian window at 160^3 the intermediates of every radius (0.8 GB) are past the caches,
+// and on a box that is expected to be all ionized at the largest radius (zeta <f_coll>)
+// its threshold launches end at once, where the all-radii form transforms every line
+// of every radius.  All radii at once, 160^3, BOX_LEN 250, by zeta <f_coll> = 1.0 / 1.1 / 1.2 / 3:
+// linear 838 831 817 809 us against 884 797 662 662, nonlinear 1069 1051 1030 1018 against
+// 1236 1162 889 884.  At 128^3 (463 against 528 at 3) and with the k-space top-hat (326
+// against 318 at 3, 353 against 467 at 1.2) all at once is as fast or faster throughout.
+bool per_radius_is_faster(int D, const cm21_bubble_params* prm) {
+    return D > 128 && prm->filter_type == 2 && prm->zeta * (double)prm->fc_mean > 1.2;
+}
+
 AllWork carve_all(void* base, int D, const float* radii, const float* denoms, int n_radii,
                   const cm21_bubble_params* prm) {
     AllWork w{};
     const FusedShape* sh = fused_shape(D);
-    if (!loop_is_fused(sh, prm)) return w;
+    if (!loop_is_fused(sh, prm) || per_radius_is_faster(D, prm)) return w;
     const size_t nt = all_radii_table(*sh, loop_delta_k(prm), radii, denoms, n_radii, prm->filter_type,
                                       prm->ref_fallthrough, loop_scale(D, prm), &w.a);
     if (nt == 0) return w;

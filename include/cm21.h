@@ -138,8 +138,10 @@ typedef struct cm21_bubble_params {
 size_t cm21_find_bubbles_workspace_bytes(int D, int n_radii, int update);
 /* The workspace with which cm21_find_bubbles is fastest for these radii and
  * parameters: at least the above, and for fused sides up to 160 what the form
- * with every radius in one launch per pass needs.  Any size from the above on
- * is accepted, with the same results bit for bit. */
+ * with every radius in one launch per pass needs, where that is the faster one (not for
+ * filter 2 at side 160 with zeta * fc_mean > 1.2, where the box is expected to be ionized
+ * at the largest radius).  Any size from the above on is accepted, with the same
+ * results bit for bit. */
 size_t cm21_find_bubbles_full_workspace_bytes(int D, const float* radii, int n_radii,
                                               const cm21_bubble_params* params);
 int cm21_find_bubbles(cm21_plan* plan, const float* delta, float* ionized,

@@ -112,3 +112,18 @@ def test_conv_bubbles_without_room_for_every_radius(gpu, graph):
         torch.cuda.set_per_process_memory_fraction(1.0)
         fb._graph_cache.clear()
     assert (want == 1).any() and want.unique().numel() > 1000  # ionized cells and partial values
+
+
+@pytest.mark.parametrize("LE", [True, False])
+def test_gaussian_window_on_a_box_ionized_at_once(gpu, LE):
+    """160^3 with filter 2: a box that is all ionized at the largest radius takes the
+    launch per radius, which ends early there (0.82 times the time); the form with
+    every radius at once asks for its workspace elsewhere, and the boxes are the same."""
+    radii = pkg("Programs.find_HII_bubbles").radius_schedule(250.0, 160)[0]
+    for mean, per_radius in ((1.0, False), (3.0, True)):
+        want, _, _ = _run(160, 250.0, LE, 2, mean, radii, False)
+        got, nbytes, least = _run(160, 250.0, LE, 2, mean, radii, True)
+        assert (nbytes == least) == per_radius and np.array_equal(got, want)
+    assert np.all(want == 1)
+    for D, fil in ((160, 1), (128, 2)):
+        assert _run(D, 250.0, LE, fil, 3.0, radii, True)[1] > _run(D, 250.0, LE, fil, 3.0, radii, False)[1]
