@@ -784,6 +784,10 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
             CM21_TRY(fused_forward(*sh, delta, a.T, a.S, tw, widest, st));
             return fused_all_radii(*sh, a, tw, st);
         }
+        // through the intermediate of the last radius, which the box before left in
+        // the caches (256^3 forward 89 us; 97 to 102 through any other), and ahead of what
+        // the host works out for the schedule
+        CM21_TRY(fused_forward(*sh, delta, w.inter[0], w.spec, tw, widest, st));
         CM21_TRY(fused_mask_clear(w.mask, (N + 63) / 64, st));
         // One launch per radius on the caller's stream, each with up to six
         // independent roles over neighbouring radii (k_fused_radius): launch
@@ -820,10 +824,11 @@ int run_loop(cm21_plan* plan, const float* delta, float* ionized, const float* r
         std::vector<int> inter_of(n_radii);
         for (int r = 0; r < n_radii; ++r)
             inter_of[r] = ahead > 0 && r <= ahead ? r % kInterMax : (r >= 5 ? inter_of[r - 5] : r);
-        auto inter = [&](int r) { return w.inter[inter_of[r]]; };
-        // through the intermediate of the last radius, which the box before left in
-        // the caches (256^3 forward 89 us; 97 to 102 through any other)
-        CM21_TRY(fused_forward(*sh, delta, inter(last), w.spec, tw, widest, st));
+        const int q_last = inter_of[last];  // takes the place of number 0
+        auto inter = [&](int r) {
+            const int q = inter_of[r];
+            return w.inter[q == q_last ? 0 : (q == 0 ? q_last : q)];
+        };
         auto col_launch = [&](int r) { return r - (r < ahead ? 3 : 2); };
         auto row_launch = [&](int r) { return r - (r < ahead ? 2 : 1); };
         // the radius whose pass falls into launch j, or -1
